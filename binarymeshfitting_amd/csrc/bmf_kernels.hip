@@ -388,33 +388,11 @@ __global__ void __launch_bounds__(256) k_csg_cull(Arenas A, int n) {
 // adaptation every
 // sample is evaluated fully (bit-identical values either way).
 // ------------------------------------------------------------------------
-// The terrain terms of the sampler and a chunk's sample geometry as values:
-// read once per tile, so the loops below never reload them after their
-// own stores.
-struct TerrainTerms {
-    float amp, y0, inv_norm;
-};
+// A chunk's sample geometry as values (like TerrainTerms): read once per
+// tile, so the loops below never reload them after their own stores.
 struct ChunkGeom {
     float ox, oy, oz, delta;
 };
-
-__device__ __forceinline__ float density_from_sum(const TerrainTerms& S, float sum, float t2) {
-    float fb = sum * S.inv_norm;
-    fb = fminf(fmaxf(fb, -1.0f), 1.0f);
-    return S.amp * fb - t2;
-}
-
-// 0: undecided, 1: certainly air (d < 0), 2: certainly solid.  The final
-// FP32 sum lies in [sum - reach[k], sum + reach[k]] (see SamplerDev::reach:
-// the interval the remaining fma steps can reach, widened by their rounding
-// and that of the two operations here, so both ends are safe bounds).
-__device__ __forceinline__ int decide_label(const TerrainTerms& S, float reach, float sum, float t2) {
-    const float lo = sum - reach, hi = sum + reach;
-    const float d0 = density_from_sum(S, lo, t2), d1 = density_from_sum(S, hi, t2);
-    if (fmaxf(d0, d1) < 0.0f) return 1;
-    if (!(fminf(d0, d1) < 0.0f)) return 2;
-    return 0;
-}
 
 __device__ __forceinline__ void sample_index(uint32_t i, uint32_t dim, uint32_t dim2, float rd, float rd2, uint32_t& x,
                                              uint32_t& y, uint32_t& z) {

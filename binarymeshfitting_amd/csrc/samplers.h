@@ -150,6 +150,30 @@ __device__ __forceinline__ float terrain_density(const SamplerDev& S, float x, f
     return t1 - t2;
 }
 
+// The terrain's terms as values, and its density from a sum of octaves
+// (terrain_density's own operations).
+struct TerrainTerms {
+    float amp, y0, inv_norm;
+};
+
+__device__ __forceinline__ float density_from_sum(const TerrainTerms& S, float sum, float t2) {
+    float fb = sum * S.inv_norm;
+    fb = fminf(fmaxf(fb, -1.0f), 1.0f);
+    return S.amp * fb - t2;
+}
+
+// 0: undecided, 1: certainly air (d < 0), 2: certainly solid.  The final
+// FP32 sum lies in [sum - reach[k], sum + reach[k]] (see SamplerDev::reach:
+// the interval the remaining fma steps can reach, widened by their rounding
+// and that of the two operations here, so both ends are safe bounds).
+__device__ __forceinline__ int decide_label(const TerrainTerms& S, float reach, float sum, float t2) {
+    const float lo = sum - reach, hi = sum + reach;
+    const float d0 = density_from_sum(S, lo, t2), d1 = density_from_sum(S, hi, t2);
+    if (fmaxf(d0, d1) < 0.0f) return 1;
+    if (!(fminf(d0, d1) < 0.0f)) return 2;
+    return 0;
+}
+
 // ImplicitFunctions (ImplicitSampler.cpp:27-65), positive inside.
 __device__ __forceinline__ float implicit_density(int kind, float res, float x, float y, float z) {
     switch (kind) {

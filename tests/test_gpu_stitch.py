@@ -111,3 +111,41 @@ def test_stitch_errors(ctx):
     assert rc == capi.ECAPACITY and need == n
     rc, _, _ = ctx.stitch(nodes, leaves, 12)  # not a power of two
     assert rc == capi.EINVAL
+
+
+@pytest.mark.parametrize("dim", [128, 256])
+def test_stitch_deep_worlds(ctx, oracle, dim):
+    """A world of 21 levels (the most a morton code holds): with 128 unit
+    nodes per chunk edge the last size of the 32-bit lattice coordinates,
+    with 256 the first of the 64-bit ones; a few of its chunks, bit-exact
+    with the oracle."""
+    nodes, leaves = _world(64.0, (0.01, 0.0, 0.0), 21)
+    assert int(nodes["level"].max()) == 21
+    level, ground = nodes["level"][leaves], nodes["pos"][leaves][:, 1] == 0.0
+    leaves = np.concatenate([leaves[(level == 2) & ground][:1], leaves[level == 21][:1]]).astype(np.int32)
+    sd = {**wl.terrain_sampler(), "y0": 0.0, "amp": 8.0, "freq": 0.05}
+    ctx.set_sampler(**sd)
+    rc, tris, n = ctx.stitch(nodes, leaves, dim, cap_triangles=1 << 18)
+    capi.check(rc, "bmf_stitch")
+    ref = oracle.stitch_points(oracle.SamplerSpec(**sd), nodes, leaves, dim, cap=1 << 18)
+    assert n == len(ref) and n > 0
+    assert np.array_equal(tris, ref)
+
+
+def test_stitch_leaf_lists_off_the_tree(ctx, oracle):
+    """Leaf list entries that a descent does not end in (an inner node, an
+    index out of range, a leaf given twice) keep their meaning."""
+    W, focus, maxl, dim = WORLDS[1]
+    nodes, leaves = _world(W, focus, maxl)
+    inner = int(np.flatnonzero(nodes["world_leaf"] == 0)[-1])
+    odd = np.concatenate([leaves[:5], [inner, leaves[2], len(nodes) + 3, -1], leaves[5:]]).astype(np.int32)
+    ctx.set_sampler(kind=capi.SAMPLER_SPHERE, world_size=2 * W)
+    rc, tris, n = ctx.stitch(nodes, odd, dim)
+    capi.check(rc, "bmf_stitch")
+    rc, plain, n0 = ctx.stitch(nodes, leaves, dim)
+    capi.check(rc, "bmf_stitch")
+    rc, twice, n2 = ctx.stitch(nodes, np.array([leaves[2]], np.int32), dim)
+    capi.check(rc, "bmf_stitch")
+    assert n == n0 + n2
+    rows = lambda a: sorted(map(tuple, a.reshape(len(a), 9).tolist()))  # noqa: E731
+    assert rows(tris) == rows(np.concatenate([plain, twice]))
