@@ -86,25 +86,11 @@ __device__ __forceinline__ ChunkMeta plan_record(const Arenas& A, const SamplerD
     m.iters = d.iters;
     m.bp = d.boundary_processing;
     m.state = kStateSampled;
-    if (allow_cull && S->kind == BMF_SAMPLER_TERRAIN) {
-        // |fbm| <= 1 exactly, so |amp*fbm| <= |amp|; sample y is monotone in j.
-        const float a = fabsf(S->amp);
+    if (allow_cull) {
         const float ylo = m.opos[1];
         const float yhi = (float)(d.dim - 1) * m.delta + m.opos[1];
-        if (ylo - S->y0 > a) m.state = kStateAir;
-        else if (yhi - S->y0 < -a) m.state = kStateSolid;
-    } else if (allow_cull && S->kind == BMF_SAMPLER_NOISE && S->cull) {
-        // d = (-dy) - n h with dy = (y g) ym monotone in y and n in
-        // [nlo, nhi]: every FP32 step is monotone, so the extremes of d
-        // over the chunk come from the end values
-        const float ylo = m.opos[1];
-        const float yhi = (float)(d.dim - 1) * m.delta + m.opos[1];
-        const float dy0 = (ylo * S->g_scale) * S->y_scale, dy1 = (yhi * S->g_scale) * S->y_scale;
-        const float p0 = S->nlo * S->height, p1 = S->nhi * S->height;
-        const float dmax = (-fminf(dy0, dy1)) - fminf(p0, p1);
-        const float dmin = (-fmaxf(dy0, dy1)) - fmaxf(p0, p1);
-        if (dmax < 0.0f) m.state = kStateAir;
-        else if (dmin >= 0.0f) m.state = kStateSolid;
+        const int sign = band_sign(*S, ylo, yhi);
+        if (sign) m.state = sign == 1 ? kStateAir : kStateSolid;
     }
     m.csg_ns = m.csg_nb = 0;  // k_csg_cull fills them
     const int64_t ns = (int64_t)d.dim * d.dim * d.dim;

@@ -62,6 +62,7 @@ struct World {
     int dim;             // unit nodes per chunk edge (a power of two)
     int log_dim;
     const int* root_level;  // device: the root's index (-1: none) and the deepest level L
+    const float* max_size;  // device: the largest size of a leaf (0: none)
 };
 
 // Integer coordinates (twice the lattice's, so that octant points are whole)
@@ -245,8 +246,9 @@ constexpr int kTileLeaves = (kStitchThreads - 1) / 26 + 2;
 // last found, so that a face point descends once); the candidates this chunk
 // stitches, about half, are compacted, and 8 lanes each take their corners'
 // signs.  Bound by the samplers' instructions within the terrain band and by
-// the descents' load latency elsewhere.  (288 chunks of 32^3 unit nodes,
-// 1.77 M candidates, 5 octaves.)
+// the descents' load latency next to it; candidates off the band descend not
+// at all.  288 chunks of 32^3 unit nodes, 1.77 M candidates, 5-octave terrain:
+// 96 us (8 descents and 8 full samplers in each candidate's lane: about 620).
 template <typename I>
 __device__ __forceinline__ void count_tile(const World& W, int L, int root, const SamplerDev& S,
                                            const int32_t* __restrict__ leaves, uint32_t per_leaf, int64_t cand0,
@@ -270,6 +272,16 @@ __device__ __forceinline__ void count_tile(const World& W, int L, int root, cons
         take = lf.b.id >= 0;
         if (take) {
             candidate_point<I>(W, lf.b, g - q * per_leaf, P2);
+            // a corner lies within one unit node (of the coarsest chunk) of
+            // its point, here with as much again for rounding: off the
+            // sampler's band all corners have one sign
+            const bmf_world_node& lq = W.nodes[lf.b.id];
+            const float part = (float)((P2[1] >> 1) - lf.b.o[1]) / (float)lf.b.e;
+            const float y = lq.pos[1] + part * lq.size;
+            const float reach = 2.0f * *W.max_size / (float)W.dim + 1e-5f * (fabsf(lq.pos[1]) + lq.size);
+            take = band_sign(S, y - reach, y + reach) == 0;
+        }
+        if (take) {
             Box<I> last = lf.b;
             if (!lf.own) last.id = -1;
             bool same = true;
@@ -384,7 +396,9 @@ __global__ void __launch_bounds__(kScanThreads) k_stitch_scan(int64_t* __restric
 // Triangles: a block takes kEmitTiles tiles, compacts their candidates with
 // triangles (a few in a hundred) and gives each 8 lanes: a corner's chunk,
 // position and density per lane, then the crossings, then the vertices.
-constexpr int kEmitTiles = 8;
+// Bound by the chain of a round (descent, octaves, two exchanges), so a block
+// has few rounds: 30 us with 2 tiles for the world above, 45 with 8.
+constexpr int kEmitTiles = 2;
 constexpr int kEmitCands = kEmitTiles * kStitchThreads;
 constexpr int kEmitRound = kStitchThreads / 8;  // candidates per round
 
@@ -413,17 +427,20 @@ __global__ void __launch_bounds__(kStitchThreads) k_stitch_emit(World W, const S
     __shared__ uint32_t s_wt[kStitchThreads / 64], s_wn[kStitchThreads / 64];
     __shared__ float4 s_corner[kEmitRound][8];
     __shared__ float s_cross[kEmitRound][12][3];
-    static_assert(kEmitCands == 1 << 11, "list entry layout");
+    static_assert(kEmitCands <= 1 << 11, "list entry layout");
+    constexpr int kPer = kEmitCands / kStitchThreads;  // consecutive candidates per thread
     if (total[0] > cap) return;  // reported by the host: nothing is written
     const int root = uniform_int(W.root_level[0]), L = uniform_int(W.root_level[1]);
     const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
     const int64_t cand0 = (int64_t)blockIdx.x * kEmitCands;
-    // 8 consecutive candidates per thread (the counts are padded to whole blocks)
-    const uint64_t cn = *reinterpret_cast<const uint64_t*>(counts + cand0 + 8 * tid);
+    // the counts are padded to whole blocks
+    uint8_t cn[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; k++) cn[k] = counts[cand0 + kPer * tid + k];
     uint32_t nt = 0, nn = 0;
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
-        const uint32_t v = cand0 + 8 * tid + k < n_cand ? (uint32_t)(cn >> (8 * k)) & 255u : 0u;
+    for (int k = 0; k < kPer; k++) {
+        const uint32_t v = cand0 + kPer * tid + k < n_cand ? cn[k] : 0u;
         nt += v;
         nn += v != 0u;
     }
@@ -451,10 +468,10 @@ __global__ void __launch_bounds__(kStitchThreads) k_stitch_emit(World W, const S
     }
     if (ns == 0) return;
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
-        const uint32_t v = cand0 + 8 * tid + k < n_cand ? (uint32_t)(cn >> (8 * k)) & 255u : 0u;
+    for (int k = 0; k < kPer; k++) {
+        const uint32_t v = cand0 + kPer * tid + k < n_cand ? cn[k] : 0u;
         if (v) {
-            s_list[on++] = (uint32_t)(8 * tid + k) | (ot << 11);
+            s_list[on++] = (uint32_t)(kPer * tid + k) | (ot << 11);
             ot += v;
         }
     }
@@ -467,7 +484,7 @@ __global__ void __launch_bounds__(kStitchThreads) k_stitch_emit(World W, const S
         const uint32_t item = r < ns ? s_list[r] : 0u;
         if (r < ns) {
             float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            const int64_t cand = cand0 + (item & (kEmitCands - 1));
+            const int64_t cand = cand0 + (item & 2047u);
             if (narrow) emit_corner<int32_t>(W, L, root, *S, leaves, per_leaf, cand, c, v);
             else emit_corner<int64_t>(W, L, root, *S, leaves, per_leaf, cand, c, v);
             s_corner[q][c] = v;
@@ -503,22 +520,27 @@ __global__ void __launch_bounds__(kStitchThreads) k_stitch_emit(World W, const S
     }
 }
 
-__global__ void k_stitch_world(const bmf_world_node* __restrict__ nodes, int n_nodes, int* __restrict__ out) {
+__global__ void k_stitch_world(const bmf_world_node* __restrict__ nodes, int n_nodes, int* __restrict__ out,
+                               float* __restrict__ max_size) {
     // out[0]: the first node without a parent, out[1]: the deepest level
-    __shared__ int s_root, s_level;
+    __shared__ int s_root, s_level, s_size;
     if (threadIdx.x == 0) {
         s_root = 0x7FFFFFFF;
         s_level = 0;
+        s_size = 0;
     }
     __syncthreads();
     for (int i = threadIdx.x; i < n_nodes; i += blockDim.x) {
         if (nodes[i].parent < 0) atomicMin(&s_root, i);
         atomicMax(&s_level, nodes[i].level);
+        // sizes are positive: their bits order as they do
+        if (nodes[i].world_leaf && nodes[i].size > 0.0f) atomicMax(&s_size, __float_as_int(nodes[i].size));
     }
     __syncthreads();
     if (threadIdx.x == 0) {
         out[0] = s_root == 0x7FFFFFFF ? -1 : s_root;
         out[1] = s_level;
+        *max_size = __int_as_float(s_size);
     }
 }
 
@@ -543,7 +565,7 @@ int bmf_stitch(bmf_ctx* c, const bmf_world_node* nodes, int32_t n_nodes, const i
     const int64_t n_cand = per_leaf * n_leaves;
     const int64_t n_tiles = (n_cand + kStitchThreads - 1) / kStitchThreads;
     if (n_tiles > 0x7FFFFFFF) return BMF_EINVAL;
-    // whole blocks of the emit kernel: it reads 8 counts per thread
+    // whole blocks of the emit kernel
     const int64_t n_room = (n_cand + kEmitCands - 1) / kEmitCands * kEmitCands;
     if (n_cand > c->stitch_cap_cand) {
         if (c->d_stitch_counts) (void)hipFree(c->d_stitch_counts);
@@ -555,17 +577,18 @@ int bmf_stitch(bmf_ctx* c, const bmf_world_node* nodes, int32_t n_nodes, const i
         BMF_HIP(hipMalloc((void**)&c->d_stitch_tiles, sizeof(int64_t) * (size_t)std::max<int64_t>(n_tiles, 1)));
         c->stitch_cap_cand = n_cand;
     }
-    if (!c->d_stitch_misc) BMF_HIP(hipMalloc((void**)&c->d_stitch_misc, sizeof(int64_t) * 2));
+    if (!c->d_stitch_misc) BMF_HIP(hipMalloc((void**)&c->d_stitch_misc, sizeof(int64_t) * 3));
     if (!c->h_stitch_total) BMF_HIP(hipHostMalloc((void**)&c->h_stitch_total, sizeof(int64_t) * 2, hipHostMallocDefault));
     // the world's root and deepest level, and the triangle total: the kernels
     // read the first two on the device, the host all three at the end
     int* dw = reinterpret_cast<int*>(c->d_stitch_misc);
     int64_t* total = c->d_stitch_misc + 1;
-    hipLaunchKernelGGL(k_stitch_world, dim3(1), dim3(1024), 0, s, nodes, n_nodes, dw);
+    float* max_size = reinterpret_cast<float*>(c->d_stitch_misc + 2);
+    hipLaunchKernelGGL(k_stitch_world, dim3(1), dim3(1024), 0, s, nodes, n_nodes, dw, max_size);
     if (n_cand > 0) {
         int log_dim = 0;
         while ((1 << log_dim) < dim) log_dim++;
-        const World W{nodes, n_nodes, dim, log_dim, dw};
+        const World W{nodes, n_nodes, dim, log_dim, dw, max_size};
         hipLaunchKernelGGL(k_stitch_count, dim3((unsigned)n_tiles), dim3(kStitchThreads), 0, s, W, c->A.sampler, leaves,
                            (uint32_t)per_leaf, n_cand, c->d_stitch_counts, c->d_stitch_tiles);
         hipLaunchKernelGGL(k_stitch_scan, dim3(1), dim3(kScanThreads), 0, s, c->d_stitch_tiles, n_tiles, total);

@@ -174,6 +174,27 @@ __device__ __forceinline__ int decide_label(const TerrainTerms& S, float reach, 
     return 0;
 }
 
+// The sign of the density at every point with y in [ylo, yhi], where the
+// sampler's range alone fixes it: 1 air (d < 0), 2 solid, 0 open.
+__device__ __forceinline__ int band_sign(const SamplerDev& S, float ylo, float yhi) {
+    if (S.kind == BMF_SAMPLER_TERRAIN) {
+        // |fbm| <= 1 exactly, so |amp*fbm| <= |amp|; sample y is monotone in j.
+        const float a = fabsf(S.amp);
+        return ylo - S.y0 > a ? 1 : (yhi - S.y0 < -a ? 2 : 0);
+    }
+    if (S.kind == BMF_SAMPLER_NOISE && S.cull) {
+        // d = (-dy) - n h with dy = (y g) ym monotone in y and n in
+        // [nlo, nhi]: every FP32 step is monotone, so the extremes of d
+        // come from the end values
+        const float dy0 = (ylo * S.g_scale) * S.y_scale, dy1 = (yhi * S.g_scale) * S.y_scale;
+        const float p0 = S.nlo * S.height, p1 = S.nhi * S.height;
+        const float dmax = (-fminf(dy0, dy1)) - fminf(p0, p1);
+        const float dmin = (-fmaxf(dy0, dy1)) - fmaxf(p0, p1);
+        return dmax < 0.0f ? 1 : (dmin >= 0.0f ? 2 : 0);
+    }
+    return 0;
+}
+
 // ImplicitFunctions (ImplicitSampler.cpp:27-65), positive inside.
 __device__ __forceinline__ float implicit_density(int kind, float res, float x, float y, float z) {
     switch (kind) {
