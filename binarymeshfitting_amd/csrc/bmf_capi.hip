@@ -35,9 +35,9 @@ hipError_t dalloc(T** p, int64_t count) {
 
 void free_arenas(bmf_ctx* c) {
     Arenas& A = c->A;
-    void* ptrs[] = {A.meta,    A.descs,     A.results,  A.tile_prefix, A.plan_part, A.plan_tmp, A.stat_blocks, A.plane_map, A.smooth_list, A.smooth_prefix,
-                    A.smooth_tprefix, A.smooth_xcd_v, A.smooth_xcd_t, A.smooth_vmap, A.smooth_tmap, A.refine, A.plane_refine_n, A.cen4,
-                    A.dens,    A.labels,    A.exact,    A.row_v,       A.row_t,        A.cell_tb,   A.cell_mask,
+    void* ptrs[] = {A.meta,    A.descs,     A.results,  A.tile_prefix, A.plan_part, A.plan_tmp, A.stat_blocks, A.item_map, A.smooth_list, A.smooth_prefix,
+                    A.smooth_tprefix, A.smooth_xcd_v, A.smooth_xcd_t, A.smooth_vmap, A.smooth_tmap, A.edges, A.word_pre, A.item_e, A.item_c, A.cen4,
+                    A.dens,    A.labels,    A.exact, A.cell_tb,   A.cell_mask,
                     A.pos,     A.pos4,      A.boundary, A.vedge,       A.vring,        A.idx,          A.ctr,
                     A.sampler, c->d_spheres, c->d_boxes, A.ring, A.ring_n, A.qef_err, A.nrm4, A.fn4, A.nrm,
                     A.csg_list};
@@ -55,8 +55,8 @@ void free_arenas(bmf_ctx* c) {
 // 1024 threads per chunk.
 int scan_blocks(const bmf_ctx* c, int n) { return std::min(n, 2 * c->cu_count); }
 
-int enqueue_pipeline(bmf_ctx* c, const Arenas& A, int n, int maxk, int wclasses, int allow_cull, int reset,
-                     int sample_blocks, int row_blocks, int scan_blocks, int smooth_blocks, hipEvent_t* ev = nullptr) {
+int enqueue_pipeline(bmf_ctx* c, const Arenas& A, int n, int maxk, int allow_cull, int reset, int sample_blocks,
+                     int row_blocks, int scan_blocks, int smooth_blocks, hipEvent_t* ev = nullptr) {
     hipStream_t s = c->stream;
 #define BMF_MARK(i) \
     if (ev) BMF_HIP(hipEventRecord(ev[i], s))
@@ -68,16 +68,12 @@ int enqueue_pipeline(bmf_ctx* c, const Arenas& A, int n, int maxk, int wclasses,
     c->stat_nrefine = row_blocks;
     BMF_MARK(2);
     const bool quads = A.mesh_mode == BMF_MESH_QUADS;
-    // the row-word classes of a mixed batch one after another on the one
-    // stream: a context is one stream (one hardware queue), so several
-    // contexts on a GPU overlap their batches
-    BMF_HIP(launch_count(A, n, row_blocks, wclasses, s));
-    BMF_HIP(launch_refine(A, n, row_blocks, s));
+    BMF_HIP(launch_count(A, row_blocks, c->h_sampler.kind == BMF_SAMPLER_TERRAIN, s));
     BMF_MARK(3);
     BMF_HIP(launch_scan(A, n, scan_blocks, s));
     BMF_MARK(4);
-    if (quads) BMF_HIP(launch_dmc_emit(A, n, row_blocks, wclasses, s));
-    else BMF_HIP(launch_emit(A, n, row_blocks, wclasses, s));
+    if (quads) BMF_HIP(launch_dmc_emit(A, row_blocks, s));
+    else BMF_HIP(launch_emit(A, row_blocks, s));
     BMF_MARK(5);
     for (int m = 0; m < maxk; m++) {
         if (quads) BMF_HIP(launch_dmc_smooth(A, m, smooth_blocks, s));
@@ -279,9 +275,9 @@ int bmf_create(bmf_ctx** out, int device, const bmf_limits* lim) {
     c->persistent_blocks = c->cu_count * 8;
     c->tune.sample_tile = kSampleTileDefault;
     c->tune.sample_blocks = c->persistent_blocks;
-    // ten per CU: the best of 4..20 per CU for count + emit on a batch of
-    // 512 64^3-cell chunks (fewer leave workgroups with a third plane item,
-    // more only add empty workgroups); the autotuner tries the others
+    // ten per CU: the best of 4..64 per CU for count + emit on a batch of
+    // 512 64^3-cell chunks (89 us; 97 at 8, 94 at 16 and more) and on 64
+    // chunks of CSG quads (150, 168, 155); the autotuner tries the others
     c->tune.row_blocks = c->cu_count * 10;
     c->tune.smooth_blocks = 4 * c->persistent_blocks;
     c->tune.row_split = -1;
@@ -289,29 +285,28 @@ int bmf_create(bmf_ctx** out, int device, const bmf_limits* lim) {
     const int64_t nc = lim->max_chunks;
     A.cap_chunks = (int32_t)nc;
     A.cap_samples = lim->max_samples;
-    A.cap_rows = lim->max_samples / 2 + nc;
+    const int64_t nw = lim->max_samples / 64 + nc, ni = nw / kItemWords + nc;  // label words, word items
     A.cap_vertices = lim->max_vertices;
     A.cap_indices = lim->max_indices;
     A.sample_tile = kSampleTileDefault;
     A.smoothing_follows = 1;
     A.stat_cap = 64 * c->cu_count;
-    A.row_split = -1;
     bool ok = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) == hipSuccess;
     ok = ok && dalloc(&A.meta, nc) == hipSuccess && dalloc(&A.descs, nc) == hipSuccess &&
          dalloc(&A.results, nc) == hipSuccess && dalloc(&A.tile_prefix, nc + 1) == hipSuccess &&
          dalloc(&A.plan_part, 40 * ((nc + 1023) / 1024) + 64) == hipSuccess &&
          dalloc(&A.plan_tmp, 2 * nc) == hipSuccess &&
          dalloc(&A.stat_blocks, 2 * (int64_t)(64 * c->cu_count)) == hipSuccess &&
-         dalloc(&A.plane_map, nc * BMF_MAX_DIM) == hipSuccess && dalloc(&A.smooth_list, nc) == hipSuccess &&
+         dalloc(&A.item_map, ni) == hipSuccess && dalloc(&A.smooth_list, nc) == hipSuccess &&
          dalloc(&A.smooth_prefix, nc + 1) == hipSuccess && dalloc(&A.smooth_tprefix, nc + 1) == hipSuccess &&
          dalloc(&A.smooth_xcd_v, kXcds + 1) == hipSuccess && dalloc(&A.smooth_xcd_t, kXcds + 1) == hipSuccess &&
          dalloc(&A.smooth_vmap, A.cap_vertices / kSmoothThreads + nc + 1) == hipSuccess &&
          dalloc(&A.smooth_tmap, A.cap_indices / 3 / kSmoothThreads + nc + 1) == hipSuccess &&
-         dalloc(&A.refine, A.cap_samples) == hipSuccess && dalloc(&A.plane_refine_n, nc * BMF_MAX_DIM * kMaxPlaneSplit) == hipSuccess &&
+         dalloc(&A.edges, nw) == hipSuccess && dalloc(&A.word_pre, nw) == hipSuccess &&
+         dalloc(&A.item_e, ni) == hipSuccess && dalloc(&A.item_c, ni) == hipSuccess &&
          dalloc(&A.cen4, A.cap_indices / 3 + 1) == hipSuccess &&
-         dalloc(&A.dens, A.cap_samples) == hipSuccess && dalloc(&A.labels, A.cap_samples / 64 + nc) == hipSuccess &&
-         dalloc(&A.exact, A.cap_samples / 64 + nc) == hipSuccess &&
-         dalloc(&A.row_v, A.cap_rows) == hipSuccess && dalloc(&A.row_t, A.cap_rows) == hipSuccess &&
+         dalloc(&A.dens, A.cap_samples) == hipSuccess && dalloc(&A.labels, nw) == hipSuccess &&
+         dalloc(&A.exact, nw) == hipSuccess &&
          dalloc(&A.cell_tb, A.cap_samples) == hipSuccess && dalloc(&A.cell_mask, A.cap_samples) == hipSuccess &&
          dalloc(&A.pos, 3 * A.cap_vertices) == hipSuccess && dalloc(&A.pos4, A.cap_vertices) == hipSuccess &&
          dalloc(&A.boundary, A.cap_vertices) == hipSuccess && dalloc(&A.vedge, A.cap_vertices) == hipSuccess &&
@@ -520,8 +515,7 @@ static int extract_impl(bmf_ctx* c, const bmf_chunk_desc* chunks, int n, int mod
         if (rc) return rc;
     }
     auto desc = [&](int j) -> const bmf_chunk_desc& { return chunks ? chunks[j] : *uni; };
-    int maxk = chunks ? max_steps(c, chunks, n) : max_steps(c, uni, 1), wclasses = 0;
-    for (int i = 0; i < (chunks ? n : 1); i++) wclasses |= row_word_class(desc(i).dim);
+    const int maxk = chunks ? max_steps(c, chunks, n) : max_steps(c, uni, 1);
     const Arenas& A = c->A;
     const int pb = c->persistent_blocks;
     if (mode == BMF_MODE_PLAIN) {
@@ -541,8 +535,7 @@ static int extract_impl(bmf_ctx* c, const bmf_chunk_desc* chunks, int n, int mod
             const int64_t dim = dj.dim;
             const int64_t ns = dim * dim * dim;
             const int sb = (int)std::min<int64_t>(ceil_div(ns, A.sample_tile), pb);
-            rc = enqueue_pipeline(c, Aj, 1, max_steps(c, &dj, 1), row_word_class(dj.dim), 1, j == 0, sb,
-                                  (int)dim * kMaxPlaneSplit, 1,
+            rc = enqueue_pipeline(c, Aj, 1, max_steps(c, &dj, 1), 1, j == 0, sb, word_blocks(dj.dim), 1,
                                   std::min(pb, 1024));
             if (rc) return rc;
         }
@@ -553,11 +546,11 @@ static int extract_impl(bmf_ctx* c, const bmf_chunk_desc* chunks, int n, int mod
     // (n, max iterations) in a hipGraph and replayed.
     GraphEntry* ge = nullptr;
     for (auto& g : c->graphs)
-        if (g.n == n && g.maxk == maxk && g.wclasses == wclasses) ge = &g;
+        if (g.n == n && g.maxk == maxk) ge = &g;
     if (!ge) {
         hipGraph_t graph = nullptr;
         BMF_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-        rc = enqueue_pipeline(c, A, n, maxk, wclasses, 1, 1, c->tune.sample_blocks, c->tune.row_blocks,
+        rc = enqueue_pipeline(c, A, n, maxk, 1, 1, c->tune.sample_blocks, c->tune.row_blocks,
                               scan_blocks(c, n), c->tune.smooth_blocks);
         hipGraph_t captured = nullptr;
         hipError_t e = hipStreamEndCapture(c->stream, &captured);
@@ -570,7 +563,6 @@ static int extract_impl(bmf_ctx* c, const bmf_chunk_desc* chunks, int n, int mod
         GraphEntry g;
         g.n = n;
         g.maxk = maxk;
-        g.wclasses = wclasses;
         e = hipGraphInstantiate(&g.exec, graph, nullptr, nullptr, 0);
         (void)hipGraphDestroy(graph);
         if (e != hipSuccess) return BMF_EHIP;
@@ -697,7 +689,7 @@ static int stage_one(bmf_ctx* c, const bmf_chunk_desc* d, bool scan) {
     BMF_HIP(launch_sample(A, 1, (int)std::min<int64_t>(ceil_div(ns, A.sample_tile), c->persistent_blocks), 0,
                           c->h_sampler.kind, c->h_sampler.noise_dims == 2, c->stream));
     if (scan) {
-        BMF_HIP(launch_count(A, 1, d->dim, row_word_class(d->dim), c->stream));
+        BMF_HIP(launch_count(A, word_blocks(d->dim), 0, c->stream));
         BMF_HIP(launch_scan(A, 1, 1, c->stream));
     }
     return BMF_OK;
@@ -790,10 +782,9 @@ int bmf_profile_stages(bmf_ctx* c, const bmf_chunk_desc* chunks, int n, float* s
     c->have_extract = true;
     rc = upload_descs(c, chunks, n);
     if (rc) return rc;
-    int maxk = max_steps(c, chunks, n), wclasses = 0;
-    for (int i = 0; i < n; i++) wclasses |= row_word_class(chunks[i].dim);
+    const int maxk = max_steps(c, chunks, n);
     BMF_HIP(hipEventRecord(c->ev0, c->stream));
-    rc = enqueue_pipeline(c, c->A, n, maxk, wclasses, 1, 1, c->tune.sample_blocks, c->tune.row_blocks,
+    rc = enqueue_pipeline(c, c->A, n, maxk, 1, 1, c->tune.sample_blocks, c->tune.row_blocks,
                           scan_blocks(c, n), c->tune.smooth_blocks, c->ev_stage);
     if (rc) return rc;
     c->stats_batch = true;
@@ -919,7 +910,6 @@ int bmf_set_tuning(bmf_ctx* c, const bmf_tuning* t) {
     BMF_HIP(hipStreamSynchronize(c->stream));
     c->tune = n;
     c->A.sample_tile = n.sample_tile;
-    c->A.row_split = n.row_split;
     drop_graphs(c);
     return BMF_OK;
 }
@@ -935,18 +925,16 @@ int bmf_autotune(bmf_ctx* c, const bmf_chunk_desc* chunks, int n, int reps, bmf_
     c->have_extract = false;
     rc = upload_descs(c, chunks, n);
     if (rc) return rc;
-    int maxk = max_steps(c, chunks, n), wclasses = 0;
-    for (int i = 0; i < n; i++) wclasses |= row_word_class(chunks[i].dim);
+    const int maxk = max_steps(c, chunks, n);
     // stage times (ms, the median of reps runs: a candidate with one lucky
     // run does not win) of the pipeline under tuning t
     float st[BMF_NUM_STAGES];
     auto run_n = [&](const bmf_tuning& t, int nrep, float* out) -> int {
         Arenas A = c->A;
         A.sample_tile = t.sample_tile;
-        A.row_split = t.row_split;
         std::vector<float> ms(static_cast<size_t>(nrep) * BMF_NUM_STAGES);
         for (int r = 0; r < nrep; r++) {
-            int e = enqueue_pipeline(c, A, n, maxk, wclasses, 1, 1, t.sample_blocks, t.row_blocks,
+            int e = enqueue_pipeline(c, A, n, maxk, 1, 1, t.sample_blocks, t.row_blocks,
                                      scan_blocks(c, n), t.smooth_blocks, c->ev_stage);
             if (e) return e;
             BMF_HIP(hipStreamSynchronize(c->stream));
@@ -985,27 +973,22 @@ int bmf_autotune(bmf_ctx* c, const bmf_chunk_desc* chunks, int n, int reps, bmf_
         cur.sample_tile = b.sample_tile;
         cur.sample_blocks = b.sample_blocks;
     }
-    // plane kernels: count (+ refine) and emit (stages 2 and 4), workgroups x row segments
+    // word kernels: count and emit (stages 2 and 4), workgroups
     {
         float bt = 1e30f;
-        int bb = cur.row_blocks, bs = cur.row_split;
+        int bb = cur.row_blocks;
         const int mult[7] = {1, 2, 4, 8, 10, 12, 16};
-        const int splits[5] = {-1, 1, 2, 4, 8};  // -1: per row-word class from its plane count
-        for (int sp : splits)
-            for (int m : mult) {
-                bmf_tuning t = cur;
-                t.row_blocks = m * cu;
-                t.row_split = sp;
-                rc = run(t, st);
-                if (rc) return rc;
-                if (st[2] + st[4] < bt) {
-                    bt = st[2] + st[4];
-                    bb = t.row_blocks;
-                    bs = t.row_split;
-                }
+        for (int m : mult) {
+            bmf_tuning t = cur;
+            t.row_blocks = m * cu;
+            rc = run(t, st);
+            if (rc) return rc;
+            if (st[2] + st[4] < bt) {
+                bt = st[2] + st[4];
+                bb = t.row_blocks;
             }
+        }
         cur.row_blocks = bb;
-        cur.row_split = bs;
     }
     // smoothing (stage 5)
     if (maxk > 0) {

@@ -13,7 +13,6 @@ namespace bmf {
 struct GraphEntry {
     int n = -1;
     int maxk = -1;
-    int wclasses = 0;
     hipGraphExec_t exec = nullptr;
 };
 

@@ -1154,7 +1154,6 @@ int bmf_forward_diff(bmf_ctx* c, const bmf_chunk_desc* d, const float* densities
     A.quad_tris = 0;
     A.smoothing_follows = 0;  // the tape smooths its own copy: every output position is written by emit
     A.normals = 0;
-    const int wcls = row_word_class(dim);
     // extraction with every octave evaluated (densities exact everywhere),
     // no smoothing: the tape smooths its own copy
     hipError_t e = launch_plan(A, 1, 0, 1, s);
@@ -1162,10 +1161,9 @@ int bmf_forward_diff(bmf_ctx* c, const bmf_chunk_desc* d, const float* densities
         e = launch_sample(A, 1, (int)std::min<int64_t>((n3 + A.sample_tile - 1) / A.sample_tile, c->persistent_blocks),
                           0, densities ? (int)BMF_SAMPLER_EXTERNAL : (int)c->h_sampler.kind,
                           !densities && c->h_sampler.noise_dims == 2, s);
-    if (e == hipSuccess) e = launch_count(A, 1, dim * kMaxPlaneSplit, wcls, s);
-    if (e == hipSuccess) e = launch_refine(A, 1, dim * kMaxPlaneSplit, s);
+    if (e == hipSuccess) e = launch_count(A, word_blocks(dim), 0, s);
     if (e == hipSuccess) e = launch_scan(A, 1, 1, s);
-    if (e == hipSuccess) e = launch_emit(A, 1, dim * kMaxPlaneSplit, wcls, s);
+    if (e == hipSuccess) e = launch_emit(A, word_blocks(dim), s);
     if (e == hipSuccess) e = hipMemcpyAsync(c->h_results, A.results, sizeof(bmf_chunk_result), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipMemcpyAsync(c->h_ctr, A.ctr, sizeof(Counters), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);

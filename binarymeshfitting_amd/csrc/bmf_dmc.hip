@@ -4,23 +4,23 @@
 // sign-changing edges, and MeshProcessor<4>/<3> smoothing over per-vertex
 // rings.
 //
-// Per batch (after sample, count and refine, which in this mode count per
-// label row the polygons of the row's cells and the quads of the row's
-// interior sign-changing edges, and leave every edge endpoint's density
-// exact):
-//   (k_scan)       row bases, arena offsets
-//   k_dmc_vertices per row: vertex positions; per surface cell its first
-//                  vertex id and mask (cell_tb / cell_mask arenas); for the
-//                  chunks that smooth, each vertex's ring (the primitives
-//                  around it in ascending id, the reference's order), from
-//                  the quad ids of its polygon's edges
-//   k_dmc_quads    per row: quad (or two-triangle) indices
+// Per batch (after sample and count, which in this mode count per item the
+// polygons of its cells and the quads of its interior sign-changing edges, and
+// leave every edge endpoint's density exact):
+//   (k_scan)       item bases, arena offsets
+//   k_dmc_vertices vertex positions; per surface cell its first vertex id
+//                  and mask (cell_tb / cell_mask arenas); for the chunks that
+//                  smooth, each vertex's ring (the primitives around it in
+//                  ascending id, the reference's order), from the quad ids of
+//                  its polygon's edges
+//   k_dmc_quads    quad (or two-triangle) indices
 //   K x (k_dual_n, k_primal_ring)
 #include <hip/hip_runtime.h>
 
 #include "bmf_device_tables.h"
 #include "bmf_internal.h"
 #include "bmf_rows.h"
+#include "bmf_words.h"
 #include "samplers.h"
 
 namespace bmf {
@@ -53,14 +53,6 @@ __device__ void load_dmc_tables(DmcTables& t) {
         t.np[m] = (uint8_t)(p + any);
         t.pe[m] = pe;
     }
-}
-
-// Sum over the wave of a per-lane count c < 8 (bit-sliced ballots), and the
-// exclusive prefix of the lanes below.
-__device__ __forceinline__ uint32_t wave_sum3(uint32_t c, uint64_t lt, uint32_t& pre) {
-    const uint64_t b0 = __ballot(c & 1u), b1 = __ballot(c & 2u), b2 = __ballot(c & 4u);
-    pre = (uint32_t)__popcll(b0 & lt) + 2u * (uint32_t)__popcll(b1 & lt) + 4u * (uint32_t)__popcll(b2 & lt);
-    return (uint32_t)__popcll(b0) + 2u * (uint32_t)__popcll(b1) + 4u * (uint32_t)__popcll(b2);
 }
 
 // ------------------------------------------------------------------------
@@ -284,34 +276,31 @@ __constant__ int8_t c_le[12][4] = {{0, 0, 0, 0}, {0, 0, 1, 0}, {0, 1, 0, 0}, {0,
 
 // ------------------------------------------------------------------------
 // Rings.  Quad ids follow the (x, y, z, axis) order of their lattice edges:
-// a row's base (row_t after the scan, per quad) plus the row's interior
-// sign-changing edges before the edge's sample (all axes) and before its axis
-// at that sample.  A vertex (a polygon of a cell) lies on the quads of its
+// an item's base plus its interior sign-changing edges before the edge's
+// sample (all axes) and before its axis at that sample.  A vertex (a polygon of a cell) lies on the quads of its
 // polygon's interior edges, so visiting the cell's local edges in the order of
 // their (dx, dy, dz, axis) offsets lists its quads in ascending id.  With
 // quads written as triangles (a, b, c), (c, d, a) (MeshProcessor.cpp:74-91) a
 // quad's first and last ring cells (corners a and c) are on both triangles,
 // the others on one, chosen by the quad's winding.
 // ------------------------------------------------------------------------
-// For label row d = 2 dx + dy of cell (x, y, z), i.e. row (x + dx, y + dy):
-// the row's first quad id plus its interior sign-changing edges before
-// sample z (all axes), and flag byte d: the interior edge bits of axes 0-2 at
-// z (bits 0-2) and at z + 1 (bits 3-5), the label at z and z + 1 (6, 7).
-// The rows come from the staged planes x, x+1, x+2.
-template <int W>
-__device__ __forceinline__ void quad_row_at(const uint64_t (*s_planes)[plane_words(W)], const uint32_t* rtc,
-                                            uint32_t div, int dim, int x, int y, int z, int d, uint32_t& pre,
-                                            uint32_t& fl) {
-    const int dx = d >> 1, dy = d & 1, xx = x + dx, yy = y + dy;
-    const RowBits<W> ra = lds_row<W>(s_planes[dx], dim, yy, true);
-    const RowBits<W> rb = lds_row<W>(s_planes[dx], dim, yy + 1, yy + 1 < dim);
-    const RowBits<W> rc = lds_row<W>(s_planes[dx + 1], dim, yy, xx + 1 < dim);
-    RowBits<W> e0, e1, e2;
-    interior_edges<W>(ra, rb, rc, dim, xx, yy, e0, e1, e2);
-    pre = rtc[(int64_t)xx * dim + yy] / div + prefix_pop<W>(e0, z) + prefix_pop<W>(e1, z) + prefix_pop<W>(e2, z);
-    const uint32_t f = bit_at<W>(e0, z) | (bit_at<W>(e1, z) << 1) | (bit_at<W>(e2, z) << 2) |
-                       (bit_at<W>(e0, z + 1) << 3) | (bit_at<W>(e1, z + 1) << 4) | (bit_at<W>(e2, z + 1) << 5) |
-                       (bit_at<W>(ra, z) << 6) | (bit_at<W>(ra, z + 1) << 7);
+// For sample row d = 2 dx + dy of the cell at the item's sample `pos`: the
+// quad id of the first edge at sample (dx, dy, 0) of the cell, and flag byte
+// d: the interior edge bits of axes 0-2 there (bits 0-2) and one sample on
+// (bits 3-5), the labels of the two (6, 7).  From the item's windows.
+__device__ __forceinline__ void quad_row_at(const ItemWindows& s, const WindowGeom& g, int dim, int pos, int d,
+                                            uint32_t& pre, uint32_t& fl) {
+    const int dx = d >> 1, dy = d & 1;
+    pre = window_edge(s, g, dim, pos, dx, dy, 0, 0);
+    const int p = pos + dy * dim + (dx ? g.off : 0);
+    uint32_t f = label_pair(s.lab + (dx ? g.n0 : 0), p) << 6;
+#pragma unroll
+    for (int dz = 0; dz < 2; dz++) {
+        const int w = ((p + dz) >> 6) + (dx ? g.n0 : 0), b = (p + dz) & 63;
+        f |= (((uint32_t)(s.ex[w] >> b) & 1u) | (((uint32_t)(s.ey[w] >> b) & 1u) << 1) |
+              (((uint32_t)(s.ez[w] >> b) & 1u) << 2))
+             << (3 * dz);
+    }
     fl |= f << (8 * d);
 }
 
@@ -365,18 +354,46 @@ __device__ __forceinline__ uint32_t dmc_ring(const Arenas& A, const uint32_t (&p
     return n;
 }
 
+// CSG primitives of one item's edge points: those of the chunk's list that
+// can reach the union's surface there.  An edge point lies within one sample
+// step of a sample with density >= 0, and the union is 1-Lipschitz, so a
+// primitive that stays below -step everywhere in the item's box never wins;
+// twice the step and a coordinate-sized slack cover the rounding.
+constexpr int kItemCsg = 16;
+
+struct DmcWave {
+    ItemWindows win;
+    uint32_t verts[4 * 64];       // a round's vertices: sample | polygon << 10 | corner mask << 12
+    float4 csg[2 * kItemCsg];     // stage_csg layout
+};
+
+// World box of the item's cells: lo and hi per axis.
+__device__ __forceinline__ void item_box(const ChunkMeta& M, int w0, float (&lo)[3], float (&hi)[3]) {
+    const int dim = M.dim, d2 = dim * dim, a = 64 * w0, b = min(a + kItemSamples, d2 * dim) - 1;
+    const int xa = a / d2, xb = b / d2;
+    const int ya = (a - xa * d2) / dim, yb = (b - xb * d2) / dim;
+    const int c0[3] = {xa, xa == xb ? ya : 0, 0};
+    const int c1[3] = {xb + 1, xa == xb ? yb + 1 : dim - 1, dim - 1};
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        lo[k] = (float)c0[k] * M.delta + M.opos[k];
+        hi[k] = (float)c1[k] * M.delta + M.opos[k];
+    }
+}
+
 // ------------------------------------------------------------------------
-// vertices: one per polygon of each surface cell.  Row pass (wave per row,
-// lane = z): per-cell first vertex id and mask, per vertex its cell and
-// polygon code and boundary flag.  The plane's vertices are a contiguous id
-// range, so a dense pass of the whole block then places them (mass point or
-// QEF), free of the row pass's idle lanes.
+// vertices: one per polygon of each active cell, a wave per item.  Rounds of
+// 64 cells: each cell's first vertex id and mask, its polygons compacted into
+// a dense list, then a lane per vertex places it (mass point or QEF) and, for
+// chunks that smooth, writes its ring.  QEF placement is bound by the
+// normals (a pass over the primitives per edge point): the item's own list
+// keeps the few that can win.  64 chunks of 64^3 cells, 300 primitives,
+// 326,882 vertices: 114 us, with the plane's rows and the chunk's list 169.
 // ------------------------------------------------------------------------
 __device__ void place_vertex(const Arenas& A, const ChunkMeta& M, const SamplerDev& S, const uint16_t* csg,
-                             const float4* s_csg, int x, uint32_t code, uint32_t mask, bool qef, float out[3],
-                             float& err) {
+                             const float4* s_csg, int ns, int nb, int x, int y, int z, int p, uint32_t mask, bool qef,
+                             float out[3], float& err) {
     const int dim = M.dim;
-    const int y = (int)((code >> 8) & 255u), z = (int)((code >> 16) & 255u), p = (int)(code >> 24);
     const float* __restrict__ D = A.dens + M.dens_off;
     const uint64_t row = c_dmc_table[mask];
     const int nn = (int)(row >> 60);
@@ -428,8 +445,8 @@ __device__ void place_vertex(const Arenas& A, const ChunkMeta& M, const SamplerD
             // unit normal of the CSG field at the point (world coordinates)
             const float wx = qx * M.delta + M.opos[0], wy = qy * M.delta + M.opos[1], wz = qz * M.delta + M.opos[2];
             float g[3];
-            if (s_csg) csg_gradient_lds(s_csg, M.csg_ns, M.csg_nb, wx, wy, wz, g);
-            else csg_gradient(S, csg, M.csg_ns, M.csg_nb, wx, wy, wz, g);
+            if (s_csg) csg_gradient_lds(s_csg, ns, nb, wx, wy, wz, g);
+            else csg_gradient(S, csg, ns, nb, wx, wy, wz, g);
             const float len = sqrtf((g[0] * g[0] + g[1] * g[1]) + g[2] * g[2]);
             float nrm[3];
             for (int c = 0; c < 3; c++) nrm[c] = len > 0.0f ? g[c] / len : 0.0f;
@@ -452,226 +469,202 @@ __device__ void place_vertex(const Arenas& A, const ChunkMeta& M, const SamplerD
     }
 }
 
-template <int W>
-__global__ void __launch_bounds__(kRowThreads) k_dmc_vertices(Arenas A, int n) {
+__global__ void __launch_bounds__(kRowThreads) k_dmc_vertices(Arenas A) {
     __shared__ DmcTables s_t;
-    __shared__ uint64_t s_planes[3][plane_words(W)];  // labels of planes x, x+1, x+2
-    __shared__ float4 s_csg[2 * kCsgStage];  // the chunk's culled CSG primitives (QEF normals)
+    __shared__ DmcWave s_wave[kWordWaves];
     load_dmc_tables(s_t);
+    __syncthreads();
     const SamplerDev* __restrict__ S = A.sampler;
-    const int wave = uniform_int(threadIdx.x >> 6);
-    const int lane = lane_id();
-    const uint64_t lt = lanemask_lt();
-    const int64_t base = A.ctr->class_base[W - 1], total = A.ctr->class_planes[W - 1];
-    for (int64_t item = blockIdx.x; item < total; item += gridDim.x) {
-        const int2 pm = A.plane_map[base + item];
-        const int j = uniform_int(pm.x);
-        const ChunkMeta M = read_chunk(A.meta, j);
-        const int dim = M.dim;
+    const int wave = uniform_int(threadIdx.x >> 6), lane = lane_id();
+    DmcWave& W = s_wave[wave];
+    ItemWindows& s = W.win;
+    const bool qef = A.placement == BMF_PLACE_QEF && S->kind == BMF_SAMPLER_CSG;
+    const bool tris = A.quad_tris != 0;
+    const int64_t total = A.ctr->total_items;
+    for (int64_t it = (int64_t)blockIdx.x * kWordWaves + wave; it < total; it += (int64_t)gridDim.x * kWordWaves) {
+        const int2 im = A.item_map[it];
+        const int chunk = uniform_int(im.x), w0 = uniform_int(im.y) * kItemWords;
+        const ChunkMeta M = read_chunk(A.meta, chunk);
         if (M.status != BMF_OK || M.V == 0) continue;
-        const int x = uniform_int(pm.y);
-        if (x >= dim - 1) continue;
-        const bool qef = A.placement == BMF_PLACE_QEF && S->kind == BMF_SAMPLER_CSG;
-        const uint16_t* csg = A.csg_list ? A.csg_list + (int64_t)j * A.csg_stride : nullptr;
-        const bool staged = qef && csg && M.csg_ns + M.csg_nb <= kCsgStage;  // uniform across the block
-        __syncthreads();
-        {
-            uint64_t* const dst[3] = {s_planes[0], s_planes[1], s_planes[2]};
-            const uint64_t* const src[3] = {A.labels + M.lab_off, A.labels + M.lab_off, A.labels + M.lab_off};
-            const int xp[3] = {x, x + 1, x + 2};
-            stage_plane_group<3>(dst, src, M.lab_words, dim, xp);
+        const int dim = M.dim, d2 = dim * dim;
+        const float rd = 1.0f / (float)dim, rd2 = 1.0f / (float)d2;
+        const WindowGeom g = stage_windows(A, M, w0, s);
+        const int nc = push_bits(s.ac[lane >> 2], s.list);
+        wave_sync();
+        if (nc == 0) continue;
+        const uint16_t* csg = A.csg_list ? A.csg_list + (int64_t)chunk * A.csg_stride : nullptr;
+        int ns = M.csg_ns, nb = M.csg_nb;
+        bool staged = false;
+        if (qef && csg) {
+            float lo[3], hi[3], far = 0.0f;
+            item_box(M, w0, lo, hi);
+#pragma unroll
+            for (int k = 0; k < 3; k++) far = fmaxf(far, fmaxf(fabsf(lo[k]), fabsf(hi[k])));
+            int is, ib;
+            staged = cull_csg(*S, csg, ns, nb, lo, hi, 2.0f * M.delta + 1e-4f * far, W.csg, kItemCsg, is, ib);
+            if (staged) {
+                ns = is;
+                nb = ib;
+            }
+            wave_sync();
         }
-        if (staged) stage_csg(*S, csg, M.csg_ns, M.csg_nb, s_csg);
-        __syncthreads();
-        const uint32_t* rv = A.row_v + M.row_off + (int64_t)x * dim;
         const int64_t vo = M.v_off;
         const uint32_t Vc = (uint32_t)M.V;
         const bool smooth = (M.iters > 0 || A.normals) && M.T > 0;  // the chunk runs the smoothing kernels
-        const bool tris = A.quad_tris != 0;
-        const uint32_t* rtc = A.row_t + M.row_off;
-        // ---- row pass ----
-        for (int y = wave; y < dim - 1; y += kRowThreads / 64) {
-            if (rv[y + 1] == rv[y]) continue;  // the row's cells have no polygon
-            const RowBits<W> r00 = lds_row<W>(s_planes[0], dim, y, true);
-            const RowBits<W> r01 = lds_row<W>(s_planes[0], dim, y + 1, true);
-            const RowBits<W> r10 = lds_row<W>(s_planes[1], dim, y, true);
-            const RowBits<W> r11 = lds_row<W>(s_planes[1], dim, y + 1, true);
-            if (quad_uniform<W>(r00, r01, r10, r11, dim)) continue;
-            uint32_t carry = rv[y];
-            for (int z0 = 0; z0 < dim - 1; z0 += 64) {
-                const int z = z0 + lane;
-                const uint32_t mask = z < dim - 1 ? cell_mask<W>(r00, r01, r10, r11, z) : 0u;
-                const uint32_t np = s_t.np[mask];
-                uint32_t pre;
-                const uint32_t tot = wave_sum3(np, lt, pre);
-                const uint32_t vb = carry + pre;
-                carry += tot;
-                if (!np) continue;
-                const int64_t ci = M.dens_off + ((int64_t)x * dim + y) * dim + z;
-                A.cell_tb[ci] = vb;
+        uint32_t vb = A.item_c[it];
+        for (int e0 = 0; e0 < nc; e0 += 64) {
+            // ---- the round's cells ----
+            int pos = 0;
+            uint32_t mask = 0, np = 0;
+            if (e0 + lane < nc) {
+                pos = s.list[e0 + lane];
+                mask = window_mask(s, g, dim, pos);
+                np = s_t.np[mask];
+            }
+            uint32_t nv;
+            const uint32_t pre = wave_prefix<3>(np, nv);
+            if (np) {
+                const int64_t ci = M.dens_off + 64ll * w0 + pos;
+                A.cell_tb[ci] = vb + pre;
                 A.cell_mask[ci] = (uint8_t)mask;
-                for (uint32_t p = 0; p < np; p++) {
-                    const uint32_t v = vb + p;
-                    if (v >= Vc) {
-                        A.ctr->error = 8;
-                        break;
-                    }
-                    A.boundary[vo + v] =
-                        (uint8_t)(x == 0 || y == 0 || z == 0 || x + 1 == dim - 1 || y + 1 == dim - 1 || z + 1 == dim - 1);
-                    A.vedge[vo + v] = (uint32_t)x | ((uint32_t)y << 8) | ((uint32_t)z << 16) | (p << 24);
+                for (uint32_t p = 0; p < np; p++) W.verts[pre + p] = (uint32_t)pos | (p << 10) | (mask << 12);
+            }
+            wave_sync();
+            // ---- their vertices ----
+            for (uint32_t e = (uint32_t)lane; e < nv; e += 64u) {
+                const uint32_t item = W.verts[e];
+                const int cpos = (int)(item & 1023u), p = (int)((item >> 10) & 3u);
+                const uint32_t cmask = item >> 12, v = vb + e;
+                if (v >= Vc) {
+                    A.ctr->error = 8;
+                    continue;
+                }
+                const uint32_t i = 64u * (uint32_t)w0 + (uint32_t)cpos;
+                const int x = (int)udiv24(i, (uint32_t)d2, rd2), r = (int)i - x * d2;
+                const int y = (int)udiv24((uint32_t)r, (uint32_t)dim, rd), z = r - y * dim;
+                A.boundary[vo + v] =
+                    (uint8_t)(x == 0 || y == 0 || z == 0 || x + 1 == dim - 1 || y + 1 == dim - 1 || z + 1 == dim - 1);
+                A.vedge[vo + v] = (uint32_t)x | ((uint32_t)y << 8) | ((uint32_t)z << 16) | ((uint32_t)p << 24);
+                float o[3], err;
+                place_vertex(A, M, *S, csg, staged ? W.csg : nullptr, ns, nb, x, y, z, p, cmask, qef, o, err);
+                float* P = A.pos + (vo + v) * 3;
+                P[0] = o[0];
+                P[1] = o[1];
+                P[2] = o[2];
+                if (smooth) A.pos4[vo + v] = make_float4(o[0], o[1], o[2], 0.0f);
+                if (A.qef_err) A.qef_err[vo + v] = err;
+                if (A.normals) {  // a vertex with no polygon keeps the zero normal
+                    A.nrm4[vo + v] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                    float* O = A.nrm + (vo + v) * 3;
+                    O[0] = 0.0f;
+                    O[1] = 0.0f;
+                    O[2] = 0.0f;
+                }
+                if (smooth) {
+                    uint32_t pre4[4], fl = 0u;
+#pragma unroll
+                    for (int d = 0; d < 4; d++) quad_row_at(s, g, dim, cpos, d, pre4[d], fl);
+                    A.ring_n[vo + v] = dmc_ring(A, pre4, fl, s_t.pe[cmask], (uint32_t)p, vo + v, tris);
                 }
             }
-        }
-        __syncthreads();  // the plane's vertex codes are written
-        // ---- dense placement of the plane's vertices [rv[0], next plane's first) ----
-        const uint32_t v0 = rv[0], v1 = min(x + 1 < dim ? rv[dim] : Vc, Vc);
-        for (uint32_t v = v0 + threadIdx.x; v < v1; v += blockDim.x) {
-            const uint32_t code = A.vedge[vo + v];
-            const int y = (int)((code >> 8) & 255u), z = (int)((code >> 16) & 255u);
-            const uint32_t mask = A.cell_mask[M.dens_off + ((int64_t)x * dim + y) * dim + z];
-            float o[3], err;
-            place_vertex(A, M, *S, csg, staged ? s_csg : nullptr, x, code, mask, qef, o, err);
-            float* P = A.pos + (vo + v) * 3;
-            P[0] = o[0];
-            P[1] = o[1];
-            P[2] = o[2];
-            if (smooth) A.pos4[vo + v] = make_float4(o[0], o[1], o[2], 0.0f);
-            if (A.qef_err) A.qef_err[vo + v] = err;
-            if (A.normals) {  // a vertex with no polygon keeps the zero normal
-                A.nrm4[vo + v] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                float* O = A.nrm + (vo + v) * 3;
-                O[0] = 0.0f;
-                O[1] = 0.0f;
-                O[2] = 0.0f;
-            }
-        }
-        if (!smooth) continue;
-        // ---- dense pass: the rings of the plane's vertices ----
-        for (uint32_t v = v0 + threadIdx.x; v < v1; v += blockDim.x) {
-            const uint32_t code = A.vedge[vo + v];
-            const int y = (int)((code >> 8) & 255u), z = (int)((code >> 16) & 255u);
-            const uint32_t mask = A.cell_mask[M.dens_off + ((int64_t)x * dim + y) * dim + z];
-            uint32_t pre[4] = {0u, 0u, 0u, 0u}, fl = 0u;
-            // one row at a time (few live registers), its prefix kept by selects
-#pragma unroll 1
-            for (int d = 0; d < 4; d++) {
-                uint32_t pd;
-                quad_row_at<W>(s_planes, rtc, tris ? 2u : 1u, dim, x, y, z, d, pd, fl);
-#pragma unroll
-                for (int q = 0; q < 4; q++) pre[q] = q == d ? pd : pre[q];
-            }
-            A.ring_n[vo + v] = dmc_ring(A, pre, fl, s_t.pe[mask], code >> 24, vo + v, tris);
+            vb += nv;
+            wave_sync();  // the round's vertices are read
         }
     }
 }
 
 // ------------------------------------------------------------------------
-// quads around the interior sign-changing edges owned by the row's samples
+// quads around the interior sign-changing edges, a wave per item, a lane per
+// sample that owns some (the batch above: 20 us, with a wave per row 71)
 // ------------------------------------------------------------------------
-template <int W>
-__global__ void __launch_bounds__(kRowThreads) k_dmc_quads(Arenas A, int n) {
+__global__ void __launch_bounds__(kRowThreads) k_dmc_quads(Arenas A) {
     __shared__ DmcTables s_t;
-    __shared__ uint64_t s_planes[2][plane_words(W)];
+    __shared__ ItemWindows s_win[kWordWaves];
     load_dmc_tables(s_t);
-    const int wave = uniform_int(threadIdx.x >> 6);
-    const int lane = lane_id();
-    const int64_t base = A.ctr->class_base[W - 1], total = A.ctr->class_planes[W - 1];
+    __syncthreads();
+    const int wave = uniform_int(threadIdx.x >> 6), lane = lane_id();
+    ItemWindows& s = s_win[wave];
     const bool tris = A.quad_tris != 0;
-    for (int64_t item = blockIdx.x; item < total; item += gridDim.x) {
-        const int2 pm = A.plane_map[base + item];
-        const ChunkMeta M = read_chunk(A.meta, pm.x);
-        const int dim = M.dim;
+    const int64_t total = A.ctr->total_items;
+    for (int64_t it = (int64_t)blockIdx.x * kWordWaves + wave; it < total; it += (int64_t)gridDim.x * kWordWaves) {
+        const ItemRef R = item_ref(A, it);
+        const ChunkMeta& M = R.M;
         if (M.status != BMF_OK || M.T == 0) continue;
-        const int x = uniform_int(pm.y);
-        __syncthreads();
-        {
-            uint64_t* const dst[2] = {s_planes[0], s_planes[1]};
-            const uint64_t* const src[2] = {A.labels + M.lab_off, A.labels + M.lab_off};
-            const int xp[2] = {x, x + 1};
-            stage_plane_group<2>(dst, src, M.lab_words, dim, xp);
-        }
-        __syncthreads();
-        const uint32_t* rt = A.row_t + M.row_off + (int64_t)x * dim;
+        const int dim = M.dim, d2 = dim * dim;
+        const float rd = 1.0f / (float)dim, rd2 = 1.0f / (float)d2;
+        (void)stage_windows(A, M, R.w0, s);
+        const int k4 = lane >> 2;
+        const int nq = push_bits(s.ex[k4] | s.ey[k4] | s.ez[k4], s.list);
+        wave_sync();
         const uint32_t Vc = (uint32_t)M.V, Tc = (uint32_t)M.T;
         uint32_t* __restrict__ I = A.idx + M.i_off;
-        for (int y = wave; y < dim; y += kRowThreads / 64) {
-            const bool x1 = x + 1 < dim, y1 = y + 1 < dim;
-            // rows whose samples own no quad (the next row's base, or the next
-            // plane's, or the chunk's total after the last row) skip the label work
-            const uint32_t next = y1 ? rt[y + 1] : (x1 ? rt[dim] : (uint32_t)M.T);
-            if (next == rt[y]) continue;
-            const RowBits<W> r00 = lds_row<W>(s_planes[0], dim, y, true);
-            const RowBits<W> r01 = lds_row<W>(s_planes[0], dim, y + 1, y1);
-            const RowBits<W> r10 = lds_row<W>(s_planes[1], dim, y, x1);
-            RowBits<W> ex, ey, ez;
-            interior_edges<W>(r00, r01, r10, dim, x, y, ex, ey, ez);
-            if (total_pop<W>(ex) + total_pop<W>(ey) + total_pop<W>(ez) == 0) continue;
-            const uint32_t qbase = rt[y] / (tris ? 2u : 1u);
-            for (int z0 = 0; z0 < dim; z0 += 64) {
-                const int z = z0 + lane;
-                if (z >= dim) continue;
-                const uint32_t f[3] = {bit_at<W>(ex, z), bit_at<W>(ey, z), bit_at<W>(ez, z)};
-                if (!(f[0] | f[1] | f[2])) continue;
-                uint32_t qid = qbase + prefix_pop<W>(ex, z) + prefix_pop<W>(ey, z) + prefix_pop<W>(ez, z);
-                const bool solid_origin = bit_at<W>(r00, z) == 0u;
-                // the rings of the sample's three edges are cells of the 2 x 2 x 2
-                // block (x-1 .. x, y-1 .. y, z-1 .. z): its eight first-vertex ids
-                // and masks load together (a cell outside the chunk reads cell 0;
-                // only the rings of interior edges, all inside, use them)
-                uint32_t tb8[8], mk8[8];
+        for (int e = lane; e < nq; e += 64) {
+            const int pos = s.list[e], w = pos >> 6;
+            const uint64_t bit = 1ull << (pos & 63), lt = bit - 1ull;
+            const uint64_t ex = s.ex[w], ey = s.ey[w], ez = s.ez[w];
+            const bool f[3] = {(ex & bit) != 0ull, (ey & bit) != 0ull, (ez & bit) != 0ull};
+            uint32_t qid = s.pre[w] + (uint32_t)(__popcll(ex & lt) + __popcll(ey & lt) + __popcll(ez & lt));
+            const bool solid_origin = (s.lab[w] & bit) == 0ull;
+            const uint32_t i = 64u * (uint32_t)R.w0 + (uint32_t)pos;
+            const int x = (int)udiv24(i, (uint32_t)d2, rd2), r0 = (int)i - x * d2;
+            const int y = (int)udiv24((uint32_t)r0, (uint32_t)dim, rd), z = r0 - y * dim;
+            // the rings of the sample's three edges are cells of the 2 x 2 x 2
+            // block (x-1 .. x, y-1 .. y, z-1 .. z): its eight first-vertex ids
+            // and masks load together (a cell outside the chunk reads cell 0;
+            // only the rings of interior edges, all inside, use them)
+            uint32_t tb8[8], mk8[8];
 #pragma unroll
-                for (int c = 0; c < 8; c++) {
-                    const int cx = x - 1 + (c >> 2), cy = y - 1 + ((c >> 1) & 1), cz = z - 1 + (c & 1);
-                    const bool in = cx >= 0 && cy >= 0 && cz >= 0 && cx <= dim - 2 && cy <= dim - 2 && cz <= dim - 2;
-                    const int64_t ci = M.dens_off + (in ? ((int64_t)cx * dim + cy) * dim + cz : 0);
-                    tb8[c] = A.cell_tb[ci];
-                    mk8[c] = A.cell_mask[ci];
+            for (int c = 0; c < 8; c++) {
+                const int cx = x - 1 + (c >> 2), cy = y - 1 + ((c >> 1) & 1), cz = z - 1 + (c & 1);
+                const bool in = cx >= 0 && cy >= 0 && cz >= 0 && cx <= dim - 2 && cy <= dim - 2 && cz <= dim - 2;
+                const int64_t ci = M.dens_off + (in ? ((int64_t)cx * dim + cy) * dim + cz : 0);
+                tb8[c] = A.cell_tb[ci];
+                mk8[c] = A.cell_mask[ci];
+            }
+#pragma unroll
+            for (int a = 0; a < 3; a++) {
+                if (!f[a]) continue;
+                uint32_t v[4];
+                bool ok = true;
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    // ring cell r of axis a: offsets (c_ring) -1 / 0 per axis -> block cell
+                    const int c = ((c_ring[a][r][0] + 1) << 2) | ((c_ring[a][r][1] + 1) << 1) | (c_ring[a][r][2] + 1);
+                    const uint32_t le = (uint32_t)c_ring[a][r][3];
+                    const uint32_t pi = (uint32_t)((s_t.pe[mk8[c]] >> (4 * le)) & 15ull);
+                    v[r] = tb8[c] + pi;
+                    if (pi == 15u || v[r] >= Vc) ok = false;
                 }
-#pragma unroll
-                for (int a = 0; a < 3; a++) {
-                    if (!f[a]) continue;
-                    uint32_t v[4];
-                    bool ok = true;
-#pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        // ring cell r of axis a: offsets (c_ring) -1 / 0 per axis -> block cell
-                        const int c = ((c_ring[a][r][0] + 1) << 2) | ((c_ring[a][r][1] + 1) << 1) | (c_ring[a][r][2] + 1);
-                        const uint32_t le = (uint32_t)c_ring[a][r][3];
-                        const uint32_t pi = (uint32_t)((s_t.pe[mk8[c]] >> (4 * le)) & 15ull);
-                        v[r] = tb8[c] + pi;
-                        if (pi == 15u || v[r] >= Vc) ok = false;
-                    }
-                    const uint32_t prim = tris ? 2u * qid : qid;
-                    if (!ok || prim + (tris ? 1u : 0u) >= Tc) {
-                        A.ctr->error = 9;
-                        qid++;
-                        continue;
-                    }
-                    // cyclic c0 c1 c3 c2: right-hand normal along -x, +y, -z;
-                    // flipped so that it points to the solid end of the edge
-                    const bool toward_origin = a != 1;
-                    uint32_t o[4] = {v[0], v[1], v[3], v[2]};
-                    if (solid_origin != toward_origin) {
-                        o[1] = v[2];
-                        o[3] = v[1];
-                    }
-                    if (tris) {  // MeshProcessor::flush_to_tris (MeshProcessor.cpp:74-91)
-                        uint32_t* t = I + 3ll * prim;
-                        t[0] = o[0];
-                        t[1] = o[1];
-                        t[2] = o[2];
-                        t[3] = o[2];
-                        t[4] = o[3];
-                        t[5] = o[0];
-                    } else {
-                        uint32_t* t = I + 4ll * prim;
-                        t[0] = o[0];
-                        t[1] = o[1];
-                        t[2] = o[2];
-                        t[3] = o[3];
-                    }
+                const uint32_t prim = tris ? 2u * qid : qid;
+                if (!ok || prim + (tris ? 1u : 0u) >= Tc) {
+                    A.ctr->error = 9;
                     qid++;
+                    continue;
                 }
+                // cyclic c0 c1 c3 c2: right-hand normal along -x, +y, -z;
+                // flipped so that it points to the solid end of the edge
+                const bool toward_origin = a != 1;
+                uint32_t o[4] = {v[0], v[1], v[3], v[2]};
+                if (solid_origin != toward_origin) {
+                    o[1] = v[2];
+                    o[3] = v[1];
+                }
+                if (tris) {  // MeshProcessor::flush_to_tris (MeshProcessor.cpp:74-91)
+                    uint32_t* t = I + 3ll * prim;
+                    t[0] = o[0];
+                    t[1] = o[1];
+                    t[2] = o[2];
+                    t[3] = o[2];
+                    t[4] = o[3];
+                    t[5] = o[0];
+                } else {
+                    uint32_t* t = I + 4ll * prim;
+                    t[0] = o[0];
+                    t[1] = o[1];
+                    t[2] = o[2];
+                    t[3] = o[3];
+                }
+                qid++;
             }
         }
     }
@@ -939,16 +932,10 @@ __global__ void __launch_bounds__(kSmoothThreads) k_primal_ring_nrm(Arenas A, in
 // launch wrappers
 // ------------------------------------------------------------------------
 
-hipError_t launch_dmc_emit(const Arenas& A, int n, int blocks, int wclasses, hipStream_t s) {
-    // per class: vertices, then the quads that index them
-    if (wclasses & 1) hipLaunchKernelGGL(k_dmc_vertices<1>, dim3(blocks), dim3(kRowThreads), 0, s, A, n);
-    if (wclasses & 2) hipLaunchKernelGGL(k_dmc_vertices<2>, dim3(blocks), dim3(kRowThreads), 0, s, A, n);
-    if (wclasses & 4) hipLaunchKernelGGL(k_dmc_vertices<3>, dim3(blocks), dim3(kRowThreads), 0, s, A, n);
-    if (wclasses & 8) hipLaunchKernelGGL(k_dmc_vertices<4>, dim3(blocks), dim3(kRowThreads), 0, s, A, n);
-    if (wclasses & 1) hipLaunchKernelGGL(k_dmc_quads<1>, dim3(blocks), dim3(kRowThreads), 0, s, A, n);
-    if (wclasses & 2) hipLaunchKernelGGL(k_dmc_quads<2>, dim3(blocks), dim3(kRowThreads), 0, s, A, n);
-    if (wclasses & 4) hipLaunchKernelGGL(k_dmc_quads<3>, dim3(blocks), dim3(kRowThreads), 0, s, A, n);
-    if (wclasses & 8) hipLaunchKernelGGL(k_dmc_quads<4>, dim3(blocks), dim3(kRowThreads), 0, s, A, n);
+hipError_t launch_dmc_emit(const Arenas& A, int blocks, hipStream_t s) {
+    // the vertices, then the quads that index them
+    hipLaunchKernelGGL(k_dmc_vertices, dim3(blocks), dim3(kRowThreads), 0, s, A);
+    hipLaunchKernelGGL(k_dmc_quads, dim3(blocks), dim3(kRowThreads), 0, s, A);
     return hipGetLastError();
 }
 

@@ -12,9 +12,9 @@ namespace bmf {
 // of 64 so that every wave owns whole label words.
 constexpr int kSampleThreads = 256;
 constexpr int kSampleTileDefault = 2048;
-constexpr int kRowThreads = 256;      // 4 waves; one x-plane (or row segment of one) per block, one label row per wave
-constexpr int kMaxPlaneSplit = 8;     // row segments per x-plane when few planes are sampled
-constexpr int kSplitTarget = 512;     // row-kernel work items aimed at before splitting stops
+constexpr int kRowThreads = 256;      // word kernels: 4 waves, an item of label words each
+constexpr int kItemWords = 16;        // label words per item: enough active cells for a wave's lanes near a surface
+constexpr int kItemSamples = 64 * kItemWords;
 constexpr int kSmoothThreads = 256;   // one vertex per thread
 constexpr int kMaxRowWords = 4;       // ceil(BMF_MAX_DIM / 64)
 constexpr int kXcds = 8;              // MI355X: 8 XCDs, each with its own L2
@@ -67,7 +67,6 @@ struct ChunkMeta {
     int64_t dens_off;   // float index into the density arena
     int64_t lab_off;    // u64 index into the label bitmap arena
     int64_t lab_words;  // u64 words of this chunk's bitmap
-    int64_t row_off;    // index into the per-row arrays (rows (x, y) in x-major order)
     uint32_t any_air;   // set by the sampling kernel
     uint32_t any_solid;
     int32_t contains_mesh;
@@ -79,7 +78,7 @@ struct ChunkMeta {
     int32_t csg_nb;     //      listed in Arenas::csg_list (sphere ids, then box ids, in order)
     int64_t v_off;      // output offsets
     int64_t i_off;
-    int64_t plane_slot; // plane_map entry of this chunk's x-plane 0 (sampled chunks)
+    int64_t item_slot;  // the chunk's first item of the word kernels (sampled chunks)
 };
 
 // Global counters, reset by the plan kernel.
@@ -96,9 +95,13 @@ struct Counters {
     int32_t n_smooth;
     int32_t overflow;
     int32_t error;
-    int32_t plane_split[4];    // row segments per x-plane item of row-word class W (index W-1)
-    int64_t class_base[4];     // first plane_map entry of class W's planes
-    int64_t class_planes[4];   // sampled planes of class W
+    int64_t total_items;       // items of the word kernels
+};
+
+// One label word's sign-changing edges per axis (in the quad mode only those
+// whose four cells lie in the chunk) and active cells, as bits of its samples.
+struct EdgeWord {
+    uint64_t ex, ey, ez, ac;
 };
 
 // Device pointers of one context.
@@ -113,8 +116,8 @@ struct Arenas {
     unsigned long long* stat_blocks;  // [2][stat_cap] terrain octaves evaluated per workgroup of
                                       // the sampling and the refinement kernels (plain stores, no atomics)
     int32_t stat_cap;
-    int2* plane_map;           // [max_chunks * BMF_MAX_DIM] (chunk, x) of each sampled x-plane, grouped by
-                               // row-word class (written by k_sample's prologue)
+    int2* item_map;            // [max_items] (chunk, item within the chunk) of the word kernels' items
+                               // (written by k_sample's prologue)
     int32_t* smooth_list;      // [max_chunks] chunks that run the smoothing
     int64_t* smooth_prefix;    // [max_chunks + 1] vertex tiles of the listed chunks
     int64_t* smooth_tprefix;   // [max_chunks + 1] triangle tiles of the listed chunks
@@ -122,15 +125,13 @@ struct Arenas {
     int64_t* smooth_xcd_t;     // [kXcds + 1] triangle-tile range of each XCD group
     int2* smooth_vmap;         // [vertex tiles] (chunk, tile within the chunk) of each smoothing vertex tile
     int2* smooth_tmap;         // [triangle tiles] the same for the triangle tiles
-    uint32_t* refine;          // [max_samples] per x-plane queue of samples (y*dim + z) to finish,
-                               // a region of rows [y0, y1) per row segment
-    int32_t row_split;         // row segments per x-plane item, or -1 for the automatic choice
-    uint32_t* plane_refine_n;  // [max_planes * kMaxPlaneSplit] queue length of each (x-plane, row segment) item
+    EdgeWord* edges;           // same layout as labels: edge and active-cell bits of each word
+    uint32_t* word_pre;        // same layout: edges of the item before the word
+    uint32_t* item_e;          // [max_items] edges of each item, then their exclusive prefix in the chunk
+    uint32_t* item_c;          // [max_items] the same for triangles (polygons in the quad mode)
     float* dens;               // [max_samples]
     uint64_t* labels;          // [max_samples / 64 + max_chunks]
     uint64_t* exact;           // same layout as labels: density of the sample is final
-    uint32_t* row_v;           // [max_rows] per label row: vertex count, then base
-    uint32_t* row_t;           // [max_rows] per label row: triangle count, then base
     uint32_t* cell_tb;         // [max_samples] first triangle of each surface cell
     uint8_t* cell_mask;        // [max_samples] corner mask of each surface cell
     float* pos;                // [max_vertices * 3]
@@ -142,7 +143,7 @@ struct Arenas {
     uint32_t* idx;             // [max_indices]
     Counters* ctr;
     SamplerDev* sampler;
-    int64_t cap_samples, cap_rows, cap_vertices, cap_indices;
+    int64_t cap_samples, cap_vertices, cap_indices;
     int32_t cap_chunks;
     int64_t ext_base;          // EXTERNAL: offset of this launch's first chunk in the caller's densities
     int32_t sample_tile;       // samples per sampling work-queue tile: 1024, 2048 or 4096
@@ -169,7 +170,11 @@ struct Arenas {
 // 7 quads, or 14 triangles when quads are written as triangles.
 constexpr int kRingSlots = 16;
 
-inline int row_word_class(int dim) { return 1 << (((dim + 63) >> 6) - 1); }
+// Workgroups that give every item of one chunk's word kernels its wave.
+inline int word_blocks(int dim) {
+    const int64_t items = ((int64_t)dim * dim * dim + kItemSamples - 1) / kItemSamples;
+    return (int)((items + kRowThreads / 64 - 1) / (kRowThreads / 64));
+}
 
 // Launch wrappers (bmf_kernels.hip).
 hipError_t launch_plan(const Arenas& A, int n, int allow_cull, int reset_bumps, hipStream_t s);
@@ -177,18 +182,16 @@ hipError_t launch_plan(const Arenas& A, int n, int allow_cull, int reset_bumps, 
 // kind: the sampler the device struct holds for this launch (BMF_SAMPLER_*)
 // slab: the sampler is a 2D noise field (its columns are evaluated once per tile)
 hipError_t launch_sample(const Arenas& A, int n, int blocks, int adaptive, int kind, int slab, hipStream_t s);
-// wclasses: bit W-1 set when the batch holds chunks with ceil(dim/64) == W
-// (the classes' kernels one after another on s).
-hipError_t launch_count(const Arenas& A, int n, int blocks, int wclasses, hipStream_t s);
+// refine: give early-labelled edge endpoints their full density (after an adaptive terrain launch_sample)
+hipError_t launch_count(const Arenas& A, int blocks, int refine, hipStream_t s);
 hipError_t launch_scan(const Arenas& A, int n, int blocks, hipStream_t s);
-hipError_t launch_emit(const Arenas& A, int n, int blocks, int wclasses, hipStream_t s);
-hipError_t launch_refine(const Arenas& A, int n, int blocks, hipStream_t s);
+hipError_t launch_emit(const Arenas& A, int blocks, hipStream_t s);
 hipError_t launch_smooth(const Arenas& A, int m, int blocks, hipStream_t s);
 // (chunk, tile) of every smoothing vertex and primitive tile, once per frame before the first step
 hipError_t launch_smooth_map(const Arenas& A, int blocks, hipStream_t s);
-// Quad mode (bmf_dmc.hip): counts after launch_count/launch_refine, emission
-// after launch_scan, smoothing over the per-vertex rings.
-hipError_t launch_dmc_emit(const Arenas& A, int n, int blocks, int wclasses, hipStream_t s);
+// Quad mode (bmf_dmc.hip): emission after launch_count / launch_scan,
+// smoothing over the per-vertex rings.
+hipError_t launch_dmc_emit(const Arenas& A, int blocks, hipStream_t s);
 hipError_t launch_dmc_smooth(const Arenas& A, int m, int blocks, hipStream_t s);
 hipError_t launch_ref_labels(const Arenas& A, uint32_t* words, hipStream_t s);
 hipError_t launch_ref_masks(const Arenas& A, uint64_t* masks, hipStream_t s);

@@ -9,19 +9,22 @@
 //   labels      flat bitmap over the sample index (x*dim + y)*dim + z,
 //               u64 word i/64, bit i%64, set when the density is < 0;
 //               one word per wave of 64 consecutive samples (one ballot)
-//   row_v/row_t per label row (x, y): vertex / triangle counts, then
-//               exclusive bases after the scan
+//   edges       per label word: bits of its samples' sign-changing edges per
+//               axis and of its active cells; word_pre its edges' prefix
+//               within its item (16 words), item_e / item_c the items' edge
+//               and cell counts, then exclusive bases after the scan
 //   cell_tb/    per surface cell (same index as the density): first triangle
 //   cell_mask   id and corner mask, written only for chunks that smooth
 //   output      positions float3, boundary u8, vertex edge code u32,
 //               chunk-local triangle indices
 // Cell masks and the reference's u32 label words are never materialised on
-// the hot path: the plane kernels rebuild them from the bitmap with shifts.
+// the hot path: the word kernels rebuild them from the bitmap with shifts.
 #include <hip/hip_runtime.h>
 
 #include "bmf_device_tables.h"
 #include "bmf_internal.h"
 #include "bmf_rows.h"
+#include "bmf_words.h"
 #include "samplers.h"
 
 namespace bmf {
@@ -69,10 +72,10 @@ __device__ __forceinline__ int64_t pick(const int64_t (&a)[N], int i) {
 
 // Plan record of one descriptor: DMCChunk::label_grid geometry
 // (DMCChunk.cpp:94-101), analytic culling, sizes; `add` gets its
-// contributions to the four arena sums (samples, label words, rows, sampling
-// tiles) and to the x-planes of its row-word class (add[4 + class]).
+// contributions to the arena sums (samples, label words, word items, sampling
+// tiles).
 __device__ __forceinline__ ChunkMeta plan_record(const Arenas& A, const SamplerDev* __restrict__ S,
-                                                 const bmf_chunk_desc& d, int allow_cull, int64_t (&add)[8]) {
+                                                 const bmf_chunk_desc& d, int allow_cull, int64_t (&add)[4]) {
     ChunkMeta m;
     float t = d.overlap * 2.0f;
     t = 1.0f + t;
@@ -107,40 +110,26 @@ __device__ __forceinline__ ChunkMeta plan_record(const Arenas& A, const SamplerD
     m.i_off = 0;
     m.dens_off = 0;
     m.lab_off = 0;
-    m.row_off = 0;
-    m.plane_slot = 0;
-#pragma unroll
-    for (int q = 0; q < 8; q++) add[q] = 0;
+    m.item_slot = 0;
     add[0] = sampled ? ns : 0;
     add[1] = m.lab_words;
-    add[2] = sampled ? (int64_t)d.dim * d.dim : 0;
+    add[2] = (m.lab_words + kItemWords - 1) / kItemWords;
     add[3] = sampled ? (ns + A.sample_tile - 1) / A.sample_tile : 0;
-    const int cls = ((d.dim + 63) >> 6) - 1;
-#pragma unroll
-    for (int q = 0; q < 4; q++) add[4 + q] = sampled && q == cls ? d.dim : 0;
     return m;
 }
 
-__device__ __forceinline__ bool plan_overflow(const Arenas& A, const int64_t (&tot)[8]) {
-    return tot[0] > A.cap_samples || tot[1] > A.cap_samples / 64 + A.cap_chunks || tot[2] > A.cap_rows;
+__device__ __forceinline__ bool plan_overflow(const Arenas& A, const int64_t (&tot)[4]) {
+    return tot[0] > A.cap_samples || tot[1] > A.cap_samples / 64 + A.cap_chunks;
 }
 
 // A record's final state once its offsets are known (base: where its block's
-// arena ranges start; cbase: its row-word class's first plane slot).
-__device__ __forceinline__ void plan_finish(const Arenas& A, int j, ChunkMeta& m, const int64_t (&base)[8],
-                                            const int64_t (&cbase)[4], bool overflow) {
+// arena ranges start).
+__device__ __forceinline__ void plan_finish(const Arenas& A, int j, ChunkMeta& m, const int64_t (&base)[4],
+                                            bool overflow) {
     m.dens_off += base[0];
     m.lab_off += base[1];
-    m.row_off += base[2];
+    m.item_slot += base[2];
     if (m.state == kStateSampled) {
-        const int q = ((m.dim + 63) >> 6) - 1;
-        int64_t cb = 0, bb = 0;
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            cb = k == q ? cbase[k] : cb;
-            bb = k == q ? base[4 + k] : bb;
-        }
-        m.plane_slot += cb + bb;
         if (overflow) {
             m.state = kStateSkipped;
             m.status = BMF_ECAPACITY;
@@ -153,11 +142,8 @@ __device__ __forceinline__ void plan_finish(const Arenas& A, int j, ChunkMeta& m
     if (m.state != kStateSampled) write_result(A, j, m);  // final: k_scan skips it
 }
 
-// The batch counters from the totals: sampling tiles, overflow, and per
-// row-word class its planes in plane_map and the row segments per plane
-// (few sampled planes, e.g. single large chunks: split each plane's rows so
-// that the class still has kSplitTarget items).
-__device__ __forceinline__ void plan_counters(const Arenas& A, int n, const int64_t (&tot)[8], bool overflow,
+// The batch counters from the totals: sampling tiles, word items, overflow.
+__device__ __forceinline__ void plan_counters(const Arenas& A, int n, const int64_t (&tot)[4], bool overflow,
                                               int reset_bumps) {
     A.tile_prefix[n] = overflow ? 0 : tot[3];
     Counters* c = A.ctr;
@@ -172,17 +158,7 @@ __device__ __forceinline__ void plan_counters(const Arenas& A, int n, const int6
     }
     if (overflow) c->overflow = 1;
     c->total_tiles = overflow ? 0 : tot[3];
-    int64_t cb = 0;
-    for (int q = 0; q < 4; q++) {
-        const int64_t np = overflow ? 0 : tot[4 + q];
-        int split = A.row_split > 0 ? A.row_split : 1;
-        if (A.row_split <= 0)
-            while (split < kMaxPlaneSplit && np * split < kSplitTarget) split <<= 1;
-        c->plane_split[q] = split;
-        c->class_base[q] = cb;
-        c->class_planes[q] = np;
-        cb += np;
-    }
+    c->total_items = overflow ? 0 : tot[2];
     c->n_smooth = 0;
     c->total_samples = tot[0];
 }
@@ -190,37 +166,29 @@ __device__ __forceinline__ void plan_counters(const Arenas& A, int n, const int6
 // Batches of up to kPlanOneBlock descriptors: one block, each thread a
 // segment of consecutive descriptors, one launch.
 __global__ void __launch_bounds__(kPlanThreads) k_plan(Arenas A, int n, int allow_cull, int reset_bumps) {
-    __shared__ int64_t s_w[8][kPlanThreads / 64 + 1];
+    __shared__ int64_t s_w[4][kPlanThreads / 64 + 1];
     const int per = (n + kPlanThreads - 1) / kPlanThreads;
     const int j0 = threadIdx.x * per, j1 = min(n, j0 + per);
-    int64_t sum[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    int64_t sum[4] = {0, 0, 0, 0};
     for (int j = j0; j < j1; j++) {
-        int64_t add[8];
+        int64_t add[4];
         ChunkMeta m = plan_record(A, A.sampler, A.descs[j], allow_cull, add);
         // offsets within the thread's segment; tile_prefix likewise
         m.dens_off = sum[0];
         m.lab_off = sum[1];
-        m.row_off = sum[2];
+        m.item_slot = sum[2];
         A.tile_prefix[j] = sum[3];
-        if (m.state == kStateSampled) m.plane_slot = pick<8>(sum, 4 + ((m.dim + 63) >> 6) - 1);
         A.meta[j] = m;
 #pragma unroll
-        for (int q = 0; q < 8; q++) sum[q] += add[q];
+        for (int q = 0; q < 4; q++) sum[q] += add[q];
     }
-    int64_t excl[8], tot[8];
-    block_scan<8, kPlanThreads>(sum, excl, tot, s_w);
+    int64_t excl[4], tot[4];
+    block_scan<4, kPlanThreads>(sum, excl, tot, s_w);
     const bool overflow = plan_overflow(A, tot);
-    // plane_map slots: the classes one after another, chunk order inside a class
-    int64_t cbase[4], cb = 0;
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-        cbase[q] = cb;
-        cb += tot[4 + q];
-    }
     for (int j = j0; j < j1; j++) {
         A.tile_prefix[j] = overflow ? 0 : A.tile_prefix[j] + excl[3];
         ChunkMeta m = A.meta[j];
-        plan_finish(A, j, m, excl, cbase, overflow);
+        plan_finish(A, j, m, excl, overflow);
     }
     if (threadIdx.x == 0) plan_counters(A, n, tot, overflow, reset_bumps);
 }
@@ -228,66 +196,57 @@ __global__ void __launch_bounds__(kPlanThreads) k_plan(Arenas A, int n, int allo
 // Larger batches, pass 1 of 3 (one descriptor per thread over many blocks):
 // records with offsets relative to their block, and each block's totals.
 __global__ void __launch_bounds__(kPlanThreads) k_plan_part(Arenas A, int n, int allow_cull) {
-    __shared__ int64_t s_w[8][kPlanThreads / 64 + 1];
+    __shared__ int64_t s_w[4][kPlanThreads / 64 + 1];
     const int j = blockIdx.x * kPlanThreads + threadIdx.x;
-    int64_t add[8];
+    int64_t add[4];
     ChunkMeta m{};
     if (j < n) m = plan_record(A, A.sampler, A.descs[j], allow_cull, add);
     else
-        for (int q = 0; q < 8; q++) add[q] = 0;
-    int64_t excl[8], tot[8];
-    block_scan<8, kPlanThreads>(add, excl, tot, s_w);
+        for (int q = 0; q < 4; q++) add[q] = 0;
+    int64_t excl[4], tot[4];
+    block_scan<4, kPlanThreads>(add, excl, tot, s_w);
     if (j < n) {
         A.tile_prefix[j] = excl[3];
         m.dens_off = excl[0];
         m.lab_off = excl[1];
-        m.row_off = excl[2];
-        if (m.state == kStateSampled) m.plane_slot = pick<8>(excl, 4 + ((m.dim + 63) >> 6) - 1);
+        m.item_slot = excl[2];
         A.meta[j] = m;
     }
-    if (threadIdx.x < 8) A.plan_part[8 * blockIdx.x + threadIdx.x] = tot[threadIdx.x];
+    if (threadIdx.x < 4) A.plan_part[4 * blockIdx.x + threadIdx.x] = pick<4>(tot, (int)threadIdx.x);
 }
 
 // Pass 2 (one block, one thread per pass-1 block, at most kPlanThreads):
 // block bases, batch totals, overflow flag, counters.  Bases go to
-// plan_part[8 (nb + b) ...], the overflow flag after them.
+// plan_part[4 (nb + b) ...], the overflow flag after them.
 __global__ void __launch_bounds__(kPlanThreads) k_plan_total(Arenas A, int n, int nb, int reset_bumps) {
-    __shared__ int64_t s_w[8][kPlanThreads / 64 + 1];
+    __shared__ int64_t s_w[4][kPlanThreads / 64 + 1];
     const int b = threadIdx.x;
-    int64_t v[8];
+    int64_t v[4];
 #pragma unroll
-    for (int q = 0; q < 8; q++) v[q] = b < nb ? A.plan_part[8 * b + q] : 0;
-    int64_t excl[8], tot[8];
-    block_scan<8, kPlanThreads>(v, excl, tot, s_w);
+    for (int q = 0; q < 4; q++) v[q] = b < nb ? A.plan_part[4 * b + q] : 0;
+    int64_t excl[4], tot[4];
+    block_scan<4, kPlanThreads>(v, excl, tot, s_w);
     const bool overflow = plan_overflow(A, tot);
     if (b < nb)
 #pragma unroll
-        for (int q = 0; q < 8; q++) A.plan_part[8 * (nb + b) + q] = excl[q];
+        for (int q = 0; q < 4; q++) A.plan_part[4 * (nb + b) + q] = excl[q];
     if (b == 0) {
-        A.plan_part[16 * nb] = overflow;
-        int64_t cb = 0;
-        for (int q = 0; q < 4; q++) {
-            A.plan_part[16 * nb + 1 + q] = cb;
-            cb += tot[4 + q];
-        }
+        A.plan_part[8 * nb] = overflow;
         plan_counters(A, n, tot, overflow, reset_bumps);
     }
 }
 
-// Pass 3: final offsets, sampling-tile prefixes, plane slots, the results
-// of culled chunks.
+// Pass 3: final offsets, sampling-tile prefixes, the results of culled chunks.
 __global__ void __launch_bounds__(kPlanThreads) k_plan_fix(Arenas A, int n, int nb) {
     const int j = blockIdx.x * kPlanThreads + threadIdx.x;
     if (j >= n) return;
-    int64_t base[8], cbase[4];
+    int64_t base[4];
 #pragma unroll
-    for (int q = 0; q < 8; q++) base[q] = A.plan_part[8 * (nb + blockIdx.x) + q];
-    const bool overflow = A.plan_part[16 * nb] != 0;
-#pragma unroll
-    for (int q = 0; q < 4; q++) cbase[q] = A.plan_part[16 * nb + 1 + q];
+    for (int q = 0; q < 4; q++) base[q] = A.plan_part[4 * (nb + blockIdx.x) + q];
+    const bool overflow = A.plan_part[8 * nb] != 0;
     A.tile_prefix[j] = overflow ? 0 : A.tile_prefix[j] + base[3];
     ChunkMeta m = A.meta[j];
-    plan_finish(A, j, m, base, cbase, overflow);
+    plan_finish(A, j, m, base, overflow);
 }
 
 // ------------------------------------------------------------------------
@@ -369,8 +328,8 @@ __global__ void __launch_bounds__(256) k_csg_cull(Arenas A, int n) {
 // samples are compacted into an LDS queue (wave ballot + popcount) so each
 // octave runs on dense waves.  Samples that run all octaves get their exact
 // density written and their bit set in the `exact` bitmap; the others only
-// get their label (k_count queues the ones that are endpoints of a
-// sign-changing edge and k_refine finishes their densities).  Without
+// get their label (k_count finishes the densities of those that are endpoints of a
+// sign-changing edge).  Without
 // adaptation every
 // sample is evaluated fully (bit-identical values either way).
 // ------------------------------------------------------------------------
@@ -461,12 +420,13 @@ __global__ void __launch_bounds__(kSampleThreads) k_sample(Arenas A, int n) {
     unsigned long long evals = 0;  // adaptive mode: octaves this wave evaluated (wave-uniform)
     __shared__ unsigned long long s_evals;
     if (threadIdx.x == 0) s_evals = 0;  // ordered before its use by the tile loop's barriers
-    // (chunk, x) of every x-plane item of the plane kernels that follow
+    // (chunk, item) of every item of the word kernels that follow
     for (int j = blockIdx.x; j < n; j += gridDim.x) {
         const ChunkMeta& M = A.meta[j];
         if (M.state != kStateSampled) continue;
-        const int64_t ps = M.plane_slot;
-        for (int x = threadIdx.x; x < M.dim; x += blockDim.x) A.plane_map[ps + x] = make_int2(j, x);
+        const int64_t ps = M.item_slot;
+        const int ni = (int)((M.lab_words + kItemWords - 1) / kItemWords);
+        for (int x = threadIdx.x; x < ni; x += blockDim.x) A.item_map[ps + x] = make_int2(j, x);
     }
     for (;;) {
         if (threadIdx.x == 0) {
@@ -692,291 +652,221 @@ __global__ void __launch_bounds__(kSampleThreads) k_sample(Arenas A, int n) {
 }
 
 // ------------------------------------------------------------------------
-// count: one block per (chunk, x-plane, row segment), one wave per label row ->
-// vertices and triangles of each row
+// count: one wave per item of kItemWords label words -> the words' edge and
+// active-cell bits, their edge prefix, and the item's edges (vertices; quads
+// in the quad mode) and cell counts (triangles; polygons in the quad mode).
+// With REFINE it also gives every endpoint of a sign-changing edge that
+// k_sample's adaptive evaluation labelled early its full density.
+//
+// All 64 labels of a word meet their neighbours in a few 64-bit operations,
+// so what is left per sample is done only for the few that the surface
+// meets, compacted into dense lanes (a terrain item of 1,024 samples holds
+// about 40 active cells).  A wave per label row with a lane per sample kept
+// 3 % of its lanes busy: 512 chunks of 64^3 cells, 64 sampled, took 70 us
+// and 23 more for the refinement as a kernel of its own; this takes 45 us.
 // ------------------------------------------------------------------------
-// Staged planes: s_lab[0..2] = labels of x-1, x, x+1; s_lab[3] = exactness
-// of x.  Counts the row's vertices and triangles (in the quad mode its
-// cells' polygons and the quads of its interior sign-changing edges, with
-// s_ntri holding polygons per mask), and queues for k_refine the row's
-// samples that are endpoints of sign-changing edges but were labelled before
-// their last octave (k_sample's adaptive evaluation).
-template <int W>
-__device__ __forceinline__ void count_row(const Arenas& A, const ChunkMeta& M, const uint64_t* const* s_lab,
-                                          const uint8_t* s_ntri, const uint8_t (*s_cls)[BMF_MAX_DIM], int x, int y,
-                                          uint32_t* __restrict__ q, uint32_t* s_qn, uint32_t& nv, uint32_t& nt) {
-    const int dim = M.dim;
-    const int lane = lane_id();
-    const bool x1 = x + 1 < dim, y1 = y + 1 < dim;
-    nv = 0;
-    nt = 0;
-    // a row inside one uniform region (the row, and its neighbours at x-1,
-    // x+1, y-1, y+1, x+1/y+1, all one constant label) has nothing; decided
-    // from the staged rows' classes (0: every label 0, 1: every label 1,
-    // 2: mixed) before any row is read
-    const uint32_t c00 = s_cls[1][y];
-    if (c00 != 2u && (!y1 || s_cls[1][y + 1] == c00) && (!x1 || s_cls[2][y] == c00) &&
-        (!(x1 && y1) || s_cls[2][y + 1] == c00) && (x < 1 || s_cls[0][y] == c00) && (y < 1 || s_cls[1][y - 1] == c00))
-        return;
-    // wave-uniform rows (the same words in every lane); per lane only single bits
-    const RowBits<W> r00 = lds_row<W>(s_lab[1], dim, y, true);
-    const RowBits<W> r01 = lds_row<W>(s_lab[1], dim, y + 1, y1);
-    const RowBits<W> r10 = lds_row<W>(s_lab[2], dim, y, x1);
-    const RowBits<W> r11 = lds_row<W>(s_lab[2], dim, y + 1, x1 && y1);
-    const RowBits<W> rxm = lds_row<W>(s_lab[0], dim, y, x >= 1);
-    const RowBits<W> rym = lds_row<W>(s_lab[1], dim, y - 1, y >= 1);
-    const RowBits<W> ex = rxor<W>(r00, r10, x1), ey = rxor<W>(r00, r01, y1), ez = zedges<W>(r00, dim);
-    const bool quads = A.mesh_mode == BMF_MESH_QUADS;
-    if (quads) {
-        RowBits<W> ix, iy, iz;
-        interior_edges<W>(r00, r01, r10, dim, x, y, ix, iy, iz);
-        nv = 0;
-        nt = (total_pop<W>(ix) + total_pop<W>(iy) + total_pop<W>(iz)) * (A.quad_tris ? 2u : 1u);
-    } else {
-        nv = total_pop<W>(ex) + total_pop<W>(ey) + total_pop<W>(ez);
-    }
-    uint32_t ncell = 0;  // triangles (polygons in the quad mode) of the row's cells
-    if (x < dim - 1 && y < dim - 1 && !quad_uniform<W>(r00, r01, r10, r11, dim)) {
-        const RowBits<W> s00 = rshr1<W>(r00), s01 = rshr1<W>(r01), s10 = rshr1<W>(r10), s11 = rshr1<W>(r11);
-#pragma unroll
-        for (int k = 0; k < W; k++) {
-            if (64 * k >= dim - 1) break;
-            const int z = 64 * k + lane;
-            // corner bit 4 dx + 2 dy + dz
-            const uint32_t c =
-                z < dim - 1 ? s_ntri[lane_bit(r00.w[k], lane) | (lane_bit(s00.w[k], lane) << 1) |
-                                     (lane_bit(r01.w[k], lane) << 2) | (lane_bit(s01.w[k], lane) << 3) |
-                                     (lane_bit(r10.w[k], lane) << 4) | (lane_bit(s10.w[k], lane) << 5) |
-                                     (lane_bit(r11.w[k], lane) << 6) | (lane_bit(s11.w[k], lane) << 7)]
-                            : 0u;
-            ncell += (uint32_t)__popcll(__ballot(c & 1u)) + 2u * (uint32_t)__popcll(__ballot(c & 2u)) +
-                     4u * (uint32_t)__popcll(__ballot(c & 4u));
-        }
-    }
-    if (quads) nv = ncell;
-    else nt = ncell;
-    // endpoints of the sign-changing edges incident to the row's samples
-    RowBits<W> ep = ror<W>(ror<W>(ex, ey), ror<W>(ez, rshl1<W>(ez)));
-    ep = ror<W>(ep, ror<W>(rxor<W>(r00, rxm, x >= 1), rxor<W>(r00, rym, y >= 1)));
-    if (total_pop<W>(ep) == 0) return;
-    const RowBits<W> done = lds_row<W>(s_lab[3], dim, y, true);
-    RowBits<W> need;
-#pragma unroll
-    for (int k = 0; k < W; k++) need.w[k] = ep.w[k] & ~done.w[k];
-    if (total_pop<W>(need) == 0) return;
-    // append them to this plane's region of the refine queue (an LDS counter
-    // per plane, no global atomics); k_refine evaluates them on dense waves.
-    // Bits past the row's last sample are clear, so word k of `need` is the
-    // set of lanes that append.
-    const uint32_t rowbase = (uint32_t)(y * dim);
-#pragma unroll
-    for (int k = 0; k < W; k++) {
-        const uint64_t b = need.w[k];
-        if (!b) continue;
-        uint32_t base = 0;
-        if (lane == 0) base = atomicAdd(s_qn, (uint32_t)__popcll(b));
-        base = __shfl(base, 0);
-        if (lane_bit(b, lane)) q[base + mbcnt64(b)] = rowbase + (uint32_t)(64 * k + lane);
-    }
-}
-
-// ------------------------------------------------------------------------
-// refine: full density of the queued samples (endpoints of sign-changing
-// edges labelled early by k_sample); one block per (x-plane, row segment) queue.
-// ------------------------------------------------------------------------
-__global__ void __launch_bounds__(kSampleThreads) k_refine(Arenas A, int n) {
-    const SamplerDev* __restrict__ S = A.sampler;
-    unsigned long long evals = 0;  // terrain octaves this workgroup evaluated (uniform)
-    for (int cw = 0; cw < 4; cw++) {  // the row-word classes in turn
-        const int split = A.ctr->plane_split[cw];
-        const int64_t base = A.ctr->class_base[cw];
-        const int64_t total = A.ctr->class_planes[cw] * split;
-        for (int64_t it = blockIdx.x; it < total; it += gridDim.x) {
-            const int64_t item = it / split;
-            const int seg = (int)(it - item * split);
-            const uint32_t cnt = A.plane_refine_n[(base + item) * kMaxPlaneSplit + seg];
-            if (cnt == 0) continue;
-            const int2 pm = A.plane_map[base + item];
-            const ChunkMeta M = read_chunk(A.meta, pm.x);
-            const uint32_t dim = (uint32_t)M.dim;
-            const uint32_t x = (uint32_t)uniform_int(pm.y);
-            const uint32_t y0 = (uint32_t)((int64_t)seg * dim / split);
-            const uint32_t* __restrict__ q = A.refine + M.dens_off + (int64_t)x * dim * dim + (int64_t)y0 * dim;
-            float* __restrict__ D = A.dens + M.dens_off + (int64_t)x * dim * dim;
-            const float px = (float)x * M.delta + M.opos[0];
-            if (S->kind == BMF_SAMPLER_TERRAIN) evals += (unsigned long long)cnt * (unsigned long long)S->octaves;
-            for (uint32_t e = threadIdx.x; e < cnt; e += blockDim.x) {
-                const uint32_t r = q[e];  // y * dim + z within the plane
-                const uint32_t y = r / dim, z = r - y * dim;
-                const float py = (float)y * M.delta + M.opos[1];
-                const float pz = (float)z * M.delta + M.opos[2];
-                D[r] = sample_density(*S, px, py, pz);
-            }
-        }
-    }
-    if (threadIdx.x == 0 && (int)blockIdx.x < A.stat_cap) A.stat_blocks[A.stat_cap + blockIdx.x] = evals;
-}
-
-// Instantiated per row-word class W = ceil(dim/64); blocks of other classes
-// skip their items (the host launches only the classes present).
-template <int W>
-__global__ void __launch_bounds__(kRowThreads) k_count(Arenas A, int n) {
-    __shared__ uint8_t s_ntri[256];
-    __shared__ uint64_t s_planes[4][plane_words(W)];
-    const uint64_t* const s_lab[4] = {s_planes[0], s_planes[1], s_planes[2], s_planes[3]};
-    __shared__ uint8_t s_cls[3][BMF_MAX_DIM];  // rows of the staged label planes: 0 / 1 every label 0 / 1, 2 mixed
-    __shared__ uint32_t s_qn;
+template <bool REFINE>
+__global__ void __launch_bounds__(kRowThreads) k_count(Arenas A) {
+    __shared__ uint8_t s_n[256];  // triangles (polygons in the quad mode) of each corner mask
+    __shared__ uint64_t s_corner[kWordWaves][kItemWords][8];
+    __shared__ uint16_t s_list[kWordWaves][kItemSamples];
+    __shared__ unsigned long long s_evals;
     const bool quads = A.mesh_mode == BMF_MESH_QUADS;
     for (int t = threadIdx.x; t < 256; t += blockDim.x)
-        s_ntri[t] = (uint8_t)(quads ? dmc_polygons(c_dmc_table[t]) : (uint32_t)((c_tri_table[t] >> 60) / 3));
-    const int wave = uniform_int(threadIdx.x >> 6);
-    const int lane = lane_id();
-    const int split = A.ctr->plane_split[W - 1];
-    const int64_t base = A.ctr->class_base[W - 1];
-    const int64_t total = A.ctr->class_planes[W - 1] * split;
-    for (int64_t it = blockIdx.x; it < total; it += gridDim.x) {
-        const int64_t item = it / split;
-        const int seg = (int)(it - item * split);
-        const int2 pm = A.plane_map[base + item];
-        const ChunkMeta M = read_chunk(A.meta, pm.x);
-        const int dim = M.dim;
-        const int x = uniform_int(pm.y);
-        const int64_t qslot = (base + item) * kMaxPlaneSplit + seg;  // this segment's refine-queue count
-        const int y0 = (int)((int64_t)seg * dim / split), y1 = (int)((int64_t)(seg + 1) * dim / split);
-        uint32_t* rv = A.row_v + M.row_off + (int64_t)x * dim;
-        uint32_t* rt = A.row_t + M.row_off + (int64_t)x * dim;
-        if (!(M.any_air && M.any_solid)) {  // no surface in this chunk
-            for (int y = y0 + threadIdx.x; y < y1; y += blockDim.x) rv[y] = rt[y] = 0u;
-            if (threadIdx.x == 0) A.plane_refine_n[qslot] = 0;
+        s_n[t] = (uint8_t)(quads ? dmc_polygons(c_dmc_table[t]) : (uint32_t)((c_tri_table[t] >> 60) / 3));
+    if (threadIdx.x == 0) s_evals = 0;
+    __syncthreads();
+    const SamplerDev* __restrict__ S = A.sampler;
+    const int wave = uniform_int(threadIdx.x >> 6), lane = lane_id(), q = lane & 3;
+    uint16_t* const list = s_list[wave];
+    unsigned long long evals = 0;  // octaves of this wave's refined samples (uniform)
+    const int64_t total = A.ctr->total_items;
+    for (int64_t it = (int64_t)blockIdx.x * kWordWaves + wave; it < total; it += (int64_t)gridDim.x * kWordWaves) {
+        const ItemRef R = item_ref(A, it);
+        const ChunkMeta& M = R.M;
+        if (!(M.any_air && M.any_solid)) {  // no surface in this chunk: nothing reads its words
+            if (lane == 0) A.item_e[it] = A.item_c[it] = 0u;
             continue;
         }
-        __syncthreads();  // previous item is done with the shared arrays
-        if (threadIdx.x == 0) s_qn = 0;
-        {
-            // label planes x-1, x, x+1 and the exact-sample plane x
-            uint64_t* const dst[4] = {s_planes[0], s_planes[1], s_planes[2], s_planes[3]};
-            const uint64_t* const src[4] = {A.labels + M.lab_off, A.labels + M.lab_off, A.labels + M.lab_off,
-                                            A.exact + M.lab_off};
-            const int xp[4] = {x - 1, x, x + 1, x};
-            stage_plane_group<4>(dst, src, M.lab_words, dim, xp);
+        const int dim = M.dim, d2 = dim * dim, nw = (int)M.lab_words;
+        const int w = R.w0 + (lane >> 2);
+        const uint64_t* __restrict__ L = A.labels + M.lab_off;
+        uint64_t c[8];
+        moved_labels(L, nw, w, 0, c[0], c[1]);
+        moved_labels(L, nw, w, dim, c[2], c[3]);
+        moved_labels(L, nw, w, d2, c[4], c[5]);
+        moved_labels(L, nw, w, d2 + dim, c[6], c[7]);
+        uint64_t lz = c[0], ly = c[0], lx = c[0];  // the neighbours below, for the refinement
+        if constexpr (REFINE) {
+            uint64_t unused;
+            moved_labels(L, nw, w, -1, lz, unused);
+            moved_labels(L, nw, w, -dim, ly, unused);
+            moved_labels(L, nw, w, -d2, lx, unused);
         }
-        __syncthreads();
-        // class of every staged label row, one thread per row
-        for (int t = threadIdx.x; t < 3 * dim; t += blockDim.x) {
-            const int p = t / dim, y = t - p * dim;
-            const uint64_t* P = s_planes[p];
-            bool any1 = false, any0 = false;
+        uint64_t diff = 0;
 #pragma unroll
-            for (int k = 0; k < W; k++) {
-                const int bit = y * dim + 64 * k, w = bit >> 6, sh = bit & 63;
-                uint64_t v = (P[w] >> sh) | ((P[w + 1] << 1) << (63 - sh));  // the pad word keeps w + 1 in bounds
-                const int nb = dim - 64 * k;
-                const uint64_t m = nb >= 64 ? ~0ull : ((1ull << nb) - 1ull);
-                v &= m;
-                any1 = any1 || v != 0ull;
-                any0 = any0 || v != m;
+        for (int k = 1; k < 8; k++) diff |= c[0] ^ c[k];
+        uint64_t field = 0ull;  // lane q of a word's four keeps its field q
+        uint32_t ne = 0u, nc = 0u;
+        // items inside one uniform region end here (labels past the bitmap
+        // and across row ends only cost the shortcut)
+        if (__any((diff | (c[0] ^ lz) | (c[0] ^ ly) | (c[0] ^ lx)) != 0ull)) {
+            const WordFaces f = word_faces(64 * w, dim, row_period(dim));
+            uint64_t ex = (c[0] ^ c[4]) & f.in & ~f.x1, ey = (c[0] ^ c[2]) & f.in & ~f.y1,
+                     ez = (c[0] ^ c[1]) & f.in & ~f.z1;
+            const uint64_t ac = diff & f.in & ~(f.x1 | f.y1 | f.z1);
+            uint64_t need = 0ull;
+            if constexpr (REFINE) {
+                const uint64_t ep = ex | ey | ez | ((c[0] ^ lz) & ~f.z0) | ((c[0] ^ ly) & ~f.y0) | ((c[0] ^ lx) & ~f.x0);
+                need = ep & f.in & ~(w < nw ? A.exact[M.lab_off + w] : 0ull);
             }
-            s_cls[p][y] = (uint8_t)(any1 ? (any0 ? 2 : 1) : 0);
-        }
-        __syncthreads();
-        // this segment's region of the plane's refine queue: its rows' samples
-        uint32_t* q = A.refine + M.dens_off + (int64_t)x * dim * dim + (int64_t)y0 * dim;
-        for (int y = y0 + wave; y < y1; y += kRowThreads / 64) {
-            uint32_t nv = 0, nt = 0;
-            count_row<W>(A, M, s_lab, s_ntri, s_cls, x, y, q, &s_qn, nv, nt);
-            if (lane == 0) {
-                rv[y] = nv;
-                rt[y] = nt;
+            if (quads) {  // only the edges whose four cells lie in the chunk carry a quad
+                const uint64_t x = f.x0 | f.x1, y = f.y0 | f.y1, z = f.z0 | f.z1;
+                ex &= ~(y | z);
+                ey &= ~(x | z);
+                ez &= ~(x | y);
             }
+            field = q == 0 ? ex : (q == 1 ? ey : (q == 2 ? ez : ac));
+            // edges before each word within the item
+            const uint32_t pre = wave_prefix<8>(
+                q == 0 ? (uint32_t)(__popcll(ex) + __popcll(ey) + __popcll(ez)) : 0u, ne);
+            if (q == 0 && w < nw) A.word_pre[M.lab_off + w] = pre;
+            // cells
+            s_corner[wave][lane >> 2][2 * q] = q == 0 ? c[0] : (q == 1 ? c[2] : (q == 2 ? c[4] : c[6]));
+            s_corner[wave][lane >> 2][2 * q + 1] = q == 0 ? c[1] : (q == 1 ? c[3] : (q == 2 ? c[5] : c[7]));
+            const int ncell = push_bits(ac, list);
+            wave_sync();
+            for (int e0 = 0; e0 < ncell; e0 += 64) {
+                uint32_t n = 0;
+                if (e0 + lane < ncell) {
+                    const uint32_t pos = list[e0 + lane];
+                    const uint32_t* cw = reinterpret_cast<const uint32_t*>(s_corner[wave][pos >> 6]) + ((pos >> 5) & 1u);
+                    uint32_t mask = 0;
+#pragma unroll
+                    for (int k = 0; k < 8; k++) mask |= ((cw[2 * k] >> (pos & 31u)) & 1u) << k;
+                    n = s_n[mask];
+                }
+                nc += (uint32_t)__popcll(__ballot(n & 1u)) + 2u * (uint32_t)__popcll(__ballot(n & 2u)) +
+                      4u * (uint32_t)__popcll(__ballot(n & 4u));
+            }
+            if constexpr (REFINE) {
+                wave_sync();  // the cells are read
+                const int nq = push_bits(need, list);
+                wave_sync();
+                evals += (unsigned long long)nq * (unsigned long long)S->octaves;
+                const float rd = 1.0f / (float)dim, rd2 = 1.0f / (float)d2;
+                for (int e = lane; e < nq; e += 64) {
+                    const uint32_t i = 64u * (uint32_t)R.w0 + list[e];
+                    const uint32_t x = udiv24(i, (uint32_t)d2, rd2), r = i - x * (uint32_t)d2;
+                    const uint32_t y = udiv24(r, (uint32_t)dim, rd), z = r - y * (uint32_t)dim;
+                    const float px = (float)x * M.delta + M.opos[0], py = (float)y * M.delta + M.opos[1],
+                                pz = (float)z * M.delta + M.opos[2];
+                    A.dens[M.dens_off + i] = terrain_density(*S, px, py, pz);
+                }
+            }
+            wave_sync();  // the next item reuses the list and the corners
+        } else if (q == 0 && w < nw) {
+            A.word_pre[M.lab_off + w] = 0u;
         }
-        __syncthreads();
-        if (threadIdx.x == 0) A.plane_refine_n[qslot] = s_qn;
+        if (w < nw) reinterpret_cast<uint64_t*>(A.edges + M.lab_off + w)[q] = field;
+        if (lane == 0) {
+            A.item_e[it] = ne;
+            A.item_c[it] = nc;
+        }
     }
+    if constexpr (REFINE) {
+        if (lane == 0 && evals) atomicAdd(&s_evals, evals);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0 && (int)blockIdx.x < A.stat_cap) A.stat_blocks[A.stat_cap + blockIdx.x] = s_evals;
 }
 
 // ------------------------------------------------------------------------
-// scan: one block per chunk -> row bases, totals, output reservation
+// scan: one block per chunk -> item bases, totals, output reservation
 // ------------------------------------------------------------------------
-constexpr int kScanThreads = 1024;
+constexpr int kScanThreads = 256;
 
 __global__ void __launch_bounds__(kScanThreads) k_scan(Arenas A, int n) {
     constexpr int NW = kScanThreads / 64;
-    __shared__ uint32_t s_wv[NW], s_wt[NW];  // wave totals
+    __shared__ uint32_t s_we[NW], s_wc[NW];  // wave totals
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     for (int j = blockIdx.x; j < n; j += gridDim.x) {
         ChunkMeta& M = A.meta[j];
         if (M.state != kStateSampled) continue;
         const int dim = M.dim;
-        const int64_t R = (int64_t)dim * dim;
-        uint32_t* rv = A.row_v + M.row_off;
-        uint32_t* rt = A.row_t + M.row_off;
-        // exclusive scan of the rows: each wave scans a contiguous run of
-        // 64-row tiles (coalesced, wave shuffles, a running carry; four tiles'
+        const int64_t R = (M.lab_words + kItemWords - 1) / kItemWords;
+        uint32_t* re = A.item_e + M.item_slot;
+        uint32_t* rc = A.item_c + M.item_slot;
+        // exclusive scan of the items: each wave scans a contiguous run of
+        // 64-item tiles (coalesced, wave shuffles, a running carry; four tiles'
         // loads issued together), then one exchange of the wave totals and a
         // second pass that adds each wave's base
         const int64_t ntile = (R + 63) / 64;
         const int64_t tpw = (ntile + NW - 1) / NW;
         const int64_t t0 = (int64_t)wave * tpw, t1 = t0 + tpw < ntile ? t0 + tpw : ntile;
-        uint32_t wv = 0, wt = 0;  // running totals of this wave's run
+        uint32_t we = 0, wc = 0;  // running totals of this wave's run
         for (int64_t tg = t0; tg < t1; tg += 4) {
-            uint32_t av[4], at[4];
+            uint32_t ae[4], ac[4];
 #pragma unroll
             for (int k = 0; k < 4; k++) {
                 const int64_t r = (tg + k) * 64 + lane;
                 const bool in = tg + k < t1 && r < R;
-                av[k] = in ? rv[r] : 0u;
-                at[k] = in ? rt[r] : 0u;
+                ae[k] = in ? re[r] : 0u;
+                ac[k] = in ? rc[r] : 0u;
             }
 #pragma unroll
             for (int k = 0; k < 4; k++) {
-                uint32_t sv = av[k], sw = at[k];
+                if (tg + k >= t1) break;
+                uint32_t se = ae[k], sc = ac[k];
 #pragma unroll
                 for (int off = 1; off < 64; off <<= 1) {
-                    const uint32_t uv = __shfl_up(sv, off), ut = __shfl_up(sw, off);
+                    const uint32_t ue = __shfl_up(se, off), uc = __shfl_up(sc, off);
                     if (lane >= off) {
-                        sv += uv;
-                        sw += ut;
+                        se += ue;
+                        sc += uc;
                     }
                 }
                 const int64_t r = (tg + k) * 64 + lane;
-                if (tg + k < t1 && r < R) {
-                    rv[r] = wv + sv - av[k];
-                    rt[r] = wt + sw - at[k];
+                if (r < R) {
+                    re[r] = we + se - ae[k];
+                    rc[r] = wc + sc - ac[k];
                 }
-                wv += (uint32_t)__shfl(sv, 63);
-                wt += (uint32_t)__shfl(sw, 63);
+                we += (uint32_t)__shfl(se, 63);
+                wc += (uint32_t)__shfl(sc, 63);
             }
         }
         if (lane == 0) {
-            s_wv[wave] = wv;
-            s_wt[wave] = wt;
+            s_we[wave] = we;
+            s_wc[wave] = wc;
         }
         __syncthreads();
-        uint32_t bv = 0, bt = 0, cv = 0, ct = 0;
+        uint32_t be = 0, bc = 0, te = 0, tc = 0;
 #pragma unroll
         for (int w = 0; w < NW; w++) {
-            const uint32_t xv = s_wv[w], xt = s_wt[w];
+            const uint32_t xe = s_we[w], xc = s_wc[w];
             if (w < wave) {
-                bv += xv;
-                bt += xt;
+                be += xe;
+                bc += xc;
             }
-            cv += xv;
-            ct += xt;
+            te += xe;
+            tc += xc;
         }
-        if (bv | bt)
+        if (be | bc)
             for (int64_t t = t0; t < t1; t++) {
                 const int64_t r = t * 64 + lane;
                 if (r < R) {
-                    rv[r] += bv;
-                    rt[r] += bt;
+                    re[r] += be;
+                    rc[r] += bc;
                 }
             }
         if (tid == 0) {
-            const uint32_t V = cv, T = ct;
+            // triangles: a vertex per edge; quads: a vertex per polygon, a
+            // quad (or two triangles) per edge
+            const bool quads = A.mesh_mode == BMF_MESH_QUADS;
+            const uint32_t V = quads ? tc : te, T = quads ? te * (A.quad_tris ? 2u : 1u) : tc;
             M.V = (int32_t)V;
             M.T = (int32_t)T;
             M.contains_mesh = M.any_air && (M.any_solid || (dim % 32 != 0));
-            int ok = 1;
             if (V > 0) {
                 const int64_t vo = (int64_t)atomicAdd(&A.ctr->v_bump, (unsigned long long)V);
                 const uint64_t ni = (uint64_t)M.ipp * T;
@@ -984,14 +874,12 @@ __global__ void __launch_bounds__(kScanThreads) k_scan(Arenas A, int n) {
                 atomicAdd(&A.ctr->need_v, (unsigned long long)V);
                 atomicAdd(&A.ctr->need_i, (unsigned long long)ni);
                 if (vo + V > A.cap_vertices || io + (int64_t)ni > A.cap_indices) {
-                    ok = 0;
                     M.status = BMF_ECAPACITY;
                     A.ctr->overflow = 1;
                 }
                 M.v_off = vo;
                 M.i_off = io;
             }
-            (void)ok;
             write_result(A, j, M);
         }
         __syncthreads();
@@ -1193,20 +1081,19 @@ __global__ void __launch_bounds__(kPlanThreads) k_smooth_prefix(Arenas A, int n,
 }
 
 // ------------------------------------------------------------------------
-// emit: one block per (chunk, x-plane, row segment), lanes = z, in slabs of
-// at most kEmitRows label rows:
-//  pass 1, one wave per row of planes x and x+1 (rows y0 .. y0 + kEmitRows):
-//    the first vertex id of every sample (row base + popcount prefix over
-//    the row's x, y and z edge masks) with its x- and y-edge bits, into an
-//    LDS table; rows of plane x owned by the slab also write their vertices.
-//  pass 2, one wave per cell row: the triangles of the row's interior cells
-//    (ids by a bit-sliced ballot prefix of the per-cell triangle counts),
-//    their corner vertex ids looked up in the table, and for chunks that
-//    smooth the per-cell triangle base and mask.
+// emit: one wave per item of kItemWords label words.  The label and edge
+// words around the item are staged in the wave's LDS windows; the samples
+// that own sign-changing edges and the active cells are compacted, and dense
+// lanes write them: a lane per sample places its up to three vertices, a
+// lane per cell writes its up to five triangles, each corner's vertex id a
+// prefix popcount of its word.  For chunks that smooth the cell's first
+// triangle and mask are kept.
+//
+// Bound by the latency of an item's chain (map, record, windows, densities,
+// stores), hidden by the waves in flight: 512 chunks of 64^3 cells, 719,423
+// vertices and 1,406,794 triangles (29 MB written), took 126 us with a wave
+// per row of samples and 3 % of its lanes busy; this takes 42 us.
 // ------------------------------------------------------------------------
-constexpr int kEmitRows = 16;
-static_assert((kEmitRows + 1) * 3 * BMF_MAX_DIM < (1 << 14), "a slab's vertex ids fit the 14-bit offsets of the id table");
-
 // Local edge e of a cell (the 12-edge numbering of DMCChunk.cpp:543-565):
 // x-edges e = 2 dy + dz, y-edges e = 4 + 2 dx + dz, z-edges e = 8 + 2 dx + dy,
 // the edge of axis `ax` starting at corner (dx, dy, dz); 5 bits per edge,
@@ -1223,239 +1110,148 @@ __host__ __device__ constexpr uint64_t edge_corner_table() {
 }
 constexpr uint64_t kEdgeCorners = edge_corner_table();
 
-// The same per edge, as emit's pass 2 uses it: the edge's id-table entry
-// relative to the cell's own (plane dx, row + dy, column + dz of the
-// [2][kEmitRows + 1][64 W] table) in bits 16-31, the entry's x- and y-edge
-// bits that precede the edge's vertex among its sample's (bits 14 and 15:
-// none for an x-edge, the x-edge for a y-edge, both for a z-edge), the
-// plane in bit 0.
-template <int W>
-__host__ __device__ constexpr uint32_t edge_decode(int e) {
-    const uint32_t g = (uint32_t)(kEdgeCorners >> (5 * e)) & 31u;
-    const uint32_t dx = g & 1u, dy = (g >> 1) & 1u, dz = (g >> 2) & 1u, ax = g >> 3;
-    const uint32_t off = dx * (uint32_t)((kEmitRows + 1) * 64 * W) + dy * (uint32_t)(64 * W) + dz;
-    return (off << 16) | (ax >= 1 ? 0x4000u : 0u) | (ax == 2 ? 0x8000u : 0u) | dx;
-}
-
-// Pass 1 for label row (x + p, y): vertex ids into s_id, and for p == 0 with
-// `own` the vertices themselves (DMCChunk::calculate_isovertex, DMCChunk.cpp:
-// 657-674; vertices of a sample in x, y, z edge order).  The row masks are
-// wave-uniform (scalar registers); per lane only the bit and the count of
-// set bits below it are taken.
-template <int W>
-__device__ __forceinline__ void emit_ids_row(const Arenas& A, const ChunkMeta& M,
-                                             const uint64_t (*s_lab)[plane_words(W)], uint32_t base,
-                                             uint16_t* s_idrow, uint32_t slab_base, int x, int p, int y, bool own) {
-    const int dim = M.dim;
-    const int lane = lane_id();
-    const int xp = x + p;
-    const bool vx = xp + 1 < dim, vy = y + 1 < dim;
-    const RowBits<W> R0 = uniform_row<W>(lds_row<W>(s_lab[p], dim, y, true));
-    const RowBits<W> EX = rxor<W>(R0, uniform_row<W>(lds_row<W>(s_lab[p + 1], dim, y, vx)), vx);
-    const RowBits<W> EY = rxor<W>(R0, uniform_row<W>(lds_row<W>(s_lab[p], dim, y + 1, vy)), vy);
-    const RowBits<W> EZ = zedges<W>(R0, dim);
+// The vertices of the item's samples (DMCChunk::calculate_isovertex,
+// DMCChunk.cpp:657-674; a sample's in x, y, z edge order).
+__device__ __forceinline__ void emit_vertices(const Arenas& A, const ChunkMeta& M, ItemWindows& s, int w0) {
+    const int lane = lane_id(), k4 = lane >> 2, dim = M.dim, d2 = dim * dim;
+    const int ns = push_bits(s.ex[k4] | s.ey[k4] | s.ez[k4], s.list);
+    wave_sync();
     const int64_t vo = M.v_off;
     const uint32_t Vc = (uint32_t)M.V;
-    float* __restrict__ P = A.pos + vo * 3;
     const bool cells = M.iters > 0 || A.normals;  // the chunk runs the smoothing kernels
     // with K > 0 the last primal step writes the output position of every
     // vertex it moves (every vertex has a ring; boundary vertices move only
     // with boundary processing), so only the others are written here
     const bool moves = M.iters > 0 && A.smoothing_follows;
     const bool moves_boundary = moves && M.bp;
+    float* __restrict__ P = A.pos + vo * 3;
     float4* __restrict__ P4 = cells ? A.pos4 + vo : nullptr;  // smoothing state
     float4* __restrict__ N4 = cells && A.normals ? A.nrm4 + vo : nullptr;
     uint8_t* __restrict__ B = A.boundary + vo;
     uint32_t* __restrict__ E = A.vedge + vo;
     const float* __restrict__ D = A.dens + M.dens_off;
-    uint32_t kb = base;  // id of the first vertex of word k's samples
-#pragma unroll
-    for (int k = 0; k < W; k++) {
-        const uint64_t ex = EX.w[k], ey = EY.w[k], ez = EZ.w[k];
-        const int z = 64 * k + lane;
-        if (z < dim) {
-            const uint32_t fx = lane_bit_u(ex), fy = lane_bit_u(ey), fz = lane_bit_u(ez);
-            uint32_t id = kb + mbcnt64(ex) + mbcnt64(ey) + mbcnt64(ez);
-            s_idrow[z] = (uint16_t)((id - slab_base) | (fx << 14) | (fy << 15));
-            if (own && (fx | fy | fz)) {
-                // the sample and the far ends of its edges load together (an
-                // edge that is not set reads the sample again)
-                const int64_t b = ((int64_t)x * dim + y) * dim + z;
-                const float s0 = D[b];
-                const float e1[3] = {D[fx ? b + (int64_t)dim * dim : b], D[fy ? b + dim : b], D[fz ? b + 1 : b]};
-                const bool fits = id + fx + fy + fz <= Vc;
-                if (!fits) A.ctr->error = 2;  // counts and ids disagree: report, never write past the chunk
-#pragma unroll
-                for (int ax = 0; ax < 3; ax++) {
-                    const uint32_t f = ax == 0 ? fx : (ax == 1 ? fy : fz);
-                    if (!f || !fits) continue;
-                    const int xe = x + (ax == 0), ye = y + (ax == 1), ze = z + (ax == 2);
-                    const float s1 = e1[ax];
-                    const float mu = (0.0f - s0) / (s1 - s0);
-                    const float dx = (float)xe - (float)x, dy = (float)ye - (float)y, dz = (float)ze - (float)z;
-                    const float qx = dx * mu + (float)x, qy = dy * mu + (float)y, qz = dz * mu + (float)z;
-                    const bool bnd = x == 0 || y == 0 || z == 0 || x == dim - 1 || y == dim - 1 || z == dim - 1 ||
-                                     xe == dim - 1 || ye == dim - 1 || ze == dim - 1;
-                    if (!(bnd ? moves_boundary : moves)) {
-                        P[3 * (int64_t)id + 0] = qx;
-                        P[3 * (int64_t)id + 1] = qy;
-                        P[3 * (int64_t)id + 2] = qz;
-                    }
-                    if (P4) P4[id] = make_float4(qx, qy, qz, 0.0f);
-                    if (N4) N4[id] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                    B[id] = (uint8_t)bnd;
-                    E[id] = (uint32_t)x | ((uint32_t)y << 8) | ((uint32_t)z << 16) | ((uint32_t)ax << 24);
-                    id++;
-                }
-            }
+    const float rd = 1.0f / (float)dim, rd2 = 1.0f / (float)d2;
+    for (int e = lane; e < ns; e += 64) {
+        const int pos = s.list[e], w = pos >> 6;
+        const uint64_t bit = 1ull << (pos & 63), lt = bit - 1ull;
+        const uint64_t ex = s.ex[w], ey = s.ey[w], ez = s.ez[w];
+        const uint32_t fx = (ex & bit) != 0ull, fy = (ey & bit) != 0ull, fz = (ez & bit) != 0ull;
+        uint32_t id = s.pre[w] + (uint32_t)(__popcll(ex & lt) + __popcll(ey & lt) + __popcll(ez & lt));
+        // the sample and the far ends of its edges load together (an edge
+        // that is not set reads the sample again)
+        const uint32_t i = 64u * (uint32_t)w0 + (uint32_t)pos;
+        const float s0 = D[i];
+        const float e1[3] = {D[fx ? i + (uint32_t)d2 : i], D[fy ? i + (uint32_t)dim : i], D[fz ? i + 1u : i]};
+        const int x = (int)udiv24(i, (uint32_t)d2, rd2), r = (int)i - x * d2;
+        const int y = (int)udiv24((uint32_t)r, (uint32_t)dim, rd), z = r - y * dim;
+        if (id + fx + fy + fz > Vc) {
+            A.ctr->error = 2;  // counts and ids disagree: report, never write past the chunk
+            continue;
         }
-        kb += (uint32_t)(__popcll(ex) + __popcll(ey) + __popcll(ez));
+#pragma unroll
+        for (int ax = 0; ax < 3; ax++) {
+            const uint32_t f = ax == 0 ? fx : (ax == 1 ? fy : fz);
+            if (!f) continue;
+            const int xe = x + (ax == 0), ye = y + (ax == 1), ze = z + (ax == 2);
+            const float s1 = e1[ax];
+            const float mu = (0.0f - s0) / (s1 - s0);
+            const float dx = (float)xe - (float)x, dy = (float)ye - (float)y, dz = (float)ze - (float)z;
+            const float qx = dx * mu + (float)x, qy = dy * mu + (float)y, qz = dz * mu + (float)z;
+            const bool bnd = x == 0 || y == 0 || z == 0 || x == dim - 1 || y == dim - 1 || z == dim - 1 ||
+                             xe == dim - 1 || ye == dim - 1 || ze == dim - 1;
+            if (!(bnd ? moves_boundary : moves)) {
+                P[3 * (int64_t)id + 0] = qx;
+                P[3 * (int64_t)id + 1] = qy;
+                P[3 * (int64_t)id + 2] = qz;
+            }
+            if (P4) P4[id] = make_float4(qx, qy, qz, 0.0f);
+            if (N4) N4[id] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            B[id] = (uint8_t)bnd;
+            E[id] = (uint32_t)x | ((uint32_t)y << 8) | ((uint32_t)z << 16) | ((uint32_t)ax << 24);
+            id++;
+        }
     }
 }
 
-// Pass 2 for cell row (x, y); s_id rows start at label row ys.
-template <int W>
-__device__ __forceinline__ void emit_tris_row(const Arenas& A, const ChunkMeta& M,
-                                              const uint64_t (*s_lab)[plane_words(W)], const uint8_t* s_ntri,
-                                              const uint64_t* s_tri, const uint32_t* s_edge, uint32_t tcarry,
-                                              const uint16_t (*s_id)[kEmitRows + 1][64 * W], uint32_t slab0,
-                                              uint32_t slab1, int x, int y, int ys) {
-    const int dim = M.dim;
-    const int lane = lane_id();
-    // corner rows of the cell row, and the same shifted by one sample (z + 1)
-    const RowBits<W> R00 = uniform_row<W>(lds_row<W>(s_lab[0], dim, y, true));
-    const RowBits<W> R01 = uniform_row<W>(lds_row<W>(s_lab[0], dim, y + 1, true));
-    const RowBits<W> R10 = uniform_row<W>(lds_row<W>(s_lab[1], dim, y, true));
-    const RowBits<W> R11 = uniform_row<W>(lds_row<W>(s_lab[1], dim, y + 1, true));
-    const RowBits<W> S00 = rshr1<W>(R00), S01 = rshr1<W>(R01), S10 = rshr1<W>(R10), S11 = rshr1<W>(R11);
-    const int64_t io = M.i_off;
+// The triangles of the item's active cells, `tbase` before them.
+__device__ __forceinline__ void emit_triangles(const Arenas& A, const ChunkMeta& M, ItemWindows& s,
+                                               const WindowGeom& g, const uint8_t* s_ntri, const uint64_t* s_tri,
+                                               int w0, uint32_t tbase) {
+    const int lane = lane_id(), dim = M.dim;
+    const int nc = push_bits(s.ac[lane >> 2], s.list);
+    wave_sync();
     const uint32_t Vc = (uint32_t)M.V, Tc = (uint32_t)M.T;
     const bool cells = M.iters > 0 || A.normals;
-#pragma unroll
-    for (int k = 0; k < W; k++) {
-        if (64 * k >= dim - 1) break;
-        const int z = 64 * k + lane;
-        // corner bit 4 dx + 2 dy + dz (DMCChunk.cpp:200-438)
-        const uint32_t mask =
-            z < dim - 1 ? lane_bit_u(R00.w[k]) | (lane_bit_u(S00.w[k]) << 1) | (lane_bit_u(R01.w[k]) << 2) |
-                              (lane_bit_u(S01.w[k]) << 3) | (lane_bit_u(R10.w[k]) << 4) |
-                              (lane_bit_u(S10.w[k]) << 5) | (lane_bit_u(R11.w[k]) << 6) |
-                              (lane_bit_u(S11.w[k]) << 7)
-                        : 0u;
-        const uint32_t nt = s_ntri[mask];
-        const uint64_t b0 = __ballot(nt & 1u), b1 = __ballot(nt & 2u), b2 = __ballot(nt & 4u);
-        if (nt) {
-            const uint32_t tb = tcarry + mbcnt64(b0) + 2u * mbcnt64(b1) + 4u * mbcnt64(b2);
-            const uint64_t row = s_tri[mask];
-            if (tb + nt > Tc) {
-                A.ctr->error = 3;
-            } else {
-                // per triangle: the three corner ids read together, written
-                // together; an id past the chunk's vertices (counts and ids
-                // disagree) is reported, its slot is inside the chunk's range
-                uint32_t* __restrict__ I = A.idx + io + 3ll * tb;
-                bool bad = false;
-                // the cell's own entry of the id table; a corner's entry is
-                // its edge's offset from it (edge_decode)
-                const uint16_t* __restrict__ cid = &s_id[0][0][0] + (y - ys) * (64 * W) + z;
-                const uint32_t sdiff = slab1 - slab0;
-                // at most 5 triangles per cell: unrolled, so each slot's table
-                // bits are a constant field of the row
-#pragma unroll
-                for (int q = 0; q < 5; q++) {
-                    if (q >= (int)nt) break;
-                    uint32_t v[3];
-#pragma unroll
-                    for (int c = 0; c < 3; c++) {
-                        const int sl = 3 * q + c;
-                        const uint32_t d = s_edge[(uint32_t)(row >> (4 * sl)) & 15u];
-                        const uint32_t e = cid[d >> 16];
-                        v[c] = slab0 + (d & 1u) * sdiff + (e & 0x3FFFu) + (uint32_t)__popc(e & d & 0xC000u);
-                        bad = bad || v[c] >= Vc;
-                    }
-                    I[3 * q] = v[0];
-                    I[3 * q + 1] = v[1];
-                    I[3 * q + 2] = v[2];
-                }
-                if (bad) A.ctr->error = 4;
-                if (cells) {
-                    const int64_t ci = M.dens_off + ((int64_t)x * dim + y) * dim + z;
-                    A.cell_tb[ci] = tb;
-                    A.cell_mask[ci] = (uint8_t)mask;
-                }
-            }
+    for (int e0 = 0; e0 < nc; e0 += 64) {
+        int pos = 0;
+        uint32_t mask = 0, nt = 0;
+        if (e0 + lane < nc) {
+            pos = s.list[e0 + lane];
+            mask = window_mask(s, g, dim, pos);
+            nt = s_ntri[mask];
         }
-        tcarry += (uint32_t)__popcll(b0) + 2u * (uint32_t)__popcll(b1) + 4u * (uint32_t)__popcll(b2);
+        uint32_t round;
+        const uint32_t tb = tbase + wave_prefix<3>(nt, round);
+        tbase += round;
+        if (!nt) continue;
+        if (tb + nt > Tc) {
+            A.ctr->error = 3;
+            continue;
+        }
+        const uint64_t row = s_tri[mask];
+        // per triangle: the three corner ids read together, written
+        // together; an id past the chunk's vertices (counts and ids
+        // disagree) is reported, its slot is inside the chunk's range
+        uint32_t* __restrict__ I = A.idx + M.i_off + 3ll * tb;
+        bool bad = false;
+        // at most 5 triangles per cell: unrolled, so each slot's table bits
+        // are a constant field of the row
+#pragma unroll
+        for (int q = 0; q < 5; q++) {
+            if (q >= (int)nt) break;
+            uint32_t v[3];
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                const uint32_t le = (uint32_t)(row >> (4 * (3 * q + c))) & 15u;
+                const uint32_t code = (uint32_t)(kEdgeCorners >> (5u * le)) & 31u;
+                v[c] = window_edge(s, g, dim, pos, (int)(code & 1u), (int)((code >> 1) & 1u), (int)((code >> 2) & 1u),
+                                   (int)(code >> 3));
+                bad = bad || v[c] >= Vc;
+            }
+            I[3 * q] = v[0];
+            I[3 * q + 1] = v[1];
+            I[3 * q + 2] = v[2];
+        }
+        if (bad) A.ctr->error = 4;
+        if (cells) {
+            const int64_t ci = M.dens_off + 64ll * w0 + pos;
+            A.cell_tb[ci] = tb;
+            A.cell_mask[ci] = (uint8_t)mask;
+        }
     }
 }
 
-template <int W>
-__global__ void __launch_bounds__(kRowThreads) k_emit(Arenas A, int n) {
-    constexpr int NW = kRowThreads / 64;
+__global__ void __launch_bounds__(kRowThreads) k_emit(Arenas A) {
+    __shared__ ItemWindows s_win[kWordWaves];
+    __shared__ uint64_t s_tri[256];  // the triangle table
     __shared__ uint8_t s_ntri[256];
-    __shared__ uint64_t s_planes[3][plane_words(W)];  // labels of planes x, x+1, x+2
-    __shared__ uint32_t s_base[3][BMF_MAX_DIM + 1];  // row vertex bases of planes x, x+1; triangle bases of plane x
-    // first vertex id of each sample of the slab's rows, less the slab's first
-    // row base of its plane (a slab's rows hold at most (kEmitRows + 1) *
-    // 3 * 256 < 2^14 vertices), | x-edge bit 14 | y-edge bit 15
-    __shared__ uint16_t s_id[2][kEmitRows + 1][64 * W];
-    __shared__ uint64_t s_tri[256];                       // the triangle table
-    __shared__ uint32_t s_edge[16];                       // edge_decode of edges 0..11
-    if (threadIdx.x < 16) s_edge[threadIdx.x] = threadIdx.x < 12 ? edge_decode<W>(threadIdx.x) : 0u;
     for (int t = threadIdx.x; t < 256; t += blockDim.x) {
         s_tri[t] = c_tri_table[t];
         s_ntri[t] = (uint8_t)((c_tri_table[t] >> 60) / 3);
     }
+    __syncthreads();
     const int wave = uniform_int(threadIdx.x >> 6);
-    const int split = A.ctr->plane_split[W - 1];
-    const int64_t base = A.ctr->class_base[W - 1];
-    const int64_t total = A.ctr->class_planes[W - 1] * split;
-    for (int64_t it = blockIdx.x; it < total; it += gridDim.x) {
-        const int64_t item = it / split;
-        const int seg = (int)(it - item * split);
-        const int2 pm = A.plane_map[base + item];
-        const ChunkMeta M = read_chunk(A.meta, pm.x);
-        const int dim = M.dim;
-        if (M.status != BMF_OK || M.V == 0) continue;  // uniform across the block
-        const int x = uniform_int(pm.y);
-        const int y0 = (int)((int64_t)seg * dim / split), y1 = (int)((int64_t)(seg + 1) * dim / split);
-        __syncthreads();  // previous item is done with the shared arrays
-        stage_planes(s_planes[0], s_planes[1], s_planes[2], A.labels + M.lab_off, M.lab_words, dim, x);
-        const uint32_t* rv = A.row_v + M.row_off + (int64_t)x * dim;
-        const uint32_t* rt = A.row_t + M.row_off + (int64_t)x * dim;
-        // row bases of planes x and x+1 and the triangle bases of plane x; the
-        // entry after a plane's last row is the next row's base (or the chunk
-        // total), so base[y+1] - base[y] is the row's count
-        const int64_t R = (int64_t)dim * dim, r0 = (int64_t)x * dim;
-        for (int y = threadIdx.x; y <= dim; y += blockDim.x) {
-            const int64_t ra = r0 + y, rb = r0 + dim + y;
-            const uint32_t va = rv[ra < R ? y : 0], vb = rv[rb < R ? dim + y : 0], ta = rt[ra < R ? y : 0];
-            s_base[0][y] = ra < R ? va : (uint32_t)M.V;
-            s_base[1][y] = rb < R ? vb : (uint32_t)M.V;
-            s_base[2][y] = ra < R ? ta : (uint32_t)M.T;
-        }
-        const bool cellsx = x < dim - 1;  // plane x has cells (and plane x+1 exists)
-        for (int ys = y0; ys < y1; ys += kEmitRows) {
-            const int ye = min(y1, ys + kEmitRows);         // cell / owned rows [ys, ye)
-            const int yl = min(dim - 1, ye);                // id rows [ys, yl]
-            __syncthreads();  // staging done; the previous slab is done with s_id
-            const uint32_t slab0 = s_base[0][ys], slab1 = s_base[1][ys];  // the id table's offsets
-            // pass 1: rows of plane x (and x+1 when it has cells); rows that own no
-            // vertex are never referenced by a triangle and skip the label work
-            const int nrow = yl - ys + 1;
-            for (int t = wave; t < (cellsx ? 2 : 1) * nrow; t += NW) {
-                const int p = t >= nrow ? 1 : 0, y = ys + (t - p * nrow);
-                if (s_base[p][y + 1] == s_base[p][y]) continue;
-                emit_ids_row<W>(A, M, s_planes, s_base[p][y], s_id[p][y - ys], p ? slab1 : slab0, x, p, y, p == 0 && y < ye);
-            }
-            if (!cellsx) continue;
-            __syncthreads();
-            // pass 2: cell rows with triangles
-            for (int y = ys + wave; y < ye && y < dim - 1; y += NW) {
-                if (s_base[2][y + 1] == s_base[2][y]) continue;
-                emit_tris_row<W>(A, M, s_planes, s_ntri, s_tri, s_edge, s_base[2][y], s_id, slab0, slab1, x, y, ys);
-            }
-        }
+    ItemWindows& s = s_win[wave];
+    const int64_t total = A.ctr->total_items;
+    for (int64_t it = (int64_t)blockIdx.x * kWordWaves + wave; it < total; it += (int64_t)gridDim.x * kWordWaves) {
+        const ItemRef R = item_ref(A, it);
+        const ChunkMeta& M = R.M;
+        if (M.status != BMF_OK || M.V == 0) continue;
+        const WindowGeom g = stage_windows(A, M, R.w0, s);
+        emit_vertices(A, M, s, R.w0);
+        wave_sync();  // the sample list is read
+        emit_triangles(A, M, s, g, s_ntri, s_tri, R.w0, A.item_c[it]);
+        wave_sync();  // the windows are read
     }
 }
 
@@ -1914,11 +1710,9 @@ hipError_t launch_sample(const Arenas& A, int n, int blocks, int adaptive, int k
 #undef BMF_SAMPLE
     return hipGetLastError();
 }
-hipError_t launch_count(const Arenas& A, int n, int blocks, int wclasses, hipStream_t s) {
-    if (wclasses & 1) hipLaunchKernelGGL(k_count<1>, dim3(blocks), dim3(kRowThreads), 0, s, A, n);
-    if (wclasses & 2) hipLaunchKernelGGL(k_count<2>, dim3(blocks), dim3(kRowThreads), 0, s, A, n);
-    if (wclasses & 4) hipLaunchKernelGGL(k_count<3>, dim3(blocks), dim3(kRowThreads), 0, s, A, n);
-    if (wclasses & 8) hipLaunchKernelGGL(k_count<4>, dim3(blocks), dim3(kRowThreads), 0, s, A, n);
+hipError_t launch_count(const Arenas& A, int blocks, int refine, hipStream_t s) {
+    if (refine) hipLaunchKernelGGL(k_count<true>, dim3(blocks), dim3(kRowThreads), 0, s, A);
+    else hipLaunchKernelGGL(k_count<false>, dim3(blocks), dim3(kRowThreads), 0, s, A);
     return hipGetLastError();
 }
 hipError_t launch_scan(const Arenas& A, int n, int blocks, hipStream_t s) {
@@ -1935,15 +1729,8 @@ hipError_t launch_scan(const Arenas& A, int n, int blocks, hipStream_t s) {
     }
     return hipGetLastError();
 }
-hipError_t launch_emit(const Arenas& A, int n, int blocks, int wclasses, hipStream_t s) {
-    if (wclasses & 1) hipLaunchKernelGGL(k_emit<1>, dim3(blocks), dim3(kRowThreads), 0, s, A, n);
-    if (wclasses & 2) hipLaunchKernelGGL(k_emit<2>, dim3(blocks), dim3(kRowThreads), 0, s, A, n);
-    if (wclasses & 4) hipLaunchKernelGGL(k_emit<3>, dim3(blocks), dim3(kRowThreads), 0, s, A, n);
-    if (wclasses & 8) hipLaunchKernelGGL(k_emit<4>, dim3(blocks), dim3(kRowThreads), 0, s, A, n);
-    return hipGetLastError();
-}
-hipError_t launch_refine(const Arenas& A, int n, int blocks, hipStream_t s) {
-    hipLaunchKernelGGL(k_refine, dim3(blocks), dim3(kSampleThreads), 0, s, A, n);
+hipError_t launch_emit(const Arenas& A, int blocks, hipStream_t s) {
+    hipLaunchKernelGGL(k_emit, dim3(blocks), dim3(kRowThreads), 0, s, A);
     return hipGetLastError();
 }
 hipError_t launch_smooth_map(const Arenas& A, int blocks, hipStream_t s) {

@@ -1,6 +1,6 @@
-// Label-row helpers shared by the plane kernels: a row of the label bitmap
-// (samples (x, y, 0..dim-1)) as W u64 words held in registers, and the
-// staging of whole label planes into LDS.
+// Helpers shared by the kernels: wave and block primitives, the chunk table
+// and sample coordinates, and label rows (samples (x, y, 0..dim-1)) as W u64
+// words for the stage inspection.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -8,10 +8,6 @@
 #include "bmf_internal.h"
 
 namespace bmf {
-
-// u64 words of one staged label plane for row-word class W (dim <= 64 W),
-// plus the zero pad word.
-__host__ __device__ constexpr int plane_words(int W) { return 64 * W * W + 1; }
 
 // ------------------------------------------------------------------------
 // small helpers
@@ -36,6 +32,11 @@ __device__ __forceinline__ ChunkMeta read_chunk(const ChunkMeta* table, int j) {
     ChunkMeta m;
     __builtin_memcpy(&m, w, sizeof(ChunkMeta));
     return m;
+}
+
+// Set bits of a wave mask below this lane.
+__device__ __forceinline__ uint32_t mbcnt64(uint64_t w) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(w >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)w, 0u));
 }
 
 __device__ __forceinline__ uint64_t lanemask_lt() {
@@ -126,17 +127,6 @@ __device__ __forceinline__ RowBits<W> zero_row() {
     return r;
 }
 
-template <int W>
-__device__ __forceinline__ RowBits<W> full_row(int dim) {
-    RowBits<W> r;
-#pragma unroll
-    for (int k = 0; k < W; k++) {
-        const int nb = dim - 64 * k;
-        r.w[k] = nb >= 64 ? ~0ull : ((1ull << nb) - 1ull);
-    }
-    return r;
-}
-
 // Row (x, y) of a chunk's flat label bitmap: bits start at (x*dim + y)*dim.
 template <int W>
 __device__ __forceinline__ RowBits<W> load_row(const uint64_t* __restrict__ L, int64_t nwords, int dim, int x, int y) {
@@ -173,74 +163,6 @@ __device__ __forceinline__ uint32_t bit_at(const RowBits<W>& r, int z) {
     return (uint32_t)((word_at<W>(r, z >> 6) >> (z & 63)) & 1ull);
 }
 
-// popcount of bits [0, z)
-template <int W>
-__device__ __forceinline__ uint32_t prefix_pop(const RowBits<W>& r, int z) {
-    const int wz = z >> 6;
-    const uint64_t m = (1ull << (z & 63)) - 1ull;
-    uint32_t c = 0;
-#pragma unroll
-    for (int k = 0; k < W; k++) {
-        const uint64_t v = r.w[k];
-        c += k < wz ? (uint32_t)__popcll(v) : (k == wz ? (uint32_t)__popcll(v & m) : 0u);
-    }
-    return c;
-}
-
-template <int W>
-__device__ __forceinline__ uint32_t total_pop(const RowBits<W>& r) {
-    uint32_t c = 0;
-#pragma unroll
-    for (int k = 0; k < W; k++) c += (uint32_t)__popcll(r.w[k]);
-    return c;
-}
-
-template <int W>
-__device__ __forceinline__ RowBits<W> rxor(const RowBits<W>& a, const RowBits<W>& b, bool valid) {
-    RowBits<W> r;
-#pragma unroll
-    for (int k = 0; k < W; k++) r.w[k] = valid ? (a.w[k] ^ b.w[k]) : 0ull;
-    return r;
-}
-
-// z-edges of a row: bit z set when labels z and z+1 differ (z <= dim-2).
-template <int W>
-__device__ __forceinline__ RowBits<W> zedges(const RowBits<W>& a, int dim) {
-    RowBits<W> r;
-#pragma unroll
-    for (int k = 0; k < W; k++) {
-        const uint64_t nxt = k + 1 < W ? a.w[k + 1] : 0ull;
-        r.w[k] = a.w[k] ^ ((a.w[k] >> 1) | (nxt << 63));
-    }
-    const int last = dim - 1;  // clear bit dim-1 and above
-#pragma unroll
-    for (int k = 0; k < W; k++) {
-        const int lo = 64 * k;
-        if (last <= lo) r.w[k] = 0ull;
-        else if (last < lo + 64) r.w[k] &= (1ull << (last - lo)) - 1ull;
-    }
-    return r;
-}
-
-template <int W>
-__device__ __forceinline__ bool row_equal(const RowBits<W>& a, const RowBits<W>& b) {
-    bool ok = true;
-#pragma unroll
-    for (int k = 0; k < W; k++) ok = ok && a.w[k] == b.w[k];
-    return ok;
-}
-
-// True when the four rows around a row of cells hold one constant label,
-// i.e. no cell of the row is mixed.
-template <int W>
-__device__ __forceinline__ bool quad_uniform(const RowBits<W>& r00, const RowBits<W>& r01, const RowBits<W>& r10,
-                                             const RowBits<W>& r11, int dim) {
-    const RowBits<W> z = zero_row<W>(), f = full_row<W>(dim);
-    const bool allz = row_equal(r00, z) && row_equal(r01, z) && row_equal(r10, z) && row_equal(r11, z);
-    const bool allf = row_equal(r00, f) && row_equal(r01, f) && row_equal(r10, f) && row_equal(r11, f);
-    return allz || allf;
-}
-
 // 8-corner mask of cell (x, y, z) from the four rows around it; corner bit
 // 4dx + 2dy + dz (DMCChunk.cpp:200-438).
 template <int W>
@@ -250,171 +172,5 @@ __device__ __forceinline__ uint32_t cell_mask(const RowBits<W>& r00, const RowBi
            (bit_at<W>(r01, z + 1) << 3) | (bit_at<W>(r10, z) << 4) | (bit_at<W>(r10, z + 1) << 5) |
            (bit_at<W>(r11, z) << 6) | (bit_at<W>(r11, z + 1) << 7);
 }
-
-// ------------------------------------------------------------------------
-// plane staging: three consecutive label planes of a chunk, realigned
-// to u64 words in LDS (coalesced funnel-shifted loads); rows are then read
-// from LDS.  Word pw of each plane is a zero pad for the funnel reads.
-// ------------------------------------------------------------------------
-// NP planes staged together: plane q is bitmap plane xp[q] of src[q] (all
-// zeros outside 0 .. dim-1) into dst[q], a zero word after each plane's
-// last; every load is issued before the first LDS write.
-template <int NP>
-__device__ __forceinline__ void stage_plane_group(uint64_t* const (&dst)[NP], const uint64_t* const (&src)[NP],
-                                                  int64_t nwords, int dim, const int (&xp)[NP]) {
-    const int64_t pbits = (int64_t)dim * dim;
-    const int pw = (int)((pbits + 63) >> 6);
-    for (int k = threadIdx.x; k <= pw; k += blockDim.x) {
-        uint64_t lo[NP], hi[NP];
-        int sh[NP];
-        bool ok[NP], has_hi[NP];
-#pragma unroll
-        for (int q = 0; q < NP; q++) {
-            ok[q] = xp[q] >= 0 && xp[q] < dim && k < pw;
-            const int64_t bit = ok[q] ? (int64_t)xp[q] * pbits + 64ll * k : 0;
-            const int64_t w = bit >> 6;
-            sh[q] = (int)(bit & 63);
-            has_hi[q] = w + 1 < nwords;
-            lo[q] = src[q][w];
-            hi[q] = src[q][has_hi[q] ? w + 1 : w];
-        }
-        const int64_t rem = pbits - 64ll * k;  // bits of the plane from word k on
-#pragma unroll
-        for (int q = 0; q < NP; q++) {
-            uint64_t v = lo[q];
-            if (sh[q]) v = (v >> sh[q]) | ((has_hi[q] ? hi[q] : 0ull) << (64 - sh[q]));
-            if (rem < 64) v &= rem > 0 ? (1ull << rem) - 1ull : 0ull;
-            dst[q][k] = ok[q] ? v : 0ull;
-        }
-    }
-}
-
-__device__ __forceinline__ void stage_planes(uint64_t* p0, uint64_t* p1, uint64_t* p2, const uint64_t* __restrict__ L,
-                                             int64_t nwords, int dim, int x0) {
-    uint64_t* const dst[3] = {p0, p1, p2};
-    const uint64_t* const src[3] = {L, L, L};
-    const int xp[3] = {x0, x0 + 1, x0 + 2};
-    stage_plane_group<3>(dst, src, nwords, dim, xp);
-}
-
-// A wave-uniform row moved to scalar registers: the bit operations on it then
-// run on the scalar unit and it holds no vector registers.
-template <int W>
-__device__ __forceinline__ RowBits<W> uniform_row(const RowBits<W>& a) {
-    RowBits<W> r;
-#pragma unroll
-    for (int k = 0; k < W; k++) {
-        const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a.w[k]);
-        const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a.w[k] >> 32));
-        r.w[k] = ((uint64_t)hi << 32) | lo;
-    }
-    return r;
-}
-
-// Row y of a staged plane.
-// Both words of every funnel read load unconditionally (the staged plane's
-// zero pad word keeps w + 1 in bounds) and an invalid row reads row 0, so
-// the reads carry no branches and issue together.
-template <int W>
-__device__ __forceinline__ RowBits<W> lds_row(const uint64_t* P, int dim, int y, bool valid) {
-    RowBits<W> r;
-    const int base = (valid ? y : 0) * dim;
-#pragma unroll
-    for (int k = 0; k < W; k++) {
-        const int bit = base + 64 * k;
-        const int w = bit >> 6;
-        const int sh = bit & 63;
-        const uint64_t lo = P[w], hi = P[w + 1];
-        uint64_t v = (lo >> sh) | ((hi << 1) << (63 - sh));  // the second term is 0 for sh == 0
-        const int nb = dim - 64 * k;
-        if (nb < 64) v &= nb > 0 ? (1ull << nb) - 1ull : 0ull;
-        r.w[k] = valid ? v : 0ull;
-    }
-    return r;
-}
-
-template <int W>
-__device__ __forceinline__ RowBits<W> rshl1(const RowBits<W>& a) {
-    RowBits<W> r;
-#pragma unroll
-    for (int k = 0; k < W; k++) r.w[k] = (a.w[k] << 1) | (k > 0 ? (a.w[k - 1] >> 63) : 0ull);
-    return r;
-}
-
-// bit z of the result = bit z + 1 of a (0 past the row)
-template <int W>
-__device__ __forceinline__ RowBits<W> rshr1(const RowBits<W>& a) {
-    RowBits<W> r;
-#pragma unroll
-    for (int k = 0; k < W; k++) r.w[k] = (a.w[k] >> 1) | (k + 1 < W ? (a.w[k + 1] << 63) : 0ull);
-    return r;
-}
-
-// Lane-wise views of a wave-uniform 64-bit word whose bit i belongs to lane
-// i (word k of a row, for samples z = 64 k + lane): the lane's bit, and the
-// number of set bits below it (v_mbcnt).
-__device__ __forceinline__ uint32_t lane_bit(uint64_t w, int lane) { return (uint32_t)(w >> lane) & 1u; }
-
-// The same for a word held in scalar registers (the same value in every
-// lane), as this lane's bit of the word used as the wave's lane mask: one
-// v_cndmask_b32 with the word as its 64-bit condition, no 64-bit shift.  The
-// caller's lane must be the executing lane.
-__device__ __forceinline__ uint32_t lane_bit_u(uint64_t w) {
-    uint32_t r;
-    asm("v_cndmask_b32_e64 %0, 0, 1, %1" : "=v"(r) : "s"(w));
-    return r;
-}
-
-__device__ __forceinline__ uint32_t mbcnt64(uint64_t w) {
-    return __builtin_amdgcn_mbcnt_hi((uint32_t)(w >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)w, 0u));
-}
-
-template <int W>
-__device__ __forceinline__ RowBits<W> ror(const RowBits<W>& a, const RowBits<W>& b) {
-    RowBits<W> r;
-#pragma unroll
-    for (int k = 0; k < W; k++) r.w[k] = a.w[k] | b.w[k];
-    return r;
-}
-
-// Samples z in [1, dim-2]: the z-range where both cells beside an x- or
-// y-edge lie in the chunk.
-template <int W>
-__device__ __forceinline__ RowBits<W> inner_z(int dim) {
-    RowBits<W> r;
-#pragma unroll
-    for (int k = 0; k < W; k++) {
-        uint64_t v = ~0ull;
-        const int lo = 64 * k;
-        if (lo == 0) v &= ~1ull;
-        const int hi = dim - 2 - lo;  // last valid bit in this word
-        if (hi < 0) v = 0ull;
-        else if (hi < 63) v &= (2ull << hi) - 1ull;
-        r.w[k] = v;
-    }
-    return r;
-}
-
-template <int W>
-__device__ __forceinline__ RowBits<W> rand_(const RowBits<W>& a, const RowBits<W>& b) {
-    RowBits<W> r;
-#pragma unroll
-    for (int k = 0; k < W; k++) r.w[k] = a.w[k] & b.w[k];
-    return r;
-}
-
-// Interior sign-changing edges owned by the samples of row (x, y): the four
-// cells around each lie in the chunk.
-template <int W>
-__device__ __forceinline__ void interior_edges(const RowBits<W>& r00, const RowBits<W>& r01, const RowBits<W>& r10,
-                                               int dim, int x, int y, RowBits<W>& ex, RowBits<W>& ey,
-                                               RowBits<W>& ez) {
-    const RowBits<W> iz = inner_z<W>(dim);
-    const bool xin = x >= 1 && x <= dim - 2, yin = y >= 1 && y <= dim - 2;
-    ex = (yin && x + 1 < dim) ? rand_<W>(rxor<W>(r00, r10, true), iz) : zero_row<W>();
-    ey = (xin && y + 1 < dim) ? rand_<W>(rxor<W>(r00, r01, true), iz) : zero_row<W>();
-    ez = (xin && yin) ? zedges<W>(r00, dim) : zero_row<W>();
-}
-
 
 }  // namespace bmf

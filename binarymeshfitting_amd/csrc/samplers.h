@@ -294,6 +294,47 @@ __device__ __forceinline__ void stage_csg(const SamplerDev& S, const uint16_t* _
     }
 }
 
+// The primitives of a chunk's list whose value can exceed -reach somewhere
+// in the box [lo, hi], by one wave, in list order into `out` (room for `cap`
+// of them): a sphere within r + reach of the box, a box that meets it grown by
+// reach.  Returns whether they fit.
+__device__ __forceinline__ bool cull_csg(const SamplerDev& S, const uint16_t* __restrict__ list, int ns, int nb,
+                                         const float (&lo)[3], const float (&hi)[3], float reach, float4* out, int cap,
+                                         int& out_s, int& out_b) {
+    const int lane = (int)(threadIdx.x & 63);
+    int n = 0;
+    out_s = 0;
+    for (int i0 = 0; i0 < ns + nb; i0 += 64) {
+        const int i = i0 + lane;
+        bool keep = false;
+        float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f), b = a;
+        if (i < ns) {
+            const float* sp = S.spheres + 4 * list[i];
+            a = make_float4(sp[0], sp[1], sp[2], sp[3]);
+            const float tx = fmaxf(fmaxf(lo[0] - a.x, a.x - hi[0]), 0.0f), ty = fmaxf(fmaxf(lo[1] - a.y, a.y - hi[1]), 0.0f),
+                        tz = fmaxf(fmaxf(lo[2] - a.z, a.z - hi[2]), 0.0f);
+            const float r = a.w + reach;
+            keep = r > 0.0f && !((tx * tx + ty * ty) + tz * tz > r * r);
+        } else if (i < ns + nb) {
+            const float* q = S.boxes + 6 * list[i];
+            a = make_float4(q[0], q[1], q[2], q[3]);
+            b = make_float4(q[4], q[5], 0.0f, 0.0f);
+            keep = !(a.x - a.w - reach > hi[0]) && !(a.x + a.w + reach < lo[0]) && !(a.y - b.x - reach > hi[1]) &&
+                   !(a.y + b.x + reach < lo[1]) && !(a.z - b.y - reach > hi[2]) && !(a.z + b.y + reach < lo[2]);
+        }
+        const uint64_t bal = __ballot(keep), spheres = __ballot(keep && i < ns);
+        const int at = n + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
+        if (keep && at < cap) {
+            out[2 * at] = a;
+            out[2 * at + 1] = b;
+        }
+        n += (int)__popcll(bal);
+        out_s += (int)__popcll(spheres);
+    }
+    out_b = n - out_s;
+    return n <= cap;
+}
+
 __device__ __forceinline__ float csg_density_lds(const float4* s_csg, int ns, int nb, float x, float y, float z) {
     float best = kCsgFloor;
     for (int k = 0; k < ns; k++) {

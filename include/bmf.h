@@ -435,10 +435,10 @@ int bmf_stitch(bmf_ctx* ctx, const bmf_world_node* nodes, int32_t n_nodes, const
 typedef struct {
     int32_t sample_tile;    /* samples per work-queue tile of the sampling kernel: 1024, 2048, 4096 */
     int32_t sample_blocks;  /* persistent workgroups of the sampling kernel */
-    int32_t row_blocks;     /* persistent workgroups of the plane kernels (count, refine, emit) */
+    int32_t row_blocks;     /* persistent workgroups of the word kernels (count, emit) */
     int32_t smooth_blocks;  /* workgroups of the smoothing kernels (rounded up to a multiple of 8) */
-    int32_t row_split;      /* row segments per x-plane item of the plane kernels: 1, 2, 4 or 8; -1
-                               doubles the split (up to 8) while sampled planes x split < 512 */
+    int32_t row_split;      /* 1, 2, 4, 8 or -1: kept for callers, without effect (the word kernels'
+                               items have one size) */
 } bmf_tuning;
 
 int bmf_get_tuning(bmf_ctx* ctx, bmf_tuning* tuning);
