@@ -35,7 +35,7 @@ hipError_t dalloc(T** p, int64_t count) {
 
 void free_arenas(bmf_ctx* c) {
     Arenas& A = c->A;
-    void* ptrs[] = {A.meta,    A.descs,     A.results,  A.tile_prefix, A.plan_part, A.plan_tmp, A.stat_blocks, A.item_map, A.smooth_list, A.smooth_prefix,
+    void* ptrs[] = {A.meta,    A.descs,     A.results,  A.tile_prefix, A.block_prefix, A.signs, A.plan_part, A.plan_tmp, A.stat_blocks, A.item_map, A.smooth_list, A.smooth_prefix,
                     A.smooth_tprefix, A.smooth_xcd_v, A.smooth_xcd_t, A.smooth_vmap, A.smooth_tmap, A.edges, A.word_pre, A.item_e, A.item_c, A.cen4,
                     A.dens,    A.labels,    A.exact, A.cell_tb,   A.cell_mask,
                     A.pos,     A.pos4,      A.boundary, A.vedge,       A.vring,        A.idx,          A.ctr,
@@ -162,6 +162,11 @@ int build_sampler(const bmf_sampler_desc* s, SamplerDev* out) {
             if ((double)rf < r) rf = std::nextafter(rf, INFINITY);
             d.reach[k] = rf;
         }
+        // k_blocks: no amplitude negative (the density's clamp never acts)
+        // and a sign that the sum decides
+        d.expand_ok = d.amp != 0.0f && std::isfinite(1.0f / (d.amp * d.inv_norm));
+        for (int o = 0; o < s->octaves; o++)
+            if (!(d.ao[o] >= 0.0f) || !finite(d.fo[o])) d.expand_ok = 0;
     }
     if (s->kind == BMF_SAMPLER_NOISE) {
         const bool dims_ok = s->noise_dims == 2 || s->noise_dims == 3;
@@ -294,9 +299,10 @@ int bmf_create(bmf_ctx** out, int device, const bmf_limits* lim) {
     bool ok = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) == hipSuccess;
     ok = ok && dalloc(&A.meta, nc) == hipSuccess && dalloc(&A.descs, nc) == hipSuccess &&
          dalloc(&A.results, nc) == hipSuccess && dalloc(&A.tile_prefix, nc + 1) == hipSuccess &&
+         dalloc(&A.block_prefix, nc + 1) == hipSuccess && dalloc(&A.signs, lim->max_samples + 16) == hipSuccess &&
          dalloc(&A.plan_part, 40 * ((nc + 1023) / 1024) + 64) == hipSuccess &&
          dalloc(&A.plan_tmp, 2 * nc) == hipSuccess &&
-         dalloc(&A.stat_blocks, 2 * (int64_t)(64 * c->cu_count)) == hipSuccess &&
+         dalloc(&A.stat_blocks, 3 * (int64_t)(64 * c->cu_count)) == hipSuccess &&
          dalloc(&A.item_map, ni) == hipSuccess && dalloc(&A.smooth_list, nc) == hipSuccess &&
          dalloc(&A.smooth_prefix, nc + 1) == hipSuccess && dalloc(&A.smooth_tprefix, nc + 1) == hipSuccess &&
          dalloc(&A.smooth_xcd_v, kXcds + 1) == hipSuccess && dalloc(&A.smooth_xcd_t, kXcds + 1) == hipSuccess &&
@@ -757,15 +763,15 @@ int bmf_get_frame_stats(bmf_ctx* c, bmf_frame_stats* out) {
     std::vector<unsigned long long> h((size_t)std::max(ns, nr));
     BMF_HIP(hipSetDevice(c->device));
     BMF_HIP(hipStreamSynchronize(c->stream));
-    int64_t sum[2] = {0, 0};
-    for (int k = 0; k < 2; k++) {
-        const int m = k == 0 ? ns : nr;
+    int64_t sum[3] = {0, 0, 0};
+    for (int k = 0; k < 3; k++) {
+        const int m = k == 1 ? nr : (k == 0 || c->h_sampler.kind == BMF_SAMPLER_TERRAIN ? ns : 0);
         if (m <= 0) continue;
         BMF_HIP(hipMemcpy(h.data(), c->A.stat_blocks + (size_t)k * c->A.stat_cap, sizeof(unsigned long long) * m,
                           hipMemcpyDeviceToHost));
         for (int b = 0; b < m; b++) sum[k] += (int64_t)h[b];
     }
-    out->octave_evals = sum[0];
+    out->octave_evals = sum[0] + sum[2];
     out->refine_evals = sum[1];
     return BMF_OK;
 }

@@ -15,6 +15,7 @@ constexpr int kSampleTileDefault = 2048;
 constexpr int kRowThreads = 256;      // word kernels: 4 waves, an item of label words each
 constexpr int kItemWords = 16;        // label words per item: enough active cells for a wave's lanes near a surface
 constexpr int kItemSamples = 64 * kItemWords;
+constexpr int kWaveBlocks = 16;       // 4 x 4 x 4 sample blocks per wave of k_blocks
 constexpr int kSmoothThreads = 256;   // one vertex per thread
 constexpr int kMaxRowWords = 4;       // ceil(BMF_MAX_DIM / 64)
 constexpr int kXcds = 8;              // MI355X: 8 XCDs, each with its own L2
@@ -40,6 +41,7 @@ struct SamplerDev {
     // reach[k] >= the most the FP32 partial sum after k octaves can still
     // move: sum of |a_o| for o >= k plus the rounding slack of those steps
     float reach[BMF_MAX_OCTAVES + 1];
+    int32_t expand_ok;          // terrain: the noise sum can be expanded about block centres (k_blocks)
     const float* spheres;       // device, n_spheres x 4
     const float* boxes;         // device, n_boxes x 6
     const float* ext;           // EXTERNAL: caller's densities, chunks packed in descriptor order
@@ -54,6 +56,14 @@ struct SamplerDev {
     // k_plan's chunk culling: n lies in [nlo, nhi] for every sample (cull = 0: no bound)
     float nlo, nhi;
     int32_t cull;
+};
+
+// How k_blocks expands a terrain chunk's noise: octaves per block and per
+// sub-block (0: the level is left out), and the error quad * r^2 + base of
+// the sum at a sample r sample steps from the centre.
+struct BlockPlan {
+    int32_t k4, k2;
+    float quad4, base4, quad2, base2;
 };
 
 // Per-chunk state in device memory.
@@ -78,6 +88,7 @@ struct ChunkMeta {
     int32_t csg_nb;     //      listed in Arenas::csg_list (sphere ids, then box ids, in order)
     int64_t v_off;      // output offsets
     int64_t i_off;
+    BlockPlan blocks;   // adaptive terrain
     int64_t item_slot;  // the chunk's first item of the word kernels (sampled chunks)
 };
 
@@ -110,11 +121,15 @@ struct Arenas {
     bmf_chunk_desc* descs;     // [max_chunks]
     bmf_chunk_result* results; // [max_chunks]
     int64_t* tile_prefix;      // [max_chunks + 1] sampling tiles
+    int64_t* block_prefix;     // [max_chunks + 1] items of kWaveBlocks sample blocks (k_blocks)
+    uint8_t* signs;            // [max_samples + 16] adaptive terrain: k_blocks' decisions, from the chunk's first
+                               // sample on a byte per four samples of a row (x, y), ceil(dim / 4) bytes a row:
+                               // undecided samples in the low bits, air samples in the high ones
     int64_t* plan_part;        // [40 nb + 64] multi-block plan passes (nb = max_chunks / 1024 rounded up):
                                // block totals and bases, flags, class and group bases
     int64_t* plan_tmp;         // [2 max_chunks] multi-block smoothing plan: per-chunk exclusive tile sums
-    unsigned long long* stat_blocks;  // [2][stat_cap] terrain octaves evaluated per workgroup of
-                                      // the sampling and the refinement kernels (plain stores, no atomics)
+    unsigned long long* stat_blocks;  // [3][stat_cap] terrain octaves evaluated per workgroup of the
+                                      // sampling, refinement and block kernels (plain stores, no atomics)
     int32_t stat_cap;
     int2* item_map;            // [max_items] (chunk, item within the chunk) of the word kernels' items
                                // (written by k_sample's prologue)

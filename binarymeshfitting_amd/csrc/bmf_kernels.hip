@@ -70,12 +70,73 @@ __device__ __forceinline__ int64_t pick(const int64_t (&a)[N], int i) {
     return r;
 }
 
+// ---- how far k_blocks expands a chunk's noise (see there) ----
+// Largest norm of the noise's Hessian: 48.21 over all positions in a simplex
+// and gradients at its corners, with a margin (tests/test_noise_bounds.py).
+constexpr float kNoiseHess = 50.0f;
+// FP32 error of two noise values and of a gradient over a block, per unit of
+// amplitude: a constant for the kernels' arithmetic (about 76.8 * 4 t^3 g.x
+// half-ulps of t, under 1e-5 each) and a part proportional to the lattice
+// coordinates, whose rounding (under 8e-7 of their sum) moves the noise by
+// its gradient (at most 7.1), twice, and the gradient by kNoiseHess.
+constexpr float kNoiseSlack = 2e-4f, kNoiseCoordSlack = 4e-5f;
+// Roundings of the sums, of the sign test and of the density from its sum,
+// relative to the sum of the amplitudes (32 ulps).
+constexpr float kSignSlack = 4e-6f;
+
+constexpr int kExpandOctaves = 4;  // a quad of lanes takes an octave each
+
+// The octaves to expand for samples at squared distance rr (in samples) from
+// their centre: the k with the least E_k, which goes out as quad * r^2 + base.
+__device__ __forceinline__ int expansion(const SamplerDev& S, float delta, float far, float rr, float& quad,
+                                         float& base) {
+    float q = 0.0f, b = 0.0f, best = S.reach[0];
+    int k = 0;
+    quad = 0.0f;
+    base = best;
+    for (int o = 0; o < min(S.octaves, kExpandOctaves); o++) {
+        const float f = S.fo[o] * delta;
+        q += S.ao[o] * (0.505f * kNoiseHess) * (f * f);
+        b += S.ao[o] * (kNoiseSlack + kNoiseCoordSlack * far * fabsf(S.fo[o]));
+        const float e = __builtin_fmaf(q, rr, b) + S.reach[o + 1];
+        if (e < best) {
+            best = e;
+            k = o + 1;
+            quad = q;
+            base = b + S.reach[o + 1];
+        }
+    }
+    base += kSignSlack * S.reach[0];
+    return k;
+}
+
+
+// The plan of a terrain chunk's blocks and sub-blocks: a level that would
+// decide hardly more than the one before is left out.
+__device__ __forceinline__ BlockPlan plan_blocks(const SamplerDev& S, const ChunkMeta& M) {
+    BlockPlan p{0, 0, 0.0f, (1.0f + kSignSlack) * S.reach[0], 0.0f, 0.0f};
+    if (!S.expand_ok) return p;
+    const float ext = (float)(M.dim - 1) * M.delta;
+    float far = 0.0f, q, e;
+#pragma unroll
+    for (int a = 0; a < 3; a++) far += fmaxf(fabsf(M.opos[a]), fabsf(M.opos[a] + ext));
+    const int k = expansion(S, M.delta, far, 3.75f, q, e);
+    if (__builtin_fmaf(q, 3.75f, e) < 0.8f * p.base4) {
+        p.k4 = k;
+        p.quad4 = q;
+        p.base4 = e;
+    }
+    p.k2 = expansion(S, M.delta, far, 0.75f, p.quad2, p.base2);
+    if (!(__builtin_fmaf(p.quad2, 0.75f, p.base2) < 0.8f * __builtin_fmaf(p.quad4, 3.75f, p.base4))) p.k2 = 0;
+    return p;
+}
+
 // Plan record of one descriptor: DMCChunk::label_grid geometry
 // (DMCChunk.cpp:94-101), analytic culling, sizes; `add` gets its
 // contributions to the arena sums (samples, label words, word items, sampling
-// tiles).
+// tiles, items of sample blocks).
 __device__ __forceinline__ ChunkMeta plan_record(const Arenas& A, const SamplerDev* __restrict__ S,
-                                                 const bmf_chunk_desc& d, int allow_cull, int64_t (&add)[4]) {
+                                                 const bmf_chunk_desc& d, int allow_cull, int64_t (&add)[5]) {
     ChunkMeta m;
     float t = d.overlap * 2.0f;
     t = 1.0f + t;
@@ -111,20 +172,23 @@ __device__ __forceinline__ ChunkMeta plan_record(const Arenas& A, const SamplerD
     m.dens_off = 0;
     m.lab_off = 0;
     m.item_slot = 0;
+    m.blocks = sampled && S->kind == BMF_SAMPLER_TERRAIN ? plan_blocks(*S, m) : BlockPlan{};
     add[0] = sampled ? ns : 0;
     add[1] = m.lab_words;
     add[2] = (m.lab_words + kItemWords - 1) / kItemWords;
     add[3] = sampled ? (ns + A.sample_tile - 1) / A.sample_tile : 0;
+    const int64_t nb = (d.dim + 3) >> 2;
+    add[4] = sampled ? (nb * nb * nb + kWaveBlocks - 1) / kWaveBlocks : 0;
     return m;
 }
 
-__device__ __forceinline__ bool plan_overflow(const Arenas& A, const int64_t (&tot)[4]) {
+__device__ __forceinline__ bool plan_overflow(const Arenas& A, const int64_t (&tot)[5]) {
     return tot[0] > A.cap_samples || tot[1] > A.cap_samples / 64 + A.cap_chunks;
 }
 
 // A record's final state once its offsets are known (base: where its block's
 // arena ranges start).
-__device__ __forceinline__ void plan_finish(const Arenas& A, int j, ChunkMeta& m, const int64_t (&base)[4],
+__device__ __forceinline__ void plan_finish(const Arenas& A, int j, ChunkMeta& m, const int64_t (&base)[5],
                                             bool overflow) {
     m.dens_off += base[0];
     m.lab_off += base[1];
@@ -143,9 +207,10 @@ __device__ __forceinline__ void plan_finish(const Arenas& A, int j, ChunkMeta& m
 }
 
 // The batch counters from the totals: sampling tiles, word items, overflow.
-__device__ __forceinline__ void plan_counters(const Arenas& A, int n, const int64_t (&tot)[4], bool overflow,
+__device__ __forceinline__ void plan_counters(const Arenas& A, int n, const int64_t (&tot)[5], bool overflow,
                                               int reset_bumps) {
     A.tile_prefix[n] = overflow ? 0 : tot[3];
+    A.block_prefix[n] = overflow ? 0 : tot[4];
     Counters* c = A.ctr;
     c->sample_head = 0;
     if (reset_bumps) {
@@ -166,27 +231,29 @@ __device__ __forceinline__ void plan_counters(const Arenas& A, int n, const int6
 // Batches of up to kPlanOneBlock descriptors: one block, each thread a
 // segment of consecutive descriptors, one launch.
 __global__ void __launch_bounds__(kPlanThreads) k_plan(Arenas A, int n, int allow_cull, int reset_bumps) {
-    __shared__ int64_t s_w[4][kPlanThreads / 64 + 1];
+    __shared__ int64_t s_w[5][kPlanThreads / 64 + 1];
     const int per = (n + kPlanThreads - 1) / kPlanThreads;
     const int j0 = threadIdx.x * per, j1 = min(n, j0 + per);
-    int64_t sum[4] = {0, 0, 0, 0};
+    int64_t sum[5] = {0, 0, 0, 0, 0};
     for (int j = j0; j < j1; j++) {
-        int64_t add[4];
+        int64_t add[5];
         ChunkMeta m = plan_record(A, A.sampler, A.descs[j], allow_cull, add);
         // offsets within the thread's segment; tile_prefix likewise
         m.dens_off = sum[0];
         m.lab_off = sum[1];
         m.item_slot = sum[2];
         A.tile_prefix[j] = sum[3];
+        A.block_prefix[j] = sum[4];
         A.meta[j] = m;
 #pragma unroll
-        for (int q = 0; q < 4; q++) sum[q] += add[q];
+        for (int q = 0; q < 5; q++) sum[q] += add[q];
     }
-    int64_t excl[4], tot[4];
-    block_scan<4, kPlanThreads>(sum, excl, tot, s_w);
+    int64_t excl[5], tot[5];
+    block_scan<5, kPlanThreads>(sum, excl, tot, s_w);
     const bool overflow = plan_overflow(A, tot);
     for (int j = j0; j < j1; j++) {
         A.tile_prefix[j] = overflow ? 0 : A.tile_prefix[j] + excl[3];
+        A.block_prefix[j] = overflow ? 0 : A.block_prefix[j] + excl[4];
         ChunkMeta m = A.meta[j];
         plan_finish(A, j, m, excl, overflow);
     }
@@ -196,42 +263,43 @@ __global__ void __launch_bounds__(kPlanThreads) k_plan(Arenas A, int n, int allo
 // Larger batches, pass 1 of 3 (one descriptor per thread over many blocks):
 // records with offsets relative to their block, and each block's totals.
 __global__ void __launch_bounds__(kPlanThreads) k_plan_part(Arenas A, int n, int allow_cull) {
-    __shared__ int64_t s_w[4][kPlanThreads / 64 + 1];
+    __shared__ int64_t s_w[5][kPlanThreads / 64 + 1];
     const int j = blockIdx.x * kPlanThreads + threadIdx.x;
-    int64_t add[4];
+    int64_t add[5];
     ChunkMeta m{};
     if (j < n) m = plan_record(A, A.sampler, A.descs[j], allow_cull, add);
     else
-        for (int q = 0; q < 4; q++) add[q] = 0;
-    int64_t excl[4], tot[4];
-    block_scan<4, kPlanThreads>(add, excl, tot, s_w);
+        for (int q = 0; q < 5; q++) add[q] = 0;
+    int64_t excl[5], tot[5];
+    block_scan<5, kPlanThreads>(add, excl, tot, s_w);
     if (j < n) {
         A.tile_prefix[j] = excl[3];
+        A.block_prefix[j] = excl[4];
         m.dens_off = excl[0];
         m.lab_off = excl[1];
         m.item_slot = excl[2];
         A.meta[j] = m;
     }
-    if (threadIdx.x < 4) A.plan_part[4 * blockIdx.x + threadIdx.x] = pick<4>(tot, (int)threadIdx.x);
+    if (threadIdx.x < 5) A.plan_part[5 * blockIdx.x + threadIdx.x] = pick<5>(tot, (int)threadIdx.x);
 }
 
 // Pass 2 (one block, one thread per pass-1 block, at most kPlanThreads):
 // block bases, batch totals, overflow flag, counters.  Bases go to
-// plan_part[4 (nb + b) ...], the overflow flag after them.
+// plan_part[5 (nb + b) ...], the overflow flag after them.
 __global__ void __launch_bounds__(kPlanThreads) k_plan_total(Arenas A, int n, int nb, int reset_bumps) {
-    __shared__ int64_t s_w[4][kPlanThreads / 64 + 1];
+    __shared__ int64_t s_w[5][kPlanThreads / 64 + 1];
     const int b = threadIdx.x;
-    int64_t v[4];
+    int64_t v[5];
 #pragma unroll
-    for (int q = 0; q < 4; q++) v[q] = b < nb ? A.plan_part[4 * b + q] : 0;
-    int64_t excl[4], tot[4];
-    block_scan<4, kPlanThreads>(v, excl, tot, s_w);
+    for (int q = 0; q < 5; q++) v[q] = b < nb ? A.plan_part[5 * b + q] : 0;
+    int64_t excl[5], tot[5];
+    block_scan<5, kPlanThreads>(v, excl, tot, s_w);
     const bool overflow = plan_overflow(A, tot);
     if (b < nb)
 #pragma unroll
-        for (int q = 0; q < 4; q++) A.plan_part[4 * (nb + b) + q] = excl[q];
+        for (int q = 0; q < 5; q++) A.plan_part[5 * (nb + b) + q] = excl[q];
     if (b == 0) {
-        A.plan_part[8 * nb] = overflow;
+        A.plan_part[10 * nb] = overflow;
         plan_counters(A, n, tot, overflow, reset_bumps);
     }
 }
@@ -240,11 +308,12 @@ __global__ void __launch_bounds__(kPlanThreads) k_plan_total(Arenas A, int n, in
 __global__ void __launch_bounds__(kPlanThreads) k_plan_fix(Arenas A, int n, int nb) {
     const int j = blockIdx.x * kPlanThreads + threadIdx.x;
     if (j >= n) return;
-    int64_t base[4];
+    int64_t base[5];
 #pragma unroll
-    for (int q = 0; q < 4; q++) base[q] = A.plan_part[4 * (nb + blockIdx.x) + q];
-    const bool overflow = A.plan_part[8 * nb] != 0;
+    for (int q = 0; q < 5; q++) base[q] = A.plan_part[5 * (nb + blockIdx.x) + q];
+    const bool overflow = A.plan_part[10 * nb] != 0;
     A.tile_prefix[j] = overflow ? 0 : A.tile_prefix[j] + base[3];
+    A.block_prefix[j] = overflow ? 0 : A.block_prefix[j] + base[4];
     ChunkMeta m = A.meta[j];
     plan_finish(A, j, m, base, overflow);
 }
@@ -312,26 +381,8 @@ __global__ void __launch_bounds__(256) k_csg_cull(Arenas A, int n) {
 }
 
 // ------------------------------------------------------------------------
-// sample: persistent; workgroups pull tiles of Arenas::sample_tile consecutive
-// samples of one chunk from an atomic work queue.
-//
-// Terrain chunks use exact adaptive octave evaluation.  After k octaves the
-// FP32 partial sum S_k bounds the final sum: each remaining step is
-// fma(a_o, n_o, S) with |n_o| <= 1 and rounding is monotone, so
-// S_O in [L, H] with L = (..(S_k - |a_k|) - ..), H = (..(S_k + |a_k|) + ..)
-// evaluated in FP32; every value involved is at most A = sum |a_o| in
-// magnitude, so L and H differ from the exact S_k -/+ sum_{o>=k} |a_o| by at
-// most (O - k) half-ulps of A, and reach[k] = that sum + (O - k + 2) ulp(A)
-// (rounded up, host side) gives FP32 bounds S_k -/+ reach[k] outside [L, H].
-// The density is monotone in S, so d(S_k - reach), d(S_k + reach) bound the
-// final density and decide the label once they agree in sign.  Undecided
-// samples are compacted into an LDS queue (wave ballot + popcount) so each
-// octave runs on dense waves.  Samples that run all octaves get their exact
-// density written and their bit set in the `exact` bitmap; the others only
-// get their label (k_count finishes the densities of those that are endpoints of a
-// sign-changing edge).  Without
-// adaptation every
-// sample is evaluated fully (bit-identical values either way).
+// sampling: the adaptive terrain through k_blocks and k_terrain, every other
+// case through k_sample
 // ------------------------------------------------------------------------
 // A chunk's sample geometry as values (like TerrainTerms): read once per
 // tile, so the loops below never reload them after their own stores.
@@ -362,64 +413,442 @@ __device__ __forceinline__ void sample_coords(const ChunkGeom& G, uint32_t i, ui
     sample_position(G, x, y, z, px, py, pz);
 }
 
-// Sampling modes, fixed per launch by the host: adaptive octaves for the
-// terrain sampler; the CSG union with the chunk's culled primitives staged in
-// LDS once per tile; a 2D noise field with the noise of the tile's (x, z)
-// columns evaluated once into LDS and broadcast along y; every other case
-// (external densities, implicit shapes, 3D noise fields, the terrain in full)
-// evaluated directly.
-constexpr int kSampleGeneric = 0, kSampleAdaptive = 1, kSampleCsg = 2, kSampleSlab = 3;
-// Adaptive mode: undecided samples of a wave (of 64) from which phase 0
-// evaluates octave 0 in place rather than queueing them: queueing costs a
-// push, a pop and the sample coordinates again, in-place evaluation the
-// idle lanes of one octave.
-constexpr int kInPlaceOctave = 52;
-// Octave queue entries: sample index within the tile (kTile <= 4096) in the
-// low 12 bits, the sample's next octave (< BMF_MAX_OCTAVES = 16) above.
-constexpr int kQueueOctaveShift = 12;
-constexpr uint32_t kQueueSampleMask = (1u << kQueueOctaveShift) - 1u;
-static_assert(16 * kSampleThreads <= (1 << kQueueOctaveShift), "tile index fits the queue entry");
-static_assert(BMF_MAX_OCTAVES <= 16, "octave index fits the queue entry");
+// ------------------------------------------------------------------------
+// blocks (adaptive terrain): the sign of most samples from a few evaluations
+// per 4 x 4 x 4 block of them.
+//
+// Simplex noise n is twice differentiable with |n| < 1 (the clamp never
+// acts) and a Hessian of norm at most kNoiseHess, so at a sample s of a block
+// with centre c
+//   |n(f s) - (n(f c) + f grad n(f c) . (s - c))| <= kNoiseHess / 2 (f |s - c|)^2,
+// and after k octaves expanded that way the sample's FP32 sum of all octaves
+// lies within
+//   E_k(r^2) = sum_{o<k} a_o (kNoiseHess / 2 (f_o r)^2 + slack_o) + reach[k]
+// of the expansion (reach: the octaves not evaluated, as in decide_label;
+// slack_o: FP32 errors of both noise values and the coordinates, see
+// kNoiseSlack).  A sample whose expansion is further than that from the sum
+// at which its density changes sign is decided.  Two levels: 4^3 blocks (one
+// per lane), then the 2^3 sub-blocks that hold undecided samples, compacted;
+// at each level the number of octaves with the least E_k.  k_terrain
+// evaluates what is left, about a thirteenth of a chunk's samples.
+//
+// A quad of lanes shares a centre, an octave each, so that a wave's chain is
+// one octave long.  Bound by VALU issue: 512 chunks of 64^3 cells, 64 sampled
+// (17.6 M samples, 5 octaves) take 52 us here and 69 in k_terrain; evaluating
+// every sample's octaves until its sign was certain (1.38 on average) took
+// 202, and 23 instead of 13 for the endpoints that it left.
+// ------------------------------------------------------------------------
+// n and its gradient at (x, y, z): snoise3's corners, without its exact
+// operation order.
+struct NoiseGrad {
+    float n, gx, gy, gz;
+};
+__device__ __forceinline__ void corner_grad(float x, float y, float z, uint32_t h, NoiseGrad& r) {
+    float t = __builtin_fmaf(-x, x, kNoiseR2);
+    t = __builtin_fmaf(-y, y, t);
+    t = __builtin_fmaf(-z, z, t);
+    t = fmaxf(t, 0.0f);
+    const float su = (h & 1u) ? -1.0f : 1.0f, sv = (h & 2u) ? -1.0f : 1.0f;
+    const bool ux = h < 8u, vy = h < 4u, vx = h == 12u || h == 14u;
+    const float gx = (ux ? su : 0.0f) + (vx ? sv : 0.0f), gy = (ux ? 0.0f : su) + (vy ? sv : 0.0f),
+                gz = vy || vx ? 0.0f : sv;
+    const float L = __builtin_fmaf(gx, x, __builtin_fmaf(gy, y, gz * z));
+    const float t2 = t * t, t4 = t2 * t2, k = -8.0f * t2 * t * L;
+    r.n = __builtin_fmaf(t4, L, r.n);
+    r.gx = __builtin_fmaf(t4, gx, __builtin_fmaf(k, x, r.gx));
+    r.gy = __builtin_fmaf(t4, gy, __builtin_fmaf(k, y, r.gy));
+    r.gz = __builtin_fmaf(t4, gz, __builtin_fmaf(k, z, r.gz));
+}
+__device__ __forceinline__ NoiseGrad snoise3_grad(float x, float y, float z, uint32_t seed) {
+    const float G3 = 1.0f / 6.0f;
+    const float s = ((x + y) + z) * (1.0f / 3.0f);
+    const float fi = floorf(x + s), fj = floorf(y + s), fk = floorf(z + s);
+    const int32_t i = (int32_t)fi, j = (int32_t)fj, k = (int32_t)fk;
+    const float t = (float)(i + j + k) * G3;
+    const float x0 = x - (fi - t), y0 = y - (fj - t), z0 = z - (fk - t);
+    const bool gxy = x0 >= y0, gyz = y0 >= z0, gxz = x0 >= z0;
+    const bool i1 = gxy && gxz, j1 = !gxy && gyz, k1 = !gxz && !gyz;
+    const bool i2 = gxy || gxz, j2 = !gxy || gyz, k2 = !gxz || !gyz;
+    const float xm = x0 - 1.0f, ym = y0 - 1.0f, zm = z0 - 1.0f;
+    const uint32_t a0 = mul24((uint32_t)i, kP1), a1 = mul24((uint32_t)(i + 1), kP1);
+    const uint32_t b0 = mul24((uint32_t)j, kP2), b1 = mul24((uint32_t)(j + 1), kP2);
+    const uint32_t c0 = mul24((uint32_t)k, kP3) ^ seed, c1 = mul24((uint32_t)(k + 1), kP3) ^ seed;
+    NoiseGrad r{0.0f, 0.0f, 0.0f, 0.0f};
+    corner_grad(x0, y0, z0, grad_mix(xor3(a0, b0, c0)), r);
+    corner_grad((i1 ? xm : x0) + G3, (j1 ? ym : y0) + G3, (k1 ? zm : z0) + G3,
+                grad_mix(xor3(i1 ? a1 : a0, j1 ? b1 : b0, k1 ? c1 : c0)), r);
+    corner_grad((i2 ? xm : x0) + 2.0f * G3, (j2 ? ym : y0) + 2.0f * G3, (k2 ? zm : z0) + 2.0f * G3,
+                grad_mix(xor3(i2 ? a1 : a0, j2 ? b1 : b0, k2 ? c1 : c0)), r);
+    corner_grad(xm + 0.5f, ym + 0.5f, zm + 0.5f, grad_mix(xor3(a1, b1, c1)), r);
+    r.n *= kNoiseScale;
+    r.gx *= kNoiseScale;
+    r.gy *= kNoiseScale;
+    r.gz *= kNoiseScale;
+    return r;
+}
+
+// Sum over the lanes of a quad, in every lane of it.
+__device__ __forceinline__ float quad_sum(float v) {
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1, 0xF, 0xF, true));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x4E, 0xF, 0xF, true));
+    return v;
+}
+
+// The first k octaves expanded about p, lane `o` of the quad taking octave
+// o: the sum and its step per sample, in every lane of the quad.
+__device__ __forceinline__ NoiseGrad expand(const SamplerDev& S, int k, int o, float delta, float px, float py,
+                                            float pz) {
+    NoiseGrad r{0.0f, 0.0f, 0.0f, 0.0f};
+    if (o < k) {
+        const float f = S.fo[o], a = S.ao[o], af = a * (f * delta);
+        const NoiseGrad g = snoise3_grad(px * f, py * f, pz * f, S.seed + (uint32_t)o);
+        r = NoiseGrad{a * g.n, af * g.gx, af * g.gy, af * g.gz};
+    }
+    return NoiseGrad{quad_sum(r.n), quad_sum(r.gx), quad_sum(r.gy), quad_sum(r.gz)};
+}
+
+__global__ void __launch_bounds__(kRowThreads) k_blocks(Arenas A, int n) {
+    // per block and plane dx of it: undecided samples in the low half, air
+    // samples in the high half, bit 4 dy + dz
+    __shared__ uint32_t s_block[kWordWaves][4 * kWaveBlocks];
+    __shared__ uint8_t s_sub[kWordWaves][8 * kWaveBlocks];
+    __shared__ unsigned long long s_evals;
+    if (threadIdx.x == 0) s_evals = 0;
+    __syncthreads();
+    const SamplerDev* __restrict__ S = A.sampler;
+    const int wave = uniform_int(threadIdx.x >> 6), lane = lane_id(), o = lane & 3;
+    unsigned long long evals = 0;  // octaves at the centres of this wave's blocks (uniform)
+    const int64_t total = A.block_prefix[n];
+    for (int64_t it = (int64_t)blockIdx.x * kWordWaves + wave; it < total; it += (int64_t)gridDim.x * kWordWaves) {
+        const int j = find_chunk_wave(A.block_prefix, n, it);
+        const ChunkMeta M = read_chunk(A.meta, j);
+        const int dim = M.dim, nb = (dim + 3) >> 2, nb2 = nb * nb;
+        const int b0 = (int)(it - A.block_prefix[j]) * kWaveBlocks, b = b0 + (lane >> 2);
+        const int bx = (int)udiv24((uint32_t)b, (uint32_t)nb2, 1.0f / (float)nb2), br = b - bx * nb2;
+        const int by = (int)udiv24((uint32_t)br, (uint32_t)nb, 1.0f / (float)nb), bz = br - by * nb;
+        const float delta = M.delta;
+        const BlockPlan& bp = M.blocks;
+        // the sum at which a sample's density amp * sum * inv_norm - t2 is 0
+        // (the clamp to [-1, 1] never acts when no amplitude is negative)
+        const float per = S->amp * S->inv_norm, inv = 1.0f / per;
+        // ---- the blocks: a quad each, lane dx = o its plane of 16 samples ----
+        const int rx = dim - 4 * bx, ry = min(4, dim - 4 * by), rz = min(4, dim - 4 * bz);
+        uint32_t und = 0u, lab = 0u;
+        if (b < nb2 * nb && o < rx) und = (0x1111u * ((1u << rz) - 1u)) & ((1u << (4 * ry)) - 1u);
+        if (S->expand_ok) {
+            const NoiseGrad g = expand(*S, bp.k4, o, delta, ((float)(4 * bx) + 1.5f) * delta + M.opos[0],
+                                       ((float)(4 * by) + 1.5f) * delta + M.opos[1],
+                                       ((float)(4 * bz) + 1.5f) * delta + M.opos[2]);
+            const float plane = __builtin_fmaf((float)o - 1.5f, g.gx, g.n);
+            const float oo = o == 0 || o == 3 ? 2.0f : 0.0f;
+            float e[3];  // by the number of the other axes on which the sample is an outer one
+#pragma unroll
+            for (int c = 0; c < 3; c++) e[c] = __builtin_fmaf(bp.quad4, 0.75f + 2.0f * (float)c + oo, bp.base4);
+            uint32_t dec = 0u, neg = 0u;
+#pragma unroll
+            for (int dy = 0; dy < 4; dy++) {
+                const float t2 = ((float)(4 * by + dy) * delta + M.opos[1]) - S->y0;
+                const float row = __builtin_fmaf((float)dy - 1.5f, g.gy, plane) - t2 * inv;
+#pragma unroll
+                for (int dz = 0; dz < 4; dz++) {
+                    const float v = __builtin_fmaf((float)dz - 1.5f, g.gz, row);
+                    const int outer = (dy == 0 || dy == 3) + (dz == 0 || dz == 3);
+                    dec |= fabsf(v) > e[outer] ? 1u << (4 * dy + dz) : 0u;
+                    neg |= v < 0.0f ? 1u << (4 * dy + dz) : 0u;
+                }
+            }
+            if (per < 0.0f) neg = ~neg;  // air below the sign change, for a positive amplitude
+            lab = und & dec & neg;
+            und &= ~dec;
+        } else {  // the band alone
+            const TerrainTerms T{S->amp, S->y0, S->inv_norm};
+#pragma unroll
+            for (int dy = 0; dy < 4; dy++) {
+                const float t2 = ((float)(4 * by + dy) * delta + M.opos[1]) - T.y0;
+                const int d = decide_label(T, S->reach[0], 0.0f, t2);
+                const uint32_t row = 0xFu << (4 * dy);
+                lab |= d == 1 ? und & row : 0u;
+                und &= d ? ~row : ~0u;
+            }
+        }
+        if (bp.k4) evals += (unsigned long long)(bp.k4 * min(kWaveBlocks, nb2 * nb - b0));
+        // ---- their sub-blocks with undecided samples: a quad each ----
+        if (bp.k2) {
+            const uint32_t pair = und | (uint32_t)__builtin_amdgcn_update_dpp(0, (int)und, 0xB1, 0xF, 0xF, true);
+            s_block[wave][lane] = und | (lab << 16);
+            uint32_t ns = 0;
+#pragma unroll
+            for (int q = 0; q < 4; q++) {  // (sy, sz); lanes 0 and 2 of the quad take sx = 0 and 1
+                const bool need = !(o & 1) && (pair & (0x33u << (8 * (q >> 1) + 2 * (q & 1)))) != 0u;
+                const uint64_t bal = __ballot(need);
+                if (need) s_sub[wave][ns + mbcnt64(bal)] = (uint8_t)((lane >> 2) * 8 + (o >> 1) * 4 + q);
+                ns += (uint32_t)__popcll(bal);
+            }
+            wave_sync();
+            evals += (unsigned long long)bp.k2 * ns;
+            const float e2 = __builtin_fmaf(bp.quad2, 0.75f, bp.base2);
+            for (uint32_t i0 = 0; i0 < ns; i0 += kWaveBlocks) {
+                const uint32_t i = i0 + (uint32_t)(lane >> 2);
+                const uint32_t sub = s_sub[wave][min(i, ns - 1u)];
+                const int sx = (int)(sub >> 2) & 1, sy = (int)(sub >> 1) & 1, sz = (int)sub & 1;
+                const int at = __shfl(bx | (by << 8) | (bz << 16), (int)(4u * (sub >> 3)));  // its block's quad
+                const int x = 4 * (at & 255) + 2 * sx, y = 4 * ((at >> 8) & 255) + 2 * sy, z = 4 * (at >> 16) + 2 * sz;
+                const NoiseGrad g = expand(*S, bp.k2, o, delta, ((float)x + 0.5f) * delta + M.opos[0],
+                                           ((float)y + 0.5f) * delta + M.opos[1], ((float)z + 0.5f) * delta + M.opos[2]);
+                // lane (dx, dy) of the quad: its two samples
+                const int dx = o >> 1, dy = o & 1;
+                const float t2 = ((float)(y + dy) * delta + M.opos[1]) - S->y0;
+                const float row = __builtin_fmaf((float)dx - 0.5f, g.gx, __builtin_fmaf((float)dy - 0.5f, g.gy, g.n)) -
+                                  t2 * inv;
+                uint32_t dec = 0u, neg = 0u;
+#pragma unroll
+                for (int dz = 0; dz < 2; dz++) {
+                    const float v = __builtin_fmaf((float)dz - 0.5f, g.gz, row);
+                    dec |= fabsf(v) > e2 ? 1u << dz : 0u;
+                    neg |= v < 0.0f ? 1u << dz : 0u;
+                }
+                if (per < 0.0f) neg = ~neg;
+                if (i < ns) {
+                    uint32_t* w = &s_block[wave][4 * (sub >> 3) + 2 * sx + dx];
+                    const int sh = 4 * (2 * sy + dy) + 2 * sz;
+                    const uint32_t hit = *w & (dec << sh);  // the other bits may be cleared meanwhile
+                    atomicAnd(w, ~hit);
+                    atomicOr(w, (hit & (neg << sh)) << 16);
+                }
+            }
+            wave_sync();
+            const uint32_t w = s_block[wave][lane];
+            und = w & 0xFFFFu;
+            lab = w >> 16;
+            wave_sync();  // before the next item's
+        }
+        // a byte per four samples of a row: undecided low, air high
+        if (b < nb2 * nb && o < rx) {
+            uint8_t* __restrict__ N = A.signs + M.dens_off + ((int64_t)(4 * bx + o) * dim + 4 * by) * nb + bz;
+            for (int dy = 0; dy < ry; dy++)
+                N[dy * nb] = (uint8_t)(((und >> (4 * dy)) & 15u) | (((lab >> (4 * dy)) & 15u) << 4));
+        }
+    }
+    if (lane == 0 && evals) atomicAdd(&s_evals, evals);
+    __syncthreads();
+    if (threadIdx.x == 0 && (int)blockIdx.x < A.stat_cap) A.stat_blocks[2 * A.stat_cap + blockIdx.x] = s_evals;
+}
+
+// ------------------------------------------------------------------------
+// terrain (adaptive): labels from k_blocks' decisions, every octave of the
+// samples it left open.
+//
+// A workgroup takes four items of label words, a wave each: a lane reads the
+// decisions of 16 consecutive samples (a byte holds four of a row), and the
+// open samples of all four items go to one list that the workgroup's lanes
+// then share.  While the list is long (a field too rough for the expansions)
+// it is evaluated octave by octave and compacted in place: after k octaves
+// the FP32 partial sum S_k bounds the final sum, each remaining step being
+// fma(a_o, n_o, S) with |n_o| <= 1 and rounding monotone, so that S_O lies in
+// [S_k - reach[k], S_k + reach[k]] (reach: sum_{o>=k} |a_o| widened by the
+// rounding of those steps and of the two bounds, host side), and the density
+// is monotone in S.  Samples that run all octaves get their exact density
+// and their bit in the `exact` bitmap; the others only their label (k_count
+// finishes the densities of those that are endpoints of a sign-changing
+// edge).  Labels and every density that a mesh reads are those of the full
+// evaluation, bit for bit.  Bound by VALU issue (49 of 69 us on the batch
+// above).  kTerrainDirect: short lists lose less to octaves that an early
+// decision would have spared than to the rounds' barriers.
+// ------------------------------------------------------------------------
+constexpr int kTerrainSamples = kWordWaves * kItemSamples;
+constexpr int kTerrainDirect = 1024;  // open samples up to which all octaves run at once
+
+__global__ void __launch_bounds__(kRowThreads) k_terrain(Arenas A, int n) {
+    struct Geom {
+        ChunkGeom G;
+        int dim, chunk, i0;
+        int64_t dens_off;
+    };
+    __shared__ Geom s_geom[kWordWaves];
+    __shared__ uint64_t s_lab[kWordWaves * kItemWords], s_exact[kWordWaves * kItemWords];
+    __shared__ uint16_t s_list[kTerrainSamples];
+    __shared__ float s_sum[kTerrainSamples];
+    __shared__ uint32_t s_n;
+    __shared__ unsigned long long s_evals;
+    __shared__ float s_oct[3][BMF_MAX_OCTAVES + 1];  // per octave: frequency, amplitude, reach
+    const SamplerDev* __restrict__ S = A.sampler;
+    const TerrainTerms TT{S->amp, S->y0, S->inv_norm};
+    const int O = S->octaves;
+    const uint32_t seed0 = S->seed;  // octave k uses seed0 + k
+    const int tid = threadIdx.x, wave = uniform_int(tid >> 6), lane = lane_id();
+    for (int t = tid; t <= O; t += blockDim.x) {
+        s_oct[0][t] = t < O ? S->fo[t] : 0.0f;
+        s_oct[1][t] = t < O ? S->ao[t] : 0.0f;
+        s_oct[2][t] = S->reach[t];
+    }
+    if (tid == 0) s_evals = 0;
+    unsigned long long evals = 0;  // octaves this lane evaluated
+    const int64_t total = A.ctr->total_items;
+    // position and y - y0 of list entry v: wave << 10 | sample of its item
+    auto locate = [&](uint32_t v, uint32_t& i, float& px, float& py, float& pz) {
+        const Geom& g = s_geom[v >> 10];
+        const uint32_t dim = (uint32_t)g.dim, dim2 = dim * dim;
+        i = (uint32_t)g.i0 + (v & 1023u);
+        sample_coords(g.G, i, dim, dim2, 1.0f / (float)dim, 1.0f / (float)dim2, px, py, pz);
+    };
+    auto set_bit = [&](uint64_t* words, uint32_t v) {
+        atomicOr(reinterpret_cast<uint32_t*>(words) + (v >> 5), 1u << (v & 31u));
+    };
+    for (int64_t it0 = (int64_t)blockIdx.x * kWordWaves; it0 < total; it0 += (int64_t)gridDim.x * kWordWaves) {
+        if (tid == 0) s_n = 0;
+        __syncthreads();
+        const int64_t it = it0 + wave;
+        uint32_t und = 0u, lab = 0u;
+        if (it < total) {
+            const int j = find_item_wave(A.meta, n, it);
+            const ChunkMeta M = read_chunk(A.meta, j);
+            const int dim = M.dim, d2 = dim * dim, n3 = d2 * dim, nb = (dim + 3) >> 2;
+            const int item = (int)(it - M.item_slot);
+            if (lane == 0) {
+                A.item_map[it] = make_int2(j, item);
+                s_geom[wave] = Geom{{M.opos[0], M.opos[1], M.opos[2], M.delta}, dim, j, item * kItemSamples, M.dens_off};
+            }
+            // the lane's 16 samples, a run within a row at a time
+            int i = item * kItemSamples + 16 * lane;
+            if (i < n3) {
+                const int x = (int)udiv24((uint32_t)i, (uint32_t)d2, 1.0f / (float)d2);
+                const int r = i - x * d2, y = (int)udiv24((uint32_t)r, (uint32_t)dim, 1.0f / (float)dim);
+                int z = r - y * dim;
+                const uint8_t* __restrict__ N = A.signs + M.dens_off + (int64_t)(x * dim + y) * nb;
+                for (int got = 0; got < 16 && i < n3;) {
+                    uint64_t w;  // the row's bytes from z on: 5 are used
+                    __builtin_memcpy(&w, N + (z >> 2), 8);
+                    const int run = min(16 - got, dim - z);
+                    const uint32_t m = (1u << run) - 1u;
+                    und |= ((low_nibbles(w) >> (z & 3)) & m) << got;
+                    lab |= ((low_nibbles(w >> 4) >> (z & 3)) & m) << got;
+                    got += run;
+                    i += run;
+                    z = 0;
+                    N += nb;
+                }
+            }
+        }
+        reinterpret_cast<uint16_t*>(s_lab)[tid] = (uint16_t)lab;
+        reinterpret_cast<uint16_t*>(s_exact)[tid] = 0u;
+        {
+            uint32_t cnt, b = und;
+            uint32_t at = wave_prefix<5>((uint32_t)__popc(b), cnt);
+            uint32_t base = 0;
+            if (lane == 0 && cnt) base = atomicAdd(&s_n, cnt);
+            at += (uint32_t)uniform_int((int)base);
+            while (b) {
+                s_list[at++] = (uint16_t)(wave << 10 | (16 * lane + __ffs(b) - 1));
+                b &= b - 1u;
+            }
+        }
+        __syncthreads();
+        uint32_t nq = s_n;
+        int k = 0;
+        // ---- a long list: an octave at a time, the survivors moved up ----
+        while (nq > (uint32_t)kTerrainDirect && k < O - 1) {
+            __syncthreads();  // every thread has read s_n
+            if (tid == 0) s_n = 0;
+            for (uint32_t e0 = 0; e0 < nq; e0 += kRowThreads) {
+                const uint32_t e = e0 + (uint32_t)tid;
+                const uint32_t v = e < nq ? s_list[e] : 0u;
+                float sum = e < nq && k > 0 ? s_sum[e] : 0.0f;
+                __syncthreads();  // this part of the list is read: it may be overwritten
+                int dec = 2;
+                if (e < nq) {
+                    uint32_t i;
+                    float px, py, pz;
+                    locate(v, i, px, py, pz);
+                    const float f = s_oct[0][k];
+                    sum = __builtin_fmaf(s_oct[1][k], snoise3(px * f, py * f, pz * f, seed0 + (uint32_t)k), sum);
+                    dec = decide_label(TT, s_oct[2][k + 1], sum, py - TT.y0);
+                    if (dec == 1) set_bit(s_lab, v);
+                    evals++;
+                }
+                const uint64_t push = __ballot(dec == 0);
+                if (push) {
+                    uint32_t base = 0;
+                    if (lane == 0) base = atomicAdd(&s_n, (uint32_t)__popcll(push));
+                    const uint32_t at = (uint32_t)uniform_int((int)base) + mbcnt64(push);
+                    if (dec == 0) {
+                        s_list[at] = (uint16_t)v;
+                        s_sum[at] = sum;
+                    }
+                }
+            }
+            __syncthreads();
+            nq = s_n;
+            k++;
+        }
+        // ---- the rest of the octaves of the open samples ----
+        for (uint32_t e = (uint32_t)tid; e < nq; e += kRowThreads) {
+            const uint32_t v = s_list[e];
+            float sum = k > 0 ? s_sum[e] : 0.0f;
+            uint32_t i;
+            float px, py, pz;
+            locate(v, i, px, py, pz);
+            for (int o = k; o < O; o++) {
+                const float f = s_oct[0][o];
+                sum = __builtin_fmaf(s_oct[1][o], snoise3(px * f, py * f, pz * f, seed0 + (uint32_t)o), sum);
+            }
+            const float d = density_from_sum(TT, sum, py - TT.y0);
+            A.dens[s_geom[v >> 10].dens_off + i] = d;
+            if (d < 0.0f) set_bit(s_lab, v);
+            set_bit(s_exact, v);
+            evals += (unsigned long long)(O - k);
+        }
+        __syncthreads();
+        // ---- the items' words ----
+        if (tid < kWordWaves * kItemWords && it0 + tid / kItemWords < total) {
+            const Geom& g = s_geom[tid / kItemWords];
+            const int i = g.i0 + 64 * (tid % kItemWords), left = g.dim * g.dim * g.dim - i;
+            const uint64_t lb = s_lab[tid];
+            if (left > 0) {
+                const int64_t w = A.meta[g.chunk].lab_off + (i >> 6);
+                A.labels[w] = lb;
+                A.exact[w] = s_exact[tid];
+            }
+            const uint64_t have = left > 0 ? ~bits_from(left) : 0ull;
+            const uint64_t group = 0xFFFFull << (lane & 48);
+            const bool air = (__ballot((lb & have) != 0ull) & group) != 0ull;
+            const bool solid = (__ballot((~lb & have) != 0ull) & group) != 0ull;
+            if ((lane & 15) == 0) {
+                if (air && !A.meta[g.chunk].any_air) atomicOr(&A.meta[g.chunk].any_air, 1u);
+                if (solid && !A.meta[g.chunk].any_solid) atomicOr(&A.meta[g.chunk].any_solid, 1u);
+            }
+        }
+        __syncthreads();  // before the next items'
+    }
+    if (evals) atomicAdd(&s_evals, evals);
+    __syncthreads();
+    if (tid == 0 && (int)blockIdx.x < A.stat_cap) A.stat_blocks[blockIdx.x] = s_evals;
+}
+
+// Sampling modes of k_sample, fixed per launch by the host: the CSG union with
+// the chunk's culled primitives staged in LDS once per tile; a 2D noise field
+// with the noise of the tile's (x, z) columns evaluated once into LDS and
+// broadcast along y; every other case (external densities, implicit shapes,
+// 3D noise fields, the terrain in full) evaluated directly.  Persistent:
+// workgroups pull tiles of Arenas::sample_tile consecutive samples of one
+// chunk from an atomic work queue.
+constexpr int kSampleGeneric = 0, kSampleCsg = 2, kSampleSlab = 3;
 
 template <int ROUNDS, int MODE>
 __global__ void __launch_bounds__(kSampleThreads) k_sample(Arenas A, int n) {
     constexpr int kTile = ROUNDS * kSampleThreads;
-    constexpr bool adapt = MODE == kSampleAdaptive;
-    constexpr int kQ = adapt ? kTile : 1;                       // octave queues (adaptive mode only)
     constexpr int kC = MODE == kSampleCsg ? 2 * kCsgStage : 1;  // staged CSG primitives
     // 2D noise columns of a tile: its samples span at most kTile / dim^2 + 2
     // x-planes of dim columns, i.e. at most kTile / dim + 2 dim <= kTile / 2 + 2 BMF_MAX_DIM
     constexpr int kSlab = MODE == kSampleSlab ? kTile / 2 + 2 * BMF_MAX_DIM : 1;
     __shared__ float s_slab[kSlab];
     __shared__ int64_t s_tile;
-    __shared__ uint32_t s_qn[2];
-    __shared__ uint16_t s_qi[2][kQ];
-    __shared__ float s_qs[2][kQ];
     __shared__ float4 s_csg[kC];
     __shared__ unsigned long long s_lab[kTile / 64];
     __shared__ unsigned long long s_exact[kTile / 64];
     __shared__ uint32_t s_flags;
     const SamplerDev* __restrict__ S = A.sampler;
-    const TerrainTerms TT{S->amp, S->y0, S->inv_norm};
-    const float reach0 = S->reach[0];
-    const int O = S->octaves;
-    const uint32_t seed0 = S->seed;  // octave k uses seed0 + k
-    // adaptive mode: per-octave frequency, amplitude and reach (visible to
-    // every thread after the first barrier of the tile loop)
-    __shared__ float s_oct[3][BMF_MAX_OCTAVES + 1];
-    if constexpr (adapt) {
-        for (int t = threadIdx.x; t <= O; t += blockDim.x) {
-            s_oct[0][t] = t < O ? S->fo[t] : 0.0f;
-            s_oct[1][t] = t < O ? S->ao[t] : 0.0f;
-            s_oct[2][t] = S->reach[t];
-        }
-    }
     const int64_t total = A.ctr->total_tiles;
     const int lane = lane_id();
-    const uint64_t lt = lanemask_lt();
-    unsigned long long evals = 0;  // adaptive mode: octaves this wave evaluated (wave-uniform)
-    __shared__ unsigned long long s_evals;
-    if (threadIdx.x == 0) s_evals = 0;  // ordered before its use by the tile loop's barriers
     // (chunk, item) of every item of the word kernels that follow
     for (int j = blockIdx.x; j < n; j += gridDim.x) {
         const ChunkMeta& M = A.meta[j];
@@ -431,8 +860,6 @@ __global__ void __launch_bounds__(kSampleThreads) k_sample(Arenas A, int n) {
     for (;;) {
         if (threadIdx.x == 0) {
             s_tile = (int64_t)atomicAdd(&A.ctr->sample_head, 1ull);
-            s_qn[0] = 0;
-            s_qn[1] = 0;
             s_flags = 0;
         }
         __syncthreads();
@@ -499,42 +926,8 @@ __global__ void __launch_bounds__(kSampleThreads) k_sample(Arenas A, int n) {
                     sample_index(i, dim, dim2, rd, rd2, cx, cy, cz);
                 }
             }
-            bool air = false, done = true, fin = false;
-            int kq = 0;         // adaptive: the next octave of the wave's undecided samples
-            float sum0 = 0.0f;  // and their partial sum
-            if constexpr (adapt) {
-                float px = 0.0f, py = 0.0f, pz = 0.0f, t2 = 0.0f;
-                int dec = 2;
-                if (valid) {
-                    sample_position(G, cx, cy, cz, px, py, pz);
-                    t2 = py - TT.y0;
-                    dec = decide_label(TT, reach0, 0.0f, t2);
-                }
-                // while nearly all of the wave's samples are undecided it
-                // evaluates their octaves here, as the rounds would (same
-                // operations); the survivors of a sparse wave are queued with
-                // their next octave, so that the rounds run on dense waves
-                for (;;) {
-                    const uint32_t live = (uint32_t)__popcll(__ballot(valid && dec == 0));
-                    if (kq >= O || live < (uint32_t)kInPlaceOctave) break;
-                    evals += live;
-                    if (valid && dec == 0) {
-                        const float f = s_oct[0][kq];
-                        sum0 = __builtin_fmaf(s_oct[1][kq], snoise3(px * f, py * f, pz * f, seed0 + (uint32_t)kq), sum0);
-                        if (kq == O - 1) {
-                            const float d = density_from_sum(TT, sum0, t2);
-                            dens[i] = d;
-                            dec = d < 0.0f ? 1 : 2;
-                            fin = true;
-                        } else {
-                            dec = decide_label(TT, s_oct[2][kq + 1], sum0, t2);
-                        }
-                    }
-                    kq++;
-                }
-                done = dec != 0;
-                air = dec == 1;
-            } else if (valid) {
+            bool air = false;
+            if (valid) {
                 float px, py, pz;
                 sample_position(G, cx, cy, cz, px, py, pz);
                 float d;
@@ -549,80 +942,14 @@ __global__ void __launch_bounds__(kSampleThreads) k_sample(Arenas A, int n) {
                 dens[i] = d;
                 air = d < 0.0f;
             }
-            const uint64_t bl = __ballot(valid && done && air);
-            const uint64_t push = __ballot(valid && !done);
+            const uint64_t bl = __ballot(valid && air);
             const uint64_t vb = __ballot(valid);
-            const uint64_t fb = __ballot(fin);
             if (lane == 0) {
                 s_lab[li >> 6] = bl;
-                s_exact[li >> 6] = adapt ? fb : vb;
-            }
-            if constexpr (adapt) {
-                if (push) {
-                    uint32_t base = 0;
-                    if (lane == 0) base = atomicAdd(&s_qn[0], (uint32_t)__popcll(push));
-                    base = __shfl(base, 0);
-                    if (valid && !done) {
-                        const uint32_t q = base + (uint32_t)__popcll(push & lt);
-                        s_qi[0][q] = (uint16_t)(li | ((uint32_t)kq << kQueueOctaveShift));
-                        s_qs[0][q] = sum0;
-                    }
-                }
+                s_exact[li >> 6] = vb;
             }
         }
         __syncthreads();
-        // ---- rounds on the compacted queue: each entry (sample, next octave,
-        // partial sum) advances one octave per round, so O rounds finish all ----
-        if constexpr (adapt) {
-            for (int rnd = 0; rnd < O; rnd++) {
-                const int cur = rnd & 1, nxt = cur ^ 1;
-                const uint32_t nq = s_qn[cur];
-                if (nq == 0) break;
-                for (uint32_t e0 = 0; e0 < nq; e0 += kSampleThreads) {
-                    const uint32_t e = e0 + threadIdx.x;
-                    const bool active = e < nq;
-                    uint32_t li = 0, k = 0;
-                    float sum = 0.0f;
-                    int dec = 2;
-                    if (active) {
-                        const uint32_t qv = s_qi[cur][e];
-                        li = qv & kQueueSampleMask;
-                        k = qv >> kQueueOctaveShift;
-                        sum = s_qs[cur][e];
-                        float px, py, pz;
-                        sample_coords(G, first + li, dim, dim2, rd, rd2, px, py, pz);
-                        const float t2 = py - TT.y0;
-                        const float f = s_oct[0][k];
-                        const float nz = snoise3(px * f, py * f, pz * f, seed0 + k);
-                        sum = __builtin_fmaf(s_oct[1][k], nz, sum);
-                        if ((int)k == O - 1) {
-                            const float d = density_from_sum(TT, sum, t2);
-                            dens[first + li] = d;
-                            dec = d < 0.0f ? 1 : 2;
-                            atomicOr(&s_exact[li >> 6], 1ull << (li & 63));
-                        } else {
-                            dec = decide_label(TT, s_oct[2][k + 1], sum, t2);
-                        }
-                        if (dec == 1) atomicOr(&s_lab[li >> 6], 1ull << (li & 63));
-                    }
-                    evals += (unsigned long long)__popcll(__ballot(active));
-                    const uint64_t push = __ballot(active && dec == 0);
-                    if (push) {
-                        uint32_t base = 0;
-                        if (lane == 0) base = atomicAdd(&s_qn[nxt], (uint32_t)__popcll(push));
-                        base = __shfl(base, 0);
-                        if (active && dec == 0) {
-                            const uint32_t q = base + (uint32_t)__popcll(push & lt);
-                            s_qi[nxt][q] = (uint16_t)(li | ((k + 1) << kQueueOctaveShift));
-                            s_qs[nxt][q] = sum;
-                        }
-                    }
-                }
-                __syncthreads();
-                if (threadIdx.x == 0) s_qn[cur] = 0;
-                __syncthreads();
-            }
-        }
         // ---- label and exactness words of the tile ----
         if (threadIdx.x < kTile / 64) {
             const uint32_t w0 = first + 64u * threadIdx.x;
@@ -645,10 +972,7 @@ __global__ void __launch_bounds__(kSampleThreads) k_sample(Arenas A, int n) {
         }
         __syncthreads();
     }
-    // the workgroup's count: one LDS add per wave, one plain store per workgroup
-    if (adapt && lane == 0 && evals) atomicAdd(&s_evals, evals);
-    __syncthreads();
-    if (threadIdx.x == 0 && (int)blockIdx.x < A.stat_cap) A.stat_blocks[blockIdx.x] = s_evals;
+    if (threadIdx.x == 0 && (int)blockIdx.x < A.stat_cap) A.stat_blocks[blockIdx.x] = 0ull;  // no octaves counted
 }
 
 // ------------------------------------------------------------------------
@@ -1689,14 +2013,17 @@ hipError_t launch_plan(const Arenas& A, int n, int allow_cull, int reset_bumps, 
     return hipGetLastError();
 }
 hipError_t launch_sample(const Arenas& A, int n, int blocks, int adaptive, int kind, int slab, hipStream_t s) {
-    const int mode = adaptive && kind == BMF_SAMPLER_TERRAIN ? kSampleAdaptive
-                     : kind == BMF_SAMPLER_CSG && A.csg_list  ? kSampleCsg
-                     : kind == BMF_SAMPLER_NOISE && slab      ? kSampleSlab
-                                                              : kSampleGeneric;
     const dim3 g(blocks), b(kSampleThreads);
+    if (adaptive && kind == BMF_SAMPLER_TERRAIN) {
+        hipLaunchKernelGGL(k_blocks, g, dim3(kRowThreads), 0, s, A, n);
+        hipLaunchKernelGGL(k_terrain, g, dim3(kRowThreads), 0, s, A, n);
+        return hipGetLastError();
+    }
+    const int mode = kind == BMF_SAMPLER_CSG && A.csg_list ? kSampleCsg
+                     : kind == BMF_SAMPLER_NOISE && slab   ? kSampleSlab
+                                                           : kSampleGeneric;
 #define BMF_SAMPLE(R)                                                                             \
     switch (mode) {                                                                               \
-        case kSampleAdaptive: hipLaunchKernelGGL((k_sample<R, kSampleAdaptive>), g, b, 0, s, A, n); break; \
         case kSampleCsg: hipLaunchKernelGGL((k_sample<R, kSampleCsg>), g, b, 0, s, A, n); break;           \
         case kSampleSlab: hipLaunchKernelGGL((k_sample<R, kSampleSlab>), g, b, 0, s, A, n); break;         \
         default: hipLaunchKernelGGL((k_sample<R, kSampleGeneric>), g, b, 0, s, A, n); break;               \

@@ -97,6 +97,29 @@ __device__ __forceinline__ int find_chunk(const int64_t* __restrict__ prefix, in
     return lo;
 }
 
+// The largest j in [0, n) with at(j) <= g, for at non-decreasing and
+// at(0) <= g, by one wave: 64 probes a round, two dependent loads up to 4,096
+// entries where a binary search has twelve.
+template <class F>
+__device__ __forceinline__ int find_wave(int n, int64_t g, F at) {
+    const int lane = lane_id();
+    int lo = 0, hi = n;
+    while (hi - lo > 1) {
+        const int step = (hi - lo + 63) >> 6, i = lo + lane * step;
+        const uint64_t ok = __ballot(i < hi && at(min(i, hi - 1)) <= g);
+        lo += ((int)__popcll(ok) - 1) * step;
+        hi = min(hi, lo + step);
+    }
+    return uniform_int(lo);
+}
+__device__ __forceinline__ int find_chunk_wave(const int64_t* __restrict__ prefix, int n, int64_t g) {
+    return find_wave(n, g, [=](int j) { return prefix[j]; });
+}
+// The chunk that item `it` of the word kernels belongs to.
+__device__ __forceinline__ int find_item_wave(const ChunkMeta* __restrict__ meta, int n, int64_t it) {
+    return find_wave(n, it, [=](int j) { return meta[j].item_slot; });
+}
+
 // q = n / d for n <= 2^24, 0 < d < 2^24 and a quotient below 2^22, with
 // rcp = 1/d correctly rounded.  (float)n is exact and fl(n * rcp) =
 // (n/d)(1 + e) with |e| <= 2^-23 + 2^-48, so the estimate is within 0.5 of

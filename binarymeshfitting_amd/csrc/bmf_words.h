@@ -26,6 +26,14 @@ __device__ __forceinline__ void wave_sync() {
 // Bits a .. 63 (any a).
 __device__ __forceinline__ uint64_t bits_from(int a) { return a <= 0 ? ~0ull : (a >= 64 ? 0ull : ~0ull << a); }
 
+// The low four bits of each byte, packed.
+__device__ __forceinline__ uint32_t low_nibbles(uint64_t w) {
+    w &= 0x0F0F0F0F0F0F0F0Full;
+    w = (w | (w >> 4)) & 0x00FF00FF00FF00FFull;
+    w = (w | (w >> 8)) & 0x0000FFFF0000FFFFull;
+    return (uint32_t)(w | (w >> 16));
+}
+
 // Exclusive prefix of a per-lane count below 2^BITS over the wave's lanes
 // (bit-sliced ballots), and its total.
 template <int BITS>

@@ -211,8 +211,9 @@ int bmf_last_timing(bmf_ctx* ctx, float* total_ms);
 
 /* Work done by the last extraction: the samples of its sampled chunks and,
  * for the terrain sampler, the noise octaves that its adaptive sampling
- * evaluated, summed over samples (every octave of every sample, as the
- * reference's block sampler computes, would be samples * octaves), and those
+ * evaluated, at samples and at the centres of sample blocks (every octave of
+ * every sample, as the reference's block sampler computes, would be
+ * samples * octaves), and those
  * the refinement of early-labelled edge endpoints evaluated (0 for the other
  * samplers).  Valid after bmf_result of a BATCHED extraction (or after
  * bmf_profile_stages); BMF_ESTATE after a PLAIN one, whose chunks run one
