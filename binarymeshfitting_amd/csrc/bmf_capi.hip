@@ -35,8 +35,7 @@ hipError_t dalloc(T** p, int64_t count) {
 
 void free_arenas(bmf_ctx* c) {
     Arenas& A = c->A;
-    void* ptrs[] = {A.meta,    A.descs,     A.results,  A.tile_prefix, A.block_prefix, A.signs, A.plan_part, A.plan_tmp, A.stat_blocks, A.item_map, A.smooth_list, A.smooth_prefix,
-                    A.smooth_tprefix, A.smooth_xcd_v, A.smooth_xcd_t, A.smooth_vmap, A.smooth_tmap, A.edges, A.word_pre, A.item_e, A.item_c, A.cen4,
+    void* ptrs[] = {A.meta,    A.descs,     A.results,  A.tile_prefix, A.block_prefix, A.signs, A.plan_part, A.stat_blocks, A.item_map, A.smooth_vmap, A.smooth_tmap, A.edges, A.word_pre, A.item_e, A.item_c, A.cen4,
                     A.dens,    A.labels,    A.exact, A.cell_tb,   A.cell_mask,
                     A.pos,     A.pos4,      A.boundary, A.vedge,       A.vring,        A.idx,          A.ctr,
                     A.sampler, c->d_spheres, c->d_boxes, A.ring, A.ring_n, A.qef_err, A.nrm4, A.fn4, A.nrm,
@@ -293,6 +292,8 @@ int bmf_create(bmf_ctx** out, int device, const bmf_limits* lim) {
     const int64_t nw = lim->max_samples / 64 + nc, ni = nw / kItemWords + nc;  // label words, word items
     A.cap_vertices = lim->max_vertices;
     A.cap_indices = lim->max_indices;
+    A.cap_vtiles = A.cap_vertices / kSmoothThreads + nc + 1;
+    A.cap_ttiles = A.cap_indices / 3 / kSmoothThreads + nc + 1;
     A.sample_tile = kSampleTileDefault;
     A.smoothing_follows = 1;
     A.stat_cap = 64 * c->cu_count;
@@ -300,14 +301,11 @@ int bmf_create(bmf_ctx** out, int device, const bmf_limits* lim) {
     ok = ok && dalloc(&A.meta, nc) == hipSuccess && dalloc(&A.descs, nc) == hipSuccess &&
          dalloc(&A.results, nc) == hipSuccess && dalloc(&A.tile_prefix, nc + 1) == hipSuccess &&
          dalloc(&A.block_prefix, nc + 1) == hipSuccess && dalloc(&A.signs, lim->max_samples + 16) == hipSuccess &&
-         dalloc(&A.plan_part, 40 * ((nc + 1023) / 1024) + 64) == hipSuccess &&
-         dalloc(&A.plan_tmp, 2 * nc) == hipSuccess &&
+         dalloc(&A.plan_part, 10 * ((nc + 1023) / 1024) + 1) == hipSuccess &&
          dalloc(&A.stat_blocks, 3 * (int64_t)(64 * c->cu_count)) == hipSuccess &&
-         dalloc(&A.item_map, ni) == hipSuccess && dalloc(&A.smooth_list, nc) == hipSuccess &&
-         dalloc(&A.smooth_prefix, nc + 1) == hipSuccess && dalloc(&A.smooth_tprefix, nc + 1) == hipSuccess &&
-         dalloc(&A.smooth_xcd_v, kXcds + 1) == hipSuccess && dalloc(&A.smooth_xcd_t, kXcds + 1) == hipSuccess &&
-         dalloc(&A.smooth_vmap, A.cap_vertices / kSmoothThreads + nc + 1) == hipSuccess &&
-         dalloc(&A.smooth_tmap, A.cap_indices / 3 / kSmoothThreads + nc + 1) == hipSuccess &&
+         dalloc(&A.item_map, ni) == hipSuccess &&
+         dalloc(&A.smooth_vmap, kXcds * A.cap_vtiles) == hipSuccess &&
+         dalloc(&A.smooth_tmap, kXcds * A.cap_ttiles) == hipSuccess &&
          dalloc(&A.edges, nw) == hipSuccess && dalloc(&A.word_pre, nw) == hipSuccess &&
          dalloc(&A.item_e, ni) == hipSuccess && dalloc(&A.item_c, ni) == hipSuccess &&
          dalloc(&A.cen4, A.cap_indices / 3 + 1) == hipSuccess &&

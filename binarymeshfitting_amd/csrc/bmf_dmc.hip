@@ -679,9 +679,10 @@ __global__ void __launch_bounds__(kRowThreads) k_dmc_quads(Arenas A) {
 // loaded together.  Tiles come from the per-frame tile map.
 __global__ void __launch_bounds__(kSmoothThreads) k_dual_n(Arenas A, int m) {
     const int xcd = blockIdx.x % kXcds;
-    const int64_t end = A.smooth_xcd_t[xcd + 1];
-    for (int64_t tile = A.smooth_xcd_t[xcd] + blockIdx.x / kXcds; tile < end; tile += gridDim.x / kXcds) {
-        const int2 tm = A.smooth_tmap[tile];  // (chunk, tile within the chunk)
+    const int end = A.ctr->xcd_ttiles[xcd];
+    const int2* __restrict__ map = A.smooth_tmap + (int64_t)xcd * A.cap_ttiles;
+    for (int tile = blockIdx.x / kXcds; tile < end; tile += gridDim.x / kXcds) {
+        const int2 tm = map[tile];  // (chunk, tile within the chunk)
         const ChunkMeta& M = A.meta[uniform_int(tm.x)];
         const int iters = uniform_int(M.iters), N = uniform_int(M.ipp), T = uniform_int(M.T);
         const uint32_t V = (uint32_t)uniform_int(M.V);
@@ -723,10 +724,11 @@ __global__ void __launch_bounds__(kSmoothThreads) k_dual_n(Arenas A, int m) {
 constexpr int kRingRoundN = 8;
 __global__ void __launch_bounds__(kSmoothThreads) k_primal_ring(Arenas A, int m) {
     const int xcd = blockIdx.x % kXcds;
-    const int64_t end = A.smooth_xcd_v[xcd + 1];
+    const int end = A.ctr->xcd_vtiles[xcd];
+    const int2* __restrict__ map = A.smooth_vmap + (int64_t)xcd * A.cap_vtiles;
     const int64_t cap = A.cap_vertices;
-    for (int64_t tile = A.smooth_xcd_v[xcd] + blockIdx.x / kXcds; tile < end; tile += gridDim.x / kXcds) {
-        const int2 tm = A.smooth_vmap[tile];  // (chunk, tile within the chunk)
+    for (int tile = blockIdx.x / kXcds; tile < end; tile += gridDim.x / kXcds) {
+        const int2 tm = map[tile];  // (chunk, tile within the chunk)
         const ChunkMeta& M = A.meta[uniform_int(tm.x)];
         const int K = uniform_int(M.iters), N = uniform_int(M.ipp), V = uniform_int(M.V), bp = uniform_int(M.bp);
         const int64_t i_off = M.i_off, v_off = M.v_off;
@@ -788,40 +790,39 @@ __device__ __forceinline__ float3 unit_cross(float ux, float uy, float uz, float
 }
 
 __global__ void __launch_bounds__(kSmoothThreads) k_dual_n_nrm(Arenas A, int m) {
-    const int nsm = A.ctr->n_smooth;
     const int xcd = blockIdx.x % kXcds;
-    const int64_t end = A.smooth_xcd_t[xcd + 1];
-    for (int64_t tile = A.smooth_xcd_t[xcd] + blockIdx.x / kXcds; tile < end; tile += gridDim.x / kXcds) {
-        const int k = find_chunk(A.smooth_tprefix, nsm, tile);
-        const ChunkMeta& M = A.meta[A.smooth_list[k]];
-        const int K = M.iters;
+    const int end = A.ctr->xcd_ttiles[xcd];
+    const int2* __restrict__ map = A.smooth_tmap + (int64_t)xcd * A.cap_ttiles;
+    for (int tile = blockIdx.x / kXcds; tile < end; tile += gridDim.x / kXcds) {
+        const int2 tm = map[tile];  // (chunk, tile within the chunk)
+        const ChunkMeta& M = A.meta[uniform_int(tm.x)];
+        const int K = uniform_int(M.iters), N = uniform_int(M.ipp), T = uniform_int(M.T);
+        const uint32_t V = (uint32_t)uniform_int(M.V);
+        const int64_t i_off = M.i_off, v_off = M.v_off;
         if (max(K, 1) <= m) continue;
-        const int64_t t = (tile - A.smooth_tprefix[k]) * kSmoothThreads + threadIdx.x;
-        if (t >= M.T) continue;
-        const int N = M.ipp;
-        const uint32_t* __restrict__ I = A.idx + M.i_off + (int64_t)N * t;
-        const float4* __restrict__ P = A.pos4 + M.v_off;
-        const float4* __restrict__ NV = A.nrm4 + M.v_off;
-        uint32_t u[4] = {0u, 0u, 0u, 0u};
-        bool ok = true;
-        for (int c = 0; c < N; c++) {
-            u[c] = I[c];
-            if (u[c] >= (uint32_t)M.V) ok = false;
-        }
-        if (!ok) {
+        const int64_t t = (int64_t)uniform_int(tm.y) * kSmoothThreads + threadIdx.x;
+        if (t >= T) continue;
+        // N = 3 or 4, one per chunk: the corner ids, then the corners, load
+        // together (a triangle's fourth repeats its first)
+        const uint32_t* __restrict__ I = A.idx + i_off + (int64_t)N * t;
+        const float4* __restrict__ P = A.pos4 + v_off;
+        const float4* __restrict__ NV = A.nrm4 + v_off;
+        const uint32_t u[4] = {I[0], I[1], I[2], I[N == 4 ? 3 : 0]};
+        if (u[0] >= V || u[1] >= V || u[2] >= V || u[3] >= V) {
             A.ctr->error = 11;
             continue;
         }
-        float4 q[4];
-        for (int c = 0; c < N; c++) q[c] = P[u[c]];
+        const float4 q[4] = {P[u[0]], P[u[1]], P[u[2]], P[u[3]]};
         float cx = 0.0f, cy = 0.0f, cz = 0.0f;
-        for (int c = 0; c < N; c++) {
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            if (c == 3 && N == 3) break;
             cx = cx + q[c].x;
             cy = cy + q[c].y;
             cz = cz + q[c].z;
         }
         const float fN = (float)N;
-        const int64_t tt = M.i_off / N + t;
+        const int64_t tt = i_off / N + t;
         A.cen4[tt] = make_float4(cx / fN, cy / fN, cz / fN, 0.0f);
         const int max_norms = min(K / 2 - 3, 10);
         float4 fn;
@@ -846,11 +847,13 @@ __global__ void __launch_bounds__(kSmoothThreads) k_dual_n_nrm(Arenas A, int m) 
             }
         } else {
             float sx = 0.0f, sy = 0.0f, sz = 0.0f;
-            for (int c = 0; c < N; c++) {
-                const float4 nc = NV[u[c]];
-                sx = sx + nc.x;
-                sy = sy + nc.y;
-                sz = sz + nc.z;
+            const float4 nc[4] = {NV[u[0]], NV[u[1]], NV[u[2]], NV[u[3]]};
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                if (c == 3 && N == 3) break;
+                sx = sx + nc[c].x;
+                sy = sy + nc[c].y;
+                sz = sz + nc[c].z;
             }
             fn = make_float4(sx, sy, sz, 0.0f);
         }
@@ -865,34 +868,47 @@ __global__ void __launch_bounds__(kSmoothThreads) k_dual_n_nrm(Arenas A, int m) 
 // boundary vertices stay unless boundary processing (K > 0 only); the last
 // step writes the unit normal (0 for a zero normal).
 __global__ void __launch_bounds__(kSmoothThreads) k_primal_ring_nrm(Arenas A, int m) {
-    const int nsm = A.ctr->n_smooth;
     const int xcd = blockIdx.x % kXcds;
-    const int64_t end = A.smooth_xcd_v[xcd + 1];
-    for (int64_t tile = A.smooth_xcd_v[xcd] + blockIdx.x / kXcds; tile < end; tile += gridDim.x / kXcds) {
-        const int k = find_chunk(A.smooth_prefix, nsm, tile);
-        const ChunkMeta& M = A.meta[A.smooth_list[k]];
-        const int K = M.iters;
+    const int end = A.ctr->xcd_vtiles[xcd];
+    const int2* __restrict__ map = A.smooth_vmap + (int64_t)xcd * A.cap_vtiles;
+    const int64_t cap = A.cap_vertices;
+    for (int tile = blockIdx.x / kXcds; tile < end; tile += gridDim.x / kXcds) {
+        const int2 tm = map[tile];  // (chunk, tile within the chunk)
+        const ChunkMeta& M = A.meta[uniform_int(tm.x)];
+        const int K = uniform_int(M.iters), N = uniform_int(M.ipp), V = uniform_int(M.V), bp = uniform_int(M.bp);
+        const int64_t i_off = M.i_off, v_off = M.v_off;
         const int steps = max(K, 1);
         if (steps <= m) continue;
-        const int64_t v = (tile - A.smooth_prefix[k]) * kSmoothThreads + threadIdx.x;
-        if (v >= M.V) continue;
-        const int64_t g = M.v_off + v;
+        const int64_t v = (int64_t)uniform_int(tm.y) * kSmoothThreads + threadIdx.x;
+        if (v >= V) continue;
+        const int64_t g = v_off + v;
+        const uint8_t bnd = A.boundary[g];
         const int n = (int)min(A.ring_n[g], (uint32_t)kRingSlots);
-        const int64_t t_off = M.i_off / M.ipp;
-        const float4* __restrict__ C = A.cen4 + t_off;
-        const float4* __restrict__ F = A.fn4 + t_off;
         float4 nv = A.nrm4[g];
+        const float4* __restrict__ C = A.cen4 + i_off / N;
+        const float4* __restrict__ F = A.fn4 + i_off / N;
         if (n > 0) {
             float sx = 0.0f, sy = 0.0f, sz = 0.0f, nx = 0.0f, ny = 0.0f, nz = 0.0f;
-            for (int i = 0; i < n; i++) {
-                const uint32_t pid = A.ring[(int64_t)i * A.cap_vertices + g];
-                const float4 q = C[pid], f = F[pid];
-                sx = sx + q.x;
-                sy = sy + q.y;
-                sz = sz + q.z;
-                nx = nx + f.x;
-                ny = ny + f.y;
-                nz = nz + f.z;
+            for (int i0 = 0; i0 < n; i0 += kRingRoundN) {
+                uint32_t id[kRingRoundN];
+#pragma unroll
+                for (int k = 0; k < kRingRoundN; k++) id[k] = A.ring[(int64_t)(i0 + k < n ? i0 + k : i0) * cap + g];
+                float4 q[kRingRoundN], f[kRingRoundN];
+#pragma unroll
+                for (int k = 0; k < kRingRoundN; k++) {
+                    q[k] = C[id[k]];
+                    f[k] = F[id[k]];
+                }
+#pragma unroll
+                for (int k = 0; k < kRingRoundN; k++) {
+                    const bool ok = i0 + k < n;
+                    sx = ok ? sx + q[k].x : sx;
+                    sy = ok ? sy + q[k].y : sy;
+                    sz = ok ? sz + q[k].z : sz;
+                    nx = ok ? nx + f[k].x : nx;
+                    ny = ok ? ny + f[k].y : ny;
+                    nz = ok ? nz + f[k].z : nz;
+                }
             }
             const float fc = (float)n;
             float ax = nx / fc, ay = ny / fc, az = nz / fc;
@@ -907,7 +923,7 @@ __global__ void __launch_bounds__(kSmoothThreads) k_primal_ring_nrm(Arenas A, in
                 nv = make_float4(ax, ay, az, 0.0f);
                 A.nrm4[g] = nv;
             }
-            if (K > 0 && (M.bp || !A.boundary[g])) {
+            if (K > 0 && (bp || !bnd)) {
                 const float px = sx / fc, py = sy / fc, pz = sz / fc;
                 A.pos4[g] = make_float4(px, py, pz, 0.0f);
                 if (m == K - 1) {
@@ -941,10 +957,6 @@ hipError_t launch_dmc_emit(const Arenas& A, int blocks, hipStream_t s) {
 
 hipError_t launch_dmc_smooth(const Arenas& A, int m, int blocks, hipStream_t s) {
     blocks = blocks < kXcds ? kXcds : blocks - blocks % kXcds;  // whole XCD groups
-    if (m == 0 && !A.normals) {
-        const hipError_t e = launch_smooth_map(A, blocks, s);
-        if (e != hipSuccess) return e;
-    }
     if (A.normals) {
         hipLaunchKernelGGL(k_dual_n_nrm, dim3(blocks), dim3(kSmoothThreads), 0, s, A, m);
         hipLaunchKernelGGL(k_primal_ring_nrm, dim3(blocks), dim3(kSmoothThreads), 0, s, A, m);

@@ -101,8 +101,8 @@ struct Counters {
     unsigned long long need_i;
     int64_t total_tiles;
     int64_t total_samples;
-    int64_t total_vtiles;
-    int64_t total_ttiles;
+    int32_t xcd_vtiles[kXcds]; // smoothing tiles of each XCD's maps
+    int32_t xcd_ttiles[kXcds];
     int32_t n_smooth;
     int32_t overflow;
     int32_t error;
@@ -125,21 +125,17 @@ struct Arenas {
     uint8_t* signs;            // [max_samples + 16] adaptive terrain: k_blocks' decisions, from the chunk's first
                                // sample on a byte per four samples of a row (x, y), ceil(dim / 4) bytes a row:
                                // undecided samples in the low bits, air samples in the high ones
-    int64_t* plan_part;        // [40 nb + 64] multi-block plan passes (nb = max_chunks / 1024 rounded up):
-                               // block totals and bases, flags, class and group bases
-    int64_t* plan_tmp;         // [2 max_chunks] multi-block smoothing plan: per-chunk exclusive tile sums
+    int64_t* plan_part;        // [10 nb + 1] multi-block plan passes (nb = max_chunks / 1024 rounded up): block
+                               // totals and bases, overflow flag
     unsigned long long* stat_blocks;  // [3][stat_cap] terrain octaves evaluated per workgroup of the
                                       // sampling, refinement and block kernels (plain stores, no atomics)
     int32_t stat_cap;
     int2* item_map;            // [max_items] (chunk, item within the chunk) of the word kernels' items
                                // (written by k_sample's prologue)
-    int32_t* smooth_list;      // [max_chunks] chunks that run the smoothing
-    int64_t* smooth_prefix;    // [max_chunks + 1] vertex tiles of the listed chunks
-    int64_t* smooth_tprefix;   // [max_chunks + 1] triangle tiles of the listed chunks
-    int64_t* smooth_xcd_v;     // [kXcds + 1] vertex-tile range of each XCD group
-    int64_t* smooth_xcd_t;     // [kXcds + 1] triangle-tile range of each XCD group
-    int2* smooth_vmap;         // [vertex tiles] (chunk, tile within the chunk) of each smoothing vertex tile
-    int2* smooth_tmap;         // [triangle tiles] the same for the triangle tiles
+    int2* smooth_vmap;         // [kXcds][cap_vtiles] (chunk, tile within the chunk) of the smoothing vertex
+                               // tiles of each XCD (k_scan)
+    int2* smooth_tmap;         // [kXcds][cap_ttiles] the same for the triangle tiles
+    int64_t cap_vtiles, cap_ttiles;
     EdgeWord* edges;           // same layout as labels: edge and active-cell bits of each word
     uint32_t* word_pre;        // same layout: edges of the item before the word
     uint32_t* item_e;          // [max_items] edges of each item, then their exclusive prefix in the chunk
@@ -202,8 +198,6 @@ hipError_t launch_count(const Arenas& A, int blocks, int refine, hipStream_t s);
 hipError_t launch_scan(const Arenas& A, int n, int blocks, hipStream_t s);
 hipError_t launch_emit(const Arenas& A, int blocks, hipStream_t s);
 hipError_t launch_smooth(const Arenas& A, int m, int blocks, hipStream_t s);
-// (chunk, tile) of every smoothing vertex and primitive tile, once per frame before the first step
-hipError_t launch_smooth_map(const Arenas& A, int blocks, hipStream_t s);
 // Quad mode (bmf_dmc.hip): emission after launch_count / launch_scan,
 // smoothing over the per-vertex rings.
 hipError_t launch_dmc_emit(const Arenas& A, int blocks, hipStream_t s);

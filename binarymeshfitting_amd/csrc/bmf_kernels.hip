@@ -30,14 +30,14 @@
 namespace bmf {
 
 // ------------------------------------------------------------------------
-// plan: geometry, culling, arena offsets, counters (one block; three passes
-// over many blocks for batches beyond one block)
+// plan: geometry, culling, arena offsets, counters
 // ------------------------------------------------------------------------
 constexpr int kPlanThreads = 1024;
-// Up to this many descriptors the plans run in one block (a few per thread,
-// one launch each); larger batches take the multi-block passes, whose extra
-// launches cost more than they save below it.
-constexpr int kPlanOneBlock = 2 * kPlanThreads;
+// Up to this many descriptors every block of the plan forms all the sums
+// itself (one launch); larger batches take three passes, whose extra launches
+// cost more than they save below it.
+constexpr int kPlanShared = 2 * kPlanThreads;
+constexpr int kPlanSlice = 64;  // records that a block then writes
 
 // The host-visible result of chunk j from its final record: written by
 // k_plan for the chunks it culls or skips and by k_scan for the sampled ones
@@ -94,7 +94,9 @@ __device__ __forceinline__ int expansion(const SamplerDev& S, float delta, float
     int k = 0;
     quad = 0.0f;
     base = best;
-    for (int o = 0; o < min(S.octaves, kExpandOctaves); o++) {
+#pragma unroll
+    for (int o = 0; o < kExpandOctaves; o++) {
+        if (o >= S.octaves) break;
         const float f = S.fo[o] * delta;
         q += S.ao[o] * (0.505f * kNoiseHess) * (f * f);
         b += S.ao[o] * (kNoiseSlack + kNoiseCoordSlack * far * fabsf(S.fo[o]));
@@ -132,11 +134,11 @@ __device__ __forceinline__ BlockPlan plan_blocks(const SamplerDev& S, const Chun
 }
 
 // Plan record of one descriptor: DMCChunk::label_grid geometry
-// (DMCChunk.cpp:94-101), analytic culling, sizes; `add` gets its
-// contributions to the arena sums (samples, label words, word items, sampling
-// tiles, items of sample blocks).
+// (DMCChunk.cpp:94-101) and analytic culling; `add` gets its contributions
+// to the arena sums (samples, label words, word items, sampling tiles, items
+// of sample blocks), each below 2^25.
 __device__ __forceinline__ ChunkMeta plan_record(const Arenas& A, const SamplerDev* __restrict__ S,
-                                                 const bmf_chunk_desc& d, int allow_cull, int64_t (&add)[5]) {
+                                                 const bmf_chunk_desc& d, int allow_cull, uint32_t (&add)[5]) {
     ChunkMeta m;
     float t = d.overlap * 2.0f;
     t = 1.0f + t;
@@ -157,9 +159,9 @@ __device__ __forceinline__ ChunkMeta plan_record(const Arenas& A, const SamplerD
         if (sign) m.state = sign == 1 ? kStateAir : kStateSolid;
     }
     m.csg_ns = m.csg_nb = 0;  // k_csg_cull fills them
-    const int64_t ns = (int64_t)d.dim * d.dim * d.dim;
+    const uint32_t ns = (uint32_t)d.dim * (uint32_t)d.dim * (uint32_t)d.dim;
     const bool sampled = m.state == kStateSampled;
-    m.lab_words = sampled ? (ns + 63) / 64 : 0;
+    m.lab_words = sampled ? (ns + 63u) / 64u : 0;
     m.any_air = m.state == kStateAir;
     m.any_solid = m.state == kStateSolid;
     m.contains_mesh = 0;
@@ -172,13 +174,12 @@ __device__ __forceinline__ ChunkMeta plan_record(const Arenas& A, const SamplerD
     m.dens_off = 0;
     m.lab_off = 0;
     m.item_slot = 0;
-    m.blocks = sampled && S->kind == BMF_SAMPLER_TERRAIN ? plan_blocks(*S, m) : BlockPlan{};
-    add[0] = sampled ? ns : 0;
-    add[1] = m.lab_words;
-    add[2] = (m.lab_words + kItemWords - 1) / kItemWords;
-    add[3] = sampled ? (ns + A.sample_tile - 1) / A.sample_tile : 0;
-    const int64_t nb = (d.dim + 3) >> 2;
-    add[4] = sampled ? (nb * nb * nb + kWaveBlocks - 1) / kWaveBlocks : 0;
+    const uint32_t nb = ((uint32_t)d.dim + 3u) >> 2;
+    add[0] = sampled ? ns : 0u;
+    add[1] = (uint32_t)m.lab_words;
+    add[2] = ((uint32_t)m.lab_words + kItemWords - 1) / kItemWords;
+    add[3] = sampled ? (ns + (uint32_t)A.sample_tile - 1) / (uint32_t)A.sample_tile : 0u;
+    add[4] = sampled ? (nb * nb * nb + kWaveBlocks - 1) / kWaveBlocks : 0u;
     return m;
 }
 
@@ -186,14 +187,17 @@ __device__ __forceinline__ bool plan_overflow(const Arenas& A, const int64_t (&t
     return tot[0] > A.cap_samples || tot[1] > A.cap_samples / 64 + A.cap_chunks;
 }
 
-// A record's final state once its offsets are known (base: where its block's
-// arena ranges start).
-__device__ __forceinline__ void plan_finish(const Arenas& A, int j, ChunkMeta& m, const int64_t (&base)[5],
-                                            bool overflow) {
-    m.dens_off += base[0];
-    m.lab_off += base[1];
-    m.item_slot += base[2];
+// A record's final state, `at` the arena sums before it.
+__device__ __forceinline__ void plan_finish(const Arenas& A, const SamplerDev* __restrict__ S, int j, ChunkMeta& m,
+                                            const int64_t (&at)[5], bool overflow) {
+    m.dens_off = at[0];
+    m.lab_off = at[1];
+    m.item_slot = at[2];
+    A.tile_prefix[j] = overflow ? 0 : at[3];
+    A.block_prefix[j] = overflow ? 0 : at[4];
+    m.blocks = BlockPlan{};
     if (m.state == kStateSampled) {
+        if (S->kind == BMF_SAMPLER_TERRAIN) m.blocks = plan_blocks(*S, m);
         if (overflow) {
             m.state = kStateSkipped;
             m.status = BMF_ECAPACITY;
@@ -225,61 +229,54 @@ __device__ __forceinline__ void plan_counters(const Arenas& A, int n, const int6
     c->total_tiles = overflow ? 0 : tot[3];
     c->total_items = overflow ? 0 : tot[2];
     c->n_smooth = 0;
+    for (int g = 0; g < kXcds; g++) c->xcd_vtiles[g] = c->xcd_ttiles[g] = 0;
     c->total_samples = tot[0];
 }
 
-// Batches of up to kPlanOneBlock descriptors: one block, each thread a
-// segment of consecutive descriptors, one launch.
+// Batches of up to kPlanShared descriptors, one launch: every block forms the
+// sums over all of them (two descriptors per thread at most, 32-bit wave
+// scans) and writes the records of its own kPlanSlice.  One block that wrote
+// every record took 14 us for 512 descriptors and 33 for 1,536 (a thread's
+// records are 120 bytes apart, written and read again across the scan);
+// this takes 6.7 and 9.9 (5.4 for one).
 __global__ void __launch_bounds__(kPlanThreads) k_plan(Arenas A, int n, int allow_cull, int reset_bumps) {
-    __shared__ int64_t s_w[5][kPlanThreads / 64 + 1];
-    const int per = (n + kPlanThreads - 1) / kPlanThreads;
-    const int j0 = threadIdx.x * per, j1 = min(n, j0 + per);
-    int64_t sum[5] = {0, 0, 0, 0, 0};
-    for (int j = j0; j < j1; j++) {
-        int64_t add[5];
-        ChunkMeta m = plan_record(A, A.sampler, A.descs[j], allow_cull, add);
-        // offsets within the thread's segment; tile_prefix likewise
-        m.dens_off = sum[0];
-        m.lab_off = sum[1];
-        m.item_slot = sum[2];
-        A.tile_prefix[j] = sum[3];
-        A.block_prefix[j] = sum[4];
-        A.meta[j] = m;
+    __shared__ uint32_t s_w[5][kPlanThreads / 64];
+    const SamplerDev* __restrict__ S = A.sampler;
+    const int per = (n + kPlanThreads - 1) / kPlanThreads;  // 1 or 2
+    const int j0 = threadIdx.x * per;
+    uint32_t sum[5] = {0u, 0u, 0u, 0u, 0u};
+    for (int i = 0; i < per; i++) {
+        if (j0 + i >= n) break;
+        uint32_t add[5];
+        (void)plan_record(A, S, A.descs[j0 + i], allow_cull, add);
 #pragma unroll
         for (int q = 0; q < 5; q++) sum[q] += add[q];
     }
     int64_t excl[5], tot[5];
-    block_scan<5, kPlanThreads>(sum, excl, tot, s_w);
+    block_scan32<5, kPlanThreads>(sum, excl, tot, s_w);
     const bool overflow = plan_overflow(A, tot);
-    for (int j = j0; j < j1; j++) {
-        A.tile_prefix[j] = overflow ? 0 : A.tile_prefix[j] + excl[3];
-        A.block_prefix[j] = overflow ? 0 : A.block_prefix[j] + excl[4];
-        ChunkMeta m = A.meta[j];
-        plan_finish(A, j, m, excl, overflow);
+    // the block's own records, formed again
+    for (int i = 0; i < per; i++) {
+        const int j = j0 + i;
+        if (j >= n || j / kPlanSlice != (int)blockIdx.x) break;  // per divides kPlanSlice
+        uint32_t add[5];
+        ChunkMeta m = plan_record(A, S, A.descs[j], allow_cull, add);
+        plan_finish(A, S, j, m, excl, overflow);
+#pragma unroll
+        for (int q = 0; q < 5; q++) excl[q] += add[q];
     }
-    if (threadIdx.x == 0) plan_counters(A, n, tot, overflow, reset_bumps);
+    if (blockIdx.x == 0 && threadIdx.x == 0) plan_counters(A, n, tot, overflow, reset_bumps);
 }
 
 // Larger batches, pass 1 of 3 (one descriptor per thread over many blocks):
-// records with offsets relative to their block, and each block's totals.
+// each block's totals.
 __global__ void __launch_bounds__(kPlanThreads) k_plan_part(Arenas A, int n, int allow_cull) {
-    __shared__ int64_t s_w[5][kPlanThreads / 64 + 1];
+    __shared__ uint32_t s_w[5][kPlanThreads / 64];
     const int j = blockIdx.x * kPlanThreads + threadIdx.x;
-    int64_t add[5];
-    ChunkMeta m{};
-    if (j < n) m = plan_record(A, A.sampler, A.descs[j], allow_cull, add);
-    else
-        for (int q = 0; q < 5; q++) add[q] = 0;
+    uint32_t add[5] = {0u, 0u, 0u, 0u, 0u};
+    if (j < n) (void)plan_record(A, A.sampler, A.descs[j], allow_cull, add);
     int64_t excl[5], tot[5];
-    block_scan<5, kPlanThreads>(add, excl, tot, s_w);
-    if (j < n) {
-        A.tile_prefix[j] = excl[3];
-        A.block_prefix[j] = excl[4];
-        m.dens_off = excl[0];
-        m.lab_off = excl[1];
-        m.item_slot = excl[2];
-        A.meta[j] = m;
-    }
+    block_scan32<5, kPlanThreads>(add, excl, tot, s_w);
     if (threadIdx.x < 5) A.plan_part[5 * blockIdx.x + threadIdx.x] = pick<5>(tot, (int)threadIdx.x);
 }
 
@@ -304,18 +301,19 @@ __global__ void __launch_bounds__(kPlanThreads) k_plan_total(Arenas A, int n, in
     }
 }
 
-// Pass 3: final offsets, sampling-tile prefixes, the results of culled chunks.
-__global__ void __launch_bounds__(kPlanThreads) k_plan_fix(Arenas A, int n, int nb) {
+// Pass 3: the records with their offsets, the results of culled chunks.
+__global__ void __launch_bounds__(kPlanThreads) k_plan_fix(Arenas A, int n, int nb, int allow_cull) {
+    __shared__ uint32_t s_w[5][kPlanThreads / 64];
     const int j = blockIdx.x * kPlanThreads + threadIdx.x;
+    uint32_t add[5] = {0u, 0u, 0u, 0u, 0u};
+    ChunkMeta m{};
+    if (j < n) m = plan_record(A, A.sampler, A.descs[j], allow_cull, add);
+    int64_t at[5], tot[5];
+    block_scan32<5, kPlanThreads>(add, at, tot, s_w);
     if (j >= n) return;
-    int64_t base[5];
 #pragma unroll
-    for (int q = 0; q < 5; q++) base[q] = A.plan_part[5 * (nb + blockIdx.x) + q];
-    const bool overflow = A.plan_part[10 * nb] != 0;
-    A.tile_prefix[j] = overflow ? 0 : A.tile_prefix[j] + base[3];
-    A.block_prefix[j] = overflow ? 0 : A.block_prefix[j] + base[4];
-    ChunkMeta m = A.meta[j];
-    plan_finish(A, j, m, base, overflow);
+    for (int q = 0; q < 5; q++) at[q] += A.plan_part[5 * (nb + blockIdx.x) + q];
+    plan_finish(A, A.sampler, j, m, at, A.plan_part[10 * nb] != 0);
 }
 
 // ------------------------------------------------------------------------
@@ -1106,13 +1104,25 @@ __global__ void __launch_bounds__(kRowThreads) k_count(Arenas A) {
 }
 
 // ------------------------------------------------------------------------
-// scan: one block per chunk -> item bases, totals, output reservation
+// scan: one block per chunk -> item bases, totals, output reservation, and the
+// chunk's entries in the smoothing tile maps: the k-th chunk to get there goes
+// to XCD k % 8, so that all its tiles run on one XCD and its positions,
+// indices and centroids stay in that XCD's L2 (workgroups are dispatched to
+// the 8 XCDs round-robin by block index; a different dispatch order only costs
+// locality, and the order of the maps only which block does which tile).  Two
+// launches that built the maps from an ordered list of the chunks took 11 us.
 // ------------------------------------------------------------------------
+// Chunks that run the smoothing kernels (K > 0 or normals, a mesh, fitted).
+__device__ __forceinline__ bool smooths(const ChunkMeta& M, int normals) {
+    return (M.iters > 0 || normals) && M.V > 0 && M.T > 0 && M.status == BMF_OK && M.state == kStateSampled;
+}
+
 constexpr int kScanThreads = 256;
 
 __global__ void __launch_bounds__(kScanThreads) k_scan(Arenas A, int n) {
     constexpr int NW = kScanThreads / 64;
     __shared__ uint32_t s_we[NW], s_wc[NW];  // wave totals
+    __shared__ int s_map[5];  // XCD, first vertex and triangle tile in its maps, their counts
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     for (int j = blockIdx.x; j < n; j += gridDim.x) {
         ChunkMeta& M = A.meta[j];
@@ -1205,203 +1215,28 @@ __global__ void __launch_bounds__(kScanThreads) k_scan(Arenas A, int n) {
                 M.i_off = io;
             }
             write_result(A, j, M);
+            const bool on = smooths(M, A.normals);
+            const int vt = on ? (int)((V + kSmoothThreads - 1) / kSmoothThreads) : 0;
+            const int tt = on ? (int)((T + kSmoothThreads - 1) / kSmoothThreads) : 0;
+            if (on) {
+                const int g = atomicAdd(&A.ctr->n_smooth, 1) & (kXcds - 1);
+                s_map[0] = g;
+                s_map[1] = atomicAdd(&A.ctr->xcd_vtiles[g], vt);
+                s_map[2] = atomicAdd(&A.ctr->xcd_ttiles[g], tt);
+            }
+            s_map[3] = vt;
+            s_map[4] = tt;
+        }
+        __syncthreads();
+        const int vt = s_map[3], tt = s_map[4];
+        if (vt) {
+            int2* __restrict__ VM = A.smooth_vmap + (int64_t)s_map[0] * A.cap_vtiles + s_map[1];
+            int2* __restrict__ TM = A.smooth_tmap + (int64_t)s_map[0] * A.cap_ttiles + s_map[2];
+            for (int r = tid; r < vt; r += kScanThreads) VM[r] = make_int2(j, r);
+            for (int r = tid; r < tt; r += kScanThreads) TM[r] = make_int2(j, r);
         }
         __syncthreads();
     }
-}
-
-// Ordered list of the chunks that run the smoothing (K > 0, a mesh, fitted)
-// and the prefix of their vertex tiles, for k_smooth (one block).
-__device__ __forceinline__ bool smooths(const ChunkMeta& M, int normals) {
-    return (M.iters > 0 || normals) && M.V > 0 && M.T > 0 && M.status == BMF_OK && M.state == kStateSampled;
-}
-
-// The list is grouped by XCD: the k-th smoothing chunk goes to XCD k % 8,
-// so that all tiles of a chunk run on one XCD and its positions, indices and
-// centroids stay in that XCD's L2 (workgroups are dispatched to the 8 XCDs
-// round-robin by block index; a different dispatch order only costs
-// locality, not correctness).
-__global__ void __launch_bounds__(kPlanThreads) k_plan_smooth(Arenas A, int n) {
-    __shared__ int64_t s_w[2][kPlanThreads / 64 + 1];
-    const int tid = threadIdx.x;
-    const int per = (n + kPlanThreads - 1) / kPlanThreads;
-    const int j0 = tid * per, j1 = min(n, j0 + per);
-    // ---- rank of each smoothing chunk (ordered compaction) ----
-    int64_t cnt = 0;
-    for (int j = j0; j < j1; j++) cnt += smooths(A.meta[j], A.normals);
-    int64_t c1[1] = {cnt}, e1[1], t1[1];
-    block_scan<1, kPlanThreads>(c1, e1, t1, s_w);
-    const int ns = (int)t1[0];
-    int k = (int)e1[0];
-    for (int j = j0; j < j1; j++) {
-        if (!smooths(A.meta[j], A.normals)) continue;
-        // grouped position: groups g = k % 8 in order, rank k / 8 inside
-        const int g = k & (kXcds - 1), q = k / kXcds;
-        int pos = q;
-        for (int h = 0; h < g; h++) pos += (ns - h + kXcds - 1) / kXcds;
-        A.smooth_list[pos] = j;
-        k++;
-    }
-    __syncthreads();  // smooth_list written by this block is visible to it
-    // ---- tile prefixes in grouped order ----
-    const int per2 = (ns + kPlanThreads - 1) / kPlanThreads;
-    const int p0 = tid * per2, p1 = min(ns, p0 + per2);
-    int64_t tv = 0, tt = 0;
-    for (int p = p0; p < p1; p++) {
-        const ChunkMeta& M = A.meta[A.smooth_list[p]];
-        tv += (M.V + kSmoothThreads - 1) / kSmoothThreads;
-        tt += (M.T + kSmoothThreads - 1) / kSmoothThreads;
-    }
-    int64_t c2[2] = {tv, tt}, e2[2], t2[2];
-    block_scan<2, kPlanThreads>(c2, e2, t2, s_w);
-    int64_t bv = e2[0], bt = e2[1];
-    for (int p = p0; p < p1; p++) {
-        const ChunkMeta& M = A.meta[A.smooth_list[p]];
-        A.smooth_prefix[p] = bv;
-        A.smooth_tprefix[p] = bt;
-        bv += (M.V + kSmoothThreads - 1) / kSmoothThreads;
-        bt += (M.T + kSmoothThreads - 1) / kSmoothThreads;
-    }
-
-    __syncthreads();
-    if (tid == kPlanThreads - 1) {
-        A.ctr->n_smooth = ns;
-        A.smooth_prefix[ns] = t2[0];
-        A.smooth_tprefix[ns] = t2[1];
-        A.ctr->total_vtiles = t2[0];
-        A.ctr->total_ttiles = t2[1];
-    }
-    __syncthreads();
-    // ---- tile range of each XCD group ----
-    if (tid <= kXcds) {
-        int pos = 0;
-        for (int h = 0; h < tid; h++) pos += (ns - h + kXcds - 1) / kXcds;
-        A.smooth_xcd_v[tid] = pos < ns ? A.smooth_prefix[pos] : A.smooth_prefix[ns];
-        A.smooth_xcd_t[tid] = pos < ns ? A.smooth_tprefix[pos] : A.smooth_tprefix[ns];
-    }
-}
-
-// Larger batches (more than kPlanOneBlock chunks): the same list and
-// prefixes in five passes over many blocks.  The grouped order puts rank k
-// (k-th smoothing chunk in chunk order) in group g = k % kXcds at place
-// k / kXcds, so the prefix at a position is the totals of the groups before
-// its own plus the sum over the earlier ranks of its residue class: block
-// scans carry one running sum per residue class.
-__device__ __forceinline__ int grouped_pos(int k, int ns) {
-    const int g = k & (kXcds - 1);
-    int pos = k / kXcds;
-    for (int h = 0; h < g; h++) pos += (ns - h + kXcds - 1) / kXcds;
-    return pos;
-}
-
-// Pass 1: smoothing chunks per block.
-__global__ void __launch_bounds__(kPlanThreads) k_smooth_count(Arenas A, int n) {
-    __shared__ int64_t s_w[1][kPlanThreads / 64 + 1];
-    const int j = blockIdx.x * kPlanThreads + threadIdx.x;
-    int64_t f[1] = {j < n && smooths(A.meta[j], A.normals)}, e[1], t[1];
-    block_scan<1, kPlanThreads>(f, e, t, s_w);
-    if (threadIdx.x == 0) A.plan_part[blockIdx.x] = t[0];
-}
-
-// Pass 2 (one block): rank base of each block, and the count.
-__global__ void __launch_bounds__(kPlanThreads) k_smooth_ranks(Arenas A, int nb) {
-    __shared__ int64_t s_w[1][kPlanThreads / 64 + 1];
-    const int b = threadIdx.x;
-    int64_t v[1] = {b < nb ? A.plan_part[b] : 0}, e[1], t[1];
-    block_scan<1, kPlanThreads>(v, e, t, s_w);
-    if (b < nb) A.plan_part[nb + b] = e[0];
-    if (b == 0) {
-        A.plan_part[2 * nb] = t[0];
-        A.ctr->n_smooth = (int)t[0];
-    }
-}
-
-// Pass 3: each smoothing chunk's rank and place in the list, and the block's
-// sums of vertex / triangle tiles per residue class (exclusive sums of the
-// chunk kept in plan_tmp).
-__global__ void __launch_bounds__(kPlanThreads) k_smooth_place(Arenas A, int n, int nb) {
-    __shared__ int64_t s_r[1][kPlanThreads / 64 + 1];
-    __shared__ int64_t s_w[2 * kXcds][kPlanThreads / 64 + 1];
-    const int j = blockIdx.x * kPlanThreads + threadIdx.x;
-    const bool on = j < n && smooths(A.meta[j], A.normals);
-    int64_t r1[1] = {on}, re[1], rt[1];
-    block_scan<1, kPlanThreads>(r1, re, rt, s_r);
-    const int k = (int)(A.plan_part[nb + blockIdx.x] + re[0]);
-    const int g = k & (kXcds - 1);
-    int64_t f[2 * kXcds], e[2 * kXcds], t[2 * kXcds];
-    int64_t vt = 0, tt = 0;
-    if (on) {
-        const ChunkMeta& M = A.meta[j];
-        vt = (M.V + kSmoothThreads - 1) / kSmoothThreads;
-        tt = (M.T + kSmoothThreads - 1) / kSmoothThreads;
-        A.smooth_list[grouped_pos(k, (int)A.plan_part[2 * nb])] = j;
-    }
-#pragma unroll
-    for (int q = 0; q < kXcds; q++) {
-        f[q] = q == g ? vt : 0;
-        f[kXcds + q] = q == g ? tt : 0;
-    }
-    block_scan<2 * kXcds, kPlanThreads>(f, e, t, s_w);
-    if (on) {
-        A.plan_tmp[2 * (int64_t)j] = pick<2 * kXcds>(e, g);
-        A.plan_tmp[2 * (int64_t)j + 1] = pick<2 * kXcds>(e, kXcds + g);
-    }
-    if (threadIdx.x < 2 * kXcds)
-        A.plan_part[2 * nb + 1 + 2 * kXcds * blockIdx.x + threadIdx.x] = pick<2 * kXcds>(t, (int)threadIdx.x);
-}
-
-// Pass 4 (one block): per block and class the sums of the blocks before it,
-// the group totals, their bases (= each XCD group's first tile) and totals.
-__global__ void __launch_bounds__(kPlanThreads) k_smooth_bases(Arenas A, int nb) {
-    __shared__ int64_t s_w[2 * kXcds][kPlanThreads / 64 + 1];
-    const int b = threadIdx.x;
-    int64_t* part = A.plan_part + 2 * nb + 1;
-    int64_t* base = part + 2 * kXcds * nb;
-    int64_t v[2 * kXcds], e[2 * kXcds], t[2 * kXcds];
-#pragma unroll
-    for (int q = 0; q < 2 * kXcds; q++) v[q] = b < nb ? part[2 * kXcds * b + q] : 0;
-    block_scan<2 * kXcds, kPlanThreads>(v, e, t, s_w);
-    if (b < nb)
-#pragma unroll
-        for (int q = 0; q < 2 * kXcds; q++) base[2 * kXcds * b + q] = e[q];
-    if (b == 0) {
-        int64_t gv = 0, gt = 0;
-        int64_t* gbase = base + 2 * kXcds * nb;
-#pragma unroll
-        for (int g = 0; g < kXcds; g++) {
-            gbase[g] = gv;
-            gbase[kXcds + g] = gt;
-            A.smooth_xcd_v[g] = gv;
-            A.smooth_xcd_t[g] = gt;
-            gv += t[g];
-            gt += t[kXcds + g];
-        }
-        A.smooth_xcd_v[kXcds] = gv;
-        A.smooth_xcd_t[kXcds] = gt;
-        const int ns = (int)A.plan_part[2 * nb];
-        A.smooth_prefix[ns] = gv;
-        A.smooth_tprefix[ns] = gt;
-        A.ctr->total_vtiles = gv;
-        A.ctr->total_ttiles = gt;
-    }
-}
-
-// Pass 5: the tile prefixes at each list position.
-__global__ void __launch_bounds__(kPlanThreads) k_smooth_prefix(Arenas A, int n, int nb) {
-    __shared__ int64_t s_r[1][kPlanThreads / 64 + 1];
-    const int j = blockIdx.x * kPlanThreads + threadIdx.x;
-    const bool on = j < n && smooths(A.meta[j], A.normals);
-    int64_t r1[1] = {on}, re[1], rt[1];
-    block_scan<1, kPlanThreads>(r1, re, rt, s_r);
-    if (!on) return;
-    const int k = (int)(A.plan_part[nb + blockIdx.x] + re[0]);
-    const int ns = (int)A.plan_part[2 * nb];
-    const int g = k & (kXcds - 1);
-    const int64_t* base = A.plan_part + 2 * nb + 1 + 2 * kXcds * nb;
-    const int64_t* gbase = base + 2 * kXcds * nb;
-    const int pos = grouped_pos(k, ns);
-    A.smooth_prefix[pos] = gbase[g] + base[2 * kXcds * blockIdx.x + g] + A.plan_tmp[2 * (int64_t)j];
-    A.smooth_tprefix[pos] = gbase[kXcds + g] + base[2 * kXcds * blockIdx.x + kXcds + g] + A.plan_tmp[2 * (int64_t)j + 1];
 }
 
 // ------------------------------------------------------------------------
@@ -1579,20 +1414,6 @@ __global__ void __launch_bounds__(kRowThreads) k_emit(Arenas A) {
     }
 }
 
-// Tile -> (chunk, tile within the chunk) for the smoothing kernels, one
-// block per listed chunk, written once per frame before the first step.
-__global__ void __launch_bounds__(kSmoothThreads) k_smooth_map(Arenas A) {
-    const int ns = A.ctr->n_smooth;
-    for (int p = blockIdx.x; p < ns; p += gridDim.x) {
-        const int j = A.smooth_list[p];
-        const ChunkMeta& M = A.meta[j];
-        const int vt = (M.V + kSmoothThreads - 1) / kSmoothThreads, tt = (M.T + kSmoothThreads - 1) / kSmoothThreads;
-        const int64_t bv = A.smooth_prefix[p], bt = A.smooth_tprefix[p];
-        for (int r = threadIdx.x; r < vt; r += blockDim.x) A.smooth_vmap[bv + r] = make_int2(j, r);
-        for (int r = threadIdx.x; r < tt; r += blockDim.x) A.smooth_tmap[bt + r] = make_int2(j, r);
-    }
-}
-
 // ------------------------------------------------------------------------
 // smoothing, iteration m of MeshProcessor<3> (MeshProcessor.cpp:130-306 as
 // driven by ChunkGenerator.cpp:112-124), over the chunks with K > m:
@@ -1625,9 +1446,10 @@ __device__ __forceinline__ SmoothChunk smooth_chunk(const ChunkMeta& M) {
 
 __global__ void __launch_bounds__(kSmoothThreads) k_dual(Arenas A, int m) {
     const int xcd = blockIdx.x % kXcds;
-    const int64_t end = A.smooth_xcd_t[xcd + 1];
-    for (int64_t tile = A.smooth_xcd_t[xcd] + blockIdx.x / kXcds; tile < end; tile += gridDim.x / kXcds) {
-        const int2 tm = A.smooth_tmap[tile];  // (chunk, tile within the chunk)
+    const int end = A.ctr->xcd_ttiles[xcd];
+    const int2* __restrict__ map = A.smooth_tmap + (int64_t)xcd * A.cap_ttiles;
+    for (int tile = blockIdx.x / kXcds; tile < end; tile += gridDim.x / kXcds) {
+        const int2 tm = map[tile];  // (chunk, tile within the chunk)
         const int chunk = uniform_int(tm.x), ty = uniform_int(tm.y);
         const SmoothChunk M = smooth_chunk(A.meta[chunk]);
         const int64_t T = M.T, i_off = M.i_off, v_off = M.v_off;
@@ -1747,9 +1569,10 @@ __device__ __forceinline__ uint32_t ring_sums(uint4 r, const float4* __restrict_
 
 __global__ void __launch_bounds__(kSmoothThreads) k_primal(Arenas A, int m) {
     const int xcd = blockIdx.x % kXcds;
-    const int64_t end = A.smooth_xcd_v[xcd + 1];
-    for (int64_t tile = A.smooth_xcd_v[xcd] + blockIdx.x / kXcds; tile < end; tile += gridDim.x / kXcds) {
-        const int2 tm = A.smooth_vmap[tile];  // (chunk, tile within the chunk)
+    const int end = A.ctr->xcd_vtiles[xcd];
+    const int2* __restrict__ map = A.smooth_vmap + (int64_t)xcd * A.cap_vtiles;
+    for (int tile = blockIdx.x / kXcds; tile < end; tile += gridDim.x / kXcds) {
+        const int2 tm = map[tile];  // (chunk, tile within the chunk)
         const int chunk = uniform_int(tm.x), ty = uniform_int(tm.y);
         const SmoothChunk M = smooth_chunk(A.meta[chunk]);
         const int K = M.iters, dim = M.dim, bp = M.bp;
@@ -1806,9 +1629,10 @@ __global__ void __launch_bounds__(kSmoothThreads) k_primal(Arenas A, int m) {
 // last step writes the unit normal.
 __global__ void __launch_bounds__(kSmoothThreads) k_dual_nrm(Arenas A, int m) {
     const int xcd = blockIdx.x % kXcds;
-    const int64_t end = A.smooth_xcd_t[xcd + 1];
-    for (int64_t tile = A.smooth_xcd_t[xcd] + blockIdx.x / kXcds; tile < end; tile += gridDim.x / kXcds) {
-        const int2 tm = A.smooth_tmap[tile];  // (chunk, tile within the chunk)
+    const int end = A.ctr->xcd_ttiles[xcd];
+    const int2* __restrict__ map = A.smooth_tmap + (int64_t)xcd * A.cap_ttiles;
+    for (int tile = blockIdx.x / kXcds; tile < end; tile += gridDim.x / kXcds) {
+        const int2 tm = map[tile];  // (chunk, tile within the chunk)
         const int chunk = uniform_int(tm.x), ty = uniform_int(tm.y);
         const SmoothChunk M = smooth_chunk(A.meta[chunk]);
         const int K = M.iters;
@@ -1869,9 +1693,10 @@ __global__ void __launch_bounds__(kSmoothThreads) k_dual_nrm(Arenas A, int m) {
 
 __global__ void __launch_bounds__(kSmoothThreads) k_primal_nrm(Arenas A, int m) {
     const int xcd = blockIdx.x % kXcds;
-    const int64_t end = A.smooth_xcd_v[xcd + 1];
-    for (int64_t tile = A.smooth_xcd_v[xcd] + blockIdx.x / kXcds; tile < end; tile += gridDim.x / kXcds) {
-        const int2 tm = A.smooth_vmap[tile];  // (chunk, tile within the chunk)
+    const int end = A.ctr->xcd_vtiles[xcd];
+    const int2* __restrict__ map = A.smooth_vmap + (int64_t)xcd * A.cap_vtiles;
+    for (int tile = blockIdx.x / kXcds; tile < end; tile += gridDim.x / kXcds) {
+        const int2 tm = map[tile];  // (chunk, tile within the chunk)
         const int chunk = uniform_int(tm.x), ty = uniform_int(tm.y);
         const SmoothChunk M = smooth_chunk(A.meta[chunk]);
         const int K = M.iters;
@@ -2000,14 +1825,15 @@ __global__ void k_ref_masks(Arenas A, uint64_t* masks) {
 // launch wrappers
 // ------------------------------------------------------------------------
 hipError_t launch_plan(const Arenas& A, int n, int allow_cull, int reset_bumps, hipStream_t s) {
-    if (n <= kPlanOneBlock) {
-        hipLaunchKernelGGL(k_plan, dim3(1), dim3(kPlanThreads), 0, s, A, n, allow_cull, reset_bumps);
+    if (n <= kPlanShared) {
+        hipLaunchKernelGGL(k_plan, dim3((n + kPlanSlice - 1) / kPlanSlice), dim3(kPlanThreads), 0, s, A, n, allow_cull,
+                           reset_bumps);
     } else {
         const int nb = (n + kPlanThreads - 1) / kPlanThreads;
         if (nb > kPlanThreads) return hipErrorInvalidValue;  // beyond BMF's 2^20 chunks
         hipLaunchKernelGGL(k_plan_part, dim3(nb), dim3(kPlanThreads), 0, s, A, n, allow_cull);
         hipLaunchKernelGGL(k_plan_total, dim3(1), dim3(kPlanThreads), 0, s, A, n, nb, reset_bumps);
-        hipLaunchKernelGGL(k_plan_fix, dim3(nb), dim3(kPlanThreads), 0, s, A, n, nb);
+        hipLaunchKernelGGL(k_plan_fix, dim3(nb), dim3(kPlanThreads), 0, s, A, n, nb, allow_cull);
     }
     if (A.csg_list) hipLaunchKernelGGL(k_csg_cull, dim3((unsigned)(n < 2048 ? n : 2048)), dim3(256), 0, s, A, n);
     return hipGetLastError();
@@ -2044,29 +1870,14 @@ hipError_t launch_count(const Arenas& A, int blocks, int refine, hipStream_t s) 
 }
 hipError_t launch_scan(const Arenas& A, int n, int blocks, hipStream_t s) {
     hipLaunchKernelGGL(k_scan, dim3(blocks), dim3(kScanThreads), 0, s, A, n);
-    if (n <= kPlanOneBlock) {
-        hipLaunchKernelGGL(k_plan_smooth, dim3(1), dim3(kPlanThreads), 0, s, A, n);
-    } else {
-        const int nb = (n + kPlanThreads - 1) / kPlanThreads;
-        hipLaunchKernelGGL(k_smooth_count, dim3(nb), dim3(kPlanThreads), 0, s, A, n);
-        hipLaunchKernelGGL(k_smooth_ranks, dim3(1), dim3(kPlanThreads), 0, s, A, nb);
-        hipLaunchKernelGGL(k_smooth_place, dim3(nb), dim3(kPlanThreads), 0, s, A, n, nb);
-        hipLaunchKernelGGL(k_smooth_bases, dim3(1), dim3(kPlanThreads), 0, s, A, nb);
-        hipLaunchKernelGGL(k_smooth_prefix, dim3(nb), dim3(kPlanThreads), 0, s, A, n, nb);
-    }
     return hipGetLastError();
 }
 hipError_t launch_emit(const Arenas& A, int blocks, hipStream_t s) {
     hipLaunchKernelGGL(k_emit, dim3(blocks), dim3(kRowThreads), 0, s, A);
     return hipGetLastError();
 }
-hipError_t launch_smooth_map(const Arenas& A, int blocks, hipStream_t s) {
-    hipLaunchKernelGGL(k_smooth_map, dim3(std::min(blocks, 1024)), dim3(kSmoothThreads), 0, s, A);
-    return hipGetLastError();
-}
 hipError_t launch_smooth(const Arenas& A, int m, int blocks, hipStream_t s) {
     blocks = blocks < kXcds ? kXcds : blocks - blocks % kXcds;  // whole XCD groups
-    if (m == 0) hipLaunchKernelGGL(k_smooth_map, dim3(std::min(blocks, 1024)), dim3(kSmoothThreads), 0, s, A);
     if (A.normals) {
         hipLaunchKernelGGL(k_dual_nrm, dim3(blocks), dim3(kSmoothThreads), 0, s, A, m);
         hipLaunchKernelGGL(k_primal_nrm, dim3(blocks), dim3(kSmoothThreads), 0, s, A, m);

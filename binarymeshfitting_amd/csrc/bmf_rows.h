@@ -86,6 +86,45 @@ __device__ __forceinline__ void block_scan(const int64_t (&v)[N], int64_t (&excl
     __syncthreads();  // the scratch may be reused
 }
 
+// Inclusive prefix over the wave's lanes (row shifts and broadcasts, no LDS).
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v) {
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, false);  // row_shr 1, 2, 4, 8
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false);  // row_bcast 15, 31
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);
+    return v;
+}
+
+// block_scan of values whose sum over a wave fits 32 bits: exclusive prefix
+// and total as 64-bit values.
+template <int N, int NT>
+__device__ __forceinline__ void block_scan32(const uint32_t (&v)[N], int64_t (&excl)[N], int64_t (&tot)[N],
+                                             uint32_t (*s_w)[NT / 64]) {
+    constexpr int NW = NT / 64;
+    const int lane = (int)(threadIdx.x & 63), w = (int)(threadIdx.x >> 6);
+    uint32_t inc[N];
+#pragma unroll
+    for (int q = 0; q < N; q++) {
+        inc[q] = wave_scan(v[q]);
+        if (lane == 63) s_w[q][w] = inc[q];
+    }
+    __syncthreads();
+    // every wave scans the (at most 16) wave totals, in 16-bit halves
+    static_assert(NW <= 16, "wave totals in one row of lanes");
+    const int uw = uniform_int(w);
+#pragma unroll
+    for (int q = 0; q < N; q++) {
+        const uint32_t x = lane < NW ? s_w[q][lane] : 0u;
+        const int lo = (int)wave_scan(x & 0xFFFFu), hi = (int)wave_scan(x >> 16);
+        const int bl = uw ? __builtin_amdgcn_readlane(lo, uw - 1) : 0, bh = uw ? __builtin_amdgcn_readlane(hi, uw - 1) : 0;
+        excl[q] = ((int64_t)bh << 16) + bl + (int64_t)(inc[q] - v[q]);
+        tot[q] = ((int64_t)__builtin_amdgcn_readlane(hi, NW - 1) << 16) + __builtin_amdgcn_readlane(lo, NW - 1);
+    }
+    __syncthreads();  // the scratch may be reused
+}
+
 // Chunk j whose half-open range [prefix[j], prefix[j+1]) holds g.
 __device__ __forceinline__ int find_chunk(const int64_t* __restrict__ prefix, int n, int64_t g) {
     int lo = 0, hi = n;
