@@ -35,7 +35,7 @@ hipError_t dalloc(T** p, int64_t count) {
 
 void free_arenas(bmf_ctx* c) {
     Arenas& A = c->A;
-    void* ptrs[] = {A.meta,    A.descs,     A.results,  A.tile_prefix, A.block_prefix, A.signs, A.plan_part, A.stat_blocks, A.item_map, A.smooth_vmap, A.smooth_tmap, A.edges, A.word_pre, A.item_e, A.item_c, A.cen4,
+    void* ptrs[] = {A.meta,    A.descs,     A.results,  A.block_prefix, A.signs, A.plan_part, A.stat_blocks, A.item_map, A.smooth_vmap, A.smooth_tmap, A.edges, A.word_pre, A.item_e, A.item_c, A.cen4,
                     A.dens,    A.labels,    A.exact, A.cell_tb,   A.cell_mask,
                     A.pos,     A.pos4,      A.boundary, A.vedge,       A.vring,        A.idx,          A.ctr,
                     A.sampler, c->d_spheres, c->d_boxes, A.ring, A.ring_n, A.qef_err, A.nrm4, A.fn4, A.nrm,
@@ -277,7 +277,7 @@ int bmf_create(bmf_ctx** out, int device, const bmf_limits* lim) {
     if (hipGetDeviceProperties(&prop, device) == hipSuccess && prop.multiProcessorCount > 0)
         c->cu_count = prop.multiProcessorCount;
     c->persistent_blocks = c->cu_count * 8;
-    c->tune.sample_tile = kSampleTileDefault;
+    c->tune.sample_tile = 2048;
     c->tune.sample_blocks = c->persistent_blocks;
     // ten per CU: the best of 4..64 per CU for count + emit on a batch of
     // 512 64^3-cell chunks (89 us; 97 at 8, 94 at 16 and more) and on 64
@@ -294,14 +294,13 @@ int bmf_create(bmf_ctx** out, int device, const bmf_limits* lim) {
     A.cap_indices = lim->max_indices;
     A.cap_vtiles = A.cap_vertices / kSmoothThreads + nc + 1;
     A.cap_ttiles = A.cap_indices / 3 / kSmoothThreads + nc + 1;
-    A.sample_tile = kSampleTileDefault;
     A.smoothing_follows = 1;
     A.stat_cap = 64 * c->cu_count;
     bool ok = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) == hipSuccess;
     ok = ok && dalloc(&A.meta, nc) == hipSuccess && dalloc(&A.descs, nc) == hipSuccess &&
-         dalloc(&A.results, nc) == hipSuccess && dalloc(&A.tile_prefix, nc + 1) == hipSuccess &&
+         dalloc(&A.results, nc) == hipSuccess &&
          dalloc(&A.block_prefix, nc + 1) == hipSuccess && dalloc(&A.signs, lim->max_samples + 16) == hipSuccess &&
-         dalloc(&A.plan_part, 10 * ((nc + 1023) / 1024) + 1) == hipSuccess &&
+         dalloc(&A.plan_part, 8 * ((nc + 1023) / 1024) + 1) == hipSuccess &&
          dalloc(&A.stat_blocks, 3 * (int64_t)(64 * c->cu_count)) == hipSuccess &&
          dalloc(&A.item_map, ni) == hipSuccess &&
          dalloc(&A.smooth_vmap, kXcds * A.cap_vtiles) == hipSuccess &&
@@ -538,7 +537,7 @@ static int extract_impl(bmf_ctx* c, const bmf_chunk_desc* chunks, int n, int mod
             Aj.results = A.results + j;
             const int64_t dim = dj.dim;
             const int64_t ns = dim * dim * dim;
-            const int sb = (int)std::min<int64_t>(ceil_div(ns, A.sample_tile), pb);
+            const int sb = sample_blocks_of(ns);
             rc = enqueue_pipeline(c, Aj, 1, max_steps(c, &dj, 1), 1, j == 0, sb, word_blocks(dj.dim), 1,
                                   std::min(pb, 1024));
             if (rc) return rc;
@@ -690,7 +689,7 @@ static int stage_one(bmf_ctx* c, const bmf_chunk_desc* d, bool scan) {
     if (rc) return rc;
     const Arenas& A = c->A;
     BMF_HIP(launch_plan(A, 1, 0, 1, c->stream));
-    BMF_HIP(launch_sample(A, 1, (int)std::min<int64_t>(ceil_div(ns, A.sample_tile), c->persistent_blocks), 0,
+    BMF_HIP(launch_sample(A, 1, sample_blocks_of(ns), 0,
                           c->h_sampler.kind, c->h_sampler.noise_dims == 2, c->stream));
     if (scan) {
         BMF_HIP(launch_count(A, word_blocks(d->dim), 0, c->stream));
@@ -913,7 +912,6 @@ int bmf_set_tuning(bmf_ctx* c, const bmf_tuning* t) {
     BMF_HIP(hipSetDevice(c->device));
     BMF_HIP(hipStreamSynchronize(c->stream));
     c->tune = n;
-    c->A.sample_tile = n.sample_tile;
     drop_graphs(c);
     return BMF_OK;
 }
@@ -934,8 +932,7 @@ int bmf_autotune(bmf_ctx* c, const bmf_chunk_desc* chunks, int n, int reps, bmf_
     // run does not win) of the pipeline under tuning t
     float st[BMF_NUM_STAGES];
     auto run_n = [&](const bmf_tuning& t, int nrep, float* out) -> int {
-        Arenas A = c->A;
-        A.sample_tile = t.sample_tile;
+        const Arenas& A = c->A;
         std::vector<float> ms(static_cast<size_t>(nrep) * BMF_NUM_STAGES);
         for (int r = 0; r < nrep; r++) {
             int e = enqueue_pipeline(c, A, n, maxk, 1, 1, t.sample_blocks, t.row_blocks,
@@ -956,25 +953,21 @@ int bmf_autotune(bmf_ctx* c, const bmf_chunk_desc* chunks, int n, int reps, bmf_
     const bmf_tuning start = c->tune;
     bmf_tuning cur = c->tune;
     const int cu = c->cu_count;
-    // sampling: tile x persistent workgroups (stage 1)
+    // sampling: persistent workgroups (stage 1)
     {
         float bt = 1e30f;
         bmf_tuning b = cur;
-        const int tiles[3] = {1024, 2048, 4096};
-        const int mult[4] = {2, 4, 8, 16};
-        for (int ti : tiles)
-            for (int m : mult) {
-                bmf_tuning t = cur;
-                t.sample_tile = ti;
-                t.sample_blocks = m * cu;
-                rc = run(t, st);
-                if (rc) return rc;
-                if (st[1] < bt) {
-                    bt = st[1];
-                    b = t;
-                }
+        const int mult[4] = {4, 8, 16, 32};
+        for (int m : mult) {
+            bmf_tuning t = cur;
+            t.sample_blocks = m * cu;
+            rc = run(t, st);
+            if (rc) return rc;
+            if (st[1] < bt) {
+                bt = st[1];
+                b = t;
             }
-        cur.sample_tile = b.sample_tile;
+        }
         cur.sample_blocks = b.sample_blocks;
     }
     // word kernels: count and emit (stages 2 and 4), workgroups

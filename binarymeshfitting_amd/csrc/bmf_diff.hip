@@ -1158,7 +1158,7 @@ int bmf_forward_diff(bmf_ctx* c, const bmf_chunk_desc* d, const float* densities
     // no smoothing: the tape smooths its own copy
     hipError_t e = launch_plan(A, 1, 0, 1, s);
     if (e == hipSuccess)
-        e = launch_sample(A, 1, (int)std::min<int64_t>((n3 + A.sample_tile - 1) / A.sample_tile, c->persistent_blocks),
+        e = launch_sample(A, 1, sample_blocks_of(n3),
                           0, densities ? (int)BMF_SAMPLER_EXTERNAL : (int)c->h_sampler.kind,
                           !densities && c->h_sampler.noise_dims == 2, s);
     if (e == hipSuccess) e = launch_count(A, word_blocks(dim), 0, s);

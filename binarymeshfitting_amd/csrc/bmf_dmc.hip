@@ -367,20 +367,6 @@ struct DmcWave {
     float4 csg[2 * kItemCsg];     // stage_csg layout
 };
 
-// World box of the item's cells: lo and hi per axis.
-__device__ __forceinline__ void item_box(const ChunkMeta& M, int w0, float (&lo)[3], float (&hi)[3]) {
-    const int dim = M.dim, d2 = dim * dim, a = 64 * w0, b = min(a + kItemSamples, d2 * dim) - 1;
-    const int xa = a / d2, xb = b / d2;
-    const int ya = (a - xa * d2) / dim, yb = (b - xb * d2) / dim;
-    const int c0[3] = {xa, xa == xb ? ya : 0, 0};
-    const int c1[3] = {xb + 1, xa == xb ? yb + 1 : dim - 1, dim - 1};
-#pragma unroll
-    for (int k = 0; k < 3; k++) {
-        lo[k] = (float)c0[k] * M.delta + M.opos[k];
-        hi[k] = (float)c1[k] * M.delta + M.opos[k];
-    }
-}
-
 // ------------------------------------------------------------------------
 // vertices: one per polygon of each active cell, a wave per item.  Rounds of
 // 64 cells: each cell's first vertex id and mask, its polygons compacted into
@@ -497,7 +483,7 @@ __global__ void __launch_bounds__(kRowThreads) k_dmc_vertices(Arenas A) {
         bool staged = false;
         if (qef && csg) {
             float lo[3], hi[3], far = 0.0f;
-            item_box(M, w0, lo, hi);
+            sample_box(M, 64 * w0, kItemSamples, 1, lo, hi);  // the cells' far corners too
 #pragma unroll
             for (int k = 0; k < 3; k++) far = fmaxf(far, fmaxf(fabsf(lo[k]), fabsf(hi[k])));
             int is, ib;

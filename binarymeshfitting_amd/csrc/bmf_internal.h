@@ -7,11 +7,6 @@
 
 namespace bmf {
 
-// Samples handled by one work-queue tile of the sampling kernel: 256 threads
-// x rounds (4, 8 or 16, chosen at run time: Arenas::sample_tile); a multiple
-// of 64 so that every wave owns whole label words.
-constexpr int kSampleThreads = 256;
-constexpr int kSampleTileDefault = 2048;
 constexpr int kRowThreads = 256;      // word kernels: 4 waves, an item of label words each
 constexpr int kItemWords = 16;        // label words per item: enough active cells for a wave's lanes near a surface
 constexpr int kItemSamples = 64 * kItemWords;
@@ -94,12 +89,10 @@ struct ChunkMeta {
 
 // Global counters, reset by the plan kernel.
 struct Counters {
-    unsigned long long sample_head;
     unsigned long long v_bump;
     unsigned long long i_bump;
     unsigned long long need_v;
     unsigned long long need_i;
-    int64_t total_tiles;
     int64_t total_samples;
     int32_t xcd_vtiles[kXcds]; // smoothing tiles of each XCD's maps
     int32_t xcd_ttiles[kXcds];
@@ -120,12 +113,12 @@ struct Arenas {
     ChunkMeta* meta;           // [max_chunks]
     bmf_chunk_desc* descs;     // [max_chunks]
     bmf_chunk_result* results; // [max_chunks]
-    int64_t* tile_prefix;      // [max_chunks + 1] sampling tiles
-    int64_t* block_prefix;     // [max_chunks + 1] items of kWaveBlocks sample blocks (k_blocks)
+    int64_t* block_prefix;     // [max_chunks + 1] items of the sampler's pre-pass: kWaveBlocks sample blocks
+                               // (k_blocks) or 64 columns (k_columns)
     uint8_t* signs;            // [max_samples + 16] adaptive terrain: k_blocks' decisions, from the chunk's first
                                // sample on a byte per four samples of a row (x, y), ceil(dim / 4) bytes a row:
                                // undecided samples in the low bits, air samples in the high ones
-    int64_t* plan_part;        // [10 nb + 1] multi-block plan passes (nb = max_chunks / 1024 rounded up): block
+    int64_t* plan_part;        // [8 nb + 1] multi-block plan passes (nb = max_chunks / 1024 rounded up): block
                                // totals and bases, overflow flag
     unsigned long long* stat_blocks;  // [3][stat_cap] terrain octaves evaluated per workgroup of the
                                       // sampling, refinement and block kernels (plain stores, no atomics)
@@ -157,7 +150,6 @@ struct Arenas {
     int64_t cap_samples, cap_vertices, cap_indices;
     int32_t cap_chunks;
     int64_t ext_base;          // EXTERNAL: offset of this launch's first chunk in the caller's densities
-    int32_t sample_tile;       // samples per sampling work-queue tile: 1024, 2048 or 4096
     int32_t smoothing_follows; // the launch runs the smoothing kernels after the emit kernel (which then
                                // leaves the output positions of the vertices they move to them)
     uint16_t* csg_list;        // CSG: [chunk][csg_stride] primitives per chunk (k_plan), or null
@@ -181,6 +173,9 @@ struct Arenas {
 // 7 quads, or 14 triangles when quads are written as triangles.
 constexpr int kRingSlots = 16;
 
+// Workgroups that sample one chunk of ns samples: a wave per 256 of them, the
+// finest of the sampling kernels' items.
+inline int sample_blocks_of(int64_t ns) { return (int)((ns + 1023) / 1024); }
 // Workgroups that give every item of one chunk's word kernels its wave.
 inline int word_blocks(int dim) {
     const int64_t items = ((int64_t)dim * dim * dim + kItemSamples - 1) / kItemSamples;
@@ -189,7 +184,7 @@ inline int word_blocks(int dim) {
 
 // Launch wrappers (bmf_kernels.hip).
 hipError_t launch_plan(const Arenas& A, int n, int allow_cull, int reset_bumps, hipStream_t s);
-// adaptive: terrain samples stop adding octaves once their label is decided
+// adaptive: signs everywhere and densities where the surface reads them (terrain, CSG); 0: every density
 // kind: the sampler the device struct holds for this launch (BMF_SAMPLER_*)
 // slab: the sampler is a 2D noise field (its columns are evaluated once per tile)
 hipError_t launch_sample(const Arenas& A, int n, int blocks, int adaptive, int kind, int slab, hipStream_t s);

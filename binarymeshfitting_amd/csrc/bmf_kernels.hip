@@ -135,10 +135,10 @@ __device__ __forceinline__ BlockPlan plan_blocks(const SamplerDev& S, const Chun
 
 // Plan record of one descriptor: DMCChunk::label_grid geometry
 // (DMCChunk.cpp:94-101) and analytic culling; `add` gets its contributions
-// to the arena sums (samples, label words, word items, sampling tiles, items
-// of sample blocks), each below 2^25.
+// to the arena sums (samples, label words, word items, items of the sampler's
+// own pre-pass: k_blocks' or k_columns'), each at most 2^24.
 __device__ __forceinline__ ChunkMeta plan_record(const Arenas& A, const SamplerDev* __restrict__ S,
-                                                 const bmf_chunk_desc& d, int allow_cull, uint32_t (&add)[5]) {
+                                                 const bmf_chunk_desc& d, int allow_cull, uint32_t (&add)[4]) {
     ChunkMeta m;
     float t = d.overlap * 2.0f;
     t = 1.0f + t;
@@ -178,23 +178,24 @@ __device__ __forceinline__ ChunkMeta plan_record(const Arenas& A, const SamplerD
     add[0] = sampled ? ns : 0u;
     add[1] = (uint32_t)m.lab_words;
     add[2] = ((uint32_t)m.lab_words + kItemWords - 1) / kItemWords;
-    add[3] = sampled ? (ns + (uint32_t)A.sample_tile - 1) / (uint32_t)A.sample_tile : 0u;
-    add[4] = sampled ? (nb * nb * nb + kWaveBlocks - 1) / kWaveBlocks : 0u;
+    add[3] = !sampled                                              ? 0u
+             : S->kind == BMF_SAMPLER_TERRAIN                     ? (nb * nb * nb + kWaveBlocks - 1) / kWaveBlocks
+             : S->kind == BMF_SAMPLER_NOISE && S->noise_dims == 2 ? ((uint32_t)d.dim * (uint32_t)d.dim + 63u) / 64u
+                                                                  : 0u;
     return m;
 }
 
-__device__ __forceinline__ bool plan_overflow(const Arenas& A, const int64_t (&tot)[5]) {
+__device__ __forceinline__ bool plan_overflow(const Arenas& A, const int64_t (&tot)[4]) {
     return tot[0] > A.cap_samples || tot[1] > A.cap_samples / 64 + A.cap_chunks;
 }
 
 // A record's final state, `at` the arena sums before it.
 __device__ __forceinline__ void plan_finish(const Arenas& A, const SamplerDev* __restrict__ S, int j, ChunkMeta& m,
-                                            const int64_t (&at)[5], bool overflow) {
+                                            const int64_t (&at)[4], bool overflow) {
     m.dens_off = at[0];
     m.lab_off = at[1];
     m.item_slot = at[2];
-    A.tile_prefix[j] = overflow ? 0 : at[3];
-    A.block_prefix[j] = overflow ? 0 : at[4];
+    A.block_prefix[j] = overflow ? 0 : at[3];
     m.blocks = BlockPlan{};
     if (m.state == kStateSampled) {
         if (S->kind == BMF_SAMPLER_TERRAIN) m.blocks = plan_blocks(*S, m);
@@ -210,13 +211,11 @@ __device__ __forceinline__ void plan_finish(const Arenas& A, const SamplerDev* _
     if (m.state != kStateSampled) write_result(A, j, m);  // final: k_scan skips it
 }
 
-// The batch counters from the totals: sampling tiles, word items, overflow.
-__device__ __forceinline__ void plan_counters(const Arenas& A, int n, const int64_t (&tot)[5], bool overflow,
+// The batch counters from the totals: word items, overflow.
+__device__ __forceinline__ void plan_counters(const Arenas& A, int n, const int64_t (&tot)[4], bool overflow,
                                               int reset_bumps) {
-    A.tile_prefix[n] = overflow ? 0 : tot[3];
-    A.block_prefix[n] = overflow ? 0 : tot[4];
+    A.block_prefix[n] = overflow ? 0 : tot[3];
     Counters* c = A.ctr;
-    c->sample_head = 0;
     if (reset_bumps) {
         c->v_bump = 0;
         c->i_bump = 0;
@@ -226,7 +225,6 @@ __device__ __forceinline__ void plan_counters(const Arenas& A, int n, const int6
         c->error = 0;
     }
     if (overflow) c->overflow = 1;
-    c->total_tiles = overflow ? 0 : tot[3];
     c->total_items = overflow ? 0 : tot[2];
     c->n_smooth = 0;
     for (int g = 0; g < kXcds; g++) c->xcd_vtiles[g] = c->xcd_ttiles[g] = 0;
@@ -240,30 +238,30 @@ __device__ __forceinline__ void plan_counters(const Arenas& A, int n, const int6
 // records are 120 bytes apart, written and read again across the scan);
 // this takes 6.7 and 9.9 (5.4 for one).
 __global__ void __launch_bounds__(kPlanThreads) k_plan(Arenas A, int n, int allow_cull, int reset_bumps) {
-    __shared__ uint32_t s_w[5][kPlanThreads / 64];
+    __shared__ uint32_t s_w[4][kPlanThreads / 64];
     const SamplerDev* __restrict__ S = A.sampler;
     const int per = (n + kPlanThreads - 1) / kPlanThreads;  // 1 or 2
     const int j0 = threadIdx.x * per;
-    uint32_t sum[5] = {0u, 0u, 0u, 0u, 0u};
+    uint32_t sum[4] = {0u, 0u, 0u, 0u};
     for (int i = 0; i < per; i++) {
         if (j0 + i >= n) break;
-        uint32_t add[5];
+        uint32_t add[4];
         (void)plan_record(A, S, A.descs[j0 + i], allow_cull, add);
 #pragma unroll
-        for (int q = 0; q < 5; q++) sum[q] += add[q];
+        for (int q = 0; q < 4; q++) sum[q] += add[q];
     }
-    int64_t excl[5], tot[5];
-    block_scan32<5, kPlanThreads>(sum, excl, tot, s_w);
+    int64_t excl[4], tot[4];
+    block_scan32<4, kPlanThreads>(sum, excl, tot, s_w);
     const bool overflow = plan_overflow(A, tot);
     // the block's own records, formed again
     for (int i = 0; i < per; i++) {
         const int j = j0 + i;
         if (j >= n || j / kPlanSlice != (int)blockIdx.x) break;  // per divides kPlanSlice
-        uint32_t add[5];
+        uint32_t add[4];
         ChunkMeta m = plan_record(A, S, A.descs[j], allow_cull, add);
         plan_finish(A, S, j, m, excl, overflow);
 #pragma unroll
-        for (int q = 0; q < 5; q++) excl[q] += add[q];
+        for (int q = 0; q < 4; q++) excl[q] += add[q];
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) plan_counters(A, n, tot, overflow, reset_bumps);
 }
@@ -271,49 +269,49 @@ __global__ void __launch_bounds__(kPlanThreads) k_plan(Arenas A, int n, int allo
 // Larger batches, pass 1 of 3 (one descriptor per thread over many blocks):
 // each block's totals.
 __global__ void __launch_bounds__(kPlanThreads) k_plan_part(Arenas A, int n, int allow_cull) {
-    __shared__ uint32_t s_w[5][kPlanThreads / 64];
+    __shared__ uint32_t s_w[4][kPlanThreads / 64];
     const int j = blockIdx.x * kPlanThreads + threadIdx.x;
-    uint32_t add[5] = {0u, 0u, 0u, 0u, 0u};
+    uint32_t add[4] = {0u, 0u, 0u, 0u};
     if (j < n) (void)plan_record(A, A.sampler, A.descs[j], allow_cull, add);
-    int64_t excl[5], tot[5];
-    block_scan32<5, kPlanThreads>(add, excl, tot, s_w);
-    if (threadIdx.x < 5) A.plan_part[5 * blockIdx.x + threadIdx.x] = pick<5>(tot, (int)threadIdx.x);
+    int64_t excl[4], tot[4];
+    block_scan32<4, kPlanThreads>(add, excl, tot, s_w);
+    if (threadIdx.x < 4) A.plan_part[4 * blockIdx.x + threadIdx.x] = pick<4>(tot, (int)threadIdx.x);
 }
 
 // Pass 2 (one block, one thread per pass-1 block, at most kPlanThreads):
 // block bases, batch totals, overflow flag, counters.  Bases go to
-// plan_part[5 (nb + b) ...], the overflow flag after them.
+// plan_part[4 (nb + b) ...], the overflow flag after them.
 __global__ void __launch_bounds__(kPlanThreads) k_plan_total(Arenas A, int n, int nb, int reset_bumps) {
-    __shared__ int64_t s_w[5][kPlanThreads / 64 + 1];
+    __shared__ int64_t s_w[4][kPlanThreads / 64 + 1];
     const int b = threadIdx.x;
-    int64_t v[5];
+    int64_t v[4];
 #pragma unroll
-    for (int q = 0; q < 5; q++) v[q] = b < nb ? A.plan_part[5 * b + q] : 0;
-    int64_t excl[5], tot[5];
-    block_scan<5, kPlanThreads>(v, excl, tot, s_w);
+    for (int q = 0; q < 4; q++) v[q] = b < nb ? A.plan_part[4 * b + q] : 0;
+    int64_t excl[4], tot[4];
+    block_scan<4, kPlanThreads>(v, excl, tot, s_w);
     const bool overflow = plan_overflow(A, tot);
     if (b < nb)
 #pragma unroll
-        for (int q = 0; q < 5; q++) A.plan_part[5 * (nb + b) + q] = excl[q];
+        for (int q = 0; q < 4; q++) A.plan_part[4 * (nb + b) + q] = excl[q];
     if (b == 0) {
-        A.plan_part[10 * nb] = overflow;
+        A.plan_part[8 * nb] = overflow;
         plan_counters(A, n, tot, overflow, reset_bumps);
     }
 }
 
 // Pass 3: the records with their offsets, the results of culled chunks.
 __global__ void __launch_bounds__(kPlanThreads) k_plan_fix(Arenas A, int n, int nb, int allow_cull) {
-    __shared__ uint32_t s_w[5][kPlanThreads / 64];
+    __shared__ uint32_t s_w[4][kPlanThreads / 64];
     const int j = blockIdx.x * kPlanThreads + threadIdx.x;
-    uint32_t add[5] = {0u, 0u, 0u, 0u, 0u};
+    uint32_t add[4] = {0u, 0u, 0u, 0u};
     ChunkMeta m{};
     if (j < n) m = plan_record(A, A.sampler, A.descs[j], allow_cull, add);
-    int64_t at[5], tot[5];
-    block_scan32<5, kPlanThreads>(add, at, tot, s_w);
+    int64_t at[4], tot[4];
+    block_scan32<4, kPlanThreads>(add, at, tot, s_w);
     if (j >= n) return;
 #pragma unroll
-    for (int q = 0; q < 5; q++) at[q] += A.plan_part[5 * (nb + blockIdx.x) + q];
-    plan_finish(A, A.sampler, j, m, at, A.plan_part[10 * nb] != 0);
+    for (int q = 0; q < 4; q++) at[q] += A.plan_part[4 * (nb + blockIdx.x) + q];
+    plan_finish(A, A.sampler, j, m, at, A.plan_part[8 * nb] != 0);
 }
 
 // ------------------------------------------------------------------------
@@ -822,153 +820,168 @@ __global__ void __launch_bounds__(kRowThreads) k_terrain(Arenas A, int n) {
     if (tid == 0 && (int)blockIdx.x < A.stat_cap) A.stat_blocks[blockIdx.x] = s_evals;
 }
 
-// Sampling modes of k_sample, fixed per launch by the host: the CSG union with
-// the chunk's culled primitives staged in LDS once per tile; a 2D noise field
-// with the noise of the tile's (x, z) columns evaluated once into LDS and
-// broadcast along y; every other case (external densities, implicit shapes,
-// 3D noise fields, the terrain in full) evaluated directly.  Persistent:
-// workgroups pull tiles of Arenas::sample_tile consecutive samples of one
-// chunk from an atomic work queue.
-constexpr int kSampleGeneric = 0, kSampleCsg = 2, kSampleSlab = 3;
+// ------------------------------------------------------------------------
+// sample: every sampler but the adaptive terrain, one wave per WORDS label
+// words (all of them in a chunk's first item, and so on): no barrier and no
+// LDS but the CSG primitives.  The words per wave balance the chip's last
+// round against the wave's own set-up.  Bound by VALU issue where a sampler is
+// evaluated, by HBM where densities only pass through.
+//   terrain in full  129^3 samples, 5 octaves: 64 us (tiles of 2,048
+//                    samples per workgroup, 1,049 of them: 95)
+//   external         48 chunks of 41^3: 12 us (tiles: 52)
+//   2D noise field   from the columns of k_columns
+//   CSG              with the item's own primitives, see below
+// ------------------------------------------------------------------------
+constexpr int kSampleImplicit = 0, kSampleTerrain = 1, kSampleCsg = 2, kSampleField2 = 3, kSampleField3 = 4,
+              kSampleExternal = 5;
+constexpr int kWaveCsg = 64;  // CSG primitives per wave staged in LDS (longer lists read global memory)
 
-template <int ROUNDS, int MODE>
-__global__ void __launch_bounds__(kSampleThreads) k_sample(Arenas A, int n) {
-    constexpr int kTile = ROUNDS * kSampleThreads;
-    constexpr int kC = MODE == kSampleCsg ? 2 * kCsgStage : 1;  // staged CSG primitives
-    // 2D noise columns of a tile: its samples span at most kTile / dim^2 + 2
-    // x-planes of dim columns, i.e. at most kTile / dim + 2 dim <= kTile / 2 + 2 BMF_MAX_DIM
-    constexpr int kSlab = MODE == kSampleSlab ? kTile / 2 + 2 * BMF_MAX_DIM : 1;
-    __shared__ float s_slab[kSlab];
-    __shared__ int64_t s_tile;
-    __shared__ float4 s_csg[kC];
-    __shared__ unsigned long long s_lab[kTile / 64];
-    __shared__ unsigned long long s_exact[kTile / 64];
-    __shared__ uint32_t s_flags;
+// 2D noise fields: n at every (x, z) column of every chunk, a lane each, into
+// the cell arena (free until the emission), from the chunk's first sample on.
+// Evaluated per tile of samples instead, the columns filled 96 of a
+// workgroup's 256 lanes: 168 chunks of 32^3 took 76 us; this and the pass
+// over the samples take 26 + 18.
+__global__ void __launch_bounds__(kRowThreads) k_columns(Arenas A, int n) {
     const SamplerDev* __restrict__ S = A.sampler;
-    const int64_t total = A.ctr->total_tiles;
+    const int64_t total = A.block_prefix[n];
     const int lane = lane_id();
-    // (chunk, item) of every item of the word kernels that follow
-    for (int j = blockIdx.x; j < n; j += gridDim.x) {
-        const ChunkMeta& M = A.meta[j];
-        if (M.state != kStateSampled) continue;
-        const int64_t ps = M.item_slot;
-        const int ni = (int)((M.lab_words + kItemWords - 1) / kItemWords);
-        for (int x = threadIdx.x; x < ni; x += blockDim.x) A.item_map[ps + x] = make_int2(j, x);
-    }
-    for (;;) {
-        if (threadIdx.x == 0) {
-            s_tile = (int64_t)atomicAdd(&A.ctr->sample_head, 1ull);
-            s_flags = 0;
-        }
-        __syncthreads();
-        const int64_t tile = s_tile;
-        if (tile >= total) break;
-        const int j = find_chunk(A.tile_prefix, n, tile);
-        const ChunkMeta& M = A.meta[j];
+    for (int64_t it = (int64_t)blockIdx.x * kWordWaves + (threadIdx.x >> 6); it < total;
+         it += (int64_t)gridDim.x * kWordWaves) {
+        const int j = find_chunk_wave(A.block_prefix, n, it);
+        const ChunkMeta M = read_chunk(A.meta, j);
+        const int c = (int)(it - A.block_prefix[j]) * 64 + lane;
+        if (c >= M.dim * M.dim) continue;
+        const int x = c / M.dim, z = c - x * M.dim;
         const ChunkGeom G{M.opos[0], M.opos[1], M.opos[2], M.delta};
+        float px, py, pz;
+        sample_position(G, (uint32_t)x, 0u, (uint32_t)z, px, py, pz);
+        A.cell_tb[M.dens_off + c] = __float_as_uint(noise_value(*S, px, 0.0f, pz));
+    }
+}
+
+// full: CSG values are wanted at every sample (stage inspection, the tape).
+// Otherwise only signs and the densities at the ends of sign-changing edges
+// are read, where the union lies within a sample step of 0 (it is
+// 1-Lipschitz): primitives that stay below -2 steps (and a coordinate-sized
+// slack) everywhere in the item's box cannot win there, and an item without
+// any is air.  64 chunks of 64^3 cells, 300 primitives: 69 us, with
+// every primitive within reach of the chunk's floor at every sample 245.
+template <int MODE, int WORDS>
+__global__ void __launch_bounds__(kRowThreads) k_sample(Arenas A, int n, int full) {
+    constexpr int kParts = kItemWords / WORDS;  // waves per item of the word kernels
+    constexpr bool kCsg = MODE == kSampleCsg;
+    __shared__ float4 s_csg[kCsg ? kWordWaves : 1][kCsg ? 2 * kWaveCsg : 1];
+    const SamplerDev* __restrict__ S = A.sampler;
+    const int wave = uniform_int(threadIdx.x >> 6), lane = lane_id();
+    const int64_t total = A.ctr->total_items * kParts;
+    for (int64_t u = (int64_t)blockIdx.x * kWordWaves + wave; u < total; u += (int64_t)gridDim.x * kWordWaves) {
+        const int64_t it = u / kParts;
+        const int part = (int)(u - it * kParts);
+        const int j = find_item_wave(A.meta, n, it);
+        const ChunkMeta M = read_chunk(A.meta, j);
+        const int item = (int)(it - M.item_slot), w0 = item * kItemWords + part * WORDS;
+        if (part == 0 && lane == 0) A.item_map[it] = make_int2(j, item);  // for the word kernels
+        if (w0 >= (int)M.lab_words) continue;
         const uint32_t dim = (uint32_t)M.dim, dim2 = dim * dim, ns = dim2 * dim;
-        const float rd = 1.0f / (float)dim, rd2 = 1.0f / (float)dim2;
+        const ChunkGeom G{M.opos[0], M.opos[1], M.opos[2], M.delta};
         float* __restrict__ dens = A.dens + M.dens_off;
-        const uint32_t first = (uint32_t)(tile - A.tile_prefix[j]) * kTile;
-        bool staged = false;
-        if constexpr (MODE == kSampleCsg) {
-            staged = M.csg_ns + M.csg_nb <= kCsgStage;  // uniform across the block
-            if (staged) {
-                stage_csg(*S, A.csg_list + (int64_t)j * A.csg_stride, M.csg_ns, M.csg_nb, s_csg);
-                __syncthreads();
+        const uint32_t first = 64u * (uint32_t)w0;
+        uint64_t mine = 0ull;  // lane r keeps word r
+        bool air = false, solid = false;
+        auto word = [&](int r, bool valid, bool is_air) {
+            const uint64_t bl = __ballot(valid && is_air), vb = __ballot(valid);
+            mine = lane == r ? bl : mine;
+            air = air || bl != 0ull;
+            solid = solid || bl != vb;
+        };
+        if constexpr (MODE == kSampleExternal) {
+            const float* __restrict__ src = S->ext + A.ext_base + M.dens_off;
+            float v[WORDS];
+#pragma unroll
+            for (int r = 0; r < WORDS; r++) v[r] = src[min(first + 64u * r + (uint32_t)lane, ns - 1u)];
+#pragma unroll
+            for (int r = 0; r < WORDS; r++) {
+                const uint32_t i = first + 64u * r + (uint32_t)lane;
+                if (i < ns) dens[i] = v[r];
+                word(r, i < ns, v[r] < 0.0f);
             }
-        }
-        uint32_t slab_x0 = 0;
-        if constexpr (MODE == kSampleSlab) {
-            const uint32_t last = min(first + (uint32_t)kTile, ns) - 1u;
-            slab_x0 = first / dim2;
-            const uint32_t ncol = (last / dim2 - slab_x0 + 1u) * dim;
-            if (ncol > (uint32_t)kSlab) {
-                if (threadIdx.x == 0) A.ctr->error = 12;  // unreachable by the bound above
-            } else {
-                for (uint32_t q = threadIdx.x; q < ncol; q += blockDim.x) {
-                    const uint32_t qx = q / dim, qz = q - qx * dim;
-                    float px, py, pz;
-                    sample_position(G, slab_x0 + qx, 0u, qz, px, py, pz);
-                    s_slab[q] = noise_value(*S, px, 0.0f, pz);
+        } else {
+            const uint16_t* list = nullptr;
+            int cs = 0, cb = 0;
+            bool staged = false, empty = false;
+            if constexpr (kCsg) {
+                list = A.csg_list ? A.csg_list + (int64_t)j * A.csg_stride : nullptr;
+                cs = M.csg_ns;
+                cb = M.csg_nb;
+                if (list && !full) {
+                    float lo[3], hi[3], far = 0.0f;
+                    sample_box(M, (int)first, 64 * WORDS, 0, lo, hi);
+#pragma unroll
+                    for (int k = 0; k < 3; k++) far = fmaxf(far, fmaxf(fabsf(lo[k]), fabsf(hi[k])));
+                    int is, ib;
+                    staged = cull_csg(*S, list, cs, cb, lo, hi, 2.0f * M.delta + 1e-4f * far, s_csg[wave], kWaveCsg, is, ib);
+                    if (staged) {
+                        cs = is;
+                        cb = ib;
+                        empty = is + ib == 0;
+                    }
+                    wave_sync();
                 }
             }
-            __syncthreads();
-        }
-        // ---- phase 0: every sample of the tile ----
-        // A thread's sample advances by kSampleThreads per round: its (x, y, z)
-        // advances by (0, q, r) with q, r = kSampleThreads / dim, % dim and at
-        // most one carry per axis while q + 1 < dim; smaller chunks divide.
-        const uint32_t step_y = kSampleThreads / dim, step_z = kSampleThreads - step_y * dim;
-        const bool stepping = step_y + 1 < dim;
-        uint32_t cx, cy, cz;
-        sample_index(first + threadIdx.x, dim, dim2, rd, rd2, cx, cy, cz);
+            // a lane's sample advances by 64 per word: its (y, z) by
+            // (64 / dim, 64 % dim) with at most one carry per axis while
+            // 64 / dim + 1 < dim; smaller chunks divide
+            const float rd = 1.0f / (float)dim, rd2 = 1.0f / (float)dim2;
+            const uint32_t step_y = 64u / dim, step_z = 64u - step_y * dim;
+            const bool stepping = step_y + 1 < dim;
+            uint32_t x, y, z;
+            sample_index(first + (uint32_t)lane, dim, dim2, rd, rd2, x, y, z);
 #pragma unroll 1
-        for (int r = 0; r < ROUNDS; r++) {
-            const uint32_t li = r * kSampleThreads + threadIdx.x;  // waves cover 64 consecutive samples
-            const uint32_t i = first + li;
-            const bool valid = i < ns;
-            if (r > 0) {
+            for (int r = 0; r < WORDS; r++) {
+                const uint32_t i = first + 64u * (uint32_t)r + (uint32_t)lane;
+                const bool valid = i < ns;
+                float d = kCsgFloor;
+                if (valid && !empty) {
+                    float px, py, pz;
+                    sample_position(G, x, y, z, px, py, pz);
+                    if constexpr (MODE == kSampleTerrain) d = terrain_density(*S, px, py, pz);
+                    else if constexpr (MODE == kSampleField2)
+                        d = noise_density_from(*S, __uint_as_float(A.cell_tb[M.dens_off + x * dim + z]), py);
+                    else if constexpr (MODE == kSampleField3) d = noise_density_from(*S, noise_value(*S, px, py, pz), py);
+                    else if constexpr (kCsg) {
+                        if (staged) d = csg_density_lds(s_csg[wave], cs, cb, px, py, pz);
+                        else if (list) d = csg_density_list(*S, list, cs, cb, px, py, pz);
+                        else d = csg_density(*S, px, py, pz);
+                    } else d = implicit_density(S->kind, S->world_size, px, py, pz);
+                    dens[i] = d;
+                }
+                word(r, valid, d < 0.0f);
                 if (stepping) {
-                    cz += step_z;
-                    cy += step_y;
-                    if (cz >= dim) {
-                        cz -= dim;
-                        cy++;
+                    z += step_z;
+                    y += step_y;
+                    if (z >= dim) {
+                        z -= dim;
+                        y++;
                     }
-                    if (cy >= dim) {
-                        cy -= dim;
-                        cx++;
+                    if (y >= dim) {
+                        y -= dim;
+                        x++;
                     }
                 } else {
-                    sample_index(i, dim, dim2, rd, rd2, cx, cy, cz);
+                    sample_index(min(i + 64u, ns), dim, dim2, rd, rd2, x, y, z);
                 }
             }
-            bool air = false;
-            if (valid) {
-                float px, py, pz;
-                sample_position(G, cx, cy, cz, px, py, pz);
-                float d;
-                if constexpr (MODE == kSampleSlab) {
-                    const uint32_t q = (cx - slab_x0) * dim + cz;
-                    d = noise_density_from(*S, q < (uint32_t)kSlab ? s_slab[q] : 0.0f, py);
-                } else if (staged) d = csg_density_lds(s_csg, M.csg_ns, M.csg_nb, px, py, pz);
-                else if (S->kind == BMF_SAMPLER_EXTERNAL) d = S->ext[A.ext_base + M.dens_off + i];
-                else if (S->kind == BMF_SAMPLER_CSG && A.csg_list)
-                    d = csg_density_list(*S, A.csg_list + (int64_t)j * A.csg_stride, M.csg_ns, M.csg_nb, px, py, pz);
-                else d = sample_density(*S, px, py, pz);
-                dens[i] = d;
-                air = d < 0.0f;
-            }
-            const uint64_t bl = __ballot(valid && air);
-            const uint64_t vb = __ballot(valid);
-            if (lane == 0) {
-                s_lab[li >> 6] = bl;
-                s_exact[li >> 6] = vb;
-            }
+            if constexpr (kCsg) wave_sync();  // the primitives are read
         }
-        __syncthreads();
-        // ---- label and exactness words of the tile ----
-        if (threadIdx.x < kTile / 64) {
-            const uint32_t w0 = first + 64u * threadIdx.x;
-            if (w0 < ns) {
-                const uint32_t nb = ns - w0;
-                const uint64_t vm = nb >= 64 ? ~0ull : ((1ull << nb) - 1ull);
-                const uint64_t lb = s_lab[threadIdx.x];
-                A.labels[M.lab_off + (w0 >> 6)] = lb;
-                A.exact[M.lab_off + (w0 >> 6)] = s_exact[threadIdx.x];
-                uint32_t fl = 0;
-                if (lb & vm) fl |= 1u;
-                if (~lb & vm) fl |= 2u;
-                if (fl) atomicOr(&s_flags, fl);
-            }
+        if (lane < WORDS && w0 + lane < (int)M.lab_words) {
+            const int left = (int)ns - 64 * (w0 + lane);
+            A.labels[M.lab_off + w0 + lane] = mine;
+            A.exact[M.lab_off + w0 + lane] = ~bits_from(left);
         }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            if (s_flags & 1u) atomicOr(&A.meta[j].any_air, 1u);
-            if (s_flags & 2u) atomicOr(&A.meta[j].any_solid, 1u);
+        if (lane == 0) {
+            if (air && !A.meta[j].any_air) atomicOr(&A.meta[j].any_air, 1u);
+            if (solid && !A.meta[j].any_solid) atomicOr(&A.meta[j].any_solid, 1u);
         }
-        __syncthreads();
     }
     if (threadIdx.x == 0 && (int)blockIdx.x < A.stat_cap) A.stat_blocks[blockIdx.x] = 0ull;  // no octaves counted
 }
@@ -1839,28 +1852,24 @@ hipError_t launch_plan(const Arenas& A, int n, int allow_cull, int reset_bumps, 
     return hipGetLastError();
 }
 hipError_t launch_sample(const Arenas& A, int n, int blocks, int adaptive, int kind, int slab, hipStream_t s) {
-    const dim3 g(blocks), b(kSampleThreads);
-    if (adaptive && kind == BMF_SAMPLER_TERRAIN) {
-        hipLaunchKernelGGL(k_blocks, g, dim3(kRowThreads), 0, s, A, n);
-        hipLaunchKernelGGL(k_terrain, g, dim3(kRowThreads), 0, s, A, n);
-        return hipGetLastError();
+    const dim3 g(blocks), b(kRowThreads);
+    if (kind == BMF_SAMPLER_TERRAIN && adaptive) {
+        hipLaunchKernelGGL(k_blocks, g, b, 0, s, A, n);
+        hipLaunchKernelGGL(k_terrain, g, b, 0, s, A, n);
+    } else if (kind == BMF_SAMPLER_TERRAIN) {
+        hipLaunchKernelGGL((k_sample<kSampleTerrain, 4>), g, b, 0, s, A, n, 1);
+    } else if (kind == BMF_SAMPLER_NOISE && slab) {
+        hipLaunchKernelGGL(k_columns, g, b, 0, s, A, n);
+        hipLaunchKernelGGL((k_sample<kSampleField2, 16>), g, b, 0, s, A, n, 1);
+    } else if (kind == BMF_SAMPLER_NOISE) {
+        hipLaunchKernelGGL((k_sample<kSampleField3, 4>), g, b, 0, s, A, n, 1);
+    } else if (kind == BMF_SAMPLER_CSG) {
+        hipLaunchKernelGGL((k_sample<kSampleCsg, 16>), g, b, 0, s, A, n, !adaptive);
+    } else if (kind == BMF_SAMPLER_EXTERNAL) {
+        hipLaunchKernelGGL((k_sample<kSampleExternal, 16>), g, b, 0, s, A, n, 1);
+    } else {
+        hipLaunchKernelGGL((k_sample<kSampleImplicit, 16>), g, b, 0, s, A, n, 1);
     }
-    const int mode = kind == BMF_SAMPLER_CSG && A.csg_list ? kSampleCsg
-                     : kind == BMF_SAMPLER_NOISE && slab   ? kSampleSlab
-                                                           : kSampleGeneric;
-#define BMF_SAMPLE(R)                                                                             \
-    switch (mode) {                                                                               \
-        case kSampleCsg: hipLaunchKernelGGL((k_sample<R, kSampleCsg>), g, b, 0, s, A, n); break;           \
-        case kSampleSlab: hipLaunchKernelGGL((k_sample<R, kSampleSlab>), g, b, 0, s, A, n); break;         \
-        default: hipLaunchKernelGGL((k_sample<R, kSampleGeneric>), g, b, 0, s, A, n); break;               \
-    }
-    switch (A.sample_tile) {
-        case 1024: BMF_SAMPLE(4) break;
-        case 2048: BMF_SAMPLE(8) break;
-        case 4096: BMF_SAMPLE(16) break;
-        default: return hipErrorInvalidValue;
-    }
-#undef BMF_SAMPLE
     return hipGetLastError();
 }
 hipError_t launch_count(const Arenas& A, int blocks, int refine, hipStream_t s) {

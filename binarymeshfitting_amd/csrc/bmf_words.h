@@ -26,6 +26,22 @@ __device__ __forceinline__ void wave_sync() {
 // Bits a .. 63 (any a).
 __device__ __forceinline__ uint64_t bits_from(int a) { return a <= 0 ? ~0ull : (a >= 64 ? 0ull : ~0ull << a); }
 
+// World box of the chunk's samples a .. a + count - 1, grown by `grow`
+// sample steps along x and y (z spans the row): lo and hi per axis.
+__device__ __forceinline__ void sample_box(const ChunkMeta& M, int a, int count, int grow, float (&lo)[3],
+                                           float (&hi)[3]) {
+    const int dim = M.dim, d2 = dim * dim, b = min(a + count, d2 * dim) - 1;
+    const int xa = a / d2, xb = b / d2;
+    const int ya = (a - xa * d2) / dim, yb = (b - xb * d2) / dim;
+    const int c0[3] = {xa, xa == xb ? ya : 0, 0};
+    const int c1[3] = {xb + grow, xa == xb ? yb + grow : dim - 1, dim - 1};
+#pragma unroll
+    for (int k = 0; k < 3; k++) {
+        lo[k] = (float)c0[k] * M.delta + M.opos[k];
+        hi[k] = (float)c1[k] * M.delta + M.opos[k];
+    }
+}
+
 // The low four bits of each byte, packed.
 __device__ __forceinline__ uint32_t low_nibbles(uint64_t w) {
     w &= 0x0F0F0F0F0F0F0F0Full;

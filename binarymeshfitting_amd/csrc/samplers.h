@@ -274,26 +274,9 @@ __device__ __forceinline__ float csg_density_list(const SamplerDev& S, const uin
     return best;
 }
 
-// Primitives of a chunk's culled list staged in LDS: two float4 per
-// primitive, (cx, cy, cz, r) and unused for a sphere, (cx, cy, cz, hx) and
-// (hy, hz, -, -) for a box; spheres first.  Same union, same operation order.
-constexpr int kCsgStage = 256;  // primitives per chunk staged in LDS (larger lists read global memory)
-
-__device__ __forceinline__ void stage_csg(const SamplerDev& S, const uint16_t* __restrict__ list, int ns, int nb,
-                                          float4* s_csg) {
-    for (int k = threadIdx.x; k < ns + nb; k += blockDim.x) {
-        if (k < ns) {
-            const float* sp = S.spheres + 4 * list[k];
-            s_csg[2 * k] = make_float4(sp[0], sp[1], sp[2], sp[3]);
-            s_csg[2 * k + 1] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        } else {
-            const float* b = S.boxes + 6 * list[k];
-            s_csg[2 * k] = make_float4(b[0], b[1], b[2], b[3]);
-            s_csg[2 * k + 1] = make_float4(b[4], b[5], 0.0f, 0.0f);
-        }
-    }
-}
-
+// Primitives staged in LDS: two float4 per primitive, (cx, cy, cz, r) and
+// unused for a sphere, (cx, cy, cz, hx) and (hy, hz, -, -) for a box; spheres
+// first.  Same union, same operation order.
 // The primitives of a chunk's list whose value can exceed -reach somewhere
 // in the box [lo, hi], by one wave, in list order into `out` (room for `cap`
 // of them): a sphere within r + reach of the box, a box that meets it grown by

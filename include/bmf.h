@@ -434,8 +434,9 @@ int bmf_stitch(bmf_ctx* ctx, const bmf_world_node* nodes, int32_t n_nodes, const
 /* Tile and workgroup shapes of the BATCHED path (the PLAIN path sizes its
  * launches per chunk).  A field left 0 keeps its current value. */
 typedef struct {
-    int32_t sample_tile;    /* samples per work-queue tile of the sampling kernel: 1024, 2048, 4096 */
-    int32_t sample_blocks;  /* persistent workgroups of the sampling kernel */
+    int32_t sample_tile;    /* 1024, 2048 or 4096: kept for callers, without effect (the sampling kernels
+                               take their work by label words) */
+    int32_t sample_blocks;  /* persistent workgroups of the sampling kernels */
     int32_t row_blocks;     /* persistent workgroups of the word kernels (count, emit) */
     int32_t smooth_blocks;  /* workgroups of the smoothing kernels (rounded up to a multiple of 8) */
     int32_t row_split;      /* 1, 2, 4, 8 or -1: kept for callers, without effect (the word kernels'
