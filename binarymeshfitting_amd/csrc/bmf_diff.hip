@@ -38,6 +38,7 @@
 #include "bmf_context.h"
 #include "bmf_device_tables.h"
 #include "bmf_internal.h"
+#include "bmf_rows.h"
 
 using namespace bmf;
 
@@ -53,9 +54,8 @@ constexpr int kMaxRing = 20;
 constexpr uint32_t kVidMask = 0x3FFFFFFFu;
 constexpr int64_t kMaxTapeVertices = int64_t(1) << 30;
 constexpr int kLeaf = 64;      // targets per leaf box of the nearest-target hierarchy
-constexpr int kNNThreads = 256;  // four vertices per workgroup, one wave each
-constexpr int kNNFan = 6;        // a wave tests 2^kNNFan = 64 boxes of one subtree level at once
-constexpr int kNNFrames = 6;     // frames of the wave's walk: root + ceil(28 / kNNFan) levels for n < 2^31
+constexpr int kNNFan = 6;      // a wave tests 2^kNNFan = 64 boxes of one subtree level at once
+constexpr int kNNFrames = 4;   // inner frames of the walk: ceil(25 / kNNFan) levels less the leaves, n < 2^31
 
 #define BMF_HIP(call)                          \
     do {                                       \
@@ -80,17 +80,57 @@ unsigned step_blocks(int64_t n) { return (unsigned)std::max<int64_t>(1, (n + kSt
 // ------------------------------------------------------------------------
 // forward
 // ------------------------------------------------------------------------
+// Vertices are ordered by lattice cells of 4^3 samples (8^3 in chunks of more
+// than 132), so that consecutive ones are near each other in every direction:
+// vertex ids follow the rows of the chunk, and a row meets a surface in few
+// and far places.  A counting order: rank within the cell (k_tape_take), the
+// cells' places in any sequence (k_order_cells), the order (k_order).
+constexpr int kOrderCells = 33 * 33 * 33;
+constexpr int kPacket = 4;  // vertices that k_nn_query takes together
+__device__ __forceinline__ uint32_t order_cell(uint32_t code, int dim) {
+    const uint32_t s = dim <= 132 ? 2u : 3u, nb = ((uint32_t)dim + (1u << s) - 1u) >> s;
+    const uint32_t x = (code & 255u) >> s, y = ((code >> 8) & 255u) >> s, z = ((code >> 16) & 255u) >> s;
+    return min((x * nb + y) * nb + z, (uint32_t)kOrderCells - 1u);
+}
+
+// The first place of each cell that holds vertices (one atomic per wave), its
+// count cleared for the next forward.  A cell takes whole packets, its spare
+// places -1: packets across two cells would hold vertices that are far apart
+// (a quarter more leaves searched per packet).
+__global__ void __launch_bounds__(kThreads) k_order_cells(uint32_t* __restrict__ cell_n, uint32_t* __restrict__ base,
+                                                          int* __restrict__ places, int32_t* __restrict__ order) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t n = i < kOrderCells ? cell_n[i] : 0u, room = (n + kPacket - 1) / kPacket * kPacket;
+    const uint32_t inc = wave_scan(room);
+    uint32_t at = 0;
+    if (lane_id() == 63 && inc) at = (uint32_t)atomicAdd(places, (int)inc);
+    at = (uint32_t)__builtin_amdgcn_readlane((int)at, 63) + inc - room;
+    if (!n) return;
+    base[i] = at;
+    cell_n[i] = 0u;
+    for (uint32_t k = n; k < room; k++) order[at + k] = -1;
+}
+__global__ void __launch_bounds__(kThreads) k_order(const uint32_t* __restrict__ vedge, int V, int dim,
+                                                    const uint32_t* __restrict__ base,
+                                                    const uint32_t* __restrict__ rank, int32_t* __restrict__ order) {
+    const int v = blockIdx.x * blockDim.x + threadIdx.x;
+    if (v < V) order[base[order_cell(vedge[v], dim)] + rank[v]] = v;
+}
+
 // Takes the chunk's extraction into the tape in one launch: densities, edge
 // codes, boundary flags and triangles copied out of the context's arenas,
 // the positions as float4 (working copy and checkpoint 0, and as float3
-// when no smoothing follows), and each sample's first vertex id (vertices
-// are numbered in sample order, x-, y-, z-edge within a sample).
+// when no smoothing follows), each sample's first vertex id (vertices
+// are numbered in sample order, x-, y-, z-edge within a sample), and each
+// vertex's rank among those of its order cell (k_nn_query's packets).
 __global__ void k_tape_take(const float* __restrict__ dens_in, const uint32_t* __restrict__ vedge_in,
                             const uint8_t* __restrict__ bnd_in, const uint32_t* __restrict__ idx_in,
                             const float* __restrict__ pos_in, int64_t n3, int V, int64_t n_idx, int dim,
                             float* __restrict__ dens, uint32_t* __restrict__ vedge, uint8_t* __restrict__ bnd,
                             uint32_t* __restrict__ idx, float4* __restrict__ p4, float4* __restrict__ ck0,
-                            float* __restrict__ pos3, uint32_t* __restrict__ vid0) {
+                            float* __restrict__ pos3, uint32_t* __restrict__ vid0, uint32_t* __restrict__ cell_n,
+                            uint32_t* __restrict__ rank, int* __restrict__ err) {
+    if (blockIdx.x == 0 && threadIdx.x < 2) err[threadIdx.x] = 0;
     const int64_t total = std::max<int64_t>(n3, std::max<int64_t>(n_idx, V));
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
         if (i < n3) dens[i] = dens_in[i];
@@ -99,6 +139,7 @@ __global__ void k_tape_take(const float* __restrict__ dens_in, const uint32_t* _
             const uint32_t code = vedge_in[i];
             vedge[i] = code;
             bnd[i] = bnd_in[i];
+            rank[i] = atomicAdd(&cell_n[order_cell(code, dim)], 1u);
             const float x = pos_in[3 * i], y = pos_in[3 * i + 1], z = pos_in[3 * i + 2];
             p4[i] = make_float4(x, y, z, 0.0f);
             ck0[i] = make_float4(x, y, z, 0.0f);
@@ -118,10 +159,14 @@ __global__ void k_tape_take(const float* __restrict__ dens_in, const uint32_t* _
 
 // Ring of each vertex from the per-cell triangle bases and masks written by
 // the emit kernel: the 4 cells around its edge in lexicographic order and,
-// in each, the table slots on its local edge in slot order.  Each triangle
+// in each, the triangles that use the edge in slot order.  Each triangle
 // is stored as its other two corners in corner order, the first with the
 // vertex's own place (0, 1, 2) in bits 30-31.  Also the vertex's backward
-// scale: 1 / (3 |ring|) if the primal step moves it, else 1.
+// scale: 1 / (3 |ring|) if the primal step moves it, else 1.  Bound by its
+// chain of gathers (edge code, cells, triangles): the four cells load
+// together, then the corners of kAdjRound triangles (44,392 vertices: 8 us;
+// a cell and a triangle at a time 21).
+constexpr int kAdjRound = 4;
 __global__ void __launch_bounds__(kStepThreads) k_tape_adj(
     const uint32_t* __restrict__ vedge, const uint8_t* __restrict__ boundary, const uint32_t* __restrict__ cell_tb,
     const uint8_t* __restrict__ cell_mask, const uint32_t* __restrict__ idx, int dim, int V, int T, int bp,
@@ -130,33 +175,60 @@ __global__ void __launch_bounds__(kStepThreads) k_tape_adj(
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
     if (v >= V) return;
     const uint32_t code = vedge[v];
+    const uint8_t bnd = boundary[v];
     const int ex = (int)(code & 255u), ey = (int)((code >> 8) & 255u), ez = (int)((code >> 16) & 255u);
     const int ax = (int)(code >> 24);
+    uint32_t tb[4], tm[4];
+    bool in[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++) {  // the rows of c_ring
+        const int u = (c >> 1) - 1, w = (c & 1) - 1;
+        const int cx = ex + (ax == 0 ? 0 : u), cy = ey + (ax == 0 ? u : (ax == 1 ? 0 : w)), cz = ez + (ax == 2 ? 0 : w);
+        in[c] = cx >= 0 && cy >= 0 && cz >= 0 && cx <= dim - 2 && cy <= dim - 2 && cz <= dim - 2;
+        const int64_t ci = in[c] ? ((int64_t)cx * dim + cy) * dim + cz : 0;
+        tb[c] = cell_tb[ci];
+        tm[c] = cell_mask[ci];
+    }
+    // the ring's triangles as bits 5 c + triangle of the cell
+    uint32_t bits = 0;
+#pragma unroll
+    for (int c = 0; c < 4; c++) bits |= (in[c] ? (uint32_t)c_edge_tris.m[tm[c]][4 * ax + 3 - c] : 0u) << (5 * c);
+    const int count = __popc(bits);
     int n = 0;
-    for (int c = 0; c < 4; c++) {
-        const int cx = ex + c_ring[ax][c][0], cy = ey + c_ring[ax][c][1], cz = ez + c_ring[ax][c][2];
-        if (cx < 0 || cy < 0 || cz < 0 || cx > dim - 2 || cy > dim - 2 || cz > dim - 2) continue;
-        const int64_t ci = ((int64_t)cx * dim + cy) * dim + cz;
-        const uint32_t le = (uint32_t)c_ring[ax][c][3];
-        const uint32_t tb = cell_tb[ci];
-        const uint64_t row = c_tri_table[cell_mask[ci]];
-        const int ns = (int)(row >> 60);
-        for (int s = 0; s < ns; s++) {
-            if (((row >> (4 * s)) & 15ull) != le) continue;
-            const uint32_t t = tb + (uint32_t)(s / 3);
-            if (t >= (uint32_t)T || n >= kMaxRing) {
+    while (bits) {
+        uint32_t t[kAdjRound], a[kAdjRound], b[kAdjRound], d[kAdjRound];
+        bool ok[kAdjRound];
+#pragma unroll
+        for (int k = 0; k < kAdjRound; k++) {
+            ok[k] = bits != 0u;
+            const uint32_t q = ok[k] ? (uint32_t)(__ffs(bits) - 1) : 0u;
+            const uint32_t f = q < 5u ? tb[0] : (q < 10u ? tb[1] - 5u : (q < 15u ? tb[2] - 10u : tb[3] - 15u));
+            t[k] = f + q;
+            bits &= bits - 1u;
+            if (ok[k] && t[k] >= (uint32_t)T) {  // counts and ids disagree
                 *err = 1;
-                continue;
+                ok[k] = false;
             }
-            const uint32_t a = idx[3 * t], b = idx[3 * t + 1], d = idx[3 * t + 2];
-            const uint32_t place = a == (uint32_t)v ? 0u : (b == (uint32_t)v ? 1u : 2u);
-            if (place == 2u && d != (uint32_t)v) *err = 1;
-            const uint32_t o1 = place == 0u ? b : a, o2 = place == 2u ? b : d;
+            if (!ok[k]) t[k] = 0u;
+        }
+#pragma unroll
+        for (int k = 0; k < kAdjRound; k++) {
+            a[k] = idx[3 * t[k]];
+            b[k] = idx[3 * t[k] + 1];
+            d[k] = idx[3 * t[k] + 2];
+        }
+#pragma unroll
+        for (int k = 0; k < kAdjRound; k++) {
+            if (!ok[k]) continue;
+            const uint32_t place = a[k] == (uint32_t)v ? 0u : (b[k] == (uint32_t)v ? 1u : 2u);
+            if (place == 2u && d[k] != (uint32_t)v) *err = 1;
+            const uint32_t o1 = place == 0u ? b[k] : a[k], o2 = place == 2u ? b[k] : d[k];
             ring[(int64_t)n * stride + v] = make_uint2(o1 | (place << 30), o2);
             n++;
         }
     }
-    const bool moved = (bp || !boundary[v]) && n > 0;
+    if (n != count) *err = 1;
+    const bool moved = (bp || !bnd) && n > 0;
     deg[v] = (uint8_t)n;
     mv[v] = (uint8_t)moved;
     bscale[v] = moved ? 1.0f / (3.0f * (float)n) : 1.0f;
@@ -302,46 +374,59 @@ __global__ void __launch_bounds__(kStepThreads) k_bwd_step(const uint2* __restri
 // edges of its -x, -y, -z neighbours.  mu = -s0 / (s1 - s0), so
 // dmu/ds0 = -s1 / (s1 - s0)^2 and dmu/ds1 = s0 / (s1 - s0)^2; the vertex
 // moves along its edge axis by mu (grid units).
-__global__ void k_bwd_place(const float* __restrict__ dens, const uint32_t* __restrict__ vid0,
-                            const float4* __restrict__ g, int dim, float* __restrict__ out) {
-    const uint32_t udim = (uint32_t)dim;
-    const uint32_t n3 = udim * udim * udim;  // dim <= 256
+// Nearly every sample has no such edge: its six neighbours are compared
+// first.  Bound by VALU issue (129^3 samples: 13 us; with 32-bit divisions
+// and both edge loops at every sample 17).
+__global__ void __launch_bounds__(kThreads) k_bwd_place(const float* __restrict__ dens,
+                                                        const uint32_t* __restrict__ vid0,
+                                                        const float4* __restrict__ g, int dim,
+                                                        float* __restrict__ out) {
+    const uint32_t d1 = (uint32_t)dim, d2 = d1 * d1, n3 = d2 * d1;  // dim <= 256
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n3) return;
-    const uint32_t row = i / udim;
-    const int z = (int)(i - row * udim), y = (int)(row % udim), x = (int)(row / udim);
-    const int64_t st[3] = {(int64_t)dim * dim, (int64_t)dim, 1};
-    const int co[3] = {x, y, z};
+    const uint32_t x = udiv24(i, d2, 1.0f / (float)d2), r = i - x * d2;
+    const uint32_t y = udiv24(r, d1, 1.0f / (float)d1), z = r - y * d1;
+    const uint32_t st[3] = {d2, d1, 1u}, co[3] = {x, y, z};
     const float di = dens[i];
     const bool li = di < 0.0f;
-    float acc = 0.0f;
-    int k = 0;
-    for (int a = 0; a < 3; a++) {  // own edges: this sample is s0
-        if (co[a] + 1 >= dim) continue;
-        const float dj = dens[i + st[a]];
-        if ((dj < 0.0f) == li) continue;
-        const float4 q = g[vid0[i] + (uint32_t)k];
-        k++;
-        const float ds = dj - di;
-        const float ga = a == 0 ? q.x : (a == 1 ? q.y : q.z);
-        acc = acc + ga * (-dj / (ds * ds));
+    float up[3], dn[3];  // neighbours along each axis, the sample itself at a face
+#pragma unroll
+    for (int a = 0; a < 3; a++) {
+        up[a] = dens[co[a] + 1 < d1 ? i + st[a] : i];
+        dn[a] = dens[co[a] > 0 ? i - st[a] : i];
     }
-    for (int a = 0; a < 3; a++) {  // edges of the -a neighbour: this sample is s1
-        if (co[a] == 0) continue;
-        const int64_t j = i - st[a];
-        const float dj = dens[j];
-        const bool lj = dj < 0.0f;
-        if (lj == li) continue;
-        // rank of j's axis-a edge among j's sign-changing edges
-        uint32_t r = 0;
-        for (int b = 0; b < a; b++) {
-            const int cb = b == 0 ? x - (a == 0) : (b == 1 ? y - (a == 1) : z);
-            if (cb + 1 < dim && ((dens[j + st[b]] < 0.0f) != lj)) r++;
+    bool any = false;
+#pragma unroll
+    for (int a = 0; a < 3; a++) any = any || (up[a] < 0.0f) != li || (dn[a] < 0.0f) != li;
+    float acc = 0.0f;
+    if (any) {
+        uint32_t k = 0;
+#pragma unroll
+        for (int a = 0; a < 3; a++) {  // own edges: this sample is s0
+            const float dj = up[a];
+            if ((dj < 0.0f) == li) continue;
+            const float4 q = g[vid0[i] + k];
+            k++;
+            const float ds = dj - di;
+            const float ga = a == 0 ? q.x : (a == 1 ? q.y : q.z);
+            acc = acc + ga * (-dj / (ds * ds));
         }
-        const float4 q = g[vid0[j] + r];
-        const float ds = di - dj;
-        const float ga = a == 0 ? q.x : (a == 1 ? q.y : q.z);
-        acc = acc + ga * (dj / (ds * ds));
+#pragma unroll
+        for (int a = 0; a < 3; a++) {  // edges of the -a neighbour: this sample is s1
+            const float dj = dn[a];
+            const bool lj = dj < 0.0f;
+            if (lj == li) continue;
+            const uint32_t j = i - st[a];
+            // rank of j's axis-a edge among j's sign-changing edges
+            uint32_t rank = 0;
+#pragma unroll
+            for (int b = 0; b < a; b++)
+                if (co[b] + 1 < d1 && ((dens[j + st[b]] < 0.0f) != lj)) rank++;
+            const float4 q = g[vid0[j] + rank];
+            const float ds = di - dj;
+            const float ga = a == 0 ? q.x : (a == 1 ? q.y : q.z);
+            acc = acc + ga * (dj / (ds * ds));
+        }
     }
     out[i] = acc;
 }
@@ -421,71 +506,99 @@ __global__ void k_nn_keys(const float* __restrict__ t, int64_t n, const int* __r
     vals[i] = (int32_t)i;
 }
 
-__global__ void k_nn_gather(const float* __restrict__ t, const int32_t* __restrict__ perm, int64_t n,
-                            float4* __restrict__ st) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int32_t p = perm[i];
-    st[i] = make_float4(t[3 * (int64_t)p], t[3 * (int64_t)p + 1], t[3 * (int64_t)p + 2], __int_as_float(p));
+// fmin with the value DPP control CTRL brings from another lane (+inf where
+// the source lane is outside the row or the row is not in ROW_MASK).
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ float dpp_fmin(float v) {
+    const int o = __builtin_amdgcn_update_dpp(__float_as_int(INFINITY), __float_as_int(v), CTRL, ROW_MASK, 0xf, false);
+    return fminf(v, __int_as_float(o));
 }
 
-// Leaf boxes of the implicit hierarchy: heap-numbered nodes 1 .. 2P-1 over
-// P (a power of two) leaves; leaf l is node P + l and holds sorted targets
-// [kLeaf l, kLeaf (l+1)); leaves past the targets are empty boxes.
-__global__ void k_nn_leaves(const float4* __restrict__ st, int64_t n, int64_t P, float4* __restrict__ lo,
-                            float4* __restrict__ hi) {
-    const int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (l >= P) return;
-    float4 a = make_float4(INFINITY, INFINITY, INFINITY, 0.0f), b = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.0f);
-    const int64_t e = std::min<int64_t>(n, (l + 1) * kLeaf);
-    for (int64_t i = l * kLeaf; i < e; i++) {
-        const float4 q = st[i];
-        a.x = fminf(a.x, q.x);
-        a.y = fminf(a.y, q.y);
-        a.z = fminf(a.z, q.z);
-        b.x = fmaxf(b.x, q.x);
-        b.y = fmaxf(b.y, q.y);
-        b.z = fmaxf(b.z, q.z);
-    }
-    lo[P + l] = a;
-    hi[P + l] = b;
+// Minimum over the 64 lanes of a wave (all lanes active): prefix minima
+// within each row of 16 lanes (row_shr 1, 2, 4, 8), then row 0's last lane
+// into row 1 and row 2's into row 3 (row_bcast:15), then lane 31 into rows 2
+// and 3 (row_bcast:31); lane 63 then holds the minimum.
+__device__ __forceinline__ float wave_min(float x) {
+    x = dpp_fmin<0x111, 0xf>(x);
+    x = dpp_fmin<0x112, 0xf>(x);
+    x = dpp_fmin<0x114, 0xf>(x);
+    x = dpp_fmin<0x118, 0xf>(x);
+    x = dpp_fmin<0x142, 0xa>(x);
+    x = dpp_fmin<0x143, 0xc>(x);
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 63));
 }
 
-// Oriented bound of each leaf: the centre c of its targets, the principal
+// Sum over the 64 lanes of a wave (all lanes active), the same way.
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ float dpp_fadd(float v) {
+    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROW_MASK, 0xf, false));
+}
+__device__ __forceinline__ float wave_sum(float x) {
+    x = dpp_fadd<0x111, 0xf>(x);
+    x = dpp_fadd<0x112, 0xf>(x);
+    x = dpp_fadd<0x114, 0xf>(x);
+    x = dpp_fadd<0x118, 0xf>(x);
+    x = dpp_fadd<0x142, 0xa>(x);
+    x = dpp_fadd<0x143, 0xc>(x);
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 63));
+}
+
+// Leaves of the implicit hierarchy: heap-numbered nodes 1 .. 2P-1 over P (a
+// power of two) leaves; leaf l is node P + l and holds sorted targets
+// [kLeaf l, kLeaf (l+1)), the last one filled up with points at infinity; leaves
+// past the targets are empty boxes.  A wave per leaf, a lane per target, which it
+// also brings into sorted order as (x, y, z, id) (a lane per leaf walked its 64
+// targets four times: 47 us for 313 leaves with the gather, this takes 12).
+//
+// Box, and oriented bound: the centre c of the targets, the principal
 // axes of their covariance (cyclic Jacobi, then re-orthonormalised) and the
 // largest |(q - c) . axis| per axis; four float4 per leaf (c, then each axis
 // with its extent in w).  A patch of a curved target set is thin along its
 // normal, where the axis-aligned box of a tilted patch is not.  Empty leaves
 // get a zero record (their axis-aligned box already excludes them).
-__global__ void k_nn_obb(const float4* __restrict__ st, int64_t n, int64_t P, float4* __restrict__ ob) {
-    const int64_t l = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (l >= P) return;
-    const int64_t b = l * kLeaf, e = std::min<int64_t>(n, (l + 1) * kLeaf);
+__global__ void __launch_bounds__(kThreads) k_nn_leaves(const float* __restrict__ t, const int32_t* __restrict__ perm,
+                                                        int64_t n, int64_t P, float4* __restrict__ st,
+                                                        float4* __restrict__ lo, float4* __restrict__ hi,
+                                                        float4* __restrict__ ob) {
+    const int64_t l = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6;
+    if (l >= P) return;  // uniform across the wave
+    const int lane = lane_id();
+    const int64_t b = l * kLeaf;
+    const bool has = b + lane < n;
     float4* o = ob + 4 * l;
-    if (b >= e) {
-        for (int k = 0; k < 4; k++) o[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (b >= n) {
+        if (lane < 4) o[lane] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (lane == 0) {
+            lo[P + l] = make_float4(INFINITY, INFINITY, INFINITY, 0.0f);
+            hi[P + l] = make_float4(-INFINITY, -INFINITY, -INFINITY, 0.0f);
+        }
         return;
     }
-    float cx = 0.0f, cy = 0.0f, cz = 0.0f;
-    for (int64_t i = b; i < e; i++) {
-        const float4 q = st[i];
-        cx += q.x;
-        cy += q.y;
-        cz += q.z;
+    float4 q = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (has) {
+        const int32_t id = perm[b + lane];
+        q = make_float4(t[3 * (int64_t)id], t[3 * (int64_t)id + 1], t[3 * (int64_t)id + 2], __int_as_float(id));
     }
-    const float inv = 1.0f / (float)(e - b);
-    cx *= inv;
-    cy *= inv;
-    cz *= inv;
-    float a[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-    for (int64_t i = b; i < e; i++) {
-        const float4 q = st[i];
-        const float d[3] = {q.x - cx, q.y - cy, q.z - cz};
+    st[b + lane] = has ? q : make_float4(INFINITY, INFINITY, INFINITY, __int_as_float(0x7FFFFFFF));
+    const float qa[3] = {q.x, q.y, q.z};
+    float bl[3], bh[3], c[3];
+    const float inv = 1.0f / (float)std::min<int64_t>(kLeaf, n - b);
 #pragma unroll
-        for (int r = 0; r < 3; r++)
-#pragma unroll
-            for (int c = 0; c < 3; c++) a[r][c] += d[r] * d[c];
+    for (int k = 0; k < 3; k++) {
+        bl[k] = wave_min(has ? qa[k] : INFINITY);
+        bh[k] = -wave_min(has ? -qa[k] : INFINITY);
+        c[k] = wave_sum(has ? qa[k] : 0.0f) * inv;
     }
+    if (lane == 0) {
+        lo[P + l] = make_float4(bl[0], bl[1], bl[2], 0.0f);
+        hi[P + l] = make_float4(bh[0], bh[1], bh[2], 0.0f);
+    }
+    const float dq[3] = {has ? q.x - c[0] : 0.0f, has ? q.y - c[1] : 0.0f, has ? q.z - c[2] : 0.0f};
+    float a[3][3];
+#pragma unroll
+    for (int r = 0; r < 3; r++)
+#pragma unroll
+        for (int k = r; k < 3; k++) a[r][k] = a[k][r] = wave_sum(dq[r] * dq[k]);
     float v[3][3] = {{1, 0, 0}, {0, 1, 0}, {0, 0, 1}};
     for (int sw = 0; sw < 8; sw++)
 #pragma unroll
@@ -524,16 +637,13 @@ __global__ void k_nn_obb(const float4* __restrict__ st, int64_t n, int64_t P, fl
     const float lw = sqrtf(w[0] * w[0] + w[1] * w[1] + w[2] * w[2]);
     for (int k = 0; k < 3; k++) w[k] /= lw;
     const float nn[3] = {u[1] * w[2] - u[2] * w[1], u[2] * w[0] - u[0] * w[2], u[0] * w[1] - u[1] * w[0]};
-    const float* ax[3] = {u, w, nn};
-    float ex[3] = {0.0f, 0.0f, 0.0f};
-    for (int64_t i = b; i < e; i++) {
-        const float4 q = st[i];
-        const float d[3] = {q.x - cx, q.y - cy, q.z - cz};
+    const float ax[3][3] = {{u[0], u[1], u[2]}, {w[0], w[1], w[2]}, {nn[0], nn[1], nn[2]}};
+    if (lane == 0) o[0] = make_float4(c[0], c[1], c[2], 0.0f);
 #pragma unroll
-        for (int k = 0; k < 3; k++) ex[k] = fmaxf(ex[k], fabsf(d[0] * ax[k][0] + d[1] * ax[k][1] + d[2] * ax[k][2]));
+    for (int k = 0; k < 3; k++) {
+        const float e = -wave_min(-fabsf(dq[0] * ax[k][0] + dq[1] * ax[k][1] + dq[2] * ax[k][2]));
+        if (lane == 0) o[1 + k] = make_float4(ax[k][0], ax[k][1], ax[k][2], e);
     }
-    o[0] = make_float4(cx, cy, cz, 0.0f);
-    for (int k = 0; k < 3; k++) o[1 + k] = make_float4(ax[k][0], ax[k][1], ax[k][2], ex[k]);
 }
 
 // Inner boxes of one wide level [level, 2 level).
@@ -562,11 +672,10 @@ __device__ __forceinline__ float dist2(float px, float py, float pz, float4 q) {
     return (dx * dx + dy * dy) + dz * dz;
 }
 
-// Squared distance from p to the box (0 inside, +inf for an empty box);
-// never above the distance to any point in the box in FP32 (every step
-// rounds monotonically).
+// Squared distance from p to the box [l, h] (0 inside, +inf for an empty box);
+// never above the distance of p to any point in it in FP32 (every step rounds
+// monotonically).
 __device__ __forceinline__ float box_lb2(float px, float py, float pz, float4 l, float4 h) {
-    if (!(l.x <= h.x)) return INFINITY;
     const float dx = fmaxf(fmaxf(l.x - px, px - h.x), 0.0f);
     const float dy = fmaxf(fmaxf(l.y - py, py - h.y), 0.0f);
     const float dz = fmaxf(fmaxf(l.z - pz, pz - h.z), 0.0f);
@@ -575,43 +684,20 @@ __device__ __forceinline__ float box_lb2(float px, float py, float pz, float4 l,
 
 // Squared-distance lower bound from p to the targets of a leaf from its
 // oriented record: per axis max(0, |(p - c) . axis| - extent - slack), summed
-// and scaled down.  The slack (1e-5 of |p - c|_1 + extent per axis, then
-// 1 - 1e-5 on the sum) is far above the FP32 errors of the projections, of
-// the axes' orthonormality and of the targets' own FP32 distances (each of
-// order 1e-7 relative), so the bound stays below the FP32 distance of every
-// target of the leaf.
-__device__ __forceinline__ float obb_lb2(float px, float py, float pz, const float4* __restrict__ o) {
-    const float4 c = o[0], u = o[1], w = o[2], nrm = o[3];
+// and scaled down.  The slack (1e-5 of |p - c|_1 and of the extent per axis,
+// then 1 - 1e-5 on the sum) is far above the FP32 errors of the projections, of
+// the axes' orthonormality and of the targets' own FP32 distances (each of order
+// 1e-7 relative), so the bound stays below the FP32 distance of p to every
+// target of the leaf.  e: the extents with their share of the slack added.
+__device__ __forceinline__ float obb_lb2(float px, float py, float pz, float4 c, float4 u, float4 w, float4 nrm,
+                                         const float (&e)[3]) {
     const float dx = px - c.x, dy = py - c.y, dz = pz - c.z;
-    const float l1 = (fabsf(dx) + fabsf(dy)) + fabsf(dz);
+    const float s = 1e-5f * ((fabsf(dx) + fabsf(dy)) + fabsf(dz));
     const float tu = fabsf((dx * u.x + dy * u.y) + dz * u.z), tw = fabsf((dx * w.x + dy * w.y) + dz * w.z),
                 tn = fabsf((dx * nrm.x + dy * nrm.y) + dz * nrm.z);
-    const float su = fmaxf(tu - u.w - 1e-5f * (l1 + u.w), 0.0f);
-    const float sw = fmaxf(tw - w.w - 1e-5f * (l1 + w.w), 0.0f);
-    const float sn = fmaxf(tn - nrm.w - 1e-5f * (l1 + nrm.w), 0.0f);
+    const float su = fmaxf((tu - e[0]) - s, 0.0f), sw = fmaxf((tw - e[1]) - s, 0.0f),
+                sn = fmaxf((tn - e[2]) - s, 0.0f);
     return ((su * su + sw * sw) + sn * sn) * (1.0f - 1e-5f);
-}
-
-// fmin with the value DPP control CTRL brings from another lane (+inf where
-// the source lane is outside the row or the row is not in ROW_MASK).
-template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ float dpp_fmin(float v) {
-    const int o = __builtin_amdgcn_update_dpp(__float_as_int(INFINITY), __float_as_int(v), CTRL, ROW_MASK, 0xf, false);
-    return fminf(v, __int_as_float(o));
-}
-
-// Minimum over the 64 lanes of a wave (all lanes active): prefix minima
-// within each row of 16 lanes (row_shr 1, 2, 4, 8), then row 0's last lane
-// into row 1 and row 2's into row 3 (row_bcast:15), then lane 31 into rows 2
-// and 3 (row_bcast:31); lane 63 then holds the minimum.
-__device__ __forceinline__ float wave_min(float x) {
-    x = dpp_fmin<0x111, 0xf>(x);
-    x = dpp_fmin<0x112, 0xf>(x);
-    x = dpp_fmin<0x114, 0xf>(x);
-    x = dpp_fmin<0x118, 0xf>(x);
-    x = dpp_fmin<0x142, 0xa>(x);
-    x = dpp_fmin<0x143, 0xc>(x);
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), 63));
 }
 
 // A wave-uniform 64-bit value held in every lane, moved to scalar registers.
@@ -628,129 +714,192 @@ __device__ __forceinline__ int wave_argmin(float x, uint64_t m, int lane) {
     return __ffsll((unsigned long long)(__ballot(y == mn) & m)) - 1;
 }
 
-// Nearest target of each vertex, one wave per vertex.  The hierarchy (heap
-// nodes 1 .. 2P-1, leaves at depth D = log2 P) is walked in frames: frame 0
-// holds the root, and each later frame holds the 2^f descendants, f <=
-// kNNFan levels down, of a node popped from the frame above (the first step
-// takes D mod kNNFan levels so that the leaf frames are full).  Lane j
-// tests descendant j; the frame keeps the set whose box is no farther than
-// the best target distance U found so far, and pops its nearest box first.
-// A frame of leaves is evaluated min(kLeaf, 64) lanes per leaf (each lane
-// taking kLeaf / 64 targets of a larger leaf), 64 / kLeaf leaves per step
-// when leaves are smaller than a wave, re-pruned against U between steps; the very first leaf frame starts
-// with its nearest leaf alone so that U is finite early.  Pruning drops a
-// box only when it is strictly farther than U, an actual target distance,
-// so every target at the minimum distance is evaluated and the result is
-// the lowest (distance, original index), as a brute-force scan gives.
-__global__ void __launch_bounds__(kNNThreads) k_nn_query(const float* __restrict__ pos, int V,
-                                                         const float4* __restrict__ st, int64_t n, int64_t P,
-                                                         const float4* __restrict__ lo, const float4* __restrict__ hi,
-                                                         const float4* __restrict__ ob,
-                                                         int32_t* __restrict__ nearest, float* __restrict__ dldp,
-                                                         double* __restrict__ d2) {
-    const int v = (int)(((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-    if (v >= V) return;  // uniform across the wave
-    const int lane = (int)(threadIdx.x & 63);
+// Value x from the lane XOR 1, 2 or (within 8 or 16 lanes, lane i <-> 7 - i, 15 - i) mirrored.
+template <int CTRL>
+__device__ __forceinline__ int dpp_lane(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
+}
+constexpr int kXor1 = 0xB1, kXor2 = 0x4E, kMirror8 = 0x141, kMirror16 = 0x140;
+
+// Nearest target of each vertex, one wave per packet of kPacket vertices that
+// are consecutive in the tape's order, so near each other.  The hierarchy
+// (heap nodes 1 .. 2P-1, leaves at depth D = log2 P) is walked once for the
+// packet, in frames of the 2^f descendants, f <= kNNFan levels down, of the
+// node popped from the frame above (the first, of the root, takes D mod kNNFan
+// levels or kNNFan so that the leaf frames are full).  Lane j holds descendant
+// j and bounds its distance from each vertex in turn (leaves also by their
+// oriented bound); it is live while some vertex's bound is no farther than that
+// vertex's best target distance U so far.  Frames pop their nearest live box
+// first.  Leaves are evaluated in pairs (one load latency and one set of
+// minima), by kPart lanes per vertex, kEach of a leaf's targets each, and the
+// frame re-pruned.  Pruning drops a box only when it is strictly farther than U
+// from every vertex, and each U is an actual target distance, so every target
+// at a vertex's minimum distance is evaluated and the result is the lowest
+// (distance, original index), as a brute-force scan gives.
+//
+// Bound by VALU issue, and with few packets by the longest walk.  A wave per
+// vertex (7 frames and 17 leaves each, a wave-wide minimum after every leaf) took
+// 168 us for 44,392 vertices and 200,000 targets, 33 us for 7,819 and 20,000;
+// packets share boxes, leaves and minima: 80 and 47 us with four
+// vertices, 92 and 86 with eight (the walks are longer and fewer).  The small
+// case pays less than its hierarchy's leaves gain.  One bound for the whole
+// packet instead of one per vertex is cheaper a box and loses all of it:
+// far from the targets, boxes differ by less than the packet's width (2,455 us).
+constexpr int kPart = 64 / kPacket;    // lanes per vertex
+constexpr int kEach = kLeaf / kPart;   // targets of a leaf per lane
+static_assert(kPart == 8 || kPart == 16, "the minima over a vertex's lanes");
+static_assert(kNNFan == 6, "a frame is a wave's lanes");
+__global__ void __launch_bounds__(64) k_nn_query(const float* __restrict__ pos, const int32_t* __restrict__ order,
+                                                 int V, const float4* __restrict__ st, int64_t n, int64_t P,
+                                                 const float4* __restrict__ lo, const float4* __restrict__ hi,
+                                                 const float4* __restrict__ ob, int32_t* __restrict__ nearest,
+                                                 float* __restrict__ dldp, double* __restrict__ d2) {
+    const int64_t first = (int64_t)blockIdx.x * kPacket;
+    const int lane = (int)threadIdx.x, slot = lane / kPart, part = lane % kPart;
+    const int mine = order[first + slot];  // -1: a packet's spare slot, which repeats its first vertex
+    const bool own = mine >= 0;
+    const int v = own ? mine : __builtin_amdgcn_readlane(mine, 0);
     const float px = pos[3 * (int64_t)v], py = pos[3 * (int64_t)v + 1], pz = pos[3 * (int64_t)v + 2];
+    // no box is near enough for a spare slot, nor for a vertex that is not a
+    // number (it has no distance)
+    const bool counts = own && px == px && py == py && pz == pz;
+    auto slot_value = [](float x, int s) {
+        return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), kPart * s));
+    };
+    float vx[kPacket], vy[kPacket], vz[kPacket], U[kPacket];  // scalar registers
+#pragma unroll
+    for (int s = 0; s < kPacket; s++) {
+        vx[s] = slot_value(px, s);
+        vy[s] = slot_value(py, s);
+        vz[s] = slot_value(pz, s);
+        U[s] = slot_value(counts ? INFINITY : -INFINITY, s);
+    }
     int D = 0;
     while ((int64_t)1 << D < P) D++;
     const int f0 = D == 0 ? 0 : D - kNNFan * ((D - 1) / kNNFan);
-    float bd = INFINITY;  // this lane's best (distance, original index, sorted position)
+    float bd = INFINITY;  // this lane's best (distance, original index, sorted position) for its vertex
     int bi = 0x7FFFFFFF;
     int bs = -1;  // sorted position (n < 2^31, heap indices < 2^30)
-    float U = INFINITY;  // best distance over the wave
-    // the frames of this wave: per-lane box distances, the live set, heap index of descendant 0
-    __shared__ float s_lb[kNNThreads / 64][kNNFrames][64];
-    __shared__ unsigned long long s_mk[kNNThreads / 64][kNNFrames];
-    __shared__ int s_base[kNNThreads / 64][kNNFrames];
-    const int w = (int)(threadIdx.x >> 6);
-    s_lb[w][0][lane] = lane == 0 ? box_lb2(px, py, pz, lo[1], hi[1]) : INFINITY;
-    s_mk[w][0] = 1;
-    s_base[w][0] = 1;
-    int depth = 1;
-    const int Pi = (int)P, ni = (int)n;
-    // a leaf's targets: kLane lanes each take kSub of them (lane, lane + kLane, ...)
-    constexpr int kLane = kLeaf < 64 ? kLeaf : 64, kSub = kLeaf / kLane;
-    auto eval = [&](int leaf) {
-        // this lane's targets of `leaf` (heap index), if any
+    // inner frames: per lane and vertex box distances, the live set, heap index of descendant 0
+    __shared__ float s_lb[kNNFrames][kPacket][64];
+    __shared__ unsigned long long s_mk[kNNFrames];
+    __shared__ int s_base[kNNFrames];
+    const int Pi = (int)P, leaves = (int)((n + kLeaf - 1) / kLeaf);
+    float lb[kPacket];
+    auto live = [&]() {
+        unsigned long long m = 0;
 #pragma unroll
-        for (int u = 0; u < kSub; u++) {
-            const int i = (leaf - Pi) * kLeaf + u * kLane + (lane & (kLane - 1));
-            if (i < ni) {
-                const float4 q = st[i];
-                const float d = dist2(px, py, pz, q);
-                const int id = __float_as_int(q.w);
-                if (d < bd || (d == bd && id < bi)) {
-                    bd = d;
-                    bi = id;
-                    bs = i;
-                }
-            }
-        }
+        for (int s = 0; s < kPacket; s++) m |= __ballot(lb[s] <= U[s]);
+        return m;
     };
-    while (depth > 0) {
-        const int k = depth - 1;
-        const int lk = k == 0 ? 0 : f0 + kNNFan * (k - 1);
-        const float lb = s_lb[w][k][lane];
-        // the frame's base and live set are the wave's (moved to scalar registers)
-        const int b0 = __builtin_amdgcn_readfirstlane(s_base[w][k]);
-        unsigned long long m = uniform_u64(s_mk[w][k]) & __ballot(lb <= U);
-        if (lk == D) {
-            if (U == INFINITY && m) {
-                const int j = wave_argmin(lb, m, lane);
-                if (lane < kLane) eval(b0 + j);
-                m &= ~(1ull << j);
-                U = wave_min(bd);
-                m &= __ballot(lb <= U);
-            }
+    auto nearest_of = [&](unsigned long long m) {
+        float x = lb[0];
+#pragma unroll
+        for (int s = 1; s < kPacket; s++) x = fminf(x, lb[s]);
+        return wave_argmin(x, m, lane);
+    };
+    auto lower = [](float& a, int& ai, int& as, float b, int bj, int bt) {
+        const bool t = (b < a) | ((b == a) & (bj < ai));
+        a = t ? b : a;
+        ai = t ? bj : ai;
+        as = t ? bt : as;
+    };
+    // The targets of two leaves (heap indices; twice the same where one is
+    // left), then every vertex's U: this lane's targets, the nearest by a tree
+    // of selects, the minimum over the vertex's lanes.
+    auto eval = [&](int leaf, int also) {
+        const uint32_t i0 = (uint32_t)(leaf - Pi) * kLeaf + (uint32_t)part;
+        const uint32_t i1 = (uint32_t)(also - Pi) * kLeaf + (uint32_t)part;
+        float4 q[2 * kEach];
+        float e[2 * kEach];
+        int ei[2 * kEach], es[2 * kEach];
+#pragma unroll
+        for (int u = 0; u < 2 * kEach; u++) {
+            es[u] = (int)((u & 1 ? i1 : i0) + kPart * (u >> 1));
+            q[u] = st[es[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < 2 * kEach; u++) {
+            const float x = dist2(px, py, pz, q[u]);
+            e[u] = x == x ? x : INFINITY;  // at a point that is not a number: as one past the targets
+            ei[u] = x == x ? __float_as_int(q[u].w) : 0x7FFFFFFF;
+        }
+#pragma unroll
+        for (int w = kEach; w; w >>= 1)
+#pragma unroll
+            for (int u = 0; u < w; u++) lower(e[u], ei[u], es[u], e[u + w], ei[u + w], es[u + w]);
+        lower(bd, bi, bs, e[0], ei[0], es[0]);
+        float m = bd;
+        m = fminf(m, __int_as_float(dpp_lane<kXor1>(__float_as_int(m))));
+        m = fminf(m, __int_as_float(dpp_lane<kXor2>(__float_as_int(m))));
+        m = fminf(m, __int_as_float(dpp_lane<kMirror8>(__float_as_int(m))));
+        if (kPart == 16) m = fminf(m, __int_as_float(dpp_lane<kMirror16>(__float_as_int(m))));
+        m = counts ? m : -INFINITY;
+#pragma unroll
+        for (int s = 0; s < kPacket; s++) U[s] = slot_value(m, s);
+    };
+    int k = 0, f = f0, base = 1 << f0;
+    while (k >= 0) {
+        const int level = f0 + kNNFan * k;
+        // a frame of leaves ends with the last that holds targets
+        const int width = level == D ? min(1 << f, Pi + leaves - base) : 1 << f;
+        const unsigned long long all = width < 64 ? (1ull << max(width, 0)) - 1ull : ~0ull;
+        const int node = lane < (1 << f) ? base + lane : base;
+        const float4 l = lo[node], h = hi[node];
+#pragma unroll
+        for (int s = 0; s < kPacket; s++) lb[s] = box_lb2(vx[s], vy[s], vz[s], l, h);
+        if (level == D) {
+            const float4* o = ob + 4 * (int64_t)(node - Pi);
+            const float4 c = o[0], u = o[1], w = o[2], nrm = o[3];
+            const float e[3] = {u.w * (1.0f + 2e-5f), w.w * (1.0f + 2e-5f), nrm.w * (1.0f + 2e-5f)};
+#pragma unroll
+            for (int s = 0; s < kPacket; s++)
+                if (__ballot(lb[s] <= U[s]))
+                    lb[s] = fmaxf(lb[s], obb_lb2(vx[s], vy[s], vz[s], c, u, w, nrm, e));
+            unsigned long long m = all & live();
             while (m) {
-                // lane group g (kLane lanes) takes the g-th lowest live leaf:
-                // the positions come off the wave-uniform mask on the scalar
-                // unit, each group selects its own
-                int j = -1;
-#pragma unroll
-                for (int t = 0; t < 64 / kLane; t++) {
-                    const int pos = m ? __ffsll((unsigned long long)m) - 1 : -1;
-                    j = lane / kLane == t ? pos : j;
-                    m &= m - 1;
-                }
-                if (j >= 0) eval(b0 + j);
-                U = wave_min(bd);
-                m &= __ballot(lb <= U);
+                // the nearest, with its sibling or else any other live one
+                const int j = nearest_of(m);
+                m &= ~(1ull << j);
+                const int h = m >> (j ^ 1) & 1 || !m ? j ^ 1 : __ffsll(m) - 1, i = m ? h : j;
+                eval(base + j, base + i);
+                m = m & ~(1ull << i) & live();
             }
-            depth--;
-            continue;
-        }
-        if (!m) {
-            depth--;
-            continue;
-        }
-        const int j = wave_argmin(lb, m, lane);
-        s_mk[w][k] = m & ~(1ull << j);
-        const int f = k == 0 ? f0 : kNNFan;
-        const int c0 = (b0 + j) << f;
-        float lc = lane < (1 << f) ? box_lb2(px, py, pz, lo[c0 + lane], hi[c0 + lane]) : INFINITY;
-        // a frame of leaves also takes each leaf's oriented bound
-        if (f0 + kNNFan * k == D && lane < (1 << f) && lc < INFINITY)
-            lc = fmaxf(lc, obb_lb2(px, py, pz, ob + 4 * (int64_t)(c0 + lane - Pi)));
-        s_lb[w][k + 1][lane] = lc;
-        s_mk[w][k + 1] = __ballot(lane < (1 << f) && lc <= U);
-        s_base[w][k + 1] = c0;
-        depth++;
-    }
-    // the wave's lowest (distance, index)
+            k--;
+        } else {
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        const float od = __shfl_xor(bd, off);
-        const int oi = __shfl_xor(bi, off);
-        const int os = __shfl_xor(bs, off);
+            for (int s = 0; s < kPacket; s++) s_lb[k][s][lane] = lb[s];
+            s_mk[k] = all;
+            s_base[k] = base;
+        }
+        // the next node: the nearest live one of the lowest frame that has any
+        for (; k >= 0; k--) {
+#pragma unroll
+            for (int s = 0; s < kPacket; s++) lb[s] = s_lb[k][s][lane];
+            const unsigned long long m = uniform_u64(s_mk[k]) & live();
+            if (!m) continue;
+            const int j = nearest_of(m);
+            s_mk[k] = m & ~(1ull << j);
+            base = (__builtin_amdgcn_readfirstlane(s_base[k]) + j) << kNNFan;
+            f = kNNFan;
+            k++;
+            break;
+        }
+    }
+    // each vertex's lowest (distance, index) over its 8 lanes
+    auto take = [&](float od, int oi, int os) {
         if (od < bd || (od == bd && oi < bi)) {
             bd = od;
             bi = oi;
             bs = os;
         }
-    }
-    if (lane != 0) return;
+    };
+    take(__int_as_float(dpp_lane<kXor1>(__float_as_int(bd))), dpp_lane<kXor1>(bi), dpp_lane<kXor1>(bs));
+    take(__int_as_float(dpp_lane<kXor2>(__float_as_int(bd))), dpp_lane<kXor2>(bi), dpp_lane<kXor2>(bs));
+    take(__int_as_float(dpp_lane<kMirror8>(__float_as_int(bd))), dpp_lane<kMirror8>(bi), dpp_lane<kMirror8>(bs));
+    if (kPart == 16)
+        take(__int_as_float(dpp_lane<kMirror16>(__float_as_int(bd))), dpp_lane<kMirror16>(bi), dpp_lane<kMirror16>(bs));
+    if (part != 0 || !own) return;
     const float4 q = bs >= 0 ? st[bs] : make_float4(px, py, pz, 0.0f);
     nearest[v] = bs >= 0 ? bi : -1;
     const float sc = 2.0f / (float)V;
@@ -797,6 +946,12 @@ struct bmf_tape {
     int32_t dim = 0, K = 0, bp = 0, V = 0, T = 0, contains_mesh = 0;
     float* dens = nullptr;
     uint32_t* vid0 = nullptr;
+    // vertices by lattice cell, for the packets of the nearest-target query
+    int32_t* order = nullptr;
+    uint32_t* rank = nullptr;     // of each vertex within its cell
+    uint32_t* cell_n = nullptr;   // [kOrderCells] vertices of each cell (0 between forwards)
+    uint32_t* cell_base = nullptr;  // [kOrderCells] first place of each cell
+    int places = 0;                 // of `order` in use, a multiple of kPacket
     uint32_t* vedge = nullptr;
     uint8_t* boundary = nullptr;
     uint32_t* idx = nullptr;
@@ -810,7 +965,7 @@ struct bmf_tape {
     float4* g = nullptr;
     float4* g2 = nullptr;   // ping-pong partner of g in the backward
     float4* r4 = nullptr;   // ping-pong partner of q4 in bmf_tape_positions
-    int* err = nullptr;
+    int* err = nullptr;           // [2]: the adjacency's check, places of `order` taken
     hipEvent_t ev[6] = {};  // start / end of the last forward, loss and backward
     bool timed[3] = {false, false, false};
     float4* ckpt = nullptr;
@@ -866,7 +1021,7 @@ int reserve_nn(bmf_tape* t, int64_t n) {
     bool ok = true;
     for (int i = 0; i < 2; i++)
         ok = ok && dalloc(&t->keys[i], n) == hipSuccess && dalloc(&t->vals[i], n) == hipSuccess;
-    ok = ok && dalloc(&t->st, n) == hipSuccess && dalloc(&t->blo, 2 * P) == hipSuccess &&
+    ok = ok && dalloc(&t->st, (n + kLeaf - 1) / kLeaf * kLeaf) == hipSuccess && dalloc(&t->blo, 2 * P) == hipSuccess &&
          dalloc(&t->bhi, 2 * P) == hipSuccess && dalloc(&t->obb, 4 * P) == hipSuccess;
     if (ok) {
         hipcub::DoubleBuffer<uint32_t> kb(t->keys[0], t->keys[1]);
@@ -917,9 +1072,8 @@ int nn_build(const float* targets, int64_t n, int* bb, const NNBuffers& b, hipSt
     hipcub::DoubleBuffer<int32_t> vb(b.vals[0], b.vals[1]);
     size_t bytes = b.cub_bytes;
     BMF_HIP(hipcub::DeviceRadixSort::SortPairs(b.cub_tmp, bytes, kb, vb, (int)n, 0, 30, s));
-    hipLaunchKernelGGL(k_nn_gather, dim3(blocks_for(n)), dim3(kThreads), 0, s, targets, vb.Current(), n, b.st);
-    hipLaunchKernelGGL(k_nn_leaves, dim3(blocks_for(P)), dim3(kThreads), 0, s, b.st, n, P, b.blo, b.bhi);
-    hipLaunchKernelGGL(k_nn_obb, dim3(blocks_for(P)), dim3(kThreads), 0, s, b.st, n, P, b.ob);
+    hipLaunchKernelGGL(k_nn_leaves, dim3(blocks_for(64 * P)), dim3(kThreads), 0, s, targets, vb.Current(), n, P, b.st,
+                       b.blo, b.bhi, b.ob);
     int64_t level = P >> 1;
     for (; level >= 2048; level >>= 1)
         hipLaunchKernelGGL(k_nn_level, dim3(blocks_for(level)), dim3(kThreads), 0, s, level, b.blo, b.bhi);
@@ -934,8 +1088,7 @@ int nn_build(const float* targets, int64_t n, int* bb, const NNBuffers& b, hipSt
 int nn_query(bmf_tape* t, const NNBuffers& b, int64_t n, float* dldp, int32_t* nearest, double* loss_out,
              hipStream_t s) {
     const int64_t P = leaf_pow2(n);
-    hipLaunchKernelGGL(k_nn_query, dim3((unsigned)(((int64_t)t->V * 64 + kNNThreads - 1) / kNNThreads)),
-                       dim3(kNNThreads), 0, s, t->pos, t->V, b.st, n, P, b.blo, b.bhi, b.ob,
+    hipLaunchKernelGGL(k_nn_query, dim3((unsigned)(t->places / kPacket)), dim3(64), 0, s, t->pos, t->order, t->V, b.st, n, P, b.blo, b.bhi, b.ob,
                        nearest ? nearest : t->nearest_tmp, dldp, t->d2);
     hipLaunchKernelGGL(k_sum, dim3(1), dim3(1024), 0, s, t->d2, t->V, loss_out);
     BMF_HIP(hipGetLastError());
@@ -1057,6 +1210,11 @@ int bmf_tape_create(bmf_tape** out, bmf_ctx* ctx, int32_t max_dim, int64_t max_v
     t->ckpt_every = checkpoint_every;
     const int64_t n3 = (int64_t)max_dim * max_dim * max_dim;
     const bool ok = dalloc(&t->dens, n3) == hipSuccess && dalloc(&t->vid0, n3) == hipSuccess &&
+                    dalloc(&t->order, max_vertices + (kPacket - 1) * std::min<int64_t>(max_vertices, kOrderCells)) ==
+                        hipSuccess && dalloc(&t->rank, max_vertices) == hipSuccess &&
+                    dalloc(&t->cell_n, kOrderCells) == hipSuccess &&
+                    dalloc(&t->cell_base, kOrderCells) == hipSuccess &&
+                    hipMemsetAsync(t->cell_n, 0, sizeof(uint32_t) * kOrderCells, ctx->stream) == hipSuccess &&
                     dalloc(&t->vedge, max_vertices) == hipSuccess && dalloc(&t->boundary, max_vertices) == hipSuccess &&
                     dalloc(&t->idx, max_indices) == hipSuccess &&
                     dalloc(&t->ring, (int64_t)kMaxRing * max_vertices) == hipSuccess &&
@@ -1065,7 +1223,7 @@ int bmf_tape_create(bmf_tape** out, bmf_ctx* ctx, int32_t max_dim, int64_t max_v
                     dalloc(&t->p4, max_vertices) == hipSuccess && dalloc(&t->q4, max_vertices) == hipSuccess &&
                     dalloc(&t->pos, 3 * max_vertices) == hipSuccess &&
                     dalloc(&t->g, max_vertices) == hipSuccess && dalloc(&t->g2, max_vertices) == hipSuccess &&
-                    dalloc(&t->r4, max_vertices) == hipSuccess && dalloc(&t->err, 1) == hipSuccess &&
+                    dalloc(&t->r4, max_vertices) == hipSuccess && dalloc(&t->err, 2) == hipSuccess &&
                     dalloc(&t->bb, 8) == hipSuccess && dalloc(&t->d2, max_vertices) == hipSuccess &&
                     dalloc(&t->loss, 1) == hipSuccess && dalloc(&t->nearest_tmp, max_vertices) == hipSuccess;
     bool evs = ok;
@@ -1087,6 +1245,10 @@ void bmf_tape_destroy(bmf_tape* t) {
     (void)hipStreamSynchronize(t->ctx->stream);
     dfree(t->dens);
     dfree(t->vid0);
+    dfree(t->order);
+    dfree(t->rank);
+    dfree(t->cell_n);
+    dfree(t->cell_base);
     dfree(t->vedge);
     dfree(t->boundary);
     dfree(t->idx);
@@ -1186,7 +1348,6 @@ int bmf_forward_diff(bmf_ctx* c, const bmf_chunk_desc* d, const float* densities
         t->ckpt_slots = slots;
     }
     const int V = t->V, T = t->T;
-    BMF_HIP(hipMemsetAsync(t->err, 0, sizeof(int), s));
     const bool smooth = t->K > 0 && T > 0;  // per-cell triangle bases and masks exist for chunks with K > 0
     {
         const int64_t most = std::max<int64_t>(n3, std::max<int64_t>(3 * (int64_t)T, V));
@@ -1194,10 +1355,15 @@ int bmf_forward_diff(bmf_ctx* c, const bmf_chunk_desc* d, const float* densities
         hipLaunchKernelGGL(k_tape_take, dim3(blocks), dim3(kThreads), 0, s, A.dens, A.vedge + r.vertex_offset,
                            A.boundary + r.vertex_offset, A.idx + r.index_offset, A.pos + 3 * r.vertex_offset, n3, V,
                            3 * (int64_t)T, dim, t->dens, t->vedge, t->boundary, t->idx, t->p4, t->ckpt,
-                           smooth ? nullptr : t->pos, t->vid0);
+                           smooth ? nullptr : t->pos, t->vid0, t->cell_n, t->rank, t->err);
         BMF_HIP(hipGetLastError());
     }
     if (V > 0) {
+        hipLaunchKernelGGL(k_order_cells, dim3(blocks_for(kOrderCells)), dim3(kThreads), 0, s, t->cell_n, t->cell_base,
+                           t->err + 1, t->order);
+        hipLaunchKernelGGL(k_order, dim3(blocks_for(V)), dim3(kThreads), 0, s, t->vedge, V, dim, t->cell_base, t->rank,
+                           t->order);
+        BMF_HIP(hipGetLastError());
         if (smooth) {
             hipLaunchKernelGGL(k_tape_adj, dim3(step_blocks(V)), dim3(kStepThreads), 0, s, t->vedge, t->boundary,
                                A.cell_tb, A.cell_mask, t->idx, dim, V, T, t->bp, (int)t->cap_v, t->ring, t->deg, t->mv,
@@ -1213,10 +1379,11 @@ int bmf_forward_diff(bmf_ctx* c, const bmf_chunk_desc* d, const float* densities
         }
     }
     BMF_HIP(hipEventRecord(t->ev[1], s));
-    int herr = 0;
-    BMF_HIP(hipMemcpyAsync(&herr, t->err, sizeof(int), hipMemcpyDeviceToHost, s));
+    int herr[2] = {0, 0};
+    BMF_HIP(hipMemcpyAsync(herr, t->err, sizeof herr, hipMemcpyDeviceToHost, s));
     BMF_HIP(hipStreamSynchronize(s));
-    if (V > 0 && herr) return BMF_EHIP;
+    if (V > 0 && herr[0]) return BMF_EHIP;
+    t->places = herr[1];
     t->valid = true;
     t->timed[0] = true;
     return BMF_OK;
