@@ -55,12 +55,13 @@ void free_arenas(bmf_ctx* c) {
 int scan_blocks(const bmf_ctx* c, int n) { return std::min(n, 2 * c->cu_count); }
 
 int enqueue_pipeline(bmf_ctx* c, const Arenas& A, int n, int maxk, int allow_cull, int reset, int sample_blocks,
-                     int row_blocks, int scan_blocks, int smooth_blocks, hipEvent_t* ev = nullptr) {
+                     int row_blocks, int scan_blocks, int smooth_blocks, hipEvent_t* ev = nullptr,
+                     const bmf_chunk_desc* one = nullptr) {
     hipStream_t s = c->stream;
 #define BMF_MARK(i) \
     if (ev) BMF_HIP(hipEventRecord(ev[i], s))
     BMF_MARK(0);
-    BMF_HIP(launch_plan(A, n, allow_cull, reset, s));
+    BMF_HIP(launch_plan(A, n, allow_cull, reset, s, one));
     BMF_MARK(1);
     BMF_HIP(launch_sample(A, n, sample_blocks, 1, c->h_sampler.kind, c->h_sampler.noise_dims == 2, s));
     c->stat_nsample = sample_blocks;
@@ -318,8 +319,8 @@ int bmf_create(bmf_ctx** out, int device, const bmf_limits* lim) {
          dalloc(&A.sampler, 1) == hipSuccess;
     ok = ok && hipHostMalloc((void**)&c->h_descs[0], sizeof(bmf_chunk_desc) * nc) == hipSuccess &&
          hipHostMalloc((void**)&c->h_descs[1], sizeof(bmf_chunk_desc) * nc) == hipSuccess &&
-         hipHostMalloc((void**)&c->h_results, sizeof(bmf_chunk_result) * nc) == hipSuccess &&
-         hipHostMalloc((void**)&c->h_ctr, sizeof(Counters)) == hipSuccess;
+         host_alloc(&c->h_results, nc, &A.host_results) == hipSuccess &&
+         host_alloc(&c->h_ctr, 1, &A.host_ctr) == hipSuccess;
     ok = ok && hipEventCreate(&c->ev0) == hipSuccess && hipEventCreate(&c->ev1) == hipSuccess &&
          hipEventCreate(&c->ev_upload[0]) == hipSuccess && hipEventCreate(&c->ev_upload[1]) == hipSuccess;
     for (int i = 0; ok && i <= BMF_NUM_STAGES; i++) ok = hipEventCreate(&c->ev_stage[i]) == hipSuccess;
@@ -351,7 +352,6 @@ void bmf_destroy(bmf_ctx* c) {
     if (c->h_fmt) (void)hipHostFree(c->h_fmt);
     if (c->d_lod_first) (void)hipFree(c->d_lod_first);
     if (c->d_lod_code) (void)hipFree(c->d_lod_code);
-    if (c->d_lod_counts) (void)hipFree(c->d_lod_counts);
     if (c->h_lod_counts) (void)hipHostFree(c->h_lod_counts);
     if (c->d_stitch_counts) (void)hipFree(c->d_stitch_counts);
     if (c->d_stitch_tiles) (void)hipFree(c->d_stitch_tiles);
@@ -513,7 +513,9 @@ static int extract_impl(bmf_ctx* c, const bmf_chunk_desc* chunks, int n, int mod
     c->stats_batch = mode == BMF_MODE_BATCHED;  // PLAIN frames run one pipeline per chunk
     if (n == 0) return BMF_OK;
     int rc = BMF_OK;
-    if (chunks) {
+    if (chunks && mode == BMF_MODE_PLAIN) {
+        c->queued_n = -1;  // as after an upload
+    } else if (chunks) {
         rc = upload_descs(c, chunks, n);
         if (rc) return rc;
     }
@@ -524,7 +526,7 @@ static int extract_impl(bmf_ctx* c, const bmf_chunk_desc* chunks, int n, int mod
     if (mode == BMF_MODE_PLAIN) {
         // one launch sequence per chunk; scratch arenas reused from offset 0,
         // output arenas bump-allocated across the chunks (ChunkGenerator.cpp:91
-        // loop body, one chunk at a time)
+        // loop body, one chunk at a time; a host descriptor goes with its launch)
         BMF_HIP(hipEventRecord(c->ev0, c->stream));
         int64_t ext_base = 0;
         for (int j = 0; j < n; j++) {
@@ -535,11 +537,12 @@ static int extract_impl(bmf_ctx* c, const bmf_chunk_desc* chunks, int n, int mod
             Aj.descs = A.descs + j;
             Aj.meta = A.meta + j;
             Aj.results = A.results + j;
+            Aj.host_results = A.host_results + j;
             const int64_t dim = dj.dim;
             const int64_t ns = dim * dim * dim;
             const int sb = sample_blocks_of(ns);
             rc = enqueue_pipeline(c, Aj, 1, max_steps(c, &dj, 1), 1, j == 0, sb, word_blocks(dj.dim), 1,
-                                  std::min(pb, 1024));
+                                  std::min(pb, 1024), nullptr, chunks ? &dj : nullptr);
             if (rc) return rc;
         }
         BMF_HIP(hipEventRecord(c->ev1, c->stream));
@@ -608,10 +611,9 @@ static int fetch_results(bmf_ctx* c) {
     if (c->results_valid) return BMF_OK;
     if (!c->have_extract) return BMF_ESTATE;
     const int n = c->last_n;
-    if (n > 0)
-        BMF_HIP(hipMemcpyAsync(c->h_results, c->A.results, sizeof(bmf_chunk_result) * n, hipMemcpyDeviceToHost,
-                               c->stream));
-    BMF_HIP(hipMemcpyAsync(c->h_ctr, c->A.ctr, sizeof(Counters), hipMemcpyDeviceToHost, c->stream));
+    // the kernels wrote both; of an empty batch only the device's counters tell
+    if (n == 0)
+        BMF_HIP(hipMemcpyAsync(c->h_ctr, c->A.ctr, sizeof(Counters), hipMemcpyDeviceToHost, c->stream));
     BMF_HIP(hipStreamSynchronize(c->stream));
     c->results_valid = true;
     return BMF_OK;

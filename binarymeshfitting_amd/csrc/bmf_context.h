@@ -28,8 +28,8 @@ struct bmf_ctx {
     hipEvent_t ev_upload[2] = {nullptr, nullptr};
     int upload_slot = 0;
     hipEvent_t ev_stage[BMF_NUM_STAGES + 1] = {};
-    bmf_chunk_result* h_results = nullptr;  // pinned
-    bmf::Counters* h_ctr = nullptr;         // pinned
+    bmf_chunk_result* h_results = nullptr;  // pinned, written by the kernels (Arenas::host_results)
+    bmf::Counters* h_ctr = nullptr;         // the same (Arenas::host_ctr)
     bmf::SamplerDev h_sampler{};
     float* d_spheres = nullptr;
     float* d_boxes = nullptr;
@@ -45,25 +45,36 @@ struct bmf_ctx {
     bmf_tuning tune{};             // BATCHED launch shapes (bmf_set_tuning / bmf_autotune)
     bmf_mesh_options mesh{0, 0, 0.1f, 0, 0};  // bmf_set_mesh_options
     int64_t* d_fmt = nullptr;  // bmf_format: per-chunk offsets and tile counts [4][max_chunks + 1]
-    int64_t* h_fmt = nullptr;  // pinned: formatted vertex and index totals
+    int64_t* h_fmt = nullptr;  // pinned, written by the kernel: formatted vertex and index totals
+    int64_t* m_fmt = nullptr;  // its device address
     // bmf_lod_queue: scratch, and the descriptors it left in the descriptor
     // arena for bmf_extract_queued (queued_n < 0: none)
     int* d_lod_first = nullptr;    // [lod_cap_nodes] lowest list position of a group candidate child
     uint8_t* d_lod_code = nullptr; // [lod_cap_list] pass-A code of each list position
     int lod_cap_nodes = 0, lod_cap_list = 0;
-    int* d_lod_counts = nullptr;   // dirty nodes, chunks
-    int* h_lod_counts = nullptr;   // pinned
+    int* h_lod_counts = nullptr;   // pinned, written by the kernel: dirty nodes, chunks
+    int* d_lod_counts = nullptr;   // its device address
     int queued_n = -1, queued_dim = 0, queued_iters = 0;
     // bmf_stitch scratch: triangles per candidate point, tile totals / offsets,
     // (root, deepest level) and the total
     uint8_t* d_stitch_counts = nullptr;
     int64_t* d_stitch_tiles = nullptr;
     int64_t* d_stitch_misc = nullptr;
-    int64_t* h_stitch_total = nullptr;  // pinned
+    int64_t* h_stitch_total = nullptr;  // pinned, written by the kernels: the pair, the total
+    int64_t* m_stitch_total = nullptr;  // its device address
     int64_t stitch_cap_cand = 0;
 };
 
 namespace bmf {
+
+// Pinned memory that kernels write for the host (coherent, so visible once
+// the stream is through), and its device address.
+template <class T>
+hipError_t host_alloc(T** host, int64_t count, T** dev) {
+    hipError_t e = hipHostMalloc((void**)host, sizeof(T) * (size_t)count, hipHostMallocMapped | hipHostMallocCoherent);
+    if (e != hipSuccess) return e;
+    return hipHostGetDevicePointer((void**)dev, *host, 0);
+}
 
 // Smoothing launches of a batch: the largest K, at least 1 with normals.
 int max_steps(const bmf_ctx* c, const bmf_chunk_desc* chunks, int n);

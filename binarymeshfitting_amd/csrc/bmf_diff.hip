@@ -112,8 +112,10 @@ __global__ void __launch_bounds__(kThreads) k_order_cells(uint32_t* __restrict__
 }
 __global__ void __launch_bounds__(kThreads) k_order(const uint32_t* __restrict__ vedge, int V, int dim,
                                                     const uint32_t* __restrict__ base,
-                                                    const uint32_t* __restrict__ rank, int32_t* __restrict__ order) {
+                                                    const uint32_t* __restrict__ rank, const int* __restrict__ taken,
+                                                    int* __restrict__ host_places, int32_t* __restrict__ order) {
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
+    if (v == 0) *host_places = *taken;
     if (v < V) order[base[order_cell(vedge[v], dim)] + rank[v]] = v;
 }
 
@@ -129,8 +131,8 @@ __global__ void k_tape_take(const float* __restrict__ dens_in, const uint32_t* _
                             float* __restrict__ dens, uint32_t* __restrict__ vedge, uint8_t* __restrict__ bnd,
                             uint32_t* __restrict__ idx, float4* __restrict__ p4, float4* __restrict__ ck0,
                             float* __restrict__ pos3, uint32_t* __restrict__ vid0, uint32_t* __restrict__ cell_n,
-                            uint32_t* __restrict__ rank, int* __restrict__ err) {
-    if (blockIdx.x == 0 && threadIdx.x < 2) err[threadIdx.x] = 0;
+                            uint32_t* __restrict__ rank, int* __restrict__ taken, int* __restrict__ err) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *taken = *err = 0;
     const int64_t total = std::max<int64_t>(n3, std::max<int64_t>(n_idx, V));
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
         if (i < n3) dens[i] = dens_in[i];
@@ -965,7 +967,15 @@ struct bmf_tape {
     float4* g = nullptr;
     float4* g2 = nullptr;   // ping-pong partner of g in the backward
     float4* r4 = nullptr;   // ping-pong partner of q4 in bmf_tape_positions
-    int* err = nullptr;           // [2]: the adjacency's check, places of `order` taken
+    int* taken = nullptr;         // places of `order` taken
+    struct Host {                 // what the host reads, written by the kernels
+        double loss;
+        int err;                  // the adjacency's check
+        int places;
+    };
+    Host* host = nullptr;         // pinned
+    Host* mhost = nullptr;        // its device address
+    SamplerDev* ext_sampler = nullptr;  // device: EXTERNAL, the densities named by each call (Arenas::ext)
     hipEvent_t ev[6] = {};  // start / end of the last forward, loss and backward
     bool timed[3] = {false, false, false};
     float4* ckpt = nullptr;
@@ -1223,12 +1233,15 @@ int bmf_tape_create(bmf_tape** out, bmf_ctx* ctx, int32_t max_dim, int64_t max_v
                     dalloc(&t->p4, max_vertices) == hipSuccess && dalloc(&t->q4, max_vertices) == hipSuccess &&
                     dalloc(&t->pos, 3 * max_vertices) == hipSuccess &&
                     dalloc(&t->g, max_vertices) == hipSuccess && dalloc(&t->g2, max_vertices) == hipSuccess &&
-                    dalloc(&t->r4, max_vertices) == hipSuccess && dalloc(&t->err, 2) == hipSuccess &&
+                    dalloc(&t->r4, max_vertices) == hipSuccess && dalloc(&t->taken, 1) == hipSuccess &&
+                    host_alloc(&t->host, 1, &t->mhost) == hipSuccess && dalloc(&t->ext_sampler, 1) == hipSuccess &&
                     dalloc(&t->bb, 8) == hipSuccess && dalloc(&t->d2, max_vertices) == hipSuccess &&
                     dalloc(&t->loss, 1) == hipSuccess && dalloc(&t->nearest_tmp, max_vertices) == hipSuccess;
     bool evs = ok;
     for (int i = 0; i < 6 && evs; i++) evs = hipEventCreate(&t->ev[i]) == hipSuccess;
-    if (!ok || !evs) {
+    SamplerDev ext{};
+    ext.kind = BMF_SAMPLER_EXTERNAL;
+    if (!evs || hipMemcpy(t->ext_sampler, &ext, sizeof ext, hipMemcpyHostToDevice) != hipSuccess) {
         bmf_tape_destroy(t);
         return BMF_EHIP;
     }
@@ -1264,7 +1277,9 @@ void bmf_tape_destroy(bmf_tape* t) {
     dfree(t->r4);
     for (int i = 0; i < 6; i++)
         if (t->ev[i]) (void)hipEventDestroy(t->ev[i]);
-    dfree(t->err);
+    dfree(t->taken);
+    dfree(t->ext_sampler);
+    if (t->host) (void)hipHostFree(t->host);
     dfree(t->ckpt);
     dfree(t->bb);
     dfree(t->d2);
@@ -1291,34 +1306,21 @@ int bmf_forward_diff(bmf_ctx* c, const bmf_chunk_desc* d, const float* densities
     BMF_HIP(hipEventRecord(t->ev[0], s));
     c->have_extract = false;
     c->results_valid = false;
-    // the sampler of this call: the context's, or the caller's densities; the
-    // context's own is put back on every way out of this call, so later
-    // extractions never read the caller's buffer
-    struct RestoreSampler {
-        bmf_ctx* c;
-        bool active = false;
-        ~RestoreSampler() {
-            if (active) (void)hipMemcpy(c->A.sampler, &c->h_sampler, sizeof(SamplerDev), hipMemcpyHostToDevice);
-        }
-    } restore{c};
-    if (densities) {
-        SamplerDev ext{};
-        ext.kind = BMF_SAMPLER_EXTERNAL;
-        ext.ext = densities;
-        restore.active = true;
-        BMF_HIP(hipMemcpy(c->A.sampler, &ext, sizeof(SamplerDev), hipMemcpyHostToDevice));
-    }
-    rc = upload_descs(c, d, 1);
-    if (rc) return rc;
+    c->queued_n = -1;  // as after an extraction
     Arenas A = c->A;
     A.ext_base = 0;
+    if (densities) {  // this call's sampler, the context's own is not touched
+        A.sampler = t->ext_sampler;
+        A.ext = densities;
+        A.csg_list = nullptr;
+    }
     A.mesh_mode = BMF_MESH_TRIANGLES;  // the adjoint is defined on the triangle path
     A.quad_tris = 0;
     A.smoothing_follows = 0;  // the tape smooths its own copy: every output position is written by emit
     A.normals = 0;
     // extraction with every octave evaluated (densities exact everywhere),
     // no smoothing: the tape smooths its own copy
-    hipError_t e = launch_plan(A, 1, 0, 1, s);
+    hipError_t e = launch_plan(A, 1, 0, 1, s, d);
     if (e == hipSuccess)
         e = launch_sample(A, 1, sample_blocks_of(n3),
                           0, densities ? (int)BMF_SAMPLER_EXTERNAL : (int)c->h_sampler.kind,
@@ -1326,8 +1328,6 @@ int bmf_forward_diff(bmf_ctx* c, const bmf_chunk_desc* d, const float* densities
     if (e == hipSuccess) e = launch_count(A, word_blocks(dim), 0, s);
     if (e == hipSuccess) e = launch_scan(A, 1, 1, s);
     if (e == hipSuccess) e = launch_emit(A, word_blocks(dim), s);
-    if (e == hipSuccess) e = hipMemcpyAsync(c->h_results, A.results, sizeof(bmf_chunk_result), hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(c->h_ctr, A.ctr, sizeof(Counters), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) return BMF_EHIP;
     const bmf_chunk_result r = c->h_results[0];
@@ -1355,19 +1355,20 @@ int bmf_forward_diff(bmf_ctx* c, const bmf_chunk_desc* d, const float* densities
         hipLaunchKernelGGL(k_tape_take, dim3(blocks), dim3(kThreads), 0, s, A.dens, A.vedge + r.vertex_offset,
                            A.boundary + r.vertex_offset, A.idx + r.index_offset, A.pos + 3 * r.vertex_offset, n3, V,
                            3 * (int64_t)T, dim, t->dens, t->vedge, t->boundary, t->idx, t->p4, t->ckpt,
-                           smooth ? nullptr : t->pos, t->vid0, t->cell_n, t->rank, t->err);
+                           smooth ? nullptr : t->pos, t->vid0, t->cell_n, t->rank, t->taken,
+                           &t->mhost->err);
         BMF_HIP(hipGetLastError());
     }
     if (V > 0) {
         hipLaunchKernelGGL(k_order_cells, dim3(blocks_for(kOrderCells)), dim3(kThreads), 0, s, t->cell_n, t->cell_base,
-                           t->err + 1, t->order);
+                           t->taken, t->order);
         hipLaunchKernelGGL(k_order, dim3(blocks_for(V)), dim3(kThreads), 0, s, t->vedge, V, dim, t->cell_base, t->rank,
-                           t->order);
+                           t->taken, &t->mhost->places, t->order);
         BMF_HIP(hipGetLastError());
         if (smooth) {
             hipLaunchKernelGGL(k_tape_adj, dim3(step_blocks(V)), dim3(kStepThreads), 0, s, t->vedge, t->boundary,
                                A.cell_tb, A.cell_mask, t->idx, dim, V, T, t->bp, (int)t->cap_v, t->ring, t->deg, t->mv,
-                               t->bscale, t->err);
+                               t->bscale, &t->mhost->err);
             BMF_HIP(hipGetLastError());
             rc = smooth_steps(t, t->p4, t->q4, t->K, s, t->pos, 0);
             if (rc) return rc;
@@ -1379,11 +1380,9 @@ int bmf_forward_diff(bmf_ctx* c, const bmf_chunk_desc* d, const float* densities
         }
     }
     BMF_HIP(hipEventRecord(t->ev[1], s));
-    int herr[2] = {0, 0};
-    BMF_HIP(hipMemcpyAsync(herr, t->err, sizeof herr, hipMemcpyDeviceToHost, s));
     BMF_HIP(hipStreamSynchronize(s));
-    if (V > 0 && herr[0]) return BMF_EHIP;
-    t->places = herr[1];
+    if (V > 0 && t->host->err) return BMF_EHIP;
+    t->places = t->host->places;
     t->valid = true;
     t->timed[0] = true;
     return BMF_OK;
@@ -1439,13 +1438,11 @@ int bmf_loss_nearest(bmf_tape* t, const float* targets, int64_t n, float* dldp, 
         if (loss) *loss = 0.0f;
         return BMF_OK;
     }
-    rc = nn_query(t, tape_nn(t), n, dldp, nearest, t->loss, s);
+    rc = nn_query(t, tape_nn(t), n, dldp, nearest, &t->mhost->loss, s);
     if (rc) return rc;
     BMF_HIP(hipEventRecord(t->ev[3], s));
-    double l = 0.0;
-    BMF_HIP(hipMemcpyAsync(&l, t->loss, sizeof(double), hipMemcpyDeviceToHost, s));
     BMF_HIP(hipStreamSynchronize(s));
-    if (loss) *loss = (float)l;
+    if (loss) *loss = (float)t->host->loss;
     t->timed[1] = true;
     return BMF_OK;
 }
@@ -1475,13 +1472,11 @@ int bmf_tape_loss_nearest(bmf_tape* t, float* dldp, int32_t* nearest, float* los
     }
     t->timed[1] = false;
     BMF_HIP(hipEventRecord(t->ev[2], s));
-    int rc = nn_query(t, tape_nn(t), t->nn_n, dldp, nearest, t->loss, s);
+    int rc = nn_query(t, tape_nn(t), t->nn_n, dldp, nearest, &t->mhost->loss, s);
     if (rc) return rc;
     BMF_HIP(hipEventRecord(t->ev[3], s));
-    double l = 0.0;
-    BMF_HIP(hipMemcpyAsync(&l, t->loss, sizeof(double), hipMemcpyDeviceToHost, s));
     BMF_HIP(hipStreamSynchronize(s));
-    if (loss) *loss = (float)l;
+    if (loss) *loss = (float)t->host->loss;
     t->timed[1] = true;
     return BMF_OK;
 }

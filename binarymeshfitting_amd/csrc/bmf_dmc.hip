@@ -350,7 +350,7 @@ __device__ __forceinline__ uint32_t dmc_ring(const Arenas& A, const uint32_t (&p
             put(prim + ((r == 1) == flip ? 1u : 0u));
         }
     }
-    if (over) A.ctr->error = 10;
+    if (over) raise_error(A, 10);
     return n;
 }
 
@@ -441,7 +441,7 @@ __device__ void place_vertex(const Arenas& A, const ChunkMeta& M, const SamplerD
     }
     err = 0.0f;
     if (k == 0 || k > 7) {
-        A.ctr->error = 8;
+        raise_error(A, 8);
         out[0] = out[1] = out[2] = 0.0f;
         return;
     }
@@ -459,6 +459,7 @@ __global__ void __launch_bounds__(kRowThreads) k_dmc_vertices(Arenas A) {
     __shared__ DmcTables s_t;
     __shared__ DmcWave s_wave[kWordWaves];
     load_dmc_tables(s_t);
+    if (blockIdx.x == 0 && threadIdx.x == 0) publish_counters(A);
     __syncthreads();
     const SamplerDev* __restrict__ S = A.sampler;
     const int wave = uniform_int(threadIdx.x >> 6), lane = lane_id();
@@ -522,7 +523,7 @@ __global__ void __launch_bounds__(kRowThreads) k_dmc_vertices(Arenas A) {
                 const int cpos = (int)(item & 1023u), p = (int)((item >> 10) & 3u);
                 const uint32_t cmask = item >> 12, v = vb + e;
                 if (v >= Vc) {
-                    A.ctr->error = 8;
+                    raise_error(A, 8);
                     continue;
                 }
                 const uint32_t i = 64u * (uint32_t)w0 + (uint32_t)cpos;
@@ -623,7 +624,7 @@ __global__ void __launch_bounds__(kRowThreads) k_dmc_quads(Arenas A) {
                 }
                 const uint32_t prim = tris ? 2u * qid : qid;
                 if (!ok || prim + (tris ? 1u : 0u) >= Tc) {
-                    A.ctr->error = 9;
+                    raise_error(A, 9);
                     qid++;
                     continue;
                 }
@@ -680,7 +681,7 @@ __global__ void __launch_bounds__(kSmoothThreads) k_dual_n(Arenas A, int m) {
         const float4* __restrict__ P = A.pos4 + v_off;
         const uint32_t u0 = I[0], u1 = I[1], u2 = I[2], u3 = N == 4 ? I[3] : u0;
         if (u0 >= V || u1 >= V || u2 >= V || u3 >= V) {
-            A.ctr->error = 11;
+            raise_error(A, 11);
             continue;
         }
         const float4 a = P[u0], b = P[u1], c = P[u2], d = P[u3];
@@ -795,7 +796,7 @@ __global__ void __launch_bounds__(kSmoothThreads) k_dual_n_nrm(Arenas A, int m) 
         const float4* __restrict__ NV = A.nrm4 + v_off;
         const uint32_t u[4] = {I[0], I[1], I[2], I[N == 4 ? 3 : 0]};
         if (u[0] >= V || u[1] >= V || u[2] >= V || u[3] >= V) {
-            A.ctr->error = 11;
+            raise_error(A, 11);
             continue;
         }
         const float4 q[4] = {P[u[0]], P[u[1]], P[u[2]], P[u[3]]};

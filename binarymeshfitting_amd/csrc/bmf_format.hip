@@ -33,6 +33,7 @@
 #include "../../include/bmf.h"
 #include "bmf_context.h"
 #include "bmf_internal.h"
+#include "bmf_rows.h"
 #include "samplers.h"
 
 namespace bmf {
@@ -84,49 +85,61 @@ __device__ __forceinline__ float3 hsv_to_rgb(float h, float s, float v) {
     }
 }
 
+// Inclusive prefix over a wave of values below 2^50, in two 32-bit scans.
+__device__ __forceinline__ int64_t wave_scan64(int64_t v) {
+    const uint32_t lo = wave_scan((uint32_t)v & 0xFFFFFFu), hi = wave_scan((uint32_t)(v >> 24));
+    return ((int64_t)hi << 24) + lo;
+}
+
 // Per chunk j of the batch (table rows of n + 1 entries, the last holding the
 // totals): 0 first formatted vertex, 1 first formatted index, 2 first vertex
-// tile, 3 first index tile.  Thread t walks a contiguous segment of chunks,
-// the segment totals are scanned across the workgroup in LDS.
+// tile, 3 first index tile; the two totals for the host too.  Thread t walks a
+// contiguous segment of chunks; one exchange of wave totals.  Bound by its
+// chain of two loads and the exchange (512 chunks 4.1 us, one 3.2; a scan
+// with two barriers per step took 7.1 and 6.4).  blockDim: the batch's whole
+// waves, at most kPlanThreads.
 __global__ void __launch_bounds__(kPlanThreads) k_format_plan(const bmf_chunk_result* __restrict__ R, int n,
-                                                               int64_t* __restrict__ tab) {
-    __shared__ int64_t s[4][kPlanThreads];
-    const int t = threadIdx.x;
-    const int seg = (n + kPlanThreads - 1) / kPlanThreads;
+                                                               int64_t* __restrict__ tab,
+                                                               int64_t* __restrict__ host) {
+    __shared__ int64_t s_w[4][kPlanThreads / 64];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6, nw = (int)blockDim.x >> 6;
+    const int seg = (n + (int)blockDim.x - 1) / (int)blockDim.x;
     const int j0 = min(n, t * seg), j1 = min(n, j0 + seg);
-    int64_t a[4] = {0, 0, 0, 0};
-    for (int j = j0; j < j1; j++) {
-        const bmf_chunk_result r = R[j];
-        const bool take = r.contains_mesh && r.status == BMF_OK;
-        const int64_t V = take ? r.vertex_count : 0, I = take ? r.index_count : 0;
+    auto add = [&](int j, int64_t (&a)[4]) {
+        const int64_t V = R[j].vertex_count, I = R[j].index_count;
+        if (!(R[j].contains_mesh && R[j].status == BMF_OK)) return;
         a[0] += V;
         a[1] += I;
         a[2] += (V + kFmtThreads - 1) / kFmtThreads;
         a[3] += (I + kFmtThreads - 1) / kFmtThreads;
+    };
+    int64_t a[4] = {0, 0, 0, 0}, run[4], tot[4] = {0, 0, 0, 0};
+    for (int j = j0; j < j1; j++) add(j, a);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int64_t inc = wave_scan64(a[k]);
+        run[k] = inc - a[k];
+        if (lane == 63) s_w[k][w] = inc;
     }
-    for (int k = 0; k < 4; k++) s[k][t] = a[k];
     __syncthreads();
-    for (int off = 1; off < kPlanThreads; off <<= 1) {  // inclusive scan (Hillis-Steele)
-        int64_t v[4];
-        for (int k = 0; k < 4; k++) v[k] = t >= off ? s[k][t - off] : 0;
-        __syncthreads();
-        for (int k = 0; k < 4; k++) s[k][t] += v[k];
-        __syncthreads();
-    }
-    int64_t run[4];
-    for (int k = 0; k < 4; k++) run[k] = s[k][t] - a[k];  // exclusive prefix of the segment
+    for (int q = 0; q < nw; q++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int64_t x = s_w[k][q];
+            run[k] += q < w ? x : 0;
+            tot[k] += x;
+        }
     for (int j = j0; j < j1; j++) {
-        const bmf_chunk_result r = R[j];
-        const bool take = r.contains_mesh && r.status == BMF_OK;
-        const int64_t V = take ? r.vertex_count : 0, I = take ? r.index_count : 0;
+#pragma unroll
         for (int k = 0; k < 4; k++) tab[(int64_t)k * (n + 1) + j] = run[k];
-        run[0] += V;
-        run[1] += I;
-        run[2] += (V + kFmtThreads - 1) / kFmtThreads;
-        run[3] += (I + kFmtThreads - 1) / kFmtThreads;
+        if (seg > 1) add(j, run);
     }
-    if (t == kPlanThreads - 1)
-        for (int k = 0; k < 4; k++) tab[(int64_t)k * (n + 1) + n] = s[k][t];
+    if (t == 0) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) tab[(int64_t)k * (n + 1) + n] = tot[k];
+        host[0] = tot[0];
+        host[1] = tot[1];
+    }
 }
 
 // The chunk j of a tile: the largest j with prefix[j] <= tile (prefix
@@ -223,7 +236,7 @@ int bmf_format(bmf_ctx* c, const bmf_format_options* o, const bmf_vbo* out, int6
         BMF_HIP(hipMalloc((void**)&c->d_fmt, sizeof(int64_t) * 4 * ((size_t)c->lim.max_chunks + 1)));
     }
     if (!c->h_fmt) {
-        BMF_HIP(hipHostMalloc((void**)&c->h_fmt, sizeof(int64_t) * 2, hipHostMallocDefault));
+        BMF_HIP(host_alloc(&c->h_fmt, 2, &c->m_fmt));
     }
     FmtParams P{};
     P.space = o->space;
@@ -250,12 +263,11 @@ int bmf_format(bmf_ctx* c, const bmf_format_options* o, const bmf_vbo* out, int6
     P.cap_i = out->cap_indices;
     hipStream_t s = c->stream;
     const int nn = std::max(n, 0);
-    hipLaunchKernelGGL(k_format_plan, dim3(1), dim3(kPlanThreads), 0, s, c->A.results, nn, c->d_fmt);
+    const int threads = std::min(kPlanThreads, std::max(64, (nn + 63) / 64 * 64));
+    hipLaunchKernelGGL(k_format_plan, dim3(1), dim3((unsigned)threads), 0, s, c->A.results, nn, c->d_fmt, c->m_fmt);
     hipLaunchKernelGGL(k_format, dim3((unsigned)std::max(1, c->persistent_blocks)), dim3(kFmtThreads), 0, s,
                        c->A.results, nn, c->d_fmt, c->A.pos, c->A.idx, c->A.nrm, P);
     BMF_HIP(hipGetLastError());
-    BMF_HIP(hipMemcpyAsync(&c->h_fmt[0], c->d_fmt + nn, sizeof(int64_t), hipMemcpyDeviceToHost, s));
-    BMF_HIP(hipMemcpyAsync(&c->h_fmt[1], c->d_fmt + (nn + 1) + nn, sizeof(int64_t), hipMemcpyDeviceToHost, s));
     BMF_HIP(hipStreamSynchronize(s));
     if (vertices) *vertices = c->h_fmt[0];
     if (indices) *indices = c->h_fmt[1];

@@ -146,7 +146,14 @@ struct Arenas {
     uint4* vring;              // [max_vertices] ring cells of each vertex, packed by the first smoothing step
     uint32_t* idx;             // [max_indices]
     Counters* ctr;
+    // The host's copies, in pinned memory that the kernels write: a result per
+    // chunk when its record is final, the counters by the emit kernel, the
+    // error flag where it is raised.  Two copies after the pipeline took 4 us of
+    // the device and 10 of the calling thread.
+    bmf_chunk_result* host_results;  // [max_chunks]
+    Counters* host_ctr;
     SamplerDev* sampler;
+    const float* ext;          // the caller's densities of this call, before the EXTERNAL sampler's own
     int64_t cap_samples, cap_vertices, cap_indices;
     int32_t cap_chunks;
     int64_t ext_base;          // EXTERNAL: offset of this launch's first chunk in the caller's densities
@@ -183,7 +190,9 @@ inline int word_blocks(int dim) {
 }
 
 // Launch wrappers (bmf_kernels.hip).
-hipError_t launch_plan(const Arenas& A, int n, int allow_cull, int reset_bumps, hipStream_t s);
+// one: the single descriptor by value (n = 1), instead of A.descs
+hipError_t launch_plan(const Arenas& A, int n, int allow_cull, int reset_bumps, hipStream_t s,
+                       const bmf_chunk_desc* one = nullptr);
 // adaptive: signs everywhere and densities where the surface reads them (terrain, CSG); 0: every density
 // kind: the sampler the device struct holds for this launch (BMF_SAMPLER_*)
 // slab: the sampler is a 2D noise field (its columns are evaluated once per tile)

@@ -58,6 +58,7 @@ __device__ __forceinline__ void write_result(const Arenas& A, int j, const Chunk
     r.overlap_pos[1] = M.opos[1];
     r.overlap_pos[2] = M.opos[2];
     A.results[j] = r;
+    A.host_results[j] = r;
 }
 
 // a[i] of a register array by unrolled selects (a runtime index into a
@@ -223,6 +224,7 @@ __device__ __forceinline__ void plan_counters(const Arenas& A, int n, const int6
         c->need_i = 0;
         c->overflow = 0;
         c->error = 0;
+        A.host_ctr->error = 0;
     }
     if (overflow) c->overflow = 1;
     c->total_items = overflow ? 0 : tot[2];
@@ -236,8 +238,10 @@ __device__ __forceinline__ void plan_counters(const Arenas& A, int n, const int6
 // scans) and writes the records of its own kPlanSlice.  One block that wrote
 // every record took 14 us for 512 descriptors and 33 for 1,536 (a thread's
 // records are 120 bytes apart, written and read again across the scan);
-// this takes 6.7 and 9.9 (5.4 for one).
-__global__ void __launch_bounds__(kPlanThreads) k_plan(Arenas A, int n, int allow_cull, int reset_bumps) {
+// this takes 6.7 and 9.9 (5.4 for one).  A single descriptor may come with the
+// launch (`by_value`), which saves its copy to the arena.
+__global__ void __launch_bounds__(kPlanThreads) k_plan(Arenas A, int n, int allow_cull, int reset_bumps,
+                                                       bmf_chunk_desc one, int by_value) {
     __shared__ uint32_t s_w[4][kPlanThreads / 64];
     const SamplerDev* __restrict__ S = A.sampler;
     const int per = (n + kPlanThreads - 1) / kPlanThreads;  // 1 or 2
@@ -246,7 +250,7 @@ __global__ void __launch_bounds__(kPlanThreads) k_plan(Arenas A, int n, int allo
     for (int i = 0; i < per; i++) {
         if (j0 + i >= n) break;
         uint32_t add[4];
-        (void)plan_record(A, S, A.descs[j0 + i], allow_cull, add);
+        (void)plan_record(A, S, by_value ? one : A.descs[j0 + i], allow_cull, add);
 #pragma unroll
         for (int q = 0; q < 4; q++) sum[q] += add[q];
     }
@@ -258,7 +262,7 @@ __global__ void __launch_bounds__(kPlanThreads) k_plan(Arenas A, int n, int allo
         const int j = j0 + i;
         if (j >= n || j / kPlanSlice != (int)blockIdx.x) break;  // per divides kPlanSlice
         uint32_t add[4];
-        ChunkMeta m = plan_record(A, S, A.descs[j], allow_cull, add);
+        ChunkMeta m = plan_record(A, S, by_value ? one : A.descs[j], allow_cull, add);
         plan_finish(A, S, j, m, excl, overflow);
 #pragma unroll
         for (int q = 0; q < 4; q++) excl[q] += add[q];
@@ -895,7 +899,7 @@ __global__ void __launch_bounds__(kRowThreads) k_sample(Arenas A, int n, int ful
             solid = solid || bl != vb;
         };
         if constexpr (MODE == kSampleExternal) {
-            const float* __restrict__ src = S->ext + A.ext_base + M.dens_off;
+            const float* __restrict__ src = (A.ext ? A.ext : S->ext) + A.ext_base + M.dens_off;
             float v[WORDS];
 #pragma unroll
             for (int r = 0; r < WORDS; r++) v[r] = src[min(first + 64u * r + (uint32_t)lane, ns - 1u)];
@@ -1317,7 +1321,7 @@ __device__ __forceinline__ void emit_vertices(const Arenas& A, const ChunkMeta& 
         const int x = (int)udiv24(i, (uint32_t)d2, rd2), r = (int)i - x * d2;
         const int y = (int)udiv24((uint32_t)r, (uint32_t)dim, rd), z = r - y * dim;
         if (id + fx + fy + fz > Vc) {
-            A.ctr->error = 2;  // counts and ids disagree: report, never write past the chunk
+            raise_error(A, 2);  // counts and ids disagree: report, never write past the chunk
             continue;
         }
 #pragma unroll
@@ -1367,7 +1371,7 @@ __device__ __forceinline__ void emit_triangles(const Arenas& A, const ChunkMeta&
         tbase += round;
         if (!nt) continue;
         if (tb + nt > Tc) {
-            A.ctr->error = 3;
+            raise_error(A, 3);
             continue;
         }
         const uint64_t row = s_tri[mask];
@@ -1394,7 +1398,7 @@ __device__ __forceinline__ void emit_triangles(const Arenas& A, const ChunkMeta&
             I[3 * q + 1] = v[1];
             I[3 * q + 2] = v[2];
         }
-        if (bad) A.ctr->error = 4;
+        if (bad) raise_error(A, 4);
         if (cells) {
             const int64_t ci = M.dens_off + 64ll * w0 + pos;
             A.cell_tb[ci] = tb;
@@ -1411,6 +1415,7 @@ __global__ void __launch_bounds__(kRowThreads) k_emit(Arenas A) {
         s_tri[t] = c_tri_table[t];
         s_ntri[t] = (uint8_t)((c_tri_table[t] >> 60) / 3);
     }
+    if (blockIdx.x == 0 && threadIdx.x == 0) publish_counters(A);
     __syncthreads();
     const int wave = uniform_int(threadIdx.x >> 6);
     ItemWindows& s = s_win[wave];
@@ -1474,7 +1479,7 @@ __global__ void __launch_bounds__(kSmoothThreads) k_dual(Arenas A, int m) {
         const float4* __restrict__ P = A.pos4 + v_off;
         const uint32_t i0 = I[0], i1 = I[1], i2 = I[2];
         if (i0 >= V || i1 >= V || i2 >= V) {
-            A.ctr->error = 5;
+            raise_error(A, 5);
             continue;
         }
         const float4 a = P[i0], b = P[i1], c = P[i2];
@@ -1603,7 +1608,7 @@ __global__ void __launch_bounds__(kSmoothThreads) k_primal(Arenas A, int m) {
         if (m == 0) {
             bool bad = false;
             r = pack_ring(A.cell_tb + dens_off, A.cell_mask + dens_off, code, dim, T, bad);
-            if (bad) A.ctr->error = 7;
+            if (bad) raise_error(A, 7);
         }
         float s[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
         const uint32_t cnt = ring_sums<false>(r, A.cen4 + t_off, nullptr, s);
@@ -1656,7 +1661,7 @@ __global__ void __launch_bounds__(kSmoothThreads) k_dual_nrm(Arenas A, int m) {
         const float4* __restrict__ P = A.pos4 + M.v_off;
         const uint32_t i0 = I[0], i1 = I[1], i2 = I[2];
         if (i0 >= (uint32_t)M.V || i1 >= (uint32_t)M.V || i2 >= (uint32_t)M.V) {
-            A.ctr->error = 5;
+            raise_error(A, 5);
             continue;
         }
         const float4 a = P[i0], b = P[i1], c = P[i2];
@@ -1724,7 +1729,7 @@ __global__ void __launch_bounds__(kSmoothThreads) k_primal_nrm(Arenas A, int m) 
         if (m == 0) {
             bool bad = false;
             r = pack_ring(A.cell_tb + dens_off, A.cell_mask + dens_off, A.vedge[g], dim, T, bad);
-            if (bad) A.ctr->error = 7;
+            if (bad) raise_error(A, 7);
         } else {
             r = A.vring[g];
         }
@@ -1837,10 +1842,11 @@ __global__ void k_ref_masks(Arenas A, uint64_t* masks) {
 // ------------------------------------------------------------------------
 // launch wrappers
 // ------------------------------------------------------------------------
-hipError_t launch_plan(const Arenas& A, int n, int allow_cull, int reset_bumps, hipStream_t s) {
+hipError_t launch_plan(const Arenas& A, int n, int allow_cull, int reset_bumps, hipStream_t s,
+                       const bmf_chunk_desc* one) {
     if (n <= kPlanShared) {
         hipLaunchKernelGGL(k_plan, dim3((n + kPlanSlice - 1) / kPlanSlice), dim3(kPlanThreads), 0, s, A, n, allow_cull,
-                           reset_bumps);
+                           reset_bumps, one ? *one : bmf_chunk_desc{}, one != nullptr);
     } else {
         const int nb = (n + kPlanThreads - 1) / kPlanThreads;
         if (nb > kPlanThreads) return hipErrorInvalidValue;  // beyond BMF's 2^20 chunks

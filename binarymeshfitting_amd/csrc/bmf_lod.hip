@@ -269,8 +269,7 @@ int bmf_lod_queue(bmf_ctx* c, const bmf_world_node* nodes, int32_t n_nodes, cons
         BMF_HIP(hipMalloc((void**)&c->d_lod_code, (size_t)n_renderables));
         c->lod_cap_list = n_renderables;
     }
-    if (!c->d_lod_counts) BMF_HIP(hipMalloc((void**)&c->d_lod_counts, sizeof(int) * 2));
-    if (!c->h_lod_counts) BMF_HIP(hipHostMalloc((void**)&c->h_lod_counts, sizeof(int) * 2, hipHostMallocDefault));
+    if (!c->h_lod_counts) BMF_HIP(host_alloc(&c->h_lod_counts, 2, &c->d_lod_counts));
     // the descriptor arena is written by this call's kernel, after any queued
     // extraction that reads it (stream order)
     const int cap = std::min(cap_items, c->lim.max_chunks);
@@ -278,7 +277,6 @@ int bmf_lod_queue(bmf_ctx* c, const bmf_world_node* nodes, int32_t n_nodes, cons
                        flags_out, c->d_lod_first, c->d_lod_code, dirty_out, items_out, c->A.descs, cap,
                        c->d_lod_counts);
     BMF_HIP(hipGetLastError());
-    BMF_HIP(hipMemcpyAsync(c->h_lod_counts, c->d_lod_counts, sizeof(int) * 2, hipMemcpyDeviceToHost, s));
     BMF_HIP(hipStreamSynchronize(s));
     if (n_dirty) *n_dirty = c->h_lod_counts[0];
     if (n_chunks) *n_chunks = c->h_lod_counts[1];

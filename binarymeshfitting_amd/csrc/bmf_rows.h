@@ -34,6 +34,25 @@ __device__ __forceinline__ ChunkMeta read_chunk(const ChunkMeta* table, int j) {
     return m;
 }
 
+// Counts and ids disagree, or a map entry is out of range: raised for the
+// host, and nothing is written past the chunk.
+__device__ __forceinline__ void raise_error(const Arenas& A, int code) {
+    A.ctr->error = code;
+    A.host_ctr->error = code;
+}
+
+// The counters the host reads, once the row scan is through.
+__device__ __forceinline__ void publish_counters(const Arenas& A) {
+    const Counters c = *A.ctr;
+    Counters* h = A.host_ctr;
+    h->v_bump = c.v_bump;
+    h->i_bump = c.i_bump;
+    h->need_v = c.need_v;
+    h->need_i = c.need_i;
+    h->total_samples = c.total_samples;
+    h->overflow = c.overflow;
+}
+
 // Set bits of a wave mask below this lane.
 __device__ __forceinline__ uint32_t mbcnt64(uint64_t w) {
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(w >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)w, 0u));

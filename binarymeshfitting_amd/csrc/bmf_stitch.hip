@@ -375,7 +375,8 @@ __global__ void __launch_bounds__(kStitchThreads) k_stitch_count(World W, const 
 
 // Exclusive scan of the tile totals in place; out_total[0] = the sum.
 __global__ void __launch_bounds__(kScanThreads) k_stitch_scan(int64_t* __restrict__ tile, int64_t n_tiles,
-                                                              int64_t* __restrict__ out_total) {
+                                                              int64_t* __restrict__ out_total,
+                                                              int64_t* __restrict__ host_total) {
     __shared__ int64_t s_w[1][kScanThreads / 64 + 1];
     const int t = threadIdx.x;
     const int64_t seg = (n_tiles + kScanThreads - 1) / kScanThreads;
@@ -390,7 +391,7 @@ __global__ void __launch_bounds__(kScanThreads) k_stitch_scan(int64_t* __restric
         tile[i] = run;
         run += v;
     }
-    if (t == 0) out_total[0] = tot[0];
+    if (t == 0) out_total[0] = host_total[0] = tot[0];
 }
 
 // Triangles: a block takes kEmitTiles tiles, compacts their candidates with
@@ -521,8 +522,8 @@ __global__ void __launch_bounds__(kStitchThreads) k_stitch_emit(World W, const S
 }
 
 __global__ void k_stitch_world(const bmf_world_node* __restrict__ nodes, int n_nodes, int* __restrict__ out,
-                               float* __restrict__ max_size) {
-    // out[0]: the first node without a parent, out[1]: the deepest level
+                               float* __restrict__ max_size, int* __restrict__ host) {
+    // out[0]: the first node without a parent, out[1]: the deepest level; both for the host too
     __shared__ int s_root, s_level, s_size;
     if (threadIdx.x == 0) {
         s_root = 0x7FFFFFFF;
@@ -540,6 +541,8 @@ __global__ void k_stitch_world(const bmf_world_node* __restrict__ nodes, int n_n
     if (threadIdx.x == 0) {
         out[0] = s_root == 0x7FFFFFFF ? -1 : s_root;
         out[1] = s_level;
+        host[0] = out[0];
+        host[1] = out[1];
         *max_size = __int_as_float(s_size);
     }
 }
@@ -578,26 +581,27 @@ int bmf_stitch(bmf_ctx* c, const bmf_world_node* nodes, int32_t n_nodes, const i
         c->stitch_cap_cand = n_cand;
     }
     if (!c->d_stitch_misc) BMF_HIP(hipMalloc((void**)&c->d_stitch_misc, sizeof(int64_t) * 3));
-    if (!c->h_stitch_total) BMF_HIP(hipHostMalloc((void**)&c->h_stitch_total, sizeof(int64_t) * 2, hipHostMallocDefault));
+    if (!c->h_stitch_total) BMF_HIP(host_alloc(&c->h_stitch_total, 2, &c->m_stitch_total));
     // the world's root and deepest level, and the triangle total: the kernels
     // read the first two on the device, the host all three at the end
     int* dw = reinterpret_cast<int*>(c->d_stitch_misc);
     int64_t* total = c->d_stitch_misc + 1;
     float* max_size = reinterpret_cast<float*>(c->d_stitch_misc + 2);
-    hipLaunchKernelGGL(k_stitch_world, dim3(1), dim3(1024), 0, s, nodes, n_nodes, dw, max_size);
+    hipLaunchKernelGGL(k_stitch_world, dim3(1), dim3(1024), 0, s, nodes, n_nodes, dw, max_size,
+                       reinterpret_cast<int*>(c->m_stitch_total));
     if (n_cand > 0) {
         int log_dim = 0;
         while ((1 << log_dim) < dim) log_dim++;
         const World W{nodes, n_nodes, dim, log_dim, dw, max_size};
         hipLaunchKernelGGL(k_stitch_count, dim3((unsigned)n_tiles), dim3(kStitchThreads), 0, s, W, c->A.sampler, leaves,
                            (uint32_t)per_leaf, n_cand, c->d_stitch_counts, c->d_stitch_tiles);
-        hipLaunchKernelGGL(k_stitch_scan, dim3(1), dim3(kScanThreads), 0, s, c->d_stitch_tiles, n_tiles, total);
+        hipLaunchKernelGGL(k_stitch_scan, dim3(1), dim3(kScanThreads), 0, s, c->d_stitch_tiles, n_tiles, total,
+                           c->m_stitch_total + 1);
         hipLaunchKernelGGL(k_stitch_emit, dim3((unsigned)(n_room / kEmitCands)), dim3(kStitchThreads), 0, s, W,
                            c->A.sampler, leaves, (uint32_t)per_leaf, n_cand, c->d_stitch_counts, c->d_stitch_tiles,
                            total, triangles, cap_triangles);
     }
     BMF_HIP(hipGetLastError());
-    BMF_HIP(hipMemcpyAsync(c->h_stitch_total, c->d_stitch_misc, sizeof(int64_t) * 2, hipMemcpyDeviceToHost, s));
     BMF_HIP(hipStreamSynchronize(s));
     int hw[2];
     std::memcpy(hw, c->h_stitch_total, sizeof(hw));
