@@ -68,7 +68,7 @@ int enqueue_pipeline(bmf_ctx* c, const Arenas& A, int n, int maxk, int allow_cul
     c->stat_nrefine = row_blocks;
     BMF_MARK(2);
     const bool quads = A.mesh_mode == BMF_MESH_QUADS;
-    BMF_HIP(launch_count(A, row_blocks, c->h_sampler.kind == BMF_SAMPLER_TERRAIN, s));
+    BMF_HIP(launch_count(A, row_blocks, refinement(c->h_sampler), s));
     BMF_MARK(3);
     BMF_HIP(launch_scan(A, n, scan_blocks, s));
     BMF_MARK(4);
@@ -216,6 +216,31 @@ int build_sampler(const bmf_sampler_desc* s, SamplerDev* out) {
             d.nlo = r;
             d.nhi = 1.0f;
         }
+    }
+    if (s->kind == BMF_SAMPLER_NOISE) {
+        // k_field's bounds: a rigid sum adds -a_o t_o with t_o in [0, 1], an
+        // FBM a_o b_o with b_o in [-1, 1] (value noise may leave them by the
+        // rounding of its blends), each step rounding a sum of at most 1 + total
+        const bool rigid = d.noise_fractal == BMF_FRACTAL_RIGID;
+        double total = 1.0;
+        for (int o = 0; o < d.octaves; o++) total += std::fabs((double)d.ao[o]);
+        for (int k = 0; k <= d.octaves; k++) {
+            double dn = 0.0, up = 0.0;
+            for (int o = k; o < d.octaves; o++) {
+                const double a = d.ao[o];
+                dn += rigid ? std::max(a, 0.0) : std::fabs(a);
+                up += rigid ? std::max(-a, 0.0) : std::fabs(a);
+            }
+            if (rigid && k == 0) up += 1.0;
+            const double slack = total * ((d.octaves - k + 2) * std::ldexp(1.0, -23) + 1e-5);
+            d.field_dn[k] = std::nextafter((float)(dn + slack), INFINITY);
+            d.field_up[k] = std::nextafter((float)(up + slack), INFINITY);
+        }
+        auto moderate = [](float x) { return std::fabs(x) < 1e9f; };
+        d.early_ok = total < 1e9 && moderate(d.height) && moderate(d.g_scale) && moderate(d.y_scale) &&
+                     moderate(d.perturb_amp) && moderate(d.inv_norm);
+        for (int o = 0; o < d.octaves; o++) d.early_ok = d.early_ok && moderate(d.fo[o]);
+        for (int k = 0; k < d.perturb_octaves; k++) d.early_ok = d.early_ok && moderate(d.pf[k]) && moderate(d.pa[k]);
     }
     if (s->kind == BMF_SAMPLER_CSG) {
         d.n_spheres = s->n_spheres;

@@ -51,6 +51,11 @@ struct SamplerDev {
     // k_plan's chunk culling: n lies in [nlo, nhi] for every sample (cull = 0: no bound)
     float nlo, nhi;
     int32_t cull;
+    // 3D NOISE (k_field): the fractal's sum after k octaves moves at most
+    // field_dn[k] down and field_up[k] up (1, then every step's rounding
+    // included); early_ok = 0: the terms are too large for such bounds
+    float field_dn[BMF_MAX_OCTAVES + 1], field_up[BMF_MAX_OCTAVES + 1];
+    int32_t early_ok;
 };
 
 // How k_blocks expands a terrain chunk's noise: octaves per block and per
@@ -187,6 +192,15 @@ inline int sample_blocks_of(int64_t ns) { return (int)((ns + 1023) / 1024); }
 inline int word_blocks(int dim) {
     const int64_t items = ((int64_t)dim * dim * dim + kItemSamples - 1) / kItemSamples;
     return (int)((items + kRowThreads / 64 - 1) / (kRowThreads / 64));
+}
+
+// What k_count evaluates again: nothing, or the endpoints of sign-changing
+// edges that the adaptive terrain or 3D field sampling labelled early.
+constexpr int kRefineNone = 0, kRefineTerrain = 1, kRefineField = 2;
+inline int refinement(const SamplerDev& S) {
+    return S.kind == BMF_SAMPLER_TERRAIN                        ? kRefineTerrain
+           : S.kind == BMF_SAMPLER_NOISE && S.noise_dims == 3 ? kRefineField
+                                                              : kRefineNone;
 }
 
 // Launch wrappers (bmf_kernels.hip).

@@ -863,6 +863,294 @@ __global__ void __launch_bounds__(kRowThreads) k_columns(Arenas A, int n) {
     }
 }
 
+// ------------------------------------------------------------------------
+// 3D noise fields (adaptive): a wave per kFieldWords label words.
+//
+// The perturbation's frequencies are low, so that a wave's samples mostly lie
+// in one simplex of it: then the four corners' gradients are the wave's, formed
+// once for all its words, and a lane is left with the corners' falloffs, shared
+// by the three fields, and three multiply-adds per corner and field.  The
+// fractal's octaves follow one at a time over the samples of the workgroup
+// whose sign is still open, compacted into dense lanes: what the rest of the
+// octaves can add bounds the density from both sides.  Once that is no more
+// than the field changes by over two sample steps (field_end), the open samples
+// are mostly ends of sign-changing edges, whose density is wanted: they get all
+// the other octaves.  k_count evaluates the ends that are left.
+//
+// Bound by VALU issue.  108 chunks of 32^3 cells (3.9 M samples, 3 x 3
+// perturbation and 8 fractal octaves, a mean of 3.4 of these taken): 203 us
+// and 18 more in k_count; every octave at every sample took 320.  With open
+// samples decided down to the last octave 199 and 50 more.
+// ------------------------------------------------------------------------
+constexpr int kFieldWords = 4;
+constexpr int kFieldSamples = 64 * kFieldWords;
+
+// The gradients at the corners of a simplex of three noise fields of one
+// frequency, as factors -1, 0, 1 of the offsets (grad_dot's choices), the same
+// in every lane.
+struct FieldSimplex {
+    int i, j, k, rank;  // rank < 0: none yet
+    float g[3][4][3];   // field, corner, axis
+};
+
+__device__ __forceinline__ float lane_value(float x, int lane) {
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
+}
+
+// One octave of the 3D gradient perturbation at (x, y, z): the three fields of
+// seeds s, s + 1, s + 2, as snoise3 gives them.  All lanes are active.
+__device__ __forceinline__ void warp_octave(float x, float y, float z, uint32_t seed, FieldSimplex& F, float (&w)[3]) {
+    const float F3 = 1.0f / 3.0f, G3 = 1.0f / 6.0f, G3x2 = 2.0f * G3;
+    const float s = ((x + y) + z) * F3;
+    const float fi = floorf(x + s), fj = floorf(y + s), fk = floorf(z + s);
+    const int i = (int32_t)fi, j = (int32_t)fj, k = (int32_t)fk;
+    const float t = (float)(i + j + k) * G3;
+    const float x0 = x - (fi - t), y0 = y - (fj - t), z0 = z - (fk - t);
+    const uint64_t gxy = __ballot(x0 >= y0), gyz = __ballot(y0 >= z0), gxz = __ballot(x0 >= z0);
+    const int ui = uniform_int(i), uj = uniform_int(j), uk = uniform_int(k);
+    const bool one = __ballot((i == ui) & (j == uj) & (k == uk)) == ~0ull && (gxy == 0ull || gxy == ~0ull) &&
+                     (gyz == 0ull || gyz == ~0ull) && (gxz == 0ull || gxz == ~0ull);
+    if (!one) {
+        for (int a = 0; a < 3; a++) w[a] = snoise3(x, y, z, seed + (uint32_t)a);
+        return;
+    }
+    const bool bxy = gxy != 0ull, byz = gyz != 0ull, bxz = gxz != 0ull;
+    const bool i1 = bxy && bxz, j1 = !bxy && byz, k1 = !bxz && !byz;
+    const bool i2 = bxy || bxz, j2 = !bxy || byz, k2 = !bxz || !byz;
+    const int rank = (int)bxy + 2 * (int)byz + 4 * (int)bxz;
+    if (F.rank != rank || F.i != ui || F.j != uj || F.k != uk) {
+        F.i = ui;
+        F.j = uj;
+        F.k = uk;
+        F.rank = rank;
+        // lane 4 a + c: field a's gradient at corner c
+        const int lane = lane_id(), c = lane & 3;
+        const uint32_t ci = (uint32_t)ui + (uint32_t)(c == 3 || (c == 1 && i1) || (c == 2 && i2));
+        const uint32_t cj = (uint32_t)uj + (uint32_t)(c == 3 || (c == 1 && j1) || (c == 2 && j2));
+        const uint32_t ck = (uint32_t)uk + (uint32_t)(c == 3 || (c == 1 && k1) || (c == 2 && k2));
+        const uint32_t h = grad_mix(xor3(mul24(ci, kP1), mul24(cj, kP2), mul24(ck, kP3) ^ (seed + (uint32_t)(lane >> 2))));
+        const bool ux = h < 8u, vy = h < 4u, vx = h == 12u || h == 14u;
+        const float su = (h & 1u) ? -1.0f : 1.0f, sv = (h & 2u) ? -1.0f : 1.0f;
+        const float gx = ux ? su : (vx ? sv : 0.0f), gy = !ux ? su : (vy ? sv : 0.0f), gz = !vy && !vx ? sv : 0.0f;
+#pragma unroll
+        for (int q = 0; q < 12; q++) {
+            F.g[q >> 2][q & 3][0] = lane_value(gx, q);
+            F.g[q >> 2][q & 3][1] = lane_value(gy, q);
+            F.g[q >> 2][q & 3][2] = lane_value(gz, q);
+        }
+    }
+    const float xm = x0 - 1.0f, ym = y0 - 1.0f, zm = z0 - 1.0f;
+    const float cx[4] = {x0, (i1 ? xm : x0) + G3, (i2 ? xm : x0) + G3x2, xm + 0.5f};
+    const float cy[4] = {y0, (j1 ? ym : y0) + G3, (j2 ? ym : y0) + G3x2, ym + 0.5f};
+    const float cz[4] = {z0, (k1 ? zm : z0) + G3, (k2 ? zm : z0) + G3x2, zm + 0.5f};
+    float n[3];
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        float q = __builtin_fmaf(-cx[c], cx[c], kNoiseR2);
+        q = __builtin_fmaf(-cy[c], cy[c], q);
+        q = __builtin_fmaf(-cz[c], cz[c], q);
+        q = fmaxf(q, 0.0f);
+        q = q * q;
+        q = q * q;
+#pragma unroll
+        for (int a = 0; a < 3; a++) {
+            // two of the factors are 1 or -1, one is 0: the sum of the two is
+            // rounded once, as grad_dot's
+            const float dot = __builtin_fmaf(
+                F.g[a][c][0], cx[c], __builtin_fmaf(F.g[a][c][1], cy[c], F.g[a][c][2] * cz[c]));
+            const float v = q * dot;
+            n[a] = c == 0 ? v : n[a] + v;
+        }
+    }
+#pragma unroll
+    for (int a = 0; a < 3; a++) w[a] = fminf(fmaxf(kNoiseScale * n[a], -1.0f), 1.0f);
+}
+
+// The octave of the fractal from which k_field decides no more signs (see
+// there): a sample step changes octave o by about a_o f_o times the step of
+// its argument, times a noise gradient of about 2.
+__device__ __forceinline__ int field_end(const SamplerDev& S, float delta) {
+    float step = 0.0f;
+    for (int o = 0; o < S.octaves; o++) step += fabsf(S.ao[o] * S.fo[o]);
+    step *= 2.0f * delta * fabsf(S.g_scale);
+    int k = 1;
+    while (k < S.octaves && S.field_dn[k] + S.field_up[k] > 2.0f * step) k++;
+    return k;
+}
+
+__global__ void __launch_bounds__(kRowThreads) k_field(Arenas A, int n) {
+    constexpr int kParts = kItemWords / kFieldWords;  // waves per item of the word kernels
+    constexpr int kList = kWordWaves * kFieldSamples;
+    struct Geom {
+        int64_t dens_off;  // of the wave's first sample
+        int end;           // octaves after which the list is taken to the end
+    };
+    __shared__ Geom s_geom[kWordWaves];
+    // open samples: perturbed position, height, fractal sum, wave << 8 | sample
+    __shared__ float s_x[kList], s_y[kList], s_z[kList], s_py[kList], s_sum[kList];
+    __shared__ uint16_t s_at[kList];
+    __shared__ uint32_t s_n;
+    __shared__ uint64_t s_lab[kWordWaves * kFieldWords], s_exact[kWordWaves * kFieldWords];
+    const SamplerDev& S = *A.sampler;
+    const bool rigid = S.noise_fractal == BMF_FRACTAL_RIGID, value = S.noise_basis == BMF_NOISE_VALUE;
+    const int tid = threadIdx.x, wave = uniform_int(tid >> 6), lane = lane_id(), O = S.octaves;
+    auto octave = [&](float sum, int o, float cx, float cy, float cz) {
+        const float f = S.fo[o], a = S.ao[o];
+        const float b = value ? value3(cx * f, cy * f, cz * f, S.seed + (uint32_t)o)
+                              : snoise3(cx * f, cy * f, cz * f, S.seed + (uint32_t)o);
+        if (!rigid) return __builtin_fmaf(a, b, sum);
+        const float t = 1.0f - fabsf(b);
+        return o == 0 ? t : __builtin_fmaf(-t, a, sum);
+    };
+    auto density = [&](float sum, float py) {
+        return noise_density_from(S, rigid ? sum : fminf(fmaxf(sum * S.inv_norm, -1.0f), 1.0f), py);
+    };
+    auto set_bit = [&](uint64_t* words, uint32_t at) {
+        atomicOr(reinterpret_cast<uint32_t*>(words) + (at >> 5), 1u << (at & 31u));
+    };
+    const int64_t total = A.ctr->total_items * kParts;
+    for (int64_t u0 = (int64_t)blockIdx.x * kWordWaves; u0 < total; u0 += (int64_t)gridDim.x * kWordWaves) {
+        // ---- each wave's samples, perturbed, into the list ----
+        if (tid == 0) s_n = 0;
+        if (tid < kWordWaves * kFieldWords) s_lab[tid] = s_exact[tid] = 0ull;
+        __syncthreads();
+        const int64_t u = u0 + wave, it = u / kParts;
+        int64_t lab_off = 0;
+        int j = 0, open = 0;
+        if (u < total) {
+            const int part = (int)(u - it * kParts);
+            j = find_item_wave(A.meta, n, it);
+            const ChunkMeta M = read_chunk(A.meta, j);
+            const int item = (int)(it - M.item_slot), w0 = item * kItemWords + part * kFieldWords;
+            if (part == 0 && lane == 0) A.item_map[it] = make_int2(j, item);  // for the word kernels
+            const uint32_t dim = (uint32_t)M.dim, dim2 = dim * dim, ns = dim2 * dim, first = 64u * (uint32_t)w0;
+            const float rd = 1.0f / (float)dim, rd2 = 1.0f / (float)dim2;
+            const ChunkGeom G{M.opos[0], M.opos[1], M.opos[2], M.delta};
+            lab_off = M.lab_off + w0;
+            open = first < ns ? (int)min((uint32_t)kFieldSamples, ns - first) : 0;
+            // no early decision where a coordinate can leave the range of the bounds
+            const float ext = (float)(dim - 1u) * M.delta;
+            const bool early = S.early_ok && fmaxf(fmaxf(fabsf(G.ox), fabsf(G.oy)), fabsf(G.oz)) + ext < 1e9f;
+            uint32_t base = 0;
+            if (lane == 0) {
+                s_geom[wave] = Geom{M.dens_off + first, early ? field_end(S, M.delta) : 0};
+                base = atomicAdd(&s_n, (uint32_t)open);
+            }
+            base = (uint32_t)uniform_int((int)base);
+            float cx[kFieldWords], cy[kFieldWords], cz[kFieldWords], ph[kFieldWords];
+#pragma unroll
+            for (int r = 0; r < kFieldWords; r++) {
+                float px, pz;
+                sample_coords(G, min(first + 64u * r + (uint32_t)lane, ns - 1u), dim, dim2, rd, rd2, px, ph[r], pz);
+                if (S.perturb == BMF_PERTURB_GRADIENT) {
+                    cx[r] = px * S.g_scale;
+                    cy[r] = ph[r] * S.g_scale;
+                    cz[r] = pz * S.g_scale;
+                } else {
+                    noise_warp(S, px, ph[r], pz, cx[r], cy[r], cz[r]);
+                }
+            }
+            if (S.perturb == BMF_PERTURB_GRADIENT) {
+                FieldSimplex F;
+                for (int k = 0; k < S.perturb_octaves; k++) {
+                    const float f = S.pf[k], a = S.pa[k];
+                    F.rank = -1;
+#pragma unroll
+                    for (int r = 0; r < kFieldWords; r++) {
+                        float w[3];
+                        warp_octave(cx[r] * f, cy[r] * f, cz[r] * f, S.seed + 1000u + 3u * (uint32_t)k, F, w);
+                        cx[r] = __builtin_fmaf(a, w[0], cx[r]);
+                        cy[r] = __builtin_fmaf(a, w[1], cy[r]);
+                        cz[r] = __builtin_fmaf(a, w[2], cz[r]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < kFieldWords; r++) {
+                const int e = 64 * r + lane;
+                if (e < open) {
+                    s_x[base + e] = cx[r];
+                    s_y[base + e] = cy[r];
+                    s_z[base + e] = cz[r];
+                    s_py[base + e] = ph[r];
+                    s_at[base + e] = (uint16_t)(wave << 8 | e);
+                }
+            }
+        }
+        __syncthreads();
+        uint32_t nq = s_n;
+        int end = O;
+        for (int w = 0; w < kWordWaves; w++)
+            if (u0 + w < total) end = min(end, s_geom[w].end);
+        // ---- an octave at a time, the samples still open moved up ----
+        int o = 0;
+        for (; o < end && o < O - 1 && nq; o++) {
+            const float dn = S.field_dn[o + 1], up = S.field_up[o + 1];
+            __syncthreads();  // every thread has read s_n
+            if (tid == 0) s_n = 0;
+            for (uint32_t e0 = 0; e0 < nq; e0 += kRowThreads) {
+                const uint32_t e = e0 + (uint32_t)tid;
+                const bool in = e < nq;
+                const float cx = s_x[in ? e : 0u], cy = s_y[in ? e : 0u], cz = s_z[in ? e : 0u], py = s_py[in ? e : 0u];
+                float sum = o > 0 && in ? s_sum[e] : 0.0f;
+                const uint32_t at = s_at[in ? e : 0u];
+                __syncthreads();  // this part of the list is read: it may be overwritten
+                bool keep = false;
+                if (in) {
+                    sum = octave(sum, o, cx, cy, cz);
+                    const float d0 = density(sum - dn, py), d1 = density(sum + up, py);
+                    const bool air = fmaxf(d0, d1) < 0.0f;
+                    if (air) set_bit(s_lab, at);
+                    keep = !(air || fminf(d0, d1) >= 0.0f);
+                }
+                const uint64_t push = __ballot(keep);
+                if (push) {
+                    uint32_t base = 0;
+                    if (lane == 0) base = atomicAdd(&s_n, (uint32_t)__popcll(push));
+                    const uint32_t k = (uint32_t)uniform_int((int)base) + mbcnt64(push);
+                    if (keep) {
+                        s_x[k] = cx;
+                        s_y[k] = cy;
+                        s_z[k] = cz;
+                        s_py[k] = py;
+                        s_sum[k] = sum;
+                        s_at[k] = (uint16_t)at;
+                    }
+                }
+            }
+            __syncthreads();
+            nq = s_n;
+        }
+        // ---- the rest of the octaves of the samples still open ----
+        for (uint32_t e = (uint32_t)tid; e < nq; e += kRowThreads) {
+            const float cx = s_x[e], cy = s_y[e], cz = s_z[e];
+            float sum = o > 0 ? s_sum[e] : 0.0f;
+            const uint32_t at = s_at[e];
+            for (int k = o; k < O; k++) sum = octave(sum, k, cx, cy, cz);
+            const float d = density(sum, s_py[e]);
+            A.dens[s_geom[at >> 8].dens_off + (at & 255u)] = d;
+            if (d < 0.0f) set_bit(s_lab, at);
+            set_bit(s_exact, at);
+        }
+        __syncthreads();
+        // ---- the words ----
+        const int left = open - 64 * lane;
+        const bool mine = lane < kFieldWords && left > 0;
+        const uint64_t lb = mine ? s_lab[wave * kFieldWords + lane] : 0ull, have = ~bits_from(left);
+        if (mine) {
+            A.labels[lab_off + lane] = lb;
+            A.exact[lab_off + lane] = s_exact[wave * kFieldWords + lane];
+        }
+        const bool air = __any(mine && lb != 0ull), solid = __any(mine && (~lb & have) != 0ull);
+        if (lane == 0) {
+            if (air && !A.meta[j].any_air) atomicOr(&A.meta[j].any_air, 1u);
+            if (solid && !A.meta[j].any_solid) atomicOr(&A.meta[j].any_solid, 1u);
+        }
+        __syncthreads();  // before the next words'
+    }
+    if (tid == 0 && (int)blockIdx.x < A.stat_cap) A.stat_blocks[blockIdx.x] = 0ull;  // no octaves counted
+}
+
 // full: CSG values are wanted at every sample (stage inspection, the tape).
 // Otherwise only signs and the densities at the ends of sign-changing edges
 // are read, where the union lies within a sample step of 0 (it is
@@ -1004,7 +1292,7 @@ __global__ void __launch_bounds__(kRowThreads) k_sample(Arenas A, int n, int ful
 // 3 % of its lanes busy: 512 chunks of 64^3 cells, 64 sampled, took 70 us
 // and 23 more for the refinement as a kernel of its own; this takes 45 us.
 // ------------------------------------------------------------------------
-template <bool REFINE>
+template <int REFINE>
 __global__ void __launch_bounds__(kRowThreads) k_count(Arenas A) {
     __shared__ uint8_t s_n[256];  // triangles (polygons in the quad mode) of each corner mask
     __shared__ uint64_t s_corner[kWordWaves][kItemWords][8];
@@ -1092,7 +1380,7 @@ __global__ void __launch_bounds__(kRowThreads) k_count(Arenas A) {
                 wave_sync();  // the cells are read
                 const int nq = push_bits(need, list);
                 wave_sync();
-                evals += (unsigned long long)nq * (unsigned long long)S->octaves;
+                if constexpr (REFINE == kRefineTerrain) evals += (unsigned long long)nq * (unsigned long long)S->octaves;
                 const float rd = 1.0f / (float)dim, rd2 = 1.0f / (float)d2;
                 for (int e = lane; e < nq; e += 64) {
                     const uint32_t i = 64u * (uint32_t)R.w0 + list[e];
@@ -1100,7 +1388,8 @@ __global__ void __launch_bounds__(kRowThreads) k_count(Arenas A) {
                     const uint32_t y = udiv24(r, (uint32_t)dim, rd), z = r - y * (uint32_t)dim;
                     const float px = (float)x * M.delta + M.opos[0], py = (float)y * M.delta + M.opos[1],
                                 pz = (float)z * M.delta + M.opos[2];
-                    A.dens[M.dens_off + i] = terrain_density(*S, px, py, pz);
+                    if constexpr (REFINE == kRefineTerrain) A.dens[M.dens_off + i] = terrain_density(*S, px, py, pz);
+                    else A.dens[M.dens_off + i] = noise_density_from(*S, noise_value(*S, px, py, pz), py);
                 }
             }
             wave_sync();  // the next item reuses the list and the corners
@@ -1867,6 +2156,8 @@ hipError_t launch_sample(const Arenas& A, int n, int blocks, int adaptive, int k
     } else if (kind == BMF_SAMPLER_NOISE && slab) {
         hipLaunchKernelGGL(k_columns, g, b, 0, s, A, n);
         hipLaunchKernelGGL((k_sample<kSampleField2, 16>), g, b, 0, s, A, n, 1);
+    } else if (kind == BMF_SAMPLER_NOISE && adaptive) {
+        hipLaunchKernelGGL(k_field, g, b, 0, s, A, n);
     } else if (kind == BMF_SAMPLER_NOISE) {
         hipLaunchKernelGGL((k_sample<kSampleField3, 4>), g, b, 0, s, A, n, 1);
     } else if (kind == BMF_SAMPLER_CSG) {
@@ -1879,8 +2170,11 @@ hipError_t launch_sample(const Arenas& A, int n, int blocks, int adaptive, int k
     return hipGetLastError();
 }
 hipError_t launch_count(const Arenas& A, int blocks, int refine, hipStream_t s) {
-    if (refine) hipLaunchKernelGGL(k_count<true>, dim3(blocks), dim3(kRowThreads), 0, s, A);
-    else hipLaunchKernelGGL(k_count<false>, dim3(blocks), dim3(kRowThreads), 0, s, A);
+    if (refine == kRefineTerrain)
+        hipLaunchKernelGGL(k_count<kRefineTerrain>, dim3(blocks), dim3(kRowThreads), 0, s, A);
+    else if (refine == kRefineField)
+        hipLaunchKernelGGL(k_count<kRefineField>, dim3(blocks), dim3(kRowThreads), 0, s, A);
+    else hipLaunchKernelGGL(k_count<kRefineNone>, dim3(blocks), dim3(kRowThreads), 0, s, A);
     return hipGetLastError();
 }
 hipError_t launch_scan(const Arenas& A, int n, int blocks, hipStream_t s) {
