@@ -158,6 +158,7 @@ __global__ void __launch_bounds__(kFmtThreads) k_format(const bmf_chunk_result* 
                                                         const int64_t* __restrict__ tab, const float* __restrict__ pos,
                                                         const uint32_t* __restrict__ idx,
                                                         const float* __restrict__ nrm, FmtParams P) {
+    if (P.colors == BMF_COLOR_NOISE) load_gradients();
     const int64_t* dv = tab;
     const int64_t* di = tab + (n + 1);
     const int64_t* vt = tab + 2 * (int64_t)(n + 1);

@@ -434,7 +434,7 @@ __device__ __forceinline__ void sample_coords(const ChunkGeom& G, uint32_t i, ui
 //
 // A quad of lanes shares a centre, an octave each, so that a wave's chain is
 // one octave long.  Bound by VALU issue: 512 chunks of 64^3 cells, 64 sampled
-// (17.6 M samples, 5 octaves) take 52 us here and 69 in k_terrain; evaluating
+// (17.6 M samples, 5 octaves) take 42 us here and 61 in k_terrain; evaluating
 // every sample's octaves until its sign was certain (1.38 on average) took
 // 202, and 23 instead of 13 for the endpoints that it left.
 // ------------------------------------------------------------------------
@@ -444,20 +444,17 @@ struct NoiseGrad {
     float n, gx, gy, gz;
 };
 __device__ __forceinline__ void corner_grad(float x, float y, float z, uint32_t h, NoiseGrad& r) {
+    const float4 g = lattice_gradient(lattice_mix(h));
     float t = __builtin_fmaf(-x, x, kNoiseR2);
     t = __builtin_fmaf(-y, y, t);
     t = __builtin_fmaf(-z, z, t);
     t = fmaxf(t, 0.0f);
-    const float su = (h & 1u) ? -1.0f : 1.0f, sv = (h & 2u) ? -1.0f : 1.0f;
-    const bool ux = h < 8u, vy = h < 4u, vx = h == 12u || h == 14u;
-    const float gx = (ux ? su : 0.0f) + (vx ? sv : 0.0f), gy = (ux ? 0.0f : su) + (vy ? sv : 0.0f),
-                gz = vy || vx ? 0.0f : sv;
-    const float L = __builtin_fmaf(gx, x, __builtin_fmaf(gy, y, gz * z));
+    const float L = __builtin_fmaf(g.x, x, __builtin_fmaf(g.y, y, g.z * z));
     const float t2 = t * t, t4 = t2 * t2, k = -8.0f * t2 * t * L;
     r.n = __builtin_fmaf(t4, L, r.n);
-    r.gx = __builtin_fmaf(t4, gx, __builtin_fmaf(k, x, r.gx));
-    r.gy = __builtin_fmaf(t4, gy, __builtin_fmaf(k, y, r.gy));
-    r.gz = __builtin_fmaf(t4, gz, __builtin_fmaf(k, z, r.gz));
+    r.gx = __builtin_fmaf(t4, g.x, __builtin_fmaf(k, x, r.gx));
+    r.gy = __builtin_fmaf(t4, g.y, __builtin_fmaf(k, y, r.gy));
+    r.gz = __builtin_fmaf(t4, g.z, __builtin_fmaf(k, z, r.gz));
 }
 __device__ __forceinline__ NoiseGrad snoise3_grad(float x, float y, float z, uint32_t seed) {
     const float G3 = 1.0f / 6.0f;
@@ -474,12 +471,12 @@ __device__ __forceinline__ NoiseGrad snoise3_grad(float x, float y, float z, uin
     const uint32_t b0 = mul24((uint32_t)j, kP2), b1 = mul24((uint32_t)(j + 1), kP2);
     const uint32_t c0 = mul24((uint32_t)k, kP3) ^ seed, c1 = mul24((uint32_t)(k + 1), kP3) ^ seed;
     NoiseGrad r{0.0f, 0.0f, 0.0f, 0.0f};
-    corner_grad(x0, y0, z0, grad_mix(xor3(a0, b0, c0)), r);
+    corner_grad(x0, y0, z0, xor3(a0, b0, c0), r);
     corner_grad((i1 ? xm : x0) + G3, (j1 ? ym : y0) + G3, (k1 ? zm : z0) + G3,
-                grad_mix(xor3(i1 ? a1 : a0, j1 ? b1 : b0, k1 ? c1 : c0)), r);
+                xor3(i1 ? a1 : a0, j1 ? b1 : b0, k1 ? c1 : c0), r);
     corner_grad((i2 ? xm : x0) + 2.0f * G3, (j2 ? ym : y0) + 2.0f * G3, (k2 ? zm : z0) + 2.0f * G3,
-                grad_mix(xor3(i2 ? a1 : a0, j2 ? b1 : b0, k2 ? c1 : c0)), r);
-    corner_grad(xm + 0.5f, ym + 0.5f, zm + 0.5f, grad_mix(xor3(a1, b1, c1)), r);
+                xor3(i2 ? a1 : a0, j2 ? b1 : b0, k2 ? c1 : c0), r);
+    corner_grad(xm + 0.5f, ym + 0.5f, zm + 0.5f, xor3(a1, b1, c1), r);
     r.n *= kNoiseScale;
     r.gx *= kNoiseScale;
     r.gy *= kNoiseScale;
@@ -515,6 +512,7 @@ __global__ void __launch_bounds__(kRowThreads) k_blocks(Arenas A, int n) {
     __shared__ unsigned long long s_evals;
     if (threadIdx.x == 0) s_evals = 0;
     __syncthreads();
+    load_gradients();
     const SamplerDev* __restrict__ S = A.sampler;
     const int wave = uniform_int(threadIdx.x >> 6), lane = lane_id(), o = lane & 3;
     unsigned long long evals = 0;  // octaves at the centres of this wave's blocks (uniform)
@@ -671,6 +669,7 @@ __global__ void __launch_bounds__(kRowThreads) k_terrain(Arenas A, int n) {
     __shared__ uint32_t s_n;
     __shared__ unsigned long long s_evals;
     __shared__ float s_oct[3][BMF_MAX_OCTAVES + 1];  // per octave: frequency, amplitude, reach
+    load_gradients();
     const SamplerDev* __restrict__ S = A.sampler;
     const TerrainTerms TT{S->amp, S->y0, S->inv_norm};
     const int O = S->octaves;
@@ -830,7 +829,7 @@ __global__ void __launch_bounds__(kRowThreads) k_terrain(Arenas A, int n) {
 // LDS but the CSG primitives.  The words per wave balance the chip's last
 // round against the wave's own set-up.  Bound by VALU issue where a sampler is
 // evaluated, by HBM where densities only pass through.
-//   terrain in full  129^3 samples, 5 octaves: 64 us (tiles of 2,048
+//   terrain in full  129^3 samples, 5 octaves: 52 us (tiles of 2,048
 //                    samples per workgroup, 1,049 of them: 95)
 //   external         48 chunks of 41^3: 12 us (tiles: 52)
 //   2D noise field   from the columns of k_columns
@@ -846,6 +845,7 @@ constexpr int kWaveCsg = 64;  // CSG primitives per wave staged in LDS (longer l
 // workgroup's 256 lanes: 168 chunks of 32^3 took 76 us; this and the pass
 // over the samples take 26 + 18.
 __global__ void __launch_bounds__(kRowThreads) k_columns(Arenas A, int n) {
+    load_gradients();
     const SamplerDev* __restrict__ S = A.sampler;
     const int64_t total = A.block_prefix[n];
     const int lane = lane_id();
@@ -878,16 +878,15 @@ __global__ void __launch_bounds__(kRowThreads) k_columns(Arenas A, int n) {
 // the other octaves.  k_count evaluates the ends that are left.
 //
 // Bound by VALU issue.  108 chunks of 32^3 cells (3.9 M samples, 3 x 3
-// perturbation and 8 fractal octaves, a mean of 3.4 of these taken): 203 us
-// and 18 more in k_count; every octave at every sample took 320.  With open
-// samples decided down to the last octave 199 and 50 more.
+// perturbation and 8 fractal octaves, a mean of 3.4 of these taken): 161 us
+// and 9 more in k_count; every octave at every sample took 255.  With open
+// samples decided down to the last octave k_count took 32 more.
 // ------------------------------------------------------------------------
 constexpr int kFieldWords = 4;
 constexpr int kFieldSamples = 64 * kFieldWords;
 
 // The gradients at the corners of a simplex of three noise fields of one
-// frequency, as factors -1, 0, 1 of the offsets (grad_dot's choices), the same
-// in every lane.
+// frequency, the same in every lane.
 struct FieldSimplex {
     int i, j, k, rank;  // rank < 0: none yet
     float g[3][4][3];   // field, corner, axis
@@ -928,15 +927,13 @@ __device__ __forceinline__ void warp_octave(float x, float y, float z, uint32_t 
         const uint32_t ci = (uint32_t)ui + (uint32_t)(c == 3 || (c == 1 && i1) || (c == 2 && i2));
         const uint32_t cj = (uint32_t)uj + (uint32_t)(c == 3 || (c == 1 && j1) || (c == 2 && j2));
         const uint32_t ck = (uint32_t)uk + (uint32_t)(c == 3 || (c == 1 && k1) || (c == 2 && k2));
-        const uint32_t h = grad_mix(xor3(mul24(ci, kP1), mul24(cj, kP2), mul24(ck, kP3) ^ (seed + (uint32_t)(lane >> 2))));
-        const bool ux = h < 8u, vy = h < 4u, vx = h == 12u || h == 14u;
-        const float su = (h & 1u) ? -1.0f : 1.0f, sv = (h & 2u) ? -1.0f : 1.0f;
-        const float gx = ux ? su : (vx ? sv : 0.0f), gy = !ux ? su : (vy ? sv : 0.0f), gz = !vy && !vx ? sv : 0.0f;
+        const float4 g = lattice_gradient(lattice_mix(
+            xor3(mul24(ci, kP1), mul24(cj, kP2), mul24(ck, kP3) ^ (seed + (uint32_t)(lane >> 2)))));
 #pragma unroll
         for (int q = 0; q < 12; q++) {
-            F.g[q >> 2][q & 3][0] = lane_value(gx, q);
-            F.g[q >> 2][q & 3][1] = lane_value(gy, q);
-            F.g[q >> 2][q & 3][2] = lane_value(gz, q);
+            F.g[q >> 2][q & 3][0] = lane_value(g.x, q);
+            F.g[q >> 2][q & 3][1] = lane_value(g.y, q);
+            F.g[q >> 2][q & 3][2] = lane_value(g.z, q);
         }
     }
     const float xm = x0 - 1.0f, ym = y0 - 1.0f, zm = z0 - 1.0f;
@@ -954,8 +951,6 @@ __device__ __forceinline__ void warp_octave(float x, float y, float z, uint32_t 
         q = q * q;
 #pragma unroll
         for (int a = 0; a < 3; a++) {
-            // two of the factors are 1 or -1, one is 0: the sum of the two is
-            // rounded once, as grad_dot's
             const float dot = __builtin_fmaf(
                 F.g[a][c][0], cx[c], __builtin_fmaf(F.g[a][c][1], cy[c], F.g[a][c][2] * cz[c]));
             const float v = q * dot;
@@ -991,6 +986,7 @@ __global__ void __launch_bounds__(kRowThreads) k_field(Arenas A, int n) {
     __shared__ uint16_t s_at[kList];
     __shared__ uint32_t s_n;
     __shared__ uint64_t s_lab[kWordWaves * kFieldWords], s_exact[kWordWaves * kFieldWords];
+    load_gradients();
     const SamplerDev& S = *A.sampler;
     const bool rigid = S.noise_fractal == BMF_FRACTAL_RIGID, value = S.noise_basis == BMF_NOISE_VALUE;
     const int tid = threadIdx.x, wave = uniform_int(tid >> 6), lane = lane_id(), O = S.octaves;
@@ -1163,6 +1159,7 @@ __global__ void __launch_bounds__(kRowThreads) k_sample(Arenas A, int n, int ful
     constexpr int kParts = kItemWords / WORDS;  // waves per item of the word kernels
     constexpr bool kCsg = MODE == kSampleCsg;
     __shared__ float4 s_csg[kCsg ? kWordWaves : 1][kCsg ? 2 * kWaveCsg : 1];
+    if constexpr (MODE == kSampleTerrain || MODE == kSampleField3) load_gradients();
     const SamplerDev* __restrict__ S = A.sampler;
     const int wave = uniform_int(threadIdx.x >> 6), lane = lane_id();
     const int64_t total = A.ctr->total_items * kParts;
@@ -1298,6 +1295,7 @@ __global__ void __launch_bounds__(kRowThreads) k_count(Arenas A) {
     __shared__ uint64_t s_corner[kWordWaves][kItemWords][8];
     __shared__ uint16_t s_list[kWordWaves][kItemSamples];
     __shared__ unsigned long long s_evals;
+    if constexpr (REFINE) load_gradients();
     const bool quads = A.mesh_mode == BMF_MESH_QUADS;
     for (int t = threadIdx.x; t < 256; t += blockDim.x)
         s_n[t] = (uint8_t)(quads ? dmc_polygons(c_dmc_table[t]) : (uint32_t)((c_tri_table[t] >> 60) / 3));

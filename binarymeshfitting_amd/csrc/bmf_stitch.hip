@@ -349,6 +349,7 @@ __global__ void __launch_bounds__(kStitchThreads) k_stitch_count(World W, const 
     __shared__ uint8_t s_cnt[kStitchThreads];
     __shared__ int s_n;
     __shared__ int s_w[kStitchThreads / 64];
+    load_gradients();
     const int root = uniform_int(W.root_level[0]), L = uniform_int(W.root_level[1]);
     const int64_t cand0 = (int64_t)blockIdx.x * kStitchThreads;
     const int ncand = (int)(n_cand - cand0 < kStitchThreads ? n_cand - cand0 : kStitchThreads);
@@ -430,6 +431,7 @@ __global__ void __launch_bounds__(kStitchThreads) k_stitch_emit(World W, const S
     __shared__ float s_cross[kEmitRound][12][3];
     static_assert(kEmitCands <= 1 << 11, "list entry layout");
     constexpr int kPer = kEmitCands / kStitchThreads;  // consecutive candidates per thread
+    load_gradients();
     if (total[0] > cap) return;  // reported by the host: nothing is written
     const int root = uniform_int(W.root_level[0]), L = uniform_int(W.root_level[1]);
     const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
