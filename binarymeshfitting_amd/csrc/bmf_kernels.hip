@@ -879,8 +879,8 @@ __global__ void __launch_bounds__(kRowThreads) k_columns(Arenas A, int n) {
 //
 // Bound by VALU issue.  108 chunks of 32^3 cells (3.9 M samples, 3 x 3
 // perturbation and 8 fractal octaves, a mean of 3.4 of these taken): 161 us
-// and 9 more in k_count; every octave at every sample took 255.  With open
-// samples decided down to the last octave k_count took 32 more.
+// and 9 more in k_count.  With compares and selects for the noise's gradients
+// (see gradient_table) it took 203 and 18, every octave at every sample 320.
 // ------------------------------------------------------------------------
 constexpr int kFieldWords = 4;
 constexpr int kFieldSamples = 64 * kFieldWords;
