@@ -22,8 +22,7 @@
 // extracted completely.
 //
 // Two launches: k_format_plan (one workgroup) forms the chunks' offsets in
-// the formatted arrays and their 256-element tile counts from the device
-// results; k_format (persistent, grid-stride over the tiles) writes the
+// the formatted arrays and their tile counts from the device results; k_format (persistent, grid-stride over the tiles) writes the
 // vertices and indices.  HBM traffic: 12 B read + 12-36 B written per
 // vertex, 4 B read + 4 B written per index.
 #include <hip/hip_runtime.h>
@@ -39,7 +38,15 @@
 namespace bmf {
 namespace {
 
-constexpr int kFmtThreads = 256;   // elements per tile, one per thread
+constexpr int kFmtThreads = 256;
+// Elements per thread of a tile: four share one search for their chunk and load
+// together where there are tiles enough to fill the chip; a few chunks, and
+// noise colours, whose octaves are a long chain, want the threads instead
+// (k_format with four and with one: one chunk 4.4 and 3.6 us, a world's 217 with
+// noise colours 14.5 and 12.4, 108 chunks 6.3 where one and a binary search took
+// 9.1).
+constexpr int kFmtEach = 4;
+constexpr int kFmtMany = 64;       // chunks from which tiles are taken to be enough
 constexpr int kPlanThreads = 1024;
 constexpr int kColorOctaves = 4;
 
@@ -99,7 +106,7 @@ __device__ __forceinline__ int64_t wave_scan64(int64_t v) {
 // with two barriers per step took 7.1 and 6.4).  blockDim: the batch's whole
 // waves, at most kPlanThreads.
 __global__ void __launch_bounds__(kPlanThreads) k_format_plan(const bmf_chunk_result* __restrict__ R, int n,
-                                                               int64_t* __restrict__ tab,
+                                                               int tile, int64_t* __restrict__ tab,
                                                                int64_t* __restrict__ host) {
     __shared__ int64_t s_w[4][kPlanThreads / 64];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6, nw = (int)blockDim.x >> 6;
@@ -110,8 +117,8 @@ __global__ void __launch_bounds__(kPlanThreads) k_format_plan(const bmf_chunk_re
         if (!(R[j].contains_mesh && R[j].status == BMF_OK)) return;
         a[0] += V;
         a[1] += I;
-        a[2] += (V + kFmtThreads - 1) / kFmtThreads;
-        a[3] += (I + kFmtThreads - 1) / kFmtThreads;
+        a[2] += (V + tile - 1) / tile;
+        a[3] += (I + tile - 1) / tile;
     };
     int64_t a[4] = {0, 0, 0, 0}, run[4], tot[4] = {0, 0, 0, 0};
     for (int j = j0; j < j1; j++) add(j, a);
@@ -142,18 +149,11 @@ __global__ void __launch_bounds__(kPlanThreads) k_format_plan(const bmf_chunk_re
     }
 }
 
-// The chunk j of a tile: the largest j with prefix[j] <= tile (prefix
-// non-decreasing, prefix[n] > tile); that chunk has a tile.
-__device__ __forceinline__ int tile_chunk(const int64_t* __restrict__ prefix, int n, int64_t tile) {
-    int lo = 0, hi = n;
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (prefix[mid] <= tile) lo = mid;
-        else hi = mid;
-    }
-    return lo;
-}
-
+// A tile's chunk is found by each wave with 64 probes a round, its elements
+// load together.  Bound by HBM with many tiles (512 chunks, 730,000 vertices
+// and 4.3 M indices, 62 MB: 15.5 us), by the chain of the search otherwise; with
+// a binary search by every lane 26.
+template <int EACH>
 __global__ void __launch_bounds__(kFmtThreads) k_format(const bmf_chunk_result* __restrict__ R, int n,
                                                         const int64_t* __restrict__ tab, const float* __restrict__ pos,
                                                         const uint32_t* __restrict__ idx,
@@ -167,49 +167,74 @@ __global__ void __launch_bounds__(kFmtThreads) k_format(const bmf_chunk_result* 
     const int64_t VT = vt[n], IT = it[n];
     for (int64_t tile = blockIdx.x; tile < VT + IT; tile += gridDim.x) {
         if (tile < VT) {
-            const int j = tile_chunk(vt, n, tile);
+            // the largest j with vt[j] <= tile: that chunk has a tile
+            const int j = find_chunk_wave(vt, n, tile);
             const bmf_chunk_result r = R[j];
-            const int64_t v = (tile - vt[j]) * kFmtThreads + threadIdx.x;
-            if (v >= r.vertex_count) continue;
-            const int64_t src = r.vertex_offset + v, dst = dv[j] + v;
-            const float px = pos[3 * src], py = pos[3 * src + 1], pz = pos[3 * src + 2];
-            float* O = P.pos + 3 * dst;
-            if (P.space == BMF_SPACE_WORLD) {
-                const float mx = px * r.delta, my = py * r.delta, mz = pz * r.delta;
-                O[0] = mx + r.overlap_pos[0];
-                O[1] = my + r.overlap_pos[1];
-                O[2] = mz + r.overlap_pos[2];
-            } else {
-                O[0] = px;
-                O[1] = py;
-                O[2] = pz;
+            const int64_t v0 = (tile - vt[j]) * (kFmtThreads * EACH) + threadIdx.x, dst0 = dv[j];
+            float p[EACH][3];
+#pragma unroll
+            for (int k = 0; k < EACH; k++) {
+                const int64_t src = r.vertex_offset + min(v0 + k * kFmtThreads, (int64_t)r.vertex_count - 1);
+#pragma unroll
+                for (int c = 0; c < 3; c++) p[k][c] = pos[3 * src + c];
             }
-            if (P.colors == BMF_COLOR_WHITE) {
-                float* C = P.col + 3 * dst;
-                C[0] = 1.0f;
-                C[1] = 1.0f;
-                C[2] = 1.0f;
-            } else if (P.colors == BMF_COLOR_NOISE) {
-                const float nz = fbm_value(P.fo, P.ao, P.inv_norm, kColorOctaves, P.seed, px, py, pz) * 4.0f;
-                const float3 c = hsv_to_rgb(((nz + 1.0f) * 0.5f) * 360.0f, 0.72f, 1.0f);
-                float* C = P.col + 3 * dst;
-                C[0] = c.x;
-                C[1] = c.y;
-                C[2] = c.z;
-            }
-            if (P.normals) {
-                float* N = P.nrm + 3 * dst;
-                N[0] = nrm[3 * src];
-                N[1] = nrm[3 * src + 1];
-                N[2] = nrm[3 * src + 2];
+#pragma unroll 1
+            for (int k = 0; k < EACH; k++) {
+                const int64_t v = v0 + k * kFmtThreads;
+                if (v >= r.vertex_count) break;
+                float px = p[0][0], py = p[0][1], pz = p[0][2];
+#pragma unroll
+                for (int q = 1; q < EACH; q++) {
+                    px = q == k ? p[q][0] : px;
+                    py = q == k ? p[q][1] : py;
+                    pz = q == k ? p[q][2] : pz;
+                }
+                const int64_t src = r.vertex_offset + v, dst = dst0 + v;
+                float* O = P.pos + 3 * dst;
+                if (P.space == BMF_SPACE_WORLD) {
+                    const float mx = px * r.delta, my = py * r.delta, mz = pz * r.delta;
+                    O[0] = mx + r.overlap_pos[0];
+                    O[1] = my + r.overlap_pos[1];
+                    O[2] = mz + r.overlap_pos[2];
+                } else {
+                    O[0] = px;
+                    O[1] = py;
+                    O[2] = pz;
+                }
+                if (P.colors == BMF_COLOR_WHITE) {
+                    float* C = P.col + 3 * dst;
+                    C[0] = 1.0f;
+                    C[1] = 1.0f;
+                    C[2] = 1.0f;
+                } else if (P.colors == BMF_COLOR_NOISE) {
+                    const float nz = fbm_value(P.fo, P.ao, P.inv_norm, kColorOctaves, P.seed, px, py, pz) * 4.0f;
+                    const float3 c = hsv_to_rgb(((nz + 1.0f) * 0.5f) * 360.0f, 0.72f, 1.0f);
+                    float* C = P.col + 3 * dst;
+                    C[0] = c.x;
+                    C[1] = c.y;
+                    C[2] = c.z;
+                }
+                if (P.normals) {
+                    float* N = P.nrm + 3 * dst;
+                    N[0] = nrm[3 * src];
+                    N[1] = nrm[3 * src + 1];
+                    N[2] = nrm[3 * src + 2];
+                }
             }
         } else {
             const int64_t tt = tile - VT;
-            const int j = tile_chunk(it, n, tt);
-            const bmf_chunk_result r = R[j];
-            const int64_t i = (tt - it[j]) * kFmtThreads + threadIdx.x;
-            if (i >= r.index_count) continue;
-            P.idx[di[j] + i] = idx[r.index_offset + i] + (P.global ? (uint32_t)dv[j] : 0u);
+            const int j = find_chunk_wave(it, n, tt);
+            const int64_t i_off = R[j].index_offset, count = R[j].index_count;
+            const int64_t i0 = (tt - it[j]) * (kFmtThreads * EACH) + threadIdx.x, dst0 = di[j];
+            const uint32_t add = P.global ? (uint32_t)dv[j] : 0u;
+            uint32_t x[EACH];
+#pragma unroll
+            for (int k = 0; k < EACH; k++) x[k] = idx[i_off + min(i0 + k * kFmtThreads, count - 1)];
+#pragma unroll
+            for (int k = 0; k < EACH; k++) {
+                const int64_t i = i0 + k * kFmtThreads;
+                if (i < count) P.idx[dst0 + i] = x[k] + add;
+            }
         }
     }
 }
@@ -265,9 +290,11 @@ int bmf_format(bmf_ctx* c, const bmf_format_options* o, const bmf_vbo* out, int6
     hipStream_t s = c->stream;
     const int nn = std::max(n, 0);
     const int threads = std::min(kPlanThreads, std::max(64, (nn + 63) / 64 * 64));
-    hipLaunchKernelGGL(k_format_plan, dim3(1), dim3((unsigned)threads), 0, s, c->A.results, nn, c->d_fmt, c->m_fmt);
-    hipLaunchKernelGGL(k_format, dim3((unsigned)std::max(1, c->persistent_blocks)), dim3(kFmtThreads), 0, s,
-                       c->A.results, nn, c->d_fmt, c->A.pos, c->A.idx, c->A.nrm, P);
+    const bool many = nn >= kFmtMany && o->colors != BMF_COLOR_NOISE;
+    hipLaunchKernelGGL(k_format_plan, dim3(1), dim3((unsigned)threads), 0, s, c->A.results, nn,
+                       kFmtThreads * (many ? kFmtEach : 1), c->d_fmt, c->m_fmt);
+    hipLaunchKernelGGL(many ? k_format<kFmtEach> : k_format<1>, dim3((unsigned)std::max(1, c->persistent_blocks)),
+                       dim3(kFmtThreads), 0, s, c->A.results, nn, c->d_fmt, c->A.pos, c->A.idx, c->A.nrm, P);
     BMF_HIP(hipGetLastError());
     BMF_HIP(hipStreamSynchronize(s));
     if (vertices) *vertices = c->h_fmt[0];

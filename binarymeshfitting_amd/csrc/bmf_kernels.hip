@@ -1497,39 +1497,55 @@ __global__ void __launch_bounds__(kScanThreads) k_scan(Arenas A, int n) {
                     rc[r] += bc;
                 }
             }
-        if (tid == 0) {
-            // triangles: a vertex per edge; quads: a vertex per polygon, a
-            // quad (or two triangles) per edge
-            const bool quads = A.mesh_mode == BMF_MESH_QUADS;
-            const uint32_t V = quads ? tc : te, T = quads ? te * (A.quad_tris ? 2u : 1u) : tc;
-            M.V = (int32_t)V;
-            M.T = (int32_t)T;
-            M.contains_mesh = M.any_air && (M.any_solid || (dim % 32 != 0));
-            if (V > 0) {
-                const int64_t vo = (int64_t)atomicAdd(&A.ctr->v_bump, (unsigned long long)V);
-                const uint64_t ni = (uint64_t)M.ipp * T;
-                const int64_t io = (int64_t)atomicAdd(&A.ctr->i_bump, (unsigned long long)ni);
-                atomicAdd(&A.ctr->need_v, (unsigned long long)V);
-                atomicAdd(&A.ctr->need_i, (unsigned long long)ni);
-                if (vo + V > A.cap_vertices || io + (int64_t)ni > A.cap_indices) {
-                    M.status = BMF_ECAPACITY;
-                    A.ctr->overflow = 1;
-                }
-                M.v_off = vo;
-                M.i_off = io;
+        // triangles: a vertex per edge; quads: a vertex per polygon, a
+        // quad (or two triangles) per edge
+        const bool quads = A.mesh_mode == BMF_MESH_QUADS;
+        const uint32_t V = quads ? tc : te, T = quads ? te * (A.quad_tris ? 2u : 1u) : tc;
+        if (wave == 0) {
+            // the chunk's output range, a lane per counter so that the four
+            // additions and the map's turn take one round trip together
+            const uint64_t ni = (uint64_t)M.ipp * T;
+            unsigned long long got = 0;
+            if (V > 0 && lane < 4) {
+                unsigned long long* at = lane == 0   ? &A.ctr->v_bump
+                                         : lane == 1 ? &A.ctr->i_bump
+                                         : lane == 2 ? &A.ctr->need_v
+                                                     : &A.ctr->need_i;
+                got = atomicAdd(at, lane & 1 ? ni : (unsigned long long)V);
             }
-            write_result(A, j, M);
-            const bool on = smooths(M, A.normals);
+            int g = 0;
+            if (V > 0 && T > 0 && lane == 4) g = atomicAdd(&A.ctr->n_smooth, 1) & (kXcds - 1);
+            const int64_t vo = (int64_t)__shfl((long long)got, 0), io = (int64_t)__shfl((long long)got, 1);
+            g = __shfl(g, 4);
+            // every lane forms the record's new fields, lane 0 writes them
+            ChunkMeta m = M;
+            m.V = (int32_t)V;
+            m.T = (int32_t)T;
+            m.contains_mesh = m.any_air && (m.any_solid || (dim % 32 != 0));
+            if (V > 0) {
+                if (vo + V > A.cap_vertices || io + (int64_t)ni > A.cap_indices) m.status = BMF_ECAPACITY;
+                m.v_off = vo;
+                m.i_off = io;
+            }
+            const bool on = smooths(m, A.normals);
             const int vt = on ? (int)((V + kSmoothThreads - 1) / kSmoothThreads) : 0;
             const int tt = on ? (int)((T + kSmoothThreads - 1) / kSmoothThreads) : 0;
-            if (on) {
-                const int g = atomicAdd(&A.ctr->n_smooth, 1) & (kXcds - 1);
+            int at = 0;
+            if (on && lane < 2) at = atomicAdd(lane == 0 ? &A.ctr->xcd_vtiles[g] : &A.ctr->xcd_ttiles[g], lane == 0 ? vt : tt);
+            if (lane == 0) {
+                if (V > 0 && m.status == BMF_ECAPACITY) A.ctr->overflow = 1;
+                M.V = m.V;
+                M.T = m.T;
+                M.contains_mesh = m.contains_mesh;
+                M.status = m.status;
+                M.v_off = m.v_off;
+                M.i_off = m.i_off;
+                write_result(A, j, m);
                 s_map[0] = g;
-                s_map[1] = atomicAdd(&A.ctr->xcd_vtiles[g], vt);
-                s_map[2] = atomicAdd(&A.ctr->xcd_ttiles[g], tt);
+                s_map[3] = vt;
+                s_map[4] = tt;
             }
-            s_map[3] = vt;
-            s_map[4] = tt;
+            if (lane < 2) s_map[1 + lane] = at;
         }
         __syncthreads();
         const int vt = s_map[3], tt = s_map[4];

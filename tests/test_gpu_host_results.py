@@ -49,7 +49,14 @@ def test_format_takes_the_chunks_in_order(ctx, n):
     rc, V, I, pos, _, _, idx = ctx.format(space=capi.SPACE_GRID, colors=capi.COLOR_NONE, global_indices=True)
     capi.check(rc, "bmf_format")
     assert V == sum(len(p) for p, _ in meshes) and I == sum(len(i) for _, i in meshes)
+    rc, _, _, world, col, _, local = ctx.format(space=capi.SPACE_WORLD, colors=capi.COLOR_WHITE, global_indices=False)
+    capi.check(rc, "bmf_format")
     if meshes:
+        took = [r for r in ctx.results(n)[1] if r.vertex_count]
+        scale = np.repeat(np.array([r.delta for r in took], np.float32), [r.vertex_count for r in took])[:, None]
+        shift = np.repeat(np.array([list(r.overlap_pos) for r in took], np.float32), [r.vertex_count for r in took], 0)
+        assert np.array_equal(world, pos * scale + shift) and np.all(col == 1.0)
+        assert np.array_equal(local, np.concatenate([i for _, i in meshes]))
         first = np.cumsum([0] + [len(p) for p, _ in meshes])
         assert np.array_equal(pos, np.concatenate([p for p, _ in meshes]))
         assert np.array_equal(idx, np.concatenate([i + np.uint32(f) for (_, i), f in zip(meshes, first)]))
