@@ -309,7 +309,10 @@ int bmf_create(bmf_ctx** out, int device, const bmf_limits* lim) {
     // 512 64^3-cell chunks (89 us; 97 at 8, 94 at 16 and more) and on 64
     // chunks of CSG quads (150, 168, 155); the autotuner tries the others
     c->tune.row_blocks = c->cu_count * 10;
-    c->tune.smooth_blocks = 4 * c->persistent_blocks;
+    // twelve per CU: all the smoothing of 512 64^3-cell chunks 91 us, of 1,536
+    // chunks of uneven LOD, whose steps have few tiles, 54; at 4 per CU 97 and
+    // 53, at 16 90 and 56, at 32 93 and 68 (dispatching blocks without a tile)
+    c->tune.smooth_blocks = c->cu_count * 12;
     c->tune.row_split = -1;
     Arenas& A = c->A;
     const int64_t nc = lim->max_chunks;

@@ -467,9 +467,9 @@ __global__ void __launch_bounds__(kRowThreads) k_dmc_vertices(Arenas A) {
     ItemWindows& s = W.win;
     const bool qef = A.placement == BMF_PLACE_QEF && S->kind == BMF_SAMPLER_CSG;
     const bool tris = A.quad_tris != 0;
-    const int64_t total = A.ctr->total_items;
+    const int64_t total = read_const(&A.ctr->total_items);
     for (int64_t it = (int64_t)blockIdx.x * kWordWaves + wave; it < total; it += (int64_t)gridDim.x * kWordWaves) {
-        const int2 im = A.item_map[it];
+        const int2 im = read_const(A.item_map + it);
         const int chunk = uniform_int(im.x), w0 = uniform_int(im.y) * kItemWords;
         const ChunkMeta M = read_chunk(A.meta, chunk);
         if (M.status != BMF_OK || M.V == 0) continue;
@@ -572,7 +572,7 @@ __global__ void __launch_bounds__(kRowThreads) k_dmc_quads(Arenas A) {
     const int wave = uniform_int(threadIdx.x >> 6), lane = lane_id();
     ItemWindows& s = s_win[wave];
     const bool tris = A.quad_tris != 0;
-    const int64_t total = A.ctr->total_items;
+    const int64_t total = read_const(&A.ctr->total_items);
     for (int64_t it = (int64_t)blockIdx.x * kWordWaves + wave; it < total; it += (int64_t)gridDim.x * kWordWaves) {
         const ItemRef R = item_ref(A, it);
         const ChunkMeta& M = R.M;
@@ -665,17 +665,13 @@ __global__ void __launch_bounds__(kRowThreads) k_dmc_quads(Arenas A) {
 // chunk): ((0 + p0) + p1 ...) / N, the corner ids and then the corners
 // loaded together.  Tiles come from the per-frame tile map.
 __global__ void __launch_bounds__(kSmoothThreads) k_dual_n(Arenas A, int m) {
-    const int xcd = blockIdx.x % kXcds;
-    const int end = A.ctr->xcd_ttiles[xcd];
-    const int2* __restrict__ map = A.smooth_tmap + (int64_t)xcd * A.cap_ttiles;
-    for (int tile = blockIdx.x / kXcds; tile < end; tile += gridDim.x / kXcds) {
-        const int2 tm = map[tile];  // (chunk, tile within the chunk)
-        const ChunkMeta& M = A.meta[uniform_int(tm.x)];
-        const int iters = uniform_int(M.iters), N = uniform_int(M.ipp), T = uniform_int(M.T);
-        const uint32_t V = (uint32_t)uniform_int(M.V);
+    for (SmoothTiles tiles(A.smooth_tmap, A.cap_ttiles, A.ctr->xcd_ttiles); tiles.next();) {
+        const SmoothTile& M = tiles.t;
+        const int iters = M.iters, N = M.ipp, T = M.T;
+        const uint32_t V = (uint32_t)M.V;
         const int64_t i_off = M.i_off, v_off = M.v_off;
         if (iters <= m) continue;
-        const int64_t t = (int64_t)uniform_int(tm.y) * kSmoothThreads + threadIdx.x;
+        const int64_t t = (int64_t)M.tile * kSmoothThreads + threadIdx.x;
         if (t >= T) continue;
         const uint32_t* __restrict__ I = A.idx + i_off + (int64_t)N * t;
         const float4* __restrict__ P = A.pos4 + v_off;
@@ -701,7 +697,7 @@ __global__ void __launch_bounds__(kSmoothThreads) k_dual_n(Arenas A, int m) {
             cz = cz + d.z;
         }
         const float fn = (float)N;
-        A.cen4[i_off / N + t] = make_float4(cx / fn, cy / fn, cz / fn, 0.0f);
+        A.cen4[M.t_off + t] = make_float4(cx / fn, cy / fn, cz / fn, 0.0f);
     }
 }
 
@@ -710,23 +706,19 @@ __global__ void __launch_bounds__(kSmoothThreads) k_dual_n(Arenas A, int m) {
 // their centroids loaded per round.
 constexpr int kRingRoundN = 8;
 __global__ void __launch_bounds__(kSmoothThreads) k_primal_ring(Arenas A, int m) {
-    const int xcd = blockIdx.x % kXcds;
-    const int end = A.ctr->xcd_vtiles[xcd];
-    const int2* __restrict__ map = A.smooth_vmap + (int64_t)xcd * A.cap_vtiles;
     const int64_t cap = A.cap_vertices;
-    for (int tile = blockIdx.x / kXcds; tile < end; tile += gridDim.x / kXcds) {
-        const int2 tm = map[tile];  // (chunk, tile within the chunk)
-        const ChunkMeta& M = A.meta[uniform_int(tm.x)];
-        const int K = uniform_int(M.iters), N = uniform_int(M.ipp), V = uniform_int(M.V), bp = uniform_int(M.bp);
-        const int64_t i_off = M.i_off, v_off = M.v_off;
+    for (SmoothTiles tiles(A.smooth_vmap, A.cap_vtiles, A.ctr->xcd_vtiles); tiles.next();) {
+        const SmoothTile& M = tiles.t;
+        const int K = M.iters, V = M.V, bp = M.bp;
+        const int64_t v_off = M.v_off;
         if (K <= m) continue;
-        const int64_t v = (int64_t)uniform_int(tm.y) * kSmoothThreads + threadIdx.x;
+        const int64_t v = (int64_t)M.tile * kSmoothThreads + threadIdx.x;
         if (v >= V) continue;
         const int64_t g = v_off + v;
         const uint8_t bnd = A.boundary[g];
         const int n = (int)min(A.ring_n[g], (uint32_t)kRingSlots);
         if ((!bp && bnd) || n == 0) continue;
-        const float4* __restrict__ C = A.cen4 + i_off / N;
+        const float4* __restrict__ C = A.cen4 + M.t_off;
         float sx = 0.0f, sy = 0.0f, sz = 0.0f;
         for (int i0 = 0; i0 < n; i0 += kRingRoundN) {
             uint32_t id[kRingRoundN];
@@ -777,17 +769,13 @@ __device__ __forceinline__ float3 unit_cross(float ux, float uy, float uz, float
 }
 
 __global__ void __launch_bounds__(kSmoothThreads) k_dual_n_nrm(Arenas A, int m) {
-    const int xcd = blockIdx.x % kXcds;
-    const int end = A.ctr->xcd_ttiles[xcd];
-    const int2* __restrict__ map = A.smooth_tmap + (int64_t)xcd * A.cap_ttiles;
-    for (int tile = blockIdx.x / kXcds; tile < end; tile += gridDim.x / kXcds) {
-        const int2 tm = map[tile];  // (chunk, tile within the chunk)
-        const ChunkMeta& M = A.meta[uniform_int(tm.x)];
-        const int K = uniform_int(M.iters), N = uniform_int(M.ipp), T = uniform_int(M.T);
-        const uint32_t V = (uint32_t)uniform_int(M.V);
+    for (SmoothTiles tiles(A.smooth_tmap, A.cap_ttiles, A.ctr->xcd_ttiles); tiles.next();) {
+        const SmoothTile& M = tiles.t;
+        const int K = M.iters, N = M.ipp, T = M.T;
+        const uint32_t V = (uint32_t)M.V;
         const int64_t i_off = M.i_off, v_off = M.v_off;
         if (max(K, 1) <= m) continue;
-        const int64_t t = (int64_t)uniform_int(tm.y) * kSmoothThreads + threadIdx.x;
+        const int64_t t = (int64_t)M.tile * kSmoothThreads + threadIdx.x;
         if (t >= T) continue;
         // N = 3 or 4, one per chunk: the corner ids, then the corners, load
         // together (a triangle's fourth repeats its first)
@@ -809,7 +797,7 @@ __global__ void __launch_bounds__(kSmoothThreads) k_dual_n_nrm(Arenas A, int m) 
             cz = cz + q[c].z;
         }
         const float fN = (float)N;
-        const int64_t tt = i_off / N + t;
+        const int64_t tt = M.t_off + t;
         A.cen4[tt] = make_float4(cx / fN, cy / fN, cz / fN, 0.0f);
         const int max_norms = min(K / 2 - 3, 10);
         float4 fn;
@@ -855,25 +843,21 @@ __global__ void __launch_bounds__(kSmoothThreads) k_dual_n_nrm(Arenas A, int m) 
 // boundary vertices stay unless boundary processing (K > 0 only); the last
 // step writes the unit normal (0 for a zero normal).
 __global__ void __launch_bounds__(kSmoothThreads) k_primal_ring_nrm(Arenas A, int m) {
-    const int xcd = blockIdx.x % kXcds;
-    const int end = A.ctr->xcd_vtiles[xcd];
-    const int2* __restrict__ map = A.smooth_vmap + (int64_t)xcd * A.cap_vtiles;
     const int64_t cap = A.cap_vertices;
-    for (int tile = blockIdx.x / kXcds; tile < end; tile += gridDim.x / kXcds) {
-        const int2 tm = map[tile];  // (chunk, tile within the chunk)
-        const ChunkMeta& M = A.meta[uniform_int(tm.x)];
-        const int K = uniform_int(M.iters), N = uniform_int(M.ipp), V = uniform_int(M.V), bp = uniform_int(M.bp);
-        const int64_t i_off = M.i_off, v_off = M.v_off;
+    for (SmoothTiles tiles(A.smooth_vmap, A.cap_vtiles, A.ctr->xcd_vtiles); tiles.next();) {
+        const SmoothTile& M = tiles.t;
+        const int K = M.iters, V = M.V, bp = M.bp;
+        const int64_t v_off = M.v_off;
         const int steps = max(K, 1);
         if (steps <= m) continue;
-        const int64_t v = (int64_t)uniform_int(tm.y) * kSmoothThreads + threadIdx.x;
+        const int64_t v = (int64_t)M.tile * kSmoothThreads + threadIdx.x;
         if (v >= V) continue;
         const int64_t g = v_off + v;
         const uint8_t bnd = A.boundary[g];
         const int n = (int)min(A.ring_n[g], (uint32_t)kRingSlots);
         float4 nv = A.nrm4[g];
-        const float4* __restrict__ C = A.cen4 + i_off / N;
-        const float4* __restrict__ F = A.fn4 + i_off / N;
+        const float4* __restrict__ C = A.cen4 + M.t_off;
+        const float4* __restrict__ F = A.fn4 + M.t_off;
         if (n > 0) {
             float sx = 0.0f, sy = 0.0f, sz = 0.0f, nx = 0.0f, ny = 0.0f, nz = 0.0f;
             for (int i0 = 0; i0 < n; i0 += kRingRoundN) {

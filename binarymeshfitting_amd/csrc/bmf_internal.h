@@ -107,6 +107,18 @@ struct Counters {
     int64_t total_items;       // items of the word kernels
 };
 
+// A tile of a chunk's vertices or primitives in the smoothing: what its
+// kernels need of the chunk, so that a tile is one load and not a tour of the
+// chunk table.
+struct alignas(16) SmoothTile {
+    int32_t chunk, tile;
+    int32_t V, T;
+    int64_t v_off, i_off, t_off;  // first vertex, index and primitive (t_off = i_off / ipp)
+    int32_t iters;
+    uint8_t bp, ipp;
+    uint16_t dim;
+};
+
 // One label word's sign-changing edges per axis (in the quad mode only those
 // whose four cells lie in the chunk) and active cells, as bits of its samples.
 struct EdgeWord {
@@ -130,9 +142,8 @@ struct Arenas {
     int32_t stat_cap;
     int2* item_map;            // [max_items] (chunk, item within the chunk) of the word kernels' items
                                // (written by k_sample's prologue)
-    int2* smooth_vmap;         // [kXcds][cap_vtiles] (chunk, tile within the chunk) of the smoothing vertex
-                               // tiles of each XCD (k_scan)
-    int2* smooth_tmap;         // [kXcds][cap_ttiles] the same for the triangle tiles
+    SmoothTile* smooth_vmap;   // [kXcds][cap_vtiles] the smoothing's vertex tiles of each XCD (k_scan)
+    SmoothTile* smooth_tmap;   // [kXcds][cap_ttiles] the same for the triangle tiles
     int64_t cap_vtiles, cap_ttiles;
     EdgeWord* edges;           // same layout as labels: edge and active-cell bits of each word
     uint32_t* word_pre;        // same layout: edges of the item before the word

@@ -682,7 +682,7 @@ __global__ void __launch_bounds__(kRowThreads) k_terrain(Arenas A, int n) {
     }
     if (tid == 0) s_evals = 0;
     unsigned long long evals = 0;  // octaves this lane evaluated
-    const int64_t total = A.ctr->total_items;
+    const int64_t total = read_const(&A.ctr->total_items);
     // position and y - y0 of list entry v: wave << 10 | sample of its item
     auto locate = [&](uint32_t v, uint32_t& i, float& px, float& py, float& pz) {
         const Geom& g = s_geom[v >> 10];
@@ -1305,7 +1305,7 @@ __global__ void __launch_bounds__(kRowThreads) k_count(Arenas A) {
     const int wave = uniform_int(threadIdx.x >> 6), lane = lane_id(), q = lane & 3;
     uint16_t* const list = s_list[wave];
     unsigned long long evals = 0;  // octaves of this wave's refined samples (uniform)
-    const int64_t total = A.ctr->total_items;
+    const int64_t total = read_const(&A.ctr->total_items);
     for (int64_t it = (int64_t)blockIdx.x * kWordWaves + wave; it < total; it += (int64_t)gridDim.x * kWordWaves) {
         const ItemRef R = item_ref(A, it);
         const ChunkMeta& M = R.M;
@@ -1426,6 +1426,7 @@ constexpr int kScanThreads = 256;
 __global__ void __launch_bounds__(kScanThreads) k_scan(Arenas A, int n) {
     constexpr int NW = kScanThreads / 64;
     __shared__ uint32_t s_we[NW], s_wc[NW];  // wave totals
+    __shared__ SmoothTile s_tile;
     __shared__ int s_map[5];  // XCD, first vertex and triangle tile in its maps, their counts
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     for (int j = blockIdx.x; j < n; j += gridDim.x) {
@@ -1541,6 +1542,8 @@ __global__ void __launch_bounds__(kScanThreads) k_scan(Arenas A, int n) {
                 M.v_off = m.v_off;
                 M.i_off = m.i_off;
                 write_result(A, j, m);
+                s_tile = SmoothTile{j,        0, m.V, m.T, m.v_off, m.i_off, m.i_off / m.ipp,
+                                    m.iters, (uint8_t)m.bp, (uint8_t)m.ipp, (uint16_t)m.dim};
                 s_map[0] = g;
                 s_map[3] = vt;
                 s_map[4] = tt;
@@ -1550,10 +1553,17 @@ __global__ void __launch_bounds__(kScanThreads) k_scan(Arenas A, int n) {
         __syncthreads();
         const int vt = s_map[3], tt = s_map[4];
         if (vt) {
-            int2* __restrict__ VM = A.smooth_vmap + (int64_t)s_map[0] * A.cap_vtiles + s_map[1];
-            int2* __restrict__ TM = A.smooth_tmap + (int64_t)s_map[0] * A.cap_ttiles + s_map[2];
-            for (int r = tid; r < vt; r += kScanThreads) VM[r] = make_int2(j, r);
-            for (int r = tid; r < tt; r += kScanThreads) TM[r] = make_int2(j, r);
+            SmoothTile* __restrict__ VM = A.smooth_vmap + (int64_t)s_map[0] * A.cap_vtiles + s_map[1];
+            SmoothTile* __restrict__ TM = A.smooth_tmap + (int64_t)s_map[0] * A.cap_ttiles + s_map[2];
+            SmoothTile t = s_tile;
+            for (int r = tid; r < vt; r += kScanThreads) {
+                t.tile = r;
+                VM[r] = t;
+            }
+            for (int r = tid; r < tt; r += kScanThreads) {
+                t.tile = r;
+                TM[r] = t;
+            }
         }
         __syncthreads();
     }
@@ -1722,7 +1732,7 @@ __global__ void __launch_bounds__(kRowThreads) k_emit(Arenas A) {
     __syncthreads();
     const int wave = uniform_int(threadIdx.x >> 6);
     ItemWindows& s = s_win[wave];
-    const int64_t total = A.ctr->total_items;
+    const int64_t total = read_const(&A.ctr->total_items);
     for (int64_t it = (int64_t)blockIdx.x * kWordWaves + wave; it < total; it += (int64_t)gridDim.x * kWordWaves) {
         const ItemRef R = item_ref(A, it);
         const ChunkMeta& M = R.M;
@@ -1748,35 +1758,13 @@ __global__ void __launch_bounds__(kRowThreads) k_emit(Arenas A) {
 // by k_primal: k_dual has consumed them); the last iteration also writes the
 // float3 output.
 // ------------------------------------------------------------------------
-// The chunk fields a smoothing tile reads, loaded together and kept in
-// scalar registers: a tile, so its chunk, is the whole block's.
-struct SmoothChunk {
-    int iters, dim, bp, V, T;
-    int64_t v_off, i_off, dens_off;
-};
-__device__ __forceinline__ int64_t uniform_i64(int64_t v) {
-    const uint64_t u = (uint64_t)v;
-    return (int64_t)(((uint64_t)(uint32_t)uniform_int((int)(u >> 32)) << 32) | (uint32_t)uniform_int((int)(uint32_t)u));
-}
-__device__ __forceinline__ SmoothChunk smooth_chunk(const ChunkMeta& M) {
-    const int iters = M.iters, dim = M.dim, bp = M.bp, V = M.V, T = M.T;
-    const int64_t v_off = M.v_off, i_off = M.i_off, dens_off = M.dens_off;
-    return SmoothChunk{uniform_int(iters), uniform_int(dim), uniform_int(bp), uniform_int(V), uniform_int(T),
-                       uniform_i64(v_off), uniform_i64(i_off), uniform_i64(dens_off)};
-}
-
 __global__ void __launch_bounds__(kSmoothThreads) k_dual(Arenas A, int m) {
-    const int xcd = blockIdx.x % kXcds;
-    const int end = A.ctr->xcd_ttiles[xcd];
-    const int2* __restrict__ map = A.smooth_tmap + (int64_t)xcd * A.cap_ttiles;
-    for (int tile = blockIdx.x / kXcds; tile < end; tile += gridDim.x / kXcds) {
-        const int2 tm = map[tile];  // (chunk, tile within the chunk)
-        const int chunk = uniform_int(tm.x), ty = uniform_int(tm.y);
-        const SmoothChunk M = smooth_chunk(A.meta[chunk]);
+    for (SmoothTiles tiles(A.smooth_tmap, A.cap_ttiles, A.ctr->xcd_ttiles); tiles.next();) {
+        const SmoothTile& M = tiles.t;
         const int64_t T = M.T, i_off = M.i_off, v_off = M.v_off;
         const uint32_t V = (uint32_t)M.V;
         if (M.iters <= m) continue;
-        const int64_t t = (int64_t)ty * kSmoothThreads + threadIdx.x;
+        const int64_t t = (int64_t)M.tile * kSmoothThreads + threadIdx.x;
         if (t >= T) continue;
         const uint32_t* __restrict__ I = A.idx + i_off + 3 * t;
         const float4* __restrict__ P = A.pos4 + v_off;
@@ -1796,7 +1784,7 @@ __global__ void __launch_bounds__(kSmoothThreads) k_dual(Arenas A, int m) {
         cx = cx + c.x;
         cy = cy + c.y;
         cz = cz + c.z;
-        A.cen4[i_off / 3 + t] = make_float4(cx / 3.0f, cy / 3.0f, cz / 3.0f, 0.0f);
+        A.cen4[M.t_off + t] = make_float4(cx / 3.0f, cy / 3.0f, cz / 3.0f, 0.0f);
     }
 }
 
@@ -1889,18 +1877,13 @@ __device__ __forceinline__ uint32_t ring_sums(uint4 r, const float4* __restrict_
 }
 
 __global__ void __launch_bounds__(kSmoothThreads) k_primal(Arenas A, int m) {
-    const int xcd = blockIdx.x % kXcds;
-    const int end = A.ctr->xcd_vtiles[xcd];
-    const int2* __restrict__ map = A.smooth_vmap + (int64_t)xcd * A.cap_vtiles;
-    for (int tile = blockIdx.x / kXcds; tile < end; tile += gridDim.x / kXcds) {
-        const int2 tm = map[tile];  // (chunk, tile within the chunk)
-        const int chunk = uniform_int(tm.x), ty = uniform_int(tm.y);
-        const SmoothChunk M = smooth_chunk(A.meta[chunk]);
+    for (SmoothTiles tiles(A.smooth_vmap, A.cap_vtiles, A.ctr->xcd_vtiles); tiles.next();) {
+        const SmoothTile& M = tiles.t;
         const int K = M.iters, dim = M.dim, bp = M.bp;
-        const int64_t V = M.V, v_off = M.v_off, dens_off = M.dens_off, t_off = M.i_off / 3;
+        const int64_t V = M.V, v_off = M.v_off, t_off = M.t_off;
         const uint32_t T = (uint32_t)M.T;
         if (K <= m) continue;
-        const int64_t v = (int64_t)ty * kSmoothThreads + threadIdx.x;
+        const int64_t v = (int64_t)M.tile * kSmoothThreads + threadIdx.x;
         if (v >= V) continue;
         const int64_t g = v_off + v;
         // the boundary flag, the lattice edge and the packed ring load together
@@ -1910,6 +1893,7 @@ __global__ void __launch_bounds__(kSmoothThreads) k_primal(Arenas A, int m) {
         if (!bp && bnd) continue;  // stays at its position in both buffers
         if (m == 0) {
             bool bad = false;
+            const int64_t dens_off = A.meta[M.chunk].dens_off;
             r = pack_ring(A.cell_tb + dens_off, A.cell_mask + dens_off, code, dim, T, bad);
             if (bad) raise_error(A, 7);
         }
@@ -1949,16 +1933,11 @@ __global__ void __launch_bounds__(kSmoothThreads) k_primal(Arenas A, int m) {
 // its y is not 0; positions move as in k_dual/k_primal (K > 0 only); the
 // last step writes the unit normal.
 __global__ void __launch_bounds__(kSmoothThreads) k_dual_nrm(Arenas A, int m) {
-    const int xcd = blockIdx.x % kXcds;
-    const int end = A.ctr->xcd_ttiles[xcd];
-    const int2* __restrict__ map = A.smooth_tmap + (int64_t)xcd * A.cap_ttiles;
-    for (int tile = blockIdx.x / kXcds; tile < end; tile += gridDim.x / kXcds) {
-        const int2 tm = map[tile];  // (chunk, tile within the chunk)
-        const int chunk = uniform_int(tm.x), ty = uniform_int(tm.y);
-        const SmoothChunk M = smooth_chunk(A.meta[chunk]);
+    for (SmoothTiles tiles(A.smooth_tmap, A.cap_ttiles, A.ctr->xcd_ttiles); tiles.next();) {
+        const SmoothTile& M = tiles.t;
         const int K = M.iters;
         if (max(K, 1) <= m) continue;
-        const int64_t t = (int64_t)ty * kSmoothThreads + threadIdx.x;
+        const int64_t t = (int64_t)M.tile * kSmoothThreads + threadIdx.x;
         if (t >= M.T) continue;
         const uint32_t* __restrict__ I = A.idx + M.i_off + 3 * t;
         const float4* __restrict__ P = A.pos4 + M.v_off;
@@ -1978,7 +1957,7 @@ __global__ void __launch_bounds__(kSmoothThreads) k_dual_nrm(Arenas A, int m) {
         cx = cx + c.x;
         cy = cy + c.y;
         cz = cz + c.z;
-        const int64_t tt = M.i_off / 3 + t;
+        const int64_t tt = M.t_off + t;
         A.cen4[tt] = make_float4(cx / 3.0f, cy / 3.0f, cz / 3.0f, 0.0f);
         const int max_norms = min(K / 2 - 3, 10);
         float4 fn;
@@ -2013,24 +1992,20 @@ __global__ void __launch_bounds__(kSmoothThreads) k_dual_nrm(Arenas A, int m) {
 }
 
 __global__ void __launch_bounds__(kSmoothThreads) k_primal_nrm(Arenas A, int m) {
-    const int xcd = blockIdx.x % kXcds;
-    const int end = A.ctr->xcd_vtiles[xcd];
-    const int2* __restrict__ map = A.smooth_vmap + (int64_t)xcd * A.cap_vtiles;
-    for (int tile = blockIdx.x / kXcds; tile < end; tile += gridDim.x / kXcds) {
-        const int2 tm = map[tile];  // (chunk, tile within the chunk)
-        const int chunk = uniform_int(tm.x), ty = uniform_int(tm.y);
-        const SmoothChunk M = smooth_chunk(A.meta[chunk]);
+    for (SmoothTiles tiles(A.smooth_vmap, A.cap_vtiles, A.ctr->xcd_vtiles); tiles.next();) {
+        const SmoothTile& M = tiles.t;
         const int K = M.iters;
         const int steps = max(K, 1);
         if (steps <= m) continue;
-        const int64_t v = (int64_t)ty * kSmoothThreads + threadIdx.x;
+        const int64_t v = (int64_t)M.tile * kSmoothThreads + threadIdx.x;
         if (v >= M.V) continue;
-        const int64_t g = M.v_off + v, dens_off = M.dens_off, t_off = M.i_off / 3;
+        const int64_t g = M.v_off + v, t_off = M.t_off;
         const int dim = M.dim, bp = M.bp;
         const uint32_t T = (uint32_t)M.T;
         uint4 r;
         if (m == 0) {
             bool bad = false;
+            const int64_t dens_off = A.meta[M.chunk].dens_off;
             r = pack_ring(A.cell_tb + dens_off, A.cell_mask + dens_off, A.vedge[g], dim, T, bad);
             if (bad) raise_error(A, 7);
         } else {

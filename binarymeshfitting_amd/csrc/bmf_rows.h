@@ -16,23 +16,55 @@ __device__ __forceinline__ int lane_id() { return (int)(threadIdx.x & 63); }
 
 __device__ __forceinline__ int uniform_int(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
-// Chunk j of the chunk table (j wave-uniform), for kernels that never write
-// the table: read through the constant address space, its fields load with
-// scalar loads into scalar registers and are not reloaded after the
-// kernel's own stores (which the compiler cannot otherwise tell apart from
-// the table).
-__device__ __forceinline__ ChunkMeta read_chunk(const ChunkMeta* table, int j) {
-    static_assert(sizeof(ChunkMeta) % 4 == 0, "ChunkMeta is copied in 32-bit words");
-    constexpr int kWords = (int)(sizeof(ChunkMeta) / 4);
+// A record at a wave-uniform address that the kernel itself never writes:
+// read through the constant address space, so by scalar loads into scalar
+// registers, whose latency is the shorter, and not again after the kernel's
+// own stores (which the compiler cannot otherwise tell apart from it).
+template <class T>
+__device__ __forceinline__ T read_const(const T* p) {
+    static_assert(sizeof(T) % 4 == 0, "records are read in 32-bit words");
+    constexpr int kWords = (int)(sizeof(T) / 4);
     using ConstWords = const __attribute__((address_space(4))) uint32_t*;
-    const ConstWords src = (ConstWords)(table + uniform_int(j));
+    const ConstWords src = (ConstWords)p;
     uint32_t w[kWords];
 #pragma unroll
     for (int i = 0; i < kWords; i++) w[i] = src[i];
-    ChunkMeta m;
-    __builtin_memcpy(&m, w, sizeof(ChunkMeta));
-    return m;
+    T r;
+    __builtin_memcpy(&r, w, sizeof(T));
+    return r;
 }
+// Chunk j of the chunk table.
+__device__ __forceinline__ ChunkMeta read_chunk(const ChunkMeta* table, int j) {
+    return read_const(table + uniform_int(j));
+}
+
+// The smoothing tiles of a block: those of its XCD's map, the record loaded
+// beside the map's end.
+struct SmoothTiles {
+    const SmoothTile* map;
+    int tile, step, last, end;
+    SmoothTile t;
+    __device__ __forceinline__ SmoothTiles(const SmoothTile* maps, int64_t cap, const int32_t* ends) {
+        const int xcd = blockIdx.x % kXcds;
+        map = maps + (int64_t)xcd * cap;
+        tile = blockIdx.x / kXcds;
+        step = gridDim.x / kXcds;
+        last = (int)cap - 1;
+        end = read_const(ends + xcd);
+    }
+    __device__ __forceinline__ bool next() {
+        uint32_t w[sizeof(SmoothTile) / 4];
+        const SmoothTile r = read_const(map + min(tile, last));
+        __builtin_memcpy(w, &r, sizeof w);
+        // all of it at once: left alone, the loads follow the branches that use them
+#pragma unroll
+        for (int i = 0; i < (int)(sizeof w / 4); i++) asm volatile("" : "+s"(w[i]));
+        __builtin_memcpy(&t, w, sizeof w);
+        const bool in = tile < end;
+        tile += step;
+        return in;
+    }
+};
 
 // Counts and ids disagree, or a map entry is out of range: raised for the
 // host, and nothing is written past the chunk.

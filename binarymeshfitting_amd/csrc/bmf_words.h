@@ -198,7 +198,7 @@ struct ItemRef {
     ChunkMeta M;
 };
 __device__ __forceinline__ ItemRef item_ref(const Arenas& A, int64_t it) {
-    const int2 m = A.item_map[it];
+    const int2 m = read_const(A.item_map + it);
     return ItemRef{uniform_int(m.y) * kItemWords, read_chunk(A.meta, m.x)};
 }
 
