@@ -35,7 +35,7 @@ hipError_t dalloc(T** p, int64_t count) {
 
 void free_arenas(bmf_ctx* c) {
     Arenas& A = c->A;
-    void* ptrs[] = {A.meta,    A.descs,     A.results,  A.block_prefix, A.signs, A.plan_part, A.stat_blocks, A.item_map, A.smooth_vmap, A.smooth_tmap, A.edges, A.word_pre, A.item_e, A.item_c, A.cen4,
+    void* ptrs[] = {A.meta,    A.descs,     A.results,  A.block_prefix, A.signs, A.plan_part, A.stat_blocks, A.item_map, A.work, A.smooth_vmap, A.smooth_tmap, A.edges, A.word_pre, A.item_e, A.item_c, A.cen4,
                     A.dens,    A.labels,    A.exact, A.cell_tb,   A.cell_mask,
                     A.pos,     A.pos4,      A.boundary, A.vedge,       A.vring,        A.idx,          A.ctr,
                     A.sampler, c->d_spheres, c->d_boxes, A.ring, A.ring_n, A.qef_err, A.nrm4, A.fn4, A.nrm,
@@ -331,7 +331,7 @@ int bmf_create(bmf_ctx** out, int device, const bmf_limits* lim) {
          dalloc(&A.block_prefix, nc + 1) == hipSuccess && dalloc(&A.signs, lim->max_samples + 16) == hipSuccess &&
          dalloc(&A.plan_part, 8 * ((nc + 1023) / 1024) + 1) == hipSuccess &&
          dalloc(&A.stat_blocks, 3 * (int64_t)(64 * c->cu_count)) == hipSuccess &&
-         dalloc(&A.item_map, ni) == hipSuccess &&
+         dalloc(&A.item_map, ni) == hipSuccess && dalloc(&A.work, ni) == hipSuccess &&
          dalloc(&A.smooth_vmap, kXcds * A.cap_vtiles) == hipSuccess &&
          dalloc(&A.smooth_tmap, kXcds * A.cap_ttiles) == hipSuccess &&
          dalloc(&A.edges, nw) == hipSuccess && dalloc(&A.word_pre, nw) == hipSuccess &&

@@ -467,9 +467,9 @@ __global__ void __launch_bounds__(kRowThreads) k_dmc_vertices(Arenas A) {
     ItemWindows& s = W.win;
     const bool qef = A.placement == BMF_PLACE_QEF && S->kind == BMF_SAMPLER_CSG;
     const bool tris = A.quad_tris != 0;
-    const int64_t total = read_const(&A.ctr->total_items);
-    for (int64_t it = (int64_t)blockIdx.x * kWordWaves + wave; it < total; it += (int64_t)gridDim.x * kWordWaves) {
-        const int2 im = read_const(A.item_map + it);
+    const int total = read_const(&A.ctr->n_work);
+    for (int wi = blockIdx.x * kWordWaves + wave; wi < total; wi += gridDim.x * kWordWaves) {
+        const int2 im = read_const(A.work + wi);
         const int chunk = uniform_int(im.x), w0 = uniform_int(im.y) * kItemWords;
         const ChunkMeta M = read_chunk(A.meta, chunk);
         if (M.status != BMF_OK || M.V == 0) continue;
@@ -498,7 +498,7 @@ __global__ void __launch_bounds__(kRowThreads) k_dmc_vertices(Arenas A) {
         const int64_t vo = M.v_off;
         const uint32_t Vc = (uint32_t)M.V;
         const bool smooth = (M.iters > 0 || A.normals) && M.T > 0;  // the chunk runs the smoothing kernels
-        uint32_t vb = A.item_c[it];
+        uint32_t vb = A.item_c[M.item_slot + im.y];
         for (int e0 = 0; e0 < nc; e0 += 64) {
             // ---- the round's cells ----
             int pos = 0;
@@ -572,9 +572,9 @@ __global__ void __launch_bounds__(kRowThreads) k_dmc_quads(Arenas A) {
     const int wave = uniform_int(threadIdx.x >> 6), lane = lane_id();
     ItemWindows& s = s_win[wave];
     const bool tris = A.quad_tris != 0;
-    const int64_t total = read_const(&A.ctr->total_items);
-    for (int64_t it = (int64_t)blockIdx.x * kWordWaves + wave; it < total; it += (int64_t)gridDim.x * kWordWaves) {
-        const ItemRef R = item_ref(A, it);
+    const int total = read_const(&A.ctr->n_work);
+    for (int wi = blockIdx.x * kWordWaves + wave; wi < total; wi += gridDim.x * kWordWaves) {
+        const ItemRef R = work_ref(A, wi);
         const ChunkMeta& M = R.M;
         if (M.status != BMF_OK || M.T == 0) continue;
         const int dim = M.dim, d2 = dim * dim;

@@ -105,6 +105,7 @@ struct Counters {
     int32_t overflow;
     int32_t error;
     int64_t total_items;       // items of the word kernels
+    int32_t n_work;            // of these, the ones with edges or cells
 };
 
 // A tile of a chunk's vertices or primitives in the smoothing: what its
@@ -142,6 +143,8 @@ struct Arenas {
     int32_t stat_cap;
     int2* item_map;            // [max_items] (chunk, item within the chunk) of the word kernels' items
                                // (written by k_sample's prologue)
+    int2* work;                // [max_items] (chunk, item within the chunk) of the items with edges or cells, a
+                               // chunk's in order (k_scan): what the emission takes
     SmoothTile* smooth_vmap;   // [kXcds][cap_vtiles] the smoothing's vertex tiles of each XCD (k_scan)
     SmoothTile* smooth_tmap;   // [kXcds][cap_ttiles] the same for the triangle tiles
     int64_t cap_vtiles, cap_ttiles;

@@ -229,6 +229,7 @@ __device__ __forceinline__ void plan_counters(const Arenas& A, int n, const int6
     if (overflow) c->overflow = 1;
     c->total_items = overflow ? 0 : tot[2];
     c->n_smooth = 0;
+    c->n_work = 0;
     for (int g = 0; g < kXcds; g++) c->xcd_vtiles[g] = c->xcd_ttiles[g] = 0;
     c->total_samples = tot[0];
 }
@@ -1425,7 +1426,11 @@ constexpr int kScanThreads = 256;
 
 __global__ void __launch_bounds__(kScanThreads) k_scan(Arenas A, int n) {
     constexpr int NW = kScanThreads / 64;
-    __shared__ uint32_t s_we[NW], s_wc[NW];  // wave totals
+    // a chunk's tiles of 64 items, and the items of each that have edges or cells
+    constexpr int kTiles = (BMF_MAX_DIM * BMF_MAX_DIM * BMF_MAX_DIM / kItemSamples + 63) / 64;
+    __shared__ uint64_t s_some[kTiles];
+    __shared__ uint32_t s_we[NW], s_wc[NW], s_wn[NW];  // wave totals
+    __shared__ int s_work;                             // the chunk's first entry of the work list
     __shared__ SmoothTile s_tile;
     __shared__ int s_map[5];  // XCD, first vertex and triangle tile in its maps, their counts
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1443,7 +1448,7 @@ __global__ void __launch_bounds__(kScanThreads) k_scan(Arenas A, int n) {
         const int64_t ntile = (R + 63) / 64;
         const int64_t tpw = (ntile + NW - 1) / NW;
         const int64_t t0 = (int64_t)wave * tpw, t1 = t0 + tpw < ntile ? t0 + tpw : ntile;
-        uint32_t we = 0, wc = 0;  // running totals of this wave's run
+        uint32_t we = 0, wc = 0, wn = 0;  // running totals of this wave's run
         for (int64_t tg = t0; tg < t1; tg += 4) {
             uint32_t ae[4], ac[4];
 #pragma unroll
@@ -1456,39 +1461,37 @@ __global__ void __launch_bounds__(kScanThreads) k_scan(Arenas A, int n) {
 #pragma unroll
             for (int k = 0; k < 4; k++) {
                 if (tg + k >= t1) break;
-                uint32_t se = ae[k], sc = ac[k];
-#pragma unroll
-                for (int off = 1; off < 64; off <<= 1) {
-                    const uint32_t ue = __shfl_up(se, off), uc = __shfl_up(sc, off);
-                    if (lane >= off) {
-                        se += ue;
-                        sc += uc;
-                    }
-                }
+                const uint32_t se = wave_scan(ae[k]), sc = wave_scan(ac[k]);
                 const int64_t r = (tg + k) * 64 + lane;
                 if (r < R) {
                     re[r] = we + se - ae[k];
                     rc[r] = wc + sc - ac[k];
                 }
-                we += (uint32_t)__shfl(se, 63);
-                wc += (uint32_t)__shfl(sc, 63);
+                we += (uint32_t)__builtin_amdgcn_readlane((int)se, 63);
+                wc += (uint32_t)__builtin_amdgcn_readlane((int)sc, 63);
+                const uint64_t some = __ballot((ae[k] | ac[k]) != 0u);
+                wn += (uint32_t)__popcll(some);
+                if (lane == 0) s_some[tg + k] = some;
             }
         }
         if (lane == 0) {
             s_we[wave] = we;
             s_wc[wave] = wc;
+            s_wn[wave] = wn;
         }
         __syncthreads();
-        uint32_t be = 0, bc = 0, te = 0, tc = 0;
+        uint32_t be = 0, bc = 0, bn = 0, te = 0, tc = 0, tn = 0;
 #pragma unroll
         for (int w = 0; w < NW; w++) {
-            const uint32_t xe = s_we[w], xc = s_wc[w];
+            const uint32_t xe = s_we[w], xc = s_wc[w], xn = s_wn[w];
             if (w < wave) {
                 be += xe;
                 bc += xc;
+                bn += xn;
             }
             te += xe;
             tc += xc;
+            tn += xn;
         }
         if (be | bc)
             for (int64_t t = t0; t < t1; t++) {
@@ -1504,7 +1507,8 @@ __global__ void __launch_bounds__(kScanThreads) k_scan(Arenas A, int n) {
         const uint32_t V = quads ? tc : te, T = quads ? te * (A.quad_tris ? 2u : 1u) : tc;
         if (wave == 0) {
             // the chunk's output range, a lane per counter so that the four
-            // additions and the map's turn take one round trip together
+            // additions, the map's turn and the work list's room take one
+            // round trip together
             const uint64_t ni = (uint64_t)M.ipp * T;
             unsigned long long got = 0;
             if (V > 0 && lane < 4) {
@@ -1516,7 +1520,9 @@ __global__ void __launch_bounds__(kScanThreads) k_scan(Arenas A, int n) {
             }
             int g = 0;
             if (V > 0 && T > 0 && lane == 4) g = atomicAdd(&A.ctr->n_smooth, 1) & (kXcds - 1);
+            if (lane == 5 && tn) g = atomicAdd(&A.ctr->n_work, (int)tn);
             const int64_t vo = (int64_t)__shfl((long long)got, 0), io = (int64_t)__shfl((long long)got, 1);
+            const int work = __shfl(g, 5);
             g = __shfl(g, 4);
             // every lane forms the record's new fields, lane 0 writes them
             ChunkMeta m = M;
@@ -1544,6 +1550,7 @@ __global__ void __launch_bounds__(kScanThreads) k_scan(Arenas A, int n) {
                 write_result(A, j, m);
                 s_tile = SmoothTile{j,        0, m.V, m.T, m.v_off, m.i_off, m.i_off / m.ipp,
                                     m.iters, (uint8_t)m.bp, (uint8_t)m.ipp, (uint16_t)m.dim};
+                s_work = work;
                 s_map[0] = g;
                 s_map[3] = vt;
                 s_map[4] = tt;
@@ -1551,6 +1558,12 @@ __global__ void __launch_bounds__(kScanThreads) k_scan(Arenas A, int n) {
             if (lane < 2) s_map[1 + lane] = at;
         }
         __syncthreads();
+        int at = s_work + (int)bn;
+        for (int64_t t = t0; t < t1; t++) {
+            const uint64_t some = s_some[t];
+            if ((some >> lane) & 1ull) A.work[at + (int)mbcnt64(some)] = make_int2(j, (int)(t * 64) + lane);
+            at += (int)__popcll(some);
+        }
         const int vt = s_map[3], tt = s_map[4];
         if (vt) {
             SmoothTile* __restrict__ VM = A.smooth_vmap + (int64_t)s_map[0] * A.cap_vtiles + s_map[1];
@@ -1732,15 +1745,15 @@ __global__ void __launch_bounds__(kRowThreads) k_emit(Arenas A) {
     __syncthreads();
     const int wave = uniform_int(threadIdx.x >> 6);
     ItemWindows& s = s_win[wave];
-    const int64_t total = read_const(&A.ctr->total_items);
-    for (int64_t it = (int64_t)blockIdx.x * kWordWaves + wave; it < total; it += (int64_t)gridDim.x * kWordWaves) {
-        const ItemRef R = item_ref(A, it);
+    const int total = read_const(&A.ctr->n_work);
+    for (int w = blockIdx.x * kWordWaves + wave; w < total; w += gridDim.x * kWordWaves) {
+        const ItemRef R = work_ref(A, w);
         const ChunkMeta& M = R.M;
         if (M.status != BMF_OK || M.V == 0) continue;
         const WindowGeom g = stage_windows(A, M, R.w0, s);
         emit_vertices(A, M, s, R.w0);
         wave_sync();  // the sample list is read
-        emit_triangles(A, M, s, g, s_ntri, s_tri, R.w0, A.item_c[it]);
+        emit_triangles(A, M, s, g, s_ntri, s_tri, R.w0, A.item_c[R.it]);
         wave_sync();  // the windows are read
     }
 }

@@ -194,12 +194,21 @@ __device__ __forceinline__ uint32_t window_edge(const ItemWindows& s, const Wind
 
 // (chunk, item within the chunk) of work item `it`, and the chunk's record.
 struct ItemRef {
-    int w0;  // the item's first word
+    int64_t it;  // the item
+    int w0;      // its first word
     ChunkMeta M;
 };
 __device__ __forceinline__ ItemRef item_ref(const Arenas& A, int64_t it) {
     const int2 m = read_const(A.item_map + it);
-    return ItemRef{uniform_int(m.y) * kItemWords, read_chunk(A.meta, m.x)};
+    return ItemRef{it, uniform_int(m.y) * kItemWords, read_chunk(A.meta, m.x)};
+}
+// Entry w of the list of items with edges or cells.
+__device__ __forceinline__ ItemRef work_ref(const Arenas& A, int w) {
+    const int2 m = read_const(A.work + w);
+    const int item = uniform_int(m.y);
+    ItemRef r{0, item * kItemWords, read_chunk(A.meta, m.x)};
+    r.it = r.M.item_slot + item;
+    return r;
 }
 
 }  // namespace bmf
