@@ -332,6 +332,38 @@ __global__ void k_bwd_init(const float* __restrict__ g3, int V, const uint8_t* _
     g[v] = make_float4(g3[3 * v] * sc, g3[3 * v + 1] * sc, g3[3 * v + 2] * sc, scaled ? (float)mv[v] : 0.0f);
 }
 
+// A round of ring records and the other corners' data.  A transposed step is
+// bound by latency (a mesh of 44,392 vertices is 0.7 waves per SIMD), so a
+// round's records load beside the vertex's own data, before its ring size is
+// known (slots past it hold anything and are not used), and their corners
+// together: two round trips, where a loop over the ring takes two for every four
+// records and the remainder one by one (4.6 us, this 4.0; the smoothing step,
+// whose arithmetic is four times that, gains nothing by it).
+constexpr int kStepRound = 8;
+struct RingRound {
+    uint2 e[kStepRound];
+    __device__ __forceinline__ void load(const uint2* __restrict__ ring, int stride, int k0, int v) {
+#pragma unroll
+        for (int k = 0; k < kStepRound; k++) e[k] = ring[(int64_t)(k0 + k < kMaxRing ? k0 + k : k0) * stride + v];
+    }
+    // the two other corners of each of the records before the n-th, v's own
+    // value for the others
+    __device__ __forceinline__ void corners(const float4* __restrict__ in, int left, int v, float4 (&a)[kStepRound],
+                                            float4 (&b)[kStepRound]) const {
+#pragma unroll
+        for (int k = 0; k < kStepRound; k++) {
+            a[k] = in[k < left ? e[k].x & kVidMask : (uint32_t)v];
+            b[k] = in[k < left ? e[k].y : (uint32_t)v];
+        }
+        // all of them at once: left alone, loads move behind the selects that use them
+#pragma unroll
+        for (int k = 0; k < kStepRound; k++) {
+            asm volatile("" : "+v"(a[k].x), "+v"(a[k].y), "+v"(a[k].z), "+v"(a[k].w));
+            asm volatile("" : "+v"(b[k].x), "+v"(b[k].y), "+v"(b[k].z), "+v"(b[k].w));
+        }
+    }
+};
+
 // One transposed smoothing iteration.  The forward step is
 // p'_u = [u not moved] p_u + [u moved] / (3 |ring(u)|) * (sum over the
 // triangles of ring(u) of their corners), so
@@ -351,23 +383,29 @@ __global__ void __launch_bounds__(kStepThreads) k_bwd_step(const uint2* __restri
                                                            float4* __restrict__ out) {
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
     if (v >= V) return;
+    RingRound R;
+    R.load(ring, stride, 0, v);
     const int n = deg[v];
     const bool moved = mv[v] != 0;
     const float4 own = in[v];
+    const float scale = bscale[v];
     const float ms = moved ? (float)n : 1.0f;
     float sx = ms * own.x, sy = ms * own.y, sz = ms * own.z;
-#pragma unroll 4
-    for (int k = 0; k < n; k++) {
-        const uint2 e = ring[(int64_t)k * stride + v];
-        const float4 a = in[e.x & kVidMask], b = in[e.y];
-        sx = __builtin_fmaf(a.w, a.x, sx);
-        sy = __builtin_fmaf(a.w, a.y, sy);
-        sz = __builtin_fmaf(a.w, a.z, sz);
-        sx = __builtin_fmaf(b.w, b.x, sx);
-        sy = __builtin_fmaf(b.w, b.y, sy);
-        sz = __builtin_fmaf(b.w, b.z, sz);
+    for (int k0 = 0; k0 < n; k0 += kStepRound) {
+        if (k0) R.load(ring, stride, k0, v);
+        float4 a[kStepRound], b[kStepRound];
+        R.corners(in, n - k0, v, a, b);
+#pragma unroll
+        for (int k = 0; k < kStepRound; k++) {
+            const bool ok = k0 + k < n;
+            const float tx = __builtin_fmaf(a[k].w, a[k].x, sx), ty = __builtin_fmaf(a[k].w, a[k].y, sy),
+                        tz = __builtin_fmaf(a[k].w, a[k].z, sz);
+            sx = ok ? __builtin_fmaf(b[k].w, b[k].x, tx) : sx;
+            sy = ok ? __builtin_fmaf(b[k].w, b[k].y, ty) : sy;
+            sz = ok ? __builtin_fmaf(b[k].w, b[k].z, tz) : sz;
+        }
     }
-    const float sc = last ? 1.0f : bscale[v];
+    const float sc = last ? 1.0f : scale;
     out[v] = make_float4(sx * sc, sy * sc, sz * sc, moved ? 1.0f : 0.0f);
 }
 
