@@ -964,7 +964,9 @@ __device__ __forceinline__ void warp_octave(float x, float y, float z, uint32_t 
 
 // The octave of the fractal from which k_field decides no more signs (see
 // there): a sample step changes octave o by about a_o f_o times the step of
-// its argument, times a noise gradient of about 2.
+// its argument, times a noise gradient of about 2.  Down to one such step,
+// two or four, the batch above with its meshing and formatting takes 300, 288
+// and 289 us.
 __device__ __forceinline__ int field_end(const SamplerDev& S, float delta) {
     float step = 0.0f;
     for (int o = 0; o < S.octaves; o++) step += fabsf(S.ao[o] * S.fo[o]);
