@@ -72,8 +72,8 @@ int enqueue_pipeline(bmf_ctx* c, const Arenas& A, int n, int maxk, int allow_cul
     BMF_MARK(3);
     BMF_HIP(launch_scan(A, n, scan_blocks, s));
     BMF_MARK(4);
-    if (quads) BMF_HIP(launch_dmc_emit(A, row_blocks, s));
-    else BMF_HIP(launch_emit(A, row_blocks, s));
+    if (quads) BMF_HIP(launch_dmc_emit(A, n, row_blocks, s));
+    else BMF_HIP(launch_emit(A, n, row_blocks, s));
     BMF_MARK(5);
     for (int m = 0; m < maxk; m++) {
         if (quads) BMF_HIP(launch_dmc_smooth(A, m, smooth_blocks, s));

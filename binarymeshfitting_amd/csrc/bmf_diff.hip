@@ -1365,7 +1365,7 @@ int bmf_forward_diff(bmf_ctx* c, const bmf_chunk_desc* d, const float* densities
                           !densities && c->h_sampler.noise_dims == 2, s);
     if (e == hipSuccess) e = launch_count(A, word_blocks(dim), 0, s);
     if (e == hipSuccess) e = launch_scan(A, 1, 1, s);
-    if (e == hipSuccess) e = launch_emit(A, word_blocks(dim), s);
+    if (e == hipSuccess) e = launch_emit(A, 1, word_blocks(dim), s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) return BMF_EHIP;
     const bmf_chunk_result r = c->h_results[0];

@@ -455,11 +455,11 @@ __device__ void place_vertex(const Arenas& A, const ChunkMeta& M, const SamplerD
     }
 }
 
-__global__ void __launch_bounds__(kRowThreads) k_dmc_vertices(Arenas A) {
+__global__ void __launch_bounds__(kRowThreads) k_dmc_vertices(Arenas A, int n) {
     __shared__ DmcTables s_t;
     __shared__ DmcWave s_wave[kWordWaves];
     load_dmc_tables(s_t);
-    if (blockIdx.x == 0 && threadIdx.x == 0) publish_counters(A);
+    publish(A, n);
     __syncthreads();
     const SamplerDev* __restrict__ S = A.sampler;
     const int wave = uniform_int(threadIdx.x >> 6), lane = lane_id();
@@ -919,9 +919,9 @@ __global__ void __launch_bounds__(kSmoothThreads) k_primal_ring_nrm(Arenas A, in
 // launch wrappers
 // ------------------------------------------------------------------------
 
-hipError_t launch_dmc_emit(const Arenas& A, int blocks, hipStream_t s) {
+hipError_t launch_dmc_emit(const Arenas& A, int n, int blocks, hipStream_t s) {
     // the vertices, then the quads that index them
-    hipLaunchKernelGGL(k_dmc_vertices, dim3(blocks), dim3(kRowThreads), 0, s, A);
+    hipLaunchKernelGGL(k_dmc_vertices, dim3(blocks), dim3(kRowThreads), 0, s, A, n);
     hipLaunchKernelGGL(k_dmc_quads, dim3(blocks), dim3(kRowThreads), 0, s, A);
     return hipGetLastError();
 }

@@ -165,9 +165,8 @@ struct Arenas {
     uint4* vring;              // [max_vertices] ring cells of each vertex, packed by the first smoothing step
     uint32_t* idx;             // [max_indices]
     Counters* ctr;
-    // The host's copies, in pinned memory that the kernels write: a result per
-    // chunk when its record is final, the counters by the emit kernel, the
-    // error flag where it is raised.  Two copies after the pipeline took 4 us of
+    // The host's copies, in pinned memory that the kernels write: the results
+    // and counters by the emit kernel, the error flag where it is raised.  Two copies after the pipeline took 4 us of
     // the device and 10 of the calling thread.
     bmf_chunk_result* host_results;  // [max_chunks]
     Counters* host_ctr;
@@ -228,11 +227,11 @@ hipError_t launch_sample(const Arenas& A, int n, int blocks, int adaptive, int k
 // refine: give early-labelled edge endpoints their full density (after an adaptive terrain launch_sample)
 hipError_t launch_count(const Arenas& A, int blocks, int refine, hipStream_t s);
 hipError_t launch_scan(const Arenas& A, int n, int blocks, hipStream_t s);
-hipError_t launch_emit(const Arenas& A, int blocks, hipStream_t s);
+hipError_t launch_emit(const Arenas& A, int n, int blocks, hipStream_t s);
 hipError_t launch_smooth(const Arenas& A, int m, int blocks, hipStream_t s);
 // Quad mode (bmf_dmc.hip): emission after launch_count / launch_scan,
 // smoothing over the per-vertex rings.
-hipError_t launch_dmc_emit(const Arenas& A, int blocks, hipStream_t s);
+hipError_t launch_dmc_emit(const Arenas& A, int n, int blocks, hipStream_t s);
 hipError_t launch_dmc_smooth(const Arenas& A, int m, int blocks, hipStream_t s);
 hipError_t launch_ref_labels(const Arenas& A, uint32_t* words, hipStream_t s);
 hipError_t launch_ref_masks(const Arenas& A, uint64_t* masks, hipStream_t s);

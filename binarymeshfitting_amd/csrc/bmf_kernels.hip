@@ -58,7 +58,6 @@ __device__ __forceinline__ void write_result(const Arenas& A, int j, const Chunk
     r.overlap_pos[1] = M.opos[1];
     r.overlap_pos[2] = M.opos[2];
     A.results[j] = r;
-    A.host_results[j] = r;
 }
 
 // a[i] of a register array by unrolled selects (a runtime index into a
@@ -1735,7 +1734,7 @@ __device__ __forceinline__ void emit_triangles(const Arenas& A, const ChunkMeta&
     }
 }
 
-__global__ void __launch_bounds__(kRowThreads) k_emit(Arenas A) {
+__global__ void __launch_bounds__(kRowThreads) k_emit(Arenas A, int n) {
     __shared__ ItemWindows s_win[kWordWaves];
     __shared__ uint64_t s_tri[256];  // the triangle table
     __shared__ uint8_t s_ntri[256];
@@ -1743,7 +1742,7 @@ __global__ void __launch_bounds__(kRowThreads) k_emit(Arenas A) {
         s_tri[t] = c_tri_table[t];
         s_ntri[t] = (uint8_t)((c_tri_table[t] >> 60) / 3);
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) publish_counters(A);
+    publish(A, n);
     __syncthreads();
     const int wave = uniform_int(threadIdx.x >> 6);
     ItemWindows& s = s_win[wave];
@@ -2185,8 +2184,8 @@ hipError_t launch_scan(const Arenas& A, int n, int blocks, hipStream_t s) {
     hipLaunchKernelGGL(k_scan, dim3(blocks), dim3(kScanThreads), 0, s, A, n);
     return hipGetLastError();
 }
-hipError_t launch_emit(const Arenas& A, int blocks, hipStream_t s) {
-    hipLaunchKernelGGL(k_emit, dim3(blocks), dim3(kRowThreads), 0, s, A);
+hipError_t launch_emit(const Arenas& A, int n, int blocks, hipStream_t s) {
+    hipLaunchKernelGGL(k_emit, dim3(blocks), dim3(kRowThreads), 0, s, A, n);
     return hipGetLastError();
 }
 hipError_t launch_smooth(const Arenas& A, int m, int blocks, hipStream_t s) {
