@@ -46,7 +46,7 @@ def parse():
     ap.add_argument("--lod-class", type=int, default=0, choices=(0, 1, 2, 3),
                     help="restrict the uneven-LOD leg to the chunks whose label rows take W u64 words "
                          "(W = ceil(dim / 64): 1 for 33^3, 2 for 65^3, 3 for 129^3 samples), so that the frame "
-                         "forks no row-word classes onto auxiliary streams; 0 = all chunks")
+                         "holds one size of chunk; 0 = all chunks")
     ap.add_argument("--world-steps", type=int, default=10,
                     help="timed batched steps of the default-world leg (0 skips it)")
     ap.add_argument("--hermite-steps", type=int, default=5,
@@ -563,7 +563,7 @@ def main():
         except (ValueError, OSError):
             traffic = None
     roof = {
-        "kernel": "k_sample",
+        "kernel": "k_blocks + k_terrain",
         "bound": "valu",
         "achieved": round(achieved_tflops, 3),
         "peak": roofline.PEAK_FP32_TFLOPS,
@@ -574,8 +574,8 @@ def main():
         "algorithmic_flops_per_launch": flops,
         "algorithmic_bytes_per_launch": int(samples * roofline.LABEL_BYTES),
         "avg_launch_ms": round(stages["sample"], 4),
-        # what the kernel executed: the adaptive evaluation stops a sample's octaves once its
-        # sign is decided (octaves counted by the kernel itself), against the FP32 peak
+        # what the kernels executed: block centres, and a sample's octaves until its sign is
+        # decided (octaves counted by the kernels themselves), against the FP32 peak
         # without packed math (the kernels are built without v_pk_* FP32 instructions)
         "executed": {"octave_evals": work["octave_evals"], "samples": work["samples"],
                      "octaves_per_sample": round(work["octave_evals"] / max(1, work["samples"]), 4),

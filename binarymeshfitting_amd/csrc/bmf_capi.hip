@@ -150,7 +150,7 @@ int build_sampler(const bmf_sampler_desc* s, SamplerDev* out) {
         }
         if (!(norm > 0.0f) || !finite(norm)) return BMF_EINVAL;
         d.inv_norm = 1.0f / norm;
-        // adaptive-octave bounds (k_sample decide_label)
+        // adaptive-octave bounds (decide_label)
         double total = 0.0;
         for (int o = 0; o < s->octaves; o++) total += std::fabs((double)d.ao[o]);
         const double ulp_total = total * std::ldexp(1.0, -23);

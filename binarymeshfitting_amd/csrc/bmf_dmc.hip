@@ -374,7 +374,7 @@ struct DmcWave {
 // chunks that smooth, writes its ring.  QEF placement is bound by the
 // normals (a pass over the primitives per edge point): the item's own list
 // keeps the few that can win.  64 chunks of 64^3 cells, 300 primitives,
-// 326,882 vertices: 114 us, with the plane's rows and the chunk's list 169.
+// 326,882 vertices: 110 us, with the plane's rows and the chunk's list 169.
 // ------------------------------------------------------------------------
 __device__ void place_vertex(const Arenas& A, const ChunkMeta& M, const SamplerDev& S, const uint16_t* csg,
                              const float4* s_csg, int ns, int nb, int x, int y, int z, int p, uint32_t mask, bool qef,
@@ -562,7 +562,7 @@ __global__ void __launch_bounds__(kRowThreads) k_dmc_vertices(Arenas A, int n) {
 
 // ------------------------------------------------------------------------
 // quads around the interior sign-changing edges, a wave per item, a lane per
-// sample that owns some (the batch above: 20 us, with a wave per row 71)
+// sample that owns some (the batch above: 18 us, with a wave per row 71)
 // ------------------------------------------------------------------------
 __global__ void __launch_bounds__(kRowThreads) k_dmc_quads(Arenas A) {
     __shared__ DmcTables s_t;

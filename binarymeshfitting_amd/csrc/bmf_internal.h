@@ -142,7 +142,7 @@ struct Arenas {
                                       // sampling, refinement and block kernels (plain stores, no atomics)
     int32_t stat_cap;
     int2* item_map;            // [max_items] (chunk, item within the chunk) of the word kernels' items
-                               // (written by k_sample's prologue)
+                               // (written by the sampling)
     int2* work;                // [max_items] (chunk, item within the chunk) of the items with edges or cells, a
                                // chunk's in order (k_scan): what the emission takes
     SmoothTile* smooth_vmap;   // [kXcds][cap_vtiles] the smoothing's vertex tiles of each XCD (k_scan)

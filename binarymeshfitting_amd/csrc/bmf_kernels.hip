@@ -2,7 +2,8 @@
 //
 // Per batch:  plan -> sample -> count -> scan -> emit -> smooth
 // (the per-chunk results are written by plan for culled or skipped chunks
-// and by scan for sampled ones, so no launch follows the smoothing)
+// and by scan for sampled ones, and go to the host with the emission, so no
+// launch and no copy follows the smoothing)
 //
 // Data layout in HBM (per sampled chunk, offsets from the plan kernel):
 //   densities   FP32 [x][y][z]                    (DMCChunk density_block)
@@ -381,8 +382,8 @@ __global__ void __launch_bounds__(256) k_csg_cull(Arenas A, int n) {
 }
 
 // ------------------------------------------------------------------------
-// sampling: the adaptive terrain through k_blocks and k_terrain, every other
-// case through k_sample
+// sampling: the adaptive terrain through k_blocks and k_terrain, adaptive 3D
+// noise fields through k_field, every other case through k_sample
 // ------------------------------------------------------------------------
 // A chunk's sample geometry as values (like TerrainTerms): read once per
 // tile, so the loops below never reload them after their own stores.
@@ -1282,14 +1283,14 @@ __global__ void __launch_bounds__(kRowThreads) k_sample(Arenas A, int n, int ful
 // active-cell bits, their edge prefix, and the item's edges (vertices; quads
 // in the quad mode) and cell counts (triangles; polygons in the quad mode).
 // With REFINE it also gives every endpoint of a sign-changing edge that
-// k_sample's adaptive evaluation labelled early its full density.
+// the adaptive sampling labelled early its full density.
 //
 // All 64 labels of a word meet their neighbours in a few 64-bit operations,
 // so what is left per sample is done only for the few that the surface
 // meets, compacted into dense lanes (a terrain item of 1,024 samples holds
 // about 40 active cells).  A wave per label row with a lane per sample kept
 // 3 % of its lanes busy: 512 chunks of 64^3 cells, 64 sampled, took 70 us
-// and 23 more for the refinement as a kernel of its own; this takes 45 us.
+// and 23 more for the refinement as a kernel of its own; this takes 31 us.
 // ------------------------------------------------------------------------
 template <int REFINE>
 __global__ void __launch_bounds__(kRowThreads) k_count(Arenas A) {
