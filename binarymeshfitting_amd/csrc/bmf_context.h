@@ -73,7 +73,13 @@ template <class T>
 hipError_t host_alloc(T** host, int64_t count, T** dev) {
     hipError_t e = hipHostMalloc((void**)host, sizeof(T) * (size_t)count, hipHostMallocMapped | hipHostMallocCoherent);
     if (e != hipSuccess) return e;
-    return hipHostGetDevicePointer((void**)dev, *host, 0);
+    e = hipHostGetDevicePointer((void**)dev, *host, 0);
+    if (e != hipSuccess) {  // both or neither
+        (void)hipHostFree(*host);
+        *host = nullptr;
+        *dev = nullptr;
+    }
+    return e;
 }
 
 // Smoothing launches of a batch: the largest K, at least 1 with normals.
