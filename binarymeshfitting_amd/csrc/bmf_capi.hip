@@ -304,7 +304,11 @@ int bmf_create(bmf_ctx** out, int device, const bmf_limits* lim) {
         c->cu_count = prop.multiProcessorCount;
     c->persistent_blocks = c->cu_count * 8;
     c->tune.sample_tile = 2048;
-    c->tune.sample_blocks = c->persistent_blocks;
+    // ten per CU: the terrain's lists and the other samplers' items leave waves
+    // idle at the end of a block (512 chunks of 64^3 cells, whole passes: 363 us at
+    // 8, 351 at 10; 64 of CSG 275 and 266, 108 of a 3D field 276 and 273; 12 and 16
+    // between the two)
+    c->tune.sample_blocks = c->cu_count * 10;
     // ten per CU: the best of 4..64 per CU for count + emit on a batch of
     // 512 64^3-cell chunks (89 us; 97 at 8, 94 at 16 and more) and on 64
     // chunks of CSG quads (150, 168, 155); the autotuner tries the others
