@@ -309,9 +309,9 @@ int bmf_create(bmf_ctx** out, int device, const bmf_limits* lim) {
     // 8, 351 at 10; 64 of CSG 275 and 266, 108 of a 3D field 276 and 273; 12 and 16
     // between the two)
     c->tune.sample_blocks = c->cu_count * 10;
-    // ten per CU: the best of 4..64 per CU for count + emit on a batch of
-    // 512 64^3-cell chunks (89 us; 97 at 8, 94 at 16 and more) and on 64
-    // chunks of CSG quads (150, 168, 155); the autotuner tries the others
+    // ten per CU: the best of 4..32 per CU for count + emit on a batch of
+    // 512 64^3-cell chunks (74 us; 87 at 4, 78 at 8, 77 at 16) and on 64
+    // chunks of CSG quads (133; 149, 139, 141); the autotuner tries the others
     c->tune.row_blocks = c->cu_count * 10;
     // twelve per CU: all the smoothing of 512 64^3-cell chunks 91 us, of 1,536
     // chunks of uneven LOD, whose steps have few tiles, 54; at 4 per CU 97 and
