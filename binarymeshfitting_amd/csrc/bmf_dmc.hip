@@ -654,6 +654,7 @@ __global__ void __launch_bounds__(kRowThreads) k_dmc_quads(Arenas A) {
                 qid++;
             }
         }
+        wave_sync();  // the windows and the list are read
     }
 }
 
