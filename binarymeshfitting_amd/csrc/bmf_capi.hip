@@ -245,6 +245,11 @@ int build_sampler(const bmf_sampler_desc* s, SamplerDev* out) {
     if (s->kind == BMF_SAMPLER_CSG) {
         d.n_spheres = s->n_spheres;
         d.n_boxes = s->n_boxes;
+        float most = 0.0f;  // (std::max drops a NaN, whose primitive never wins)
+        for (int i = 0; i < s->n_spheres; i++) most = std::max(most, std::fabs(s->spheres[4 * i + 3]));
+        for (int i = 0; i < s->n_boxes; i++)
+            for (int k = 3; k < 6; k++) most = std::max(most, std::fabs(s->boxes[6 * i + k]));
+        d.csg_slack = 4e-6f * most;
     }
     if (s->kind == BMF_SAMPLER_EXTERNAL) d.ext = s->densities;
     *out = d;

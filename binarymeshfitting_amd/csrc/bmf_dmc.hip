@@ -355,10 +355,7 @@ __device__ __forceinline__ uint32_t dmc_ring(const Arenas& A, const uint32_t (&p
 }
 
 // CSG primitives of one item's edge points: those of the chunk's list that
-// can reach the union's surface there.  An edge point lies within one sample
-// step of a sample with density >= 0, and the union is 1-Lipschitz, so a
-// primitive that stays below -step everywhere in the item's box never wins;
-// twice the step and a coordinate-sized slack cover the rounding.
+// can reach the union's surface there (csg_reach).
 constexpr int kItemCsg = 16;
 
 struct DmcWave {
@@ -483,12 +480,10 @@ __global__ void __launch_bounds__(kRowThreads) k_dmc_vertices(Arenas A, int n) {
         int ns = M.csg_ns, nb = M.csg_nb;
         bool staged = false;
         if (qef && csg) {
-            float lo[3], hi[3], far = 0.0f;
+            float lo[3], hi[3];
             sample_box(M, 64 * w0, kItemSamples, 1, lo, hi);  // the cells' far corners too
-#pragma unroll
-            for (int k = 0; k < 3; k++) far = fmaxf(far, fmaxf(fabsf(lo[k]), fabsf(hi[k])));
             int is, ib;
-            staged = cull_csg(*S, csg, ns, nb, lo, hi, 2.0f * M.delta + 1e-4f * far, W.csg, kItemCsg, is, ib);
+            staged = cull_csg(*S, csg, ns, nb, lo, hi, csg_reach(*S, M.delta, lo, hi), W.csg, kItemCsg, is, ib);
             if (staged) {
                 ns = is;
                 nb = ib;

@@ -39,6 +39,7 @@ struct SamplerDev {
     int32_t expand_ok;          // terrain: the noise sum can be expanded about block centres (k_blocks)
     const float* spheres;       // device, n_spheres x 4
     const float* boxes;         // device, n_boxes x 6
+    float csg_slack;            // CSG: bounds the FP32 error of a primitive's value and of its cull (csg_reach)
     const float* ext;           // EXTERNAL: caller's densities, chunks packed in descriptor order
     // NOISE: basis, fractal, density map and perturbation (bmf_sampler_desc)
     int32_t noise_dims, noise_basis, noise_fractal;

@@ -322,7 +322,8 @@ __global__ void __launch_bounds__(kPlanThreads) k_plan_fix(Arenas A, int n, int 
 // ------------------------------------------------------------------------
 // CSG culling: per chunk, the primitives whose value can exceed the floor
 // inside its sample box (spheres within r + |floor| of the box, boxes whose
-// box grown by |floor| meets it; 0.5 of slack covers FP32 rounding), in
+// box grown by |floor| meets it; 0.5 and the slack of csg_reach cover FP32
+// rounding), in
 // their original order (sphere ids, then box ids).  Block per chunk; order
 // kept by a ballot prefix per 256 primitives.
 // ------------------------------------------------------------------------
@@ -336,7 +337,9 @@ __global__ void __launch_bounds__(256) k_csg_cull(Arenas A, int n) {
         ChunkMeta& M = A.meta[j];
         const float lo[3] = {M.opos[0], M.opos[1], M.opos[2]};
         const float ext = (float)(M.dim - 1) * M.delta;
-        const float reach = -kCsgFloor + 0.5f;
+        float far = 0.0f;
+        for (int a = 0; a < 3; a++) far = fmaxf(far, fmaxf(fabsf(lo[a]), fabsf(lo[a] + ext)));
+        const float reach = -kCsgFloor + 0.5f + 4e-6f * far + S->csg_slack;
         uint16_t* L = A.csg_list + (int64_t)j * A.csg_stride;
         if (threadIdx.x == 0) s_base = 0;
         __syncthreads();
@@ -1152,10 +1155,9 @@ __global__ void __launch_bounds__(kRowThreads) k_field(Arenas A, int n) {
 
 // full: CSG values are wanted at every sample (stage inspection, the tape).
 // Otherwise only signs and the densities at the ends of sign-changing edges
-// are read, where the union lies within a sample step of 0 (it is
-// 1-Lipschitz): primitives that stay below -2 steps (and a coordinate-sized
-// slack) everywhere in the item's box cannot win there, and an item without
-// any is air.  64 chunks of 64^3 cells, 300 primitives: 69 us, with
+// are read, where the union lies within a sample step of 0 (csg_reach):
+// primitives that stay further below it everywhere in the item's box cannot win
+// there, and an item without any is air.  64 chunks of 64^3 cells, 300 primitives: 69 us, with
 // every primitive within reach of the chunk's floor at every sample 245.
 template <int MODE, int WORDS>
 __global__ void __launch_bounds__(kRowThreads) k_sample(Arenas A, int n, int full) {
@@ -1206,12 +1208,11 @@ __global__ void __launch_bounds__(kRowThreads) k_sample(Arenas A, int n, int ful
                 cs = M.csg_ns;
                 cb = M.csg_nb;
                 if (list && !full) {
-                    float lo[3], hi[3], far = 0.0f;
+                    float lo[3], hi[3];
                     sample_box(M, (int)first, 64 * WORDS, 0, lo, hi);
-#pragma unroll
-                    for (int k = 0; k < 3; k++) far = fmaxf(far, fmaxf(fabsf(lo[k]), fabsf(hi[k])));
                     int is, ib;
-                    staged = cull_csg(*S, list, cs, cb, lo, hi, 2.0f * M.delta + 1e-4f * far, s_csg[wave], kWaveCsg, is, ib);
+                    staged = cull_csg(*S, list, cs, cb, lo, hi, csg_reach(*S, M.delta, lo, hi), s_csg[wave], kWaveCsg,
+                                      is, ib);
                     if (staged) {
                         cs = is;
                         cb = ib;

@@ -293,6 +293,23 @@ __device__ __forceinline__ float csg_density_list(const SamplerDev& S, const uin
     return best;
 }
 
+// How far below 0 a primitive's value may lie in the box [lo, hi] for it still
+// to matter at the ends of sign-changing edges there, and on those edges.  Such
+// a point lies within one sample step of a sample with density >= 0.  Exact
+// values change by at most the step from there (each primitive is 1-Lipschitz),
+// the FP32 ones by their error more: near its surface a primitive of radius
+// (half extent) r has its value within 7 half-ulps of r, 4.2e-7 r, twice for
+// the winner and once for the one left out, and the cull's own test is within
+// 3e-7 r.  csg_slack is 4e-6 of the largest r of all, half a step more than one
+// and 1e-4 of the coordinates, whose rounding moves the samples by 5e-7 of them.
+__device__ __forceinline__ float csg_reach(const SamplerDev& S, float delta, const float (&lo)[3],
+                                           const float (&hi)[3]) {
+    float far = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 3; k++) far = fmaxf(far, fmaxf(fabsf(lo[k]), fabsf(hi[k])));
+    return 2.0f * delta + 1e-4f * far + S.csg_slack;
+}
+
 // Primitives staged in LDS: two float4 per primitive, (cx, cy, cz, r) and
 // unused for a sphere, (cx, cy, cz, hx) and (hy, hz, -, -) for a box; spheres
 // first.  Same union, same operation order.
