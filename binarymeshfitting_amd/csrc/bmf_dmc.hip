@@ -17,6 +17,8 @@
 //   K x (k_dual_n, k_primal_ring)
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "bmf_device_tables.h"
 #include "bmf_internal.h"
 #include "bmf_rows.h"
@@ -109,9 +111,40 @@ __device__ void csg_gradient(const SamplerDev& S, const uint16_t* list, int ns, 
     }
 }
 
-// The same with the chunk's primitives staged in LDS (stage_csg layout):
-// the loop finds the winning primitive (first index on ties), whose
-// gradient is then formed once, with the same operations as above.
+// Gradient of one primitive, as cull_csg writes it.
+__device__ __forceinline__ void primitive_gradient(bool sphere, float4 b0, float4 b1, float x, float y, float z,
+                                                   float g[3]) {
+    g[0] = g[1] = g[2] = 0.0f;
+    const float px = x - b0.x, py = y - b0.y, pz = z - b0.z;
+    if (sphere) {
+        const float l = sqrtf((px * px + py * py) + pz * pz);
+        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+        g[0] = -px * inv;
+        g[1] = -py * inv;
+        g[2] = -pz * inv;
+        return;
+    }
+    const float qx = fabsf(px) - b0.w, qy = fabsf(py) - b1.x, qz = fabsf(pz) - b1.y;
+    const float mx = fmaxf(qx, 0.0f), my = fmaxf(qy, 0.0f), mz = fmaxf(qz, 0.0f);
+    const float outside = sqrtf((mx * mx + my * my) + mz * mz);
+    const float sx = px < 0.0f ? -1.0f : 1.0f, sy = py < 0.0f ? -1.0f : 1.0f, sz = pz < 0.0f ? -1.0f : 1.0f;
+    if (outside > 0.0f) {
+        const float inv = 1.0f / outside;
+        g[0] = -mx * sx * inv;
+        g[1] = -my * sy * inv;
+        g[2] = -mz * sz * inv;
+    } else if (qx >= qy && qx >= qz) {
+        g[0] = -sx;
+    } else if (qy >= qz) {
+        g[1] = -sy;
+    } else {
+        g[2] = -sz;
+    }
+}
+
+// The same with the item's primitives in LDS (cull_csg's layout): the loop
+// finds the winning primitive (first index on ties), whose gradient is then
+// formed once, with the same operations as above.
 __device__ void csg_gradient_lds(const float4* s_csg, int ns, int nb, float x, float y, float z, float g[3]) {
     float best = kCsgFloor;
     int win = -1;
@@ -140,34 +173,52 @@ __device__ void csg_gradient_lds(const float4* s_csg, int ns, int nb, float x, f
     }
     g[0] = g[1] = g[2] = 0.0f;
     if (win < 0) return;  // the floor
-    if (win < ns) {
-        const float4 sp = s_csg[2 * win];
-        const float dx = x - sp.x, dy = y - sp.y, dz = z - sp.z;
-        const float l = sqrtf((dx * dx + dy * dy) + dz * dz);
-        const float inv = l > 0.0f ? 1.0f / l : 0.0f;
-        g[0] = -dx * inv;
-        g[1] = -dy * inv;
-        g[2] = -dz * inv;
-        return;
+    primitive_gradient(win < ns, s_csg[2 * win], s_csg[2 * win + 1], x, y, z, g);
+}
+
+// The same over the item's ids (cull_csg_ids).
+__device__ void csg_gradient_ids(const SamplerDev& S, const uint16_t* ids, int ns, int nb, float x, float y, float z,
+                                 float g[3]) {
+    const int b0 = (ns + 3) & ~3;
+    float best = kCsgFloor;
+    int win = -1;
+    for (int k = 0; k < ns; k += 4) {
+        float p[4][4];
+        csg_fetch<4>(S.spheres, ids, k, ns, p);
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            if (k + u >= ns) break;
+            const float dx = x - p[u][0], dy = y - p[u][1], dz = z - p[u][2];
+            const float l = sqrtf((dx * dx + dy * dy) + dz * dz);
+            const float v = p[u][3] - l;
+            win = v > best ? k + u : win;
+            best = v > best ? v : best;
+        }
     }
-    const float4 b0 = s_csg[2 * win], b1 = s_csg[2 * win + 1];
-    const float px = x - b0.x, py = y - b0.y, pz = z - b0.z;
-    const float qx = fabsf(px) - b0.w, qy = fabsf(py) - b1.x, qz = fabsf(pz) - b1.y;
-    const float mx = fmaxf(qx, 0.0f), my = fmaxf(qy, 0.0f), mz = fmaxf(qz, 0.0f);
-    const float outside = sqrtf((mx * mx + my * my) + mz * mz);
-    const float sx = px < 0.0f ? -1.0f : 1.0f, sy = py < 0.0f ? -1.0f : 1.0f, sz = pz < 0.0f ? -1.0f : 1.0f;
-    if (outside > 0.0f) {
-        const float inv = 1.0f / outside;
-        g[0] = -mx * sx * inv;
-        g[1] = -my * sy * inv;
-        g[2] = -mz * sz * inv;
-    } else if (qx >= qy && qx >= qz) {
-        g[0] = -sx;
-    } else if (qy >= qz) {
-        g[1] = -sy;
-    } else {
-        g[2] = -sz;
+    for (int k = 0; k < nb; k += 4) {
+        float p[4][6];
+        csg_fetch<6>(S.boxes, ids + b0, k, nb, p);
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            if (k + u >= nb) break;
+            const float px = x - p[u][0], py = y - p[u][1], pz = z - p[u][2];
+            const float qx = fabsf(px) - p[u][3], qy = fabsf(py) - p[u][4], qz = fabsf(pz) - p[u][5];
+            const float mx = fmaxf(qx, 0.0f), my = fmaxf(qy, 0.0f), mz = fmaxf(qz, 0.0f);
+            const float outside = sqrtf((mx * mx + my * my) + mz * mz);
+            const float inside = fminf(fmaxf(qx, fmaxf(qy, qz)), 0.0f);
+            const float v = -(outside + inside);
+            win = v > best ? b0 + k + u : win;
+            best = v > best ? v : best;
+        }
     }
+    g[0] = g[1] = g[2] = 0.0f;
+    if (win < 0) return;  // the floor
+    const bool sphere = win < ns;
+    const uint32_t id = ids[win];
+    const float* q = sphere ? S.spheres + 4 * id : S.boxes + 6 * id;
+    const float4 a = make_float4(q[0], q[1], q[2], q[3]);
+    const float4 b = sphere ? a : make_float4(q[4], q[5], 0.0f, 0.0f);
+    primitive_gradient(sphere, a, b, x, y, z, g);
 }
 
 // QEF of `count` (point, unit normal) pairs (qef_simd.h:392-579): normal
@@ -355,13 +406,18 @@ __device__ __forceinline__ uint32_t dmc_ring(const Arenas& A, const uint32_t (&p
 }
 
 // CSG primitives of one item's edge points: those of the chunk's list that
-// can reach the union's surface there (csg_reach).
+// can reach the union's surface there (csg_reach).  Up to kItemCsg are staged
+// themselves, more as their ids (kCsgIds; more than those: the chunk's list).  A
+// larger stage gains a tenth on items of 17 to 64 primitives (98 us instead of
+// 108 for 45^3 cells with 90) and costs 118 instead of 115 on thinly spread
+// ones (64 chunks of 64^3 cells, 300 primitives).
 constexpr int kItemCsg = 16;
 
 struct DmcWave {
     ItemWindows win;
     uint32_t verts[4 * 64];       // a round's vertices: sample | polygon << 10 | corner mask << 12
-    float4 csg[2 * kItemCsg];     // stage_csg layout
+    float4 csg[2 * kItemCsg];     // cull_csg's layout
+    uint16_t ids[kCsgIds] __attribute__((aligned(8)));  // cull_csg_ids'
 };
 
 // ------------------------------------------------------------------------
@@ -374,8 +430,8 @@ struct DmcWave {
 // 326,882 vertices: 110 us, with the plane's rows and the chunk's list 169.
 // ------------------------------------------------------------------------
 __device__ void place_vertex(const Arenas& A, const ChunkMeta& M, const SamplerDev& S, const uint16_t* csg,
-                             const float4* s_csg, int ns, int nb, int x, int y, int z, int p, uint32_t mask, bool qef,
-                             float out[3], float& err) {
+                             const float4* s_csg, const uint16_t* ids, int ns, int nb, int x, int y, int z, int p,
+                             uint32_t mask, bool qef, float out[3], float& err) {
     const int dim = M.dim;
     const float* __restrict__ D = A.dens + M.dens_off;
     const uint64_t row = c_dmc_table[mask];
@@ -429,6 +485,7 @@ __device__ void place_vertex(const Arenas& A, const ChunkMeta& M, const SamplerD
             const float wx = qx * M.delta + M.opos[0], wy = qy * M.delta + M.opos[1], wz = qz * M.delta + M.opos[2];
             float g[3];
             if (s_csg) csg_gradient_lds(s_csg, ns, nb, wx, wy, wz, g);
+            else if (ids) csg_gradient_ids(S, ids, ns, nb, wx, wy, wz, g);
             else csg_gradient(S, csg, ns, nb, wx, wy, wz, g);
             const float len = sqrtf((g[0] * g[0] + g[1] * g[1]) + g[2] * g[2]);
             float nrm[3];
@@ -452,6 +509,16 @@ __device__ void place_vertex(const Arenas& A, const ChunkMeta& M, const SamplerD
     }
 }
 
+// Few items with QEF placement: kVertexParts waves stage each of them and take
+// every kVertexParts-th of its rounds of cells, so that a detailed object in
+// one chunk is not left to as many waves as it has items.  Stage times with four
+// waves and with one: 33^3 cells with 60 primitives on the surface 119 and
+// 260 us, 100^3 with 400 208 and 321, 8 chunks of 45^3 with 90 58 and 104.
+// kVertexFew: a wave per SIMD without.  Twice as many still gain where the lists
+// are long (128^3 cells with 250: 137 and 223) and lose where they are short and
+// staging is most of the work (64 chunks of 64^3, 300 spread thinly: 119 and 115).
+constexpr int kVertexParts = 4;
+constexpr int kVertexFew = 1024;
 __global__ void __launch_bounds__(kRowThreads) k_dmc_vertices(Arenas A, int n) {
     __shared__ DmcTables s_t;
     __shared__ DmcWave s_wave[kWordWaves];
@@ -465,7 +532,9 @@ __global__ void __launch_bounds__(kRowThreads) k_dmc_vertices(Arenas A, int n) {
     const bool qef = A.placement == BMF_PLACE_QEF && S->kind == BMF_SAMPLER_CSG;
     const bool tris = A.quad_tris != 0;
     const int total = read_const(&A.ctr->n_work);
-    for (int wi = blockIdx.x * kWordWaves + wave; wi < total; wi += gridDim.x * kWordWaves) {
+    const int parts = qef && total <= kVertexFew ? kVertexParts : 1;
+    for (int wu = blockIdx.x * kWordWaves + wave; wu < total * parts; wu += gridDim.x * kWordWaves) {
+        const int wi = wu / parts, part = wu - wi * parts;
         const int2 im = read_const(A.work + wi);
         const int chunk = uniform_int(im.x), w0 = uniform_int(im.y) * kItemWords;
         const ChunkMeta M = read_chunk(A.meta, chunk);
@@ -475,16 +544,18 @@ __global__ void __launch_bounds__(kRowThreads) k_dmc_vertices(Arenas A, int n) {
         const WindowGeom g = stage_windows(A, M, w0, s);
         const int nc = push_bits(s.ac[lane >> 2], s.list);
         wave_sync();
-        if (nc == 0) continue;
+        if (nc <= 64 * part) continue;
         const uint16_t* csg = A.csg_list ? A.csg_list + (int64_t)chunk * A.csg_stride : nullptr;
         int ns = M.csg_ns, nb = M.csg_nb;
-        bool staged = false;
+        bool staged = false, listed = false;
         if (qef && csg) {
             float lo[3], hi[3];
             sample_box(M, 64 * w0, kItemSamples, 1, lo, hi);  // the cells' far corners too
+            const float reach = csg_reach(*S, M.delta, lo, hi);
             int is, ib;
-            staged = cull_csg(*S, csg, ns, nb, lo, hi, csg_reach(*S, M.delta, lo, hi), W.csg, kItemCsg, is, ib);
-            if (staged) {
+            staged = cull_csg(*S, csg, ns, nb, lo, hi, reach, W.csg, kItemCsg, is, ib);
+            if (!staged) listed = cull_csg_ids(*S, csg, ns, nb, lo, hi, reach, W.ids, is, ib);
+            if (staged || listed) {
                 ns = is;
                 nb = ib;
             }
@@ -505,6 +576,10 @@ __global__ void __launch_bounds__(kRowThreads) k_dmc_vertices(Arenas A, int n) {
             }
             uint32_t nv;
             const uint32_t pre = wave_prefix<3>(np, nv);
+            if (parts > 1 && (e0 >> 6) % parts != part) {  // another wave's
+                vb += nv;
+                continue;
+            }
             if (np) {
                 const int64_t ci = M.dens_off + 64ll * w0 + pos;
                 A.cell_tb[ci] = vb + pre;
@@ -528,7 +603,8 @@ __global__ void __launch_bounds__(kRowThreads) k_dmc_vertices(Arenas A, int n) {
                     (uint8_t)(x == 0 || y == 0 || z == 0 || x + 1 == dim - 1 || y + 1 == dim - 1 || z + 1 == dim - 1);
                 A.vedge[vo + v] = (uint32_t)x | ((uint32_t)y << 8) | ((uint32_t)z << 16) | ((uint32_t)p << 24);
                 float o[3], err;
-                place_vertex(A, M, *S, csg, staged ? W.csg : nullptr, ns, nb, x, y, z, p, cmask, qef, o, err);
+                place_vertex(A, M, *S, csg, staged ? W.csg : nullptr, listed ? W.ids : nullptr, ns, nb, x, y, z, p, cmask, qef,
+                             o, err);
                 float* P = A.pos + (vo + v) * 3;
                 P[0] = o[0];
                 P[1] = o[1];
@@ -917,7 +993,10 @@ __global__ void __launch_bounds__(kSmoothThreads) k_primal_ring_nrm(Arenas A, in
 
 hipError_t launch_dmc_emit(const Arenas& A, int n, int blocks, hipStream_t s) {
     // the vertices, then the quads that index them
-    hipLaunchKernelGGL(k_dmc_vertices, dim3(blocks), dim3(kRowThreads), 0, s, A, n);
+    // a grid sized to one chunk's items: four times that for their parts, as far as they go
+    constexpr int kMost = kVertexParts * kVertexFew / kWordWaves;
+    const int vblocks = A.placement == BMF_PLACE_QEF ? std::max(blocks, std::min(kVertexParts * blocks, kMost)) : blocks;
+    hipLaunchKernelGGL(k_dmc_vertices, dim3(vblocks), dim3(kRowThreads), 0, s, A, n);
     hipLaunchKernelGGL(k_dmc_quads, dim3(blocks), dim3(kRowThreads), 0, s, A);
     return hipGetLastError();
 }

@@ -839,9 +839,7 @@ __global__ void __launch_bounds__(kRowThreads) k_terrain(Arenas A, int n) {
 //   2D noise field   from the columns of k_columns
 //   CSG              with the item's own primitives, see below
 // ------------------------------------------------------------------------
-constexpr int kSampleImplicit = 0, kSampleTerrain = 1, kSampleCsg = 2, kSampleField2 = 3, kSampleField3 = 4,
-              kSampleExternal = 5;
-constexpr int kWaveCsg = 64;  // CSG primitives per wave staged in LDS (longer lists read global memory)
+constexpr int kSampleImplicit = 0, kSampleTerrain = 1, kSampleField2 = 2, kSampleField3 = 3, kSampleExternal = 4;
 
 // 2D noise fields: n at every (x, z) column of every chunk, a lane each, into
 // the cell arena (free until the emission), from the chunk's first sample on.
@@ -1153,17 +1151,9 @@ __global__ void __launch_bounds__(kRowThreads) k_field(Arenas A, int n) {
     if (tid == 0 && (int)blockIdx.x < A.stat_cap) A.stat_blocks[blockIdx.x] = 0ull;  // no octaves counted
 }
 
-// full: CSG values are wanted at every sample (stage inspection, the tape).
-// Otherwise only signs and the densities at the ends of sign-changing edges
-// are read, where the union lies within a sample step of 0 (csg_reach):
-// primitives that stay further below it everywhere in the item's box cannot win
-// there, and an item without any is air.  64 chunks of 64^3 cells, 300 primitives: 69 us, with
-// every primitive within reach of the chunk's floor at every sample 245.
 template <int MODE, int WORDS>
-__global__ void __launch_bounds__(kRowThreads) k_sample(Arenas A, int n, int full) {
+__global__ void __launch_bounds__(kRowThreads) k_sample(Arenas A, int n) {
     constexpr int kParts = kItemWords / WORDS;  // waves per item of the word kernels
-    constexpr bool kCsg = MODE == kSampleCsg;
-    __shared__ float4 s_csg[kCsg ? kWordWaves : 1][kCsg ? 2 * kWaveCsg : 1];
     if constexpr (MODE == kSampleTerrain || MODE == kSampleField3) load_gradients();
     const SamplerDev* __restrict__ S = A.sampler;
     const int wave = uniform_int(threadIdx.x >> 6), lane = lane_id();
@@ -1200,27 +1190,6 @@ __global__ void __launch_bounds__(kRowThreads) k_sample(Arenas A, int n, int ful
                 word(r, i < ns, v[r] < 0.0f);
             }
         } else {
-            const uint16_t* list = nullptr;
-            int cs = 0, cb = 0;
-            bool staged = false, empty = false;
-            if constexpr (kCsg) {
-                list = A.csg_list ? A.csg_list + (int64_t)j * A.csg_stride : nullptr;
-                cs = M.csg_ns;
-                cb = M.csg_nb;
-                if (list && !full) {
-                    float lo[3], hi[3];
-                    sample_box(M, (int)first, 64 * WORDS, 0, lo, hi);
-                    int is, ib;
-                    staged = cull_csg(*S, list, cs, cb, lo, hi, csg_reach(*S, M.delta, lo, hi), s_csg[wave], kWaveCsg,
-                                      is, ib);
-                    if (staged) {
-                        cs = is;
-                        cb = ib;
-                        empty = is + ib == 0;
-                    }
-                    wave_sync();
-                }
-            }
             // a lane's sample advances by 64 per word: its (y, z) by
             // (64 / dim, 64 % dim) with at most one carry per axis while
             // 64 / dim + 1 < dim; smaller chunks divide
@@ -1233,19 +1202,15 @@ __global__ void __launch_bounds__(kRowThreads) k_sample(Arenas A, int n, int ful
             for (int r = 0; r < WORDS; r++) {
                 const uint32_t i = first + 64u * (uint32_t)r + (uint32_t)lane;
                 const bool valid = i < ns;
-                float d = kCsgFloor;
-                if (valid && !empty) {
+                float d = 0.0f;
+                if (valid) {
                     float px, py, pz;
                     sample_position(G, x, y, z, px, py, pz);
                     if constexpr (MODE == kSampleTerrain) d = terrain_density(*S, px, py, pz);
                     else if constexpr (MODE == kSampleField2)
                         d = noise_density_from(*S, __uint_as_float(A.cell_tb[M.dens_off + x * dim + z]), py);
                     else if constexpr (MODE == kSampleField3) d = noise_density_from(*S, noise_value(*S, px, py, pz), py);
-                    else if constexpr (kCsg) {
-                        if (staged) d = csg_density_lds(s_csg[wave], cs, cb, px, py, pz);
-                        else if (list) d = csg_density_list(*S, list, cs, cb, px, py, pz);
-                        else d = csg_density(*S, px, py, pz);
-                    } else d = implicit_density(S->kind, S->world_size, px, py, pz);
+                    else d = implicit_density(S->kind, S->world_size, px, py, pz);
                     dens[i] = d;
                 }
                 word(r, valid, d < 0.0f);
@@ -1264,9 +1229,106 @@ __global__ void __launch_bounds__(kRowThreads) k_sample(Arenas A, int n, int ful
                     sample_index(min(i + 64u, ns), dim, dim2, rd, rd2, x, y, z);
                 }
             }
-            if constexpr (kCsg) wave_sync();  // the primitives are read
         }
         if (lane < WORDS && w0 + lane < (int)M.lab_words) {
+            const int left = (int)ns - 64 * (w0 + lane);
+            A.labels[M.lab_off + w0 + lane] = mine;
+            A.exact[M.lab_off + w0 + lane] = ~bits_from(left);
+        }
+        if (lane == 0) {
+            if (air && !A.meta[j].any_air) atomicOr(&A.meta[j].any_air, 1u);
+            if (solid && !A.meta[j].any_solid) atomicOr(&A.meta[j].any_solid, 1u);
+        }
+    }
+    if (threadIdx.x == 0 && (int)blockIdx.x < A.stat_cap) A.stat_blocks[blockIdx.x] = 0ull;  // no octaves counted
+}
+
+// ------------------------------------------------------------------------
+// CSG: a wave per item of label words with the item's own primitives, culled
+// from its chunk's list.  full: values are wanted at every sample (stage
+// inspection, the tape) and nothing is culled.  Otherwise only signs and the
+// densities at the ends of sign-changing edges are read, where the union lies
+// within a sample step of 0 (csg_reach): primitives that stay further below it
+// everywhere in the item's box cannot win there, and an item without any is air.
+// Bound by VALU issue (the square root of each primitive's distance).
+// ------------------------------------------------------------------------
+// A wave takes its item's words in groups whose samples share a primitive's
+// loads; batches of up to kCsgFew items have a wave, and a cull, per group.
+// Sampling with a group and with an item per wave: one chunk of 20^3 cells with
+// 300 primitives 84 and 314 us, of 64^3 (269 items) 42 and 135, 8 of 45^3 (760)
+// 29 and 51 (with 30 primitives 23 and 17), 8 of 64^3 (2,145) 72 and 47.
+constexpr int kCsgGroup = 4;
+constexpr int kCsgFew = 1024;
+__global__ void __launch_bounds__(kRowThreads) k_csg(Arenas A, int n, int full) {
+    __shared__ __attribute__((aligned(8))) uint16_t s_ids[kWordWaves][kCsgIds];
+    const SamplerDev& S = *A.sampler;
+    const int wave = uniform_int(threadIdx.x >> 6), lane = lane_id();
+    const int64_t items = read_const(&A.ctr->total_items);
+    const int words = items <= kCsgFew ? kCsgGroup : kItemWords, parts = kItemWords / words;
+    uint16_t* const ids = s_ids[wave];
+    for (int64_t u = (int64_t)blockIdx.x * kWordWaves + wave; u < items * parts; u += (int64_t)gridDim.x * kWordWaves) {
+        const int64_t it = u / parts;
+        const int part = (int)(u - it * parts);
+        const int j = find_item_wave(A.meta, n, it);
+        const ChunkMeta M = read_chunk(A.meta, j);
+        const int item = (int)(it - M.item_slot), w0 = item * kItemWords + part * words;
+        if (part == 0 && lane == 0) A.item_map[it] = make_int2(j, item);  // for the word kernels
+        if (w0 >= (int)M.lab_words) continue;
+        const uint32_t dim = (uint32_t)M.dim, dim2 = dim * dim, ns = dim2 * dim;
+        const float rd = 1.0f / (float)dim, rd2 = 1.0f / (float)dim2;
+        const ChunkGeom G{M.opos[0], M.opos[1], M.opos[2], M.delta};
+        float* __restrict__ dens = A.dens + M.dens_off;
+        const uint32_t first = 64u * (uint32_t)w0;
+        const uint16_t* list = A.csg_list ? A.csg_list + (int64_t)j * A.csg_stride : nullptr;
+        int cs = M.csg_ns, cb = M.csg_nb;
+        bool fits = false;
+        if (list) {
+            float lo[3], hi[3];
+            sample_box(M, (int)first, 64 * words, 0, lo, hi);
+            int is, ib;
+            fits = cull_csg_ids(S, list, cs, cb, lo, hi, full ? INFINITY : csg_reach(S, M.delta, lo, hi), ids, is, ib);
+            if (fits) {
+                cs = is;
+                cb = ib;
+            }
+            wave_sync();
+        }
+        const bool empty = fits && cs + cb == 0 && !full;
+        uint64_t mine = 0ull;  // lane r keeps word r
+        bool air = false, solid = false;
+#pragma unroll 1
+        for (int r0 = 0; r0 < words; r0 += kCsgGroup) {
+            float px[kCsgGroup], py[kCsgGroup], pz[kCsgGroup], d[kCsgGroup];
+            if (empty) {
+#pragma unroll
+                for (int r = 0; r < kCsgGroup; r++) d[r] = kCsgFloor;
+            } else {
+#pragma unroll
+                for (int r = 0; r < kCsgGroup; r++)
+                    sample_coords(G, min(first + 64u * (uint32_t)(r0 + r) + (uint32_t)lane, ns - 1u), dim, dim2, rd, rd2,
+                                  px[r], py[r], pz[r]);
+                if (fits) {
+                    csg_density_ids<kCsgGroup>(S, ids, cs, cb, px, py, pz, d);
+                } else {
+#pragma unroll
+                    for (int r = 0; r < kCsgGroup; r++)
+                        d[r] = list ? csg_density_list(S, list, cs, cb, px[r], py[r], pz[r])
+                                    : csg_density(S, px[r], py[r], pz[r]);
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < kCsgGroup; r++) {
+                const uint32_t i = first + 64u * (uint32_t)(r0 + r) + (uint32_t)lane;
+                const bool valid = i < ns;
+                if (valid && !empty) dens[i] = d[r];
+                const uint64_t bl = __ballot(valid && d[r] < 0.0f), vb = __ballot(valid);
+                mine = lane == r0 + r ? bl : mine;
+                air = air || bl != 0ull;
+                solid = solid || bl != vb;
+            }
+        }
+        wave_sync();  // the ids are read
+        if (lane < words && w0 + lane < (int)M.lab_words) {
             const int left = (int)ns - 64 * (w0 + lane);
             A.labels[M.lab_off + w0 + lane] = mine;
             A.exact[M.lab_off + w0 + lane] = ~bits_from(left);
@@ -2157,20 +2219,20 @@ hipError_t launch_sample(const Arenas& A, int n, int blocks, int adaptive, int k
         hipLaunchKernelGGL(k_blocks, g, b, 0, s, A, n);
         hipLaunchKernelGGL(k_terrain, g, b, 0, s, A, n);
     } else if (kind == BMF_SAMPLER_TERRAIN) {
-        hipLaunchKernelGGL((k_sample<kSampleTerrain, 4>), g, b, 0, s, A, n, 1);
+        hipLaunchKernelGGL((k_sample<kSampleTerrain, 4>), g, b, 0, s, A, n);
     } else if (kind == BMF_SAMPLER_NOISE && slab) {
         hipLaunchKernelGGL(k_columns, g, b, 0, s, A, n);
-        hipLaunchKernelGGL((k_sample<kSampleField2, 16>), g, b, 0, s, A, n, 1);
+        hipLaunchKernelGGL((k_sample<kSampleField2, 16>), g, b, 0, s, A, n);
     } else if (kind == BMF_SAMPLER_NOISE && adaptive) {
         hipLaunchKernelGGL(k_field, g, b, 0, s, A, n);
     } else if (kind == BMF_SAMPLER_NOISE) {
-        hipLaunchKernelGGL((k_sample<kSampleField3, 4>), g, b, 0, s, A, n, 1);
+        hipLaunchKernelGGL((k_sample<kSampleField3, 4>), g, b, 0, s, A, n);
     } else if (kind == BMF_SAMPLER_CSG) {
-        hipLaunchKernelGGL((k_sample<kSampleCsg, 16>), g, b, 0, s, A, n, !adaptive);
+        hipLaunchKernelGGL(k_csg, g, b, 0, s, A, n, !adaptive);
     } else if (kind == BMF_SAMPLER_EXTERNAL) {
-        hipLaunchKernelGGL((k_sample<kSampleExternal, 16>), g, b, 0, s, A, n, 1);
+        hipLaunchKernelGGL((k_sample<kSampleExternal, 16>), g, b, 0, s, A, n);
     } else {
-        hipLaunchKernelGGL((k_sample<kSampleImplicit, 16>), g, b, 0, s, A, n, 1);
+        hipLaunchKernelGGL((k_sample<kSampleImplicit, 16>), g, b, 0, s, A, n);
     }
     return hipGetLastError();
 }

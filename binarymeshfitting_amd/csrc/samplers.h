@@ -18,6 +18,7 @@
 #include <stdint.h>
 
 #include "bmf_internal.h"
+#include "bmf_rows.h"
 
 namespace bmf {
 
@@ -310,39 +311,45 @@ __device__ __forceinline__ float csg_reach(const SamplerDev& S, float delta, con
     return 2.0f * delta + 1e-4f * far + S.csg_slack;
 }
 
-// Primitives staged in LDS: two float4 per primitive, (cx, cy, cz, r) and
-// unused for a sphere, (cx, cy, cz, hx) and (hy, hz, -, -) for a box; spheres
-// first.  Same union, same operation order.
-// The primitives of a chunk's list whose value can exceed -reach somewhere
-// in the box [lo, hi], by one wave, in list order into `out` (room for `cap`
-// of them): a sphere within r + reach of the box, a box that meets it grown by
-// reach.  Returns whether they fit.
+// Whether primitive i of a chunk's list (sphere ids, then box ids) can exceed
+// -reach somewhere in the box [lo, hi]: a sphere within r + reach of the box, a
+// box that meets it grown by reach.  a and b get the primitive as cull_csg
+// writes it.
+__device__ __forceinline__ bool csg_reaches(const SamplerDev& S, const uint16_t* __restrict__ list, int i, int ns, int nb,
+                                            const float (&lo)[3], const float (&hi)[3], float reach, float4& a,
+                                            float4& b) {
+    a = b = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (i < ns) {
+        const float* sp = S.spheres + 4 * list[i];
+        a = make_float4(sp[0], sp[1], sp[2], sp[3]);
+        const float tx = fmaxf(fmaxf(lo[0] - a.x, a.x - hi[0]), 0.0f), ty = fmaxf(fmaxf(lo[1] - a.y, a.y - hi[1]), 0.0f),
+                    tz = fmaxf(fmaxf(lo[2] - a.z, a.z - hi[2]), 0.0f);
+        const float r = a.w + reach;
+        return r > 0.0f && !((tx * tx + ty * ty) + tz * tz > r * r);
+    }
+    if (i >= ns + nb) return false;
+    const float* q = S.boxes + 6 * list[i];
+    a = make_float4(q[0], q[1], q[2], q[3]);
+    b = make_float4(q[4], q[5], 0.0f, 0.0f);
+    return !(a.x - a.w - reach > hi[0]) && !(a.x + a.w + reach < lo[0]) && !(a.y - b.x - reach > hi[1]) &&
+           !(a.y + b.x + reach < lo[1]) && !(a.z - b.y - reach > hi[2]) && !(a.z + b.y + reach < lo[2]);
+}
+
+// The primitives of a chunk's list that reach the box, by one wave, in list
+// order into LDS (room for `cap` of them): two float4 per primitive,
+// (cx, cy, cz, r) and unused for a sphere, (cx, cy, cz, hx) and (hy, hz, -, -)
+// for a box; spheres first.  Returns whether they fit.
 __device__ __forceinline__ bool cull_csg(const SamplerDev& S, const uint16_t* __restrict__ list, int ns, int nb,
                                          const float (&lo)[3], const float (&hi)[3], float reach, float4* out, int cap,
                                          int& out_s, int& out_b) {
-    const int lane = (int)(threadIdx.x & 63);
     int n = 0;
     out_s = 0;
     for (int i0 = 0; i0 < ns + nb; i0 += 64) {
-        const int i = i0 + lane;
-        bool keep = false;
-        float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f), b = a;
-        if (i < ns) {
-            const float* sp = S.spheres + 4 * list[i];
-            a = make_float4(sp[0], sp[1], sp[2], sp[3]);
-            const float tx = fmaxf(fmaxf(lo[0] - a.x, a.x - hi[0]), 0.0f), ty = fmaxf(fmaxf(lo[1] - a.y, a.y - hi[1]), 0.0f),
-                        tz = fmaxf(fmaxf(lo[2] - a.z, a.z - hi[2]), 0.0f);
-            const float r = a.w + reach;
-            keep = r > 0.0f && !((tx * tx + ty * ty) + tz * tz > r * r);
-        } else if (i < ns + nb) {
-            const float* q = S.boxes + 6 * list[i];
-            a = make_float4(q[0], q[1], q[2], q[3]);
-            b = make_float4(q[4], q[5], 0.0f, 0.0f);
-            keep = !(a.x - a.w - reach > hi[0]) && !(a.x + a.w + reach < lo[0]) && !(a.y - b.x - reach > hi[1]) &&
-                   !(a.y + b.x + reach < lo[1]) && !(a.z - b.y - reach > hi[2]) && !(a.z + b.y + reach < lo[2]);
-        }
+        const int i = i0 + lane_id();
+        float4 a, b;
+        const bool keep = csg_reaches(S, list, i, ns, nb, lo, hi, reach, a, b);
         const uint64_t bal = __ballot(keep), spheres = __ballot(keep && i < ns);
-        const int at = n + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
+        const int at = n + (int)mbcnt64(bal);
         if (keep && at < cap) {
             out[2 * at] = a;
             out[2 * at + 1] = b;
@@ -354,24 +361,87 @@ __device__ __forceinline__ bool cull_csg(const SamplerDev& S, const uint16_t* __
     return n <= cap;
 }
 
-__device__ __forceinline__ float csg_density_lds(const float4* s_csg, int ns, int nb, float x, float y, float z) {
-    float best = kCsgFloor;
-    for (int k = 0; k < ns; k++) {
-        const float4 sp = s_csg[2 * k];
-        float dx = x - sp.x, dy = y - sp.y, dz = z - sp.z;
-        float l = sqrtf((dx * dx + dy * dy) + dz * dz);
-        best = fmaxf(best, sp.w - l);
+// Their ids instead, which take a sixteenth of the room: the spheres' from 0
+// on, the boxes' from the next multiple of four.  The primitives themselves are
+// then read by the whole wave at once, through scalar loads.  kCsgIds: 2 KiB per
+// wave, the most that costs neither kernel a workgroup per CU.
+constexpr int kCsgIds = 1024;
+__device__ __forceinline__ bool cull_csg_ids(const SamplerDev& S, const uint16_t* __restrict__ list, int ns, int nb,
+                                             const float (&lo)[3], const float (&hi)[3], float reach, uint16_t* ids,
+                                             int& out_s, int& out_b) {
+    out_s = out_b = 0;
+    for (int i0 = 0; i0 < ns + nb; i0 += 64) {
+        const int i = i0 + lane_id();
+        float4 a, b;
+        const bool keep = csg_reaches(S, list, i, ns, nb, lo, hi, reach, a, b), sphere = i < ns;
+        const uint64_t spheres = __ballot(keep && sphere), boxes = __ballot(keep && !sphere);
+        const int at = sphere ? out_s + (int)mbcnt64(spheres)
+                              : ((out_s + (int)__popcll(spheres) + 3) & ~3) + out_b + (int)mbcnt64(boxes);
+        if (keep && at < kCsgIds) ids[at] = list[i];
+        out_s += (int)__popcll(spheres);
+        out_b += (int)__popcll(boxes);
     }
-    for (int k = ns; k < ns + nb; k++) {
-        const float4 b0 = s_csg[2 * k], b1 = s_csg[2 * k + 1];
-        float px = x - b0.x, py = y - b0.y, pz = z - b0.z;
-        float qx = fabsf(px) - b0.w, qy = fabsf(py) - b1.x, qz = fabsf(pz) - b1.y;
-        float mx = fmaxf(qx, 0.0f), my = fmaxf(qy, 0.0f), mz = fmaxf(qz, 0.0f);
-        float outside = sqrtf((mx * mx + my * my) + mz * mz);
-        float inside = fminf(fmaxf(qx, fmaxf(qy, qz)), 0.0f);
-        best = fmaxf(best, -(outside + inside));
+    return ((out_s + 3) & ~3) + out_b <= kCsgIds;
+}
+
+// Four primitives' FP32 words from id position k on (a multiple of four) of n,
+// N words each: the id and the primitives are the same in every lane.  A
+// position past the end repeats the first.
+template <int N>
+__device__ __forceinline__ void csg_fetch(const float* prims, const uint16_t* ids, int k, int n, float (&p)[4][N]) {
+    const uint2 w = *reinterpret_cast<const uint2*>(ids + k);
+    const uint32_t w0 = (uint32_t)uniform_int((int)w.x), w1 = (uint32_t)uniform_int((int)w.y);
+    const uint32_t id[4] = {w0 & 0xFFFFu, w0 >> 16, w1 & 0xFFFFu, w1 >> 16};
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+        struct Words {
+            float v[N];
+        };
+        const Words r = read_const(reinterpret_cast<const Words*>(prims) + (k + u < n ? id[u] : id[0]));
+#pragma unroll
+        for (int q = 0; q < N; q++) p[u][q] = r.v[q];
     }
-    return best;
+}
+
+// The union at G points of each lane over a wave's list of ids.
+template <int G>
+__device__ __forceinline__ void csg_density_ids(const SamplerDev& S, const uint16_t* ids, int ns, int nb,
+                                                const float (&x)[G], const float (&y)[G], const float (&z)[G],
+                                                float (&best)[G]) {
+#pragma unroll
+    for (int g = 0; g < G; g++) best[g] = kCsgFloor;
+    for (int k = 0; k < ns; k += 4) {
+        float p[4][4];
+        csg_fetch<4>(S.spheres, ids, k, ns, p);
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            if (k + u >= ns) break;
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+                const float dx = x[g] - p[u][0], dy = y[g] - p[u][1], dz = z[g] - p[u][2];
+                const float l = sqrtf((dx * dx + dy * dy) + dz * dz);
+                best[g] = fmaxf(best[g], p[u][3] - l);
+            }
+        }
+    }
+    ids += (ns + 3) & ~3;
+    for (int k = 0; k < nb; k += 4) {
+        float p[4][6];
+        csg_fetch<6>(S.boxes, ids, k, nb, p);
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            if (k + u >= nb) break;
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+                const float px = x[g] - p[u][0], py = y[g] - p[u][1], pz = z[g] - p[u][2];
+                const float qx = fabsf(px) - p[u][3], qy = fabsf(py) - p[u][4], qz = fabsf(pz) - p[u][5];
+                const float mx = fmaxf(qx, 0.0f), my = fmaxf(qy, 0.0f), mz = fmaxf(qz, 0.0f);
+                const float outside = sqrtf((mx * mx + my * my) + mz * mz);
+                const float inside = fminf(fmaxf(qx, fmaxf(qy, qz)), 0.0f);
+                best[g] = fmaxf(best[g], -(outside + inside));
+            }
+        }
+    }
 }
 
 // ---- noise fields: the NoiseSamplers block shapes (NoiseSampler.cpp:113-318)
