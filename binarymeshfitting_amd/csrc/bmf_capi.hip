@@ -6,6 +6,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <initializer_list>
 #include <mutex>
 #include <new>
 #include <vector>
@@ -992,58 +993,38 @@ int bmf_autotune(bmf_ctx* c, const bmf_chunk_desc* chunks, int n, int reps, bmf_
     const bmf_tuning start = c->tune;
     bmf_tuning cur = c->tune;
     const int cu = c->cu_count;
-    // sampling: persistent workgroups (stage 1)
-    {
-        float bt = 1e30f;
-        bmf_tuning b = cur;
-        const int mult[4] = {4, 8, 16, 32};
-        for (int m : mult) {
+    // one shape at a time: the present one, then the others, by the time of its stages
+    const auto search = [&](int32_t bmf_tuning::* shape, std::initializer_list<int> others, int stage, int also) -> int {
+        float best_ms = 1e30f;
+        int32_t best_shape = cur.*shape;
+        const auto attempt = [&](int32_t blocks) -> int {
             bmf_tuning t = cur;
-            t.sample_blocks = m * cu;
-            rc = run(t, st);
-            if (rc) return rc;
-            if (st[1] < bt) {
-                bt = st[1];
-                b = t;
+            t.*shape = blocks;
+            const int e = run(t, st);
+            if (e) return e;
+            const float ms = st[stage] + (also >= 0 ? st[also] : 0.0f);
+            if (ms < best_ms) {
+                best_ms = ms;
+                best_shape = blocks;
             }
+            return BMF_OK;
+        };
+        int e = attempt(cur.*shape);
+        for (int b : others) {
+            const int blocks = (b + kXcds - 1) / kXcds * kXcds;
+            if (!e && blocks != cur.*shape) e = attempt(blocks);
         }
-        cur.sample_blocks = b.sample_blocks;
-    }
-    // word kernels: count and emit (stages 2 and 4), workgroups
-    {
-        float bt = 1e30f;
-        int bb = cur.row_blocks;
-        const int mult[7] = {1, 2, 4, 8, 10, 12, 16};
-        for (int m : mult) {
-            bmf_tuning t = cur;
-            t.row_blocks = m * cu;
-            rc = run(t, st);
-            if (rc) return rc;
-            if (st[2] + st[4] < bt) {
-                bt = st[2] + st[4];
-                bb = t.row_blocks;
-            }
-        }
-        cur.row_blocks = bb;
-    }
-    // smoothing (stage 5)
-    if (maxk > 0) {
-        float bt = 1e30f;
-        int bb = cur.smooth_blocks;
-        // from 64 workgroups (a few small meshes) to 32 per CU
-        const int cand[7] = {8 * kXcds, cu, 2 * cu, 4 * cu, 8 * cu, 16 * cu, 32 * cu};
-        for (int b : cand) {
-            bmf_tuning t = cur;
-            t.smooth_blocks = (b + kXcds - 1) / kXcds * kXcds;
-            rc = run(t, st);
-            if (rc) return rc;
-            if (st[5] < bt) {
-                bt = st[5];
-                bb = t.smooth_blocks;
-            }
-        }
-        cur.smooth_blocks = bb;
-    }
+        cur.*shape = best_shape;
+        return e;
+    };
+    // sampling (stage 1); count and emit (stages 2 and 4); smoothing (stage 5),
+    // from 64 workgroups (a few small meshes) to 32 per CU
+    rc = search(&bmf_tuning::sample_blocks, {4 * cu, 8 * cu, 10 * cu, 12 * cu, 16 * cu, 32 * cu}, 1, -1);
+    if (!rc) rc = search(&bmf_tuning::row_blocks, {cu, 2 * cu, 4 * cu, 8 * cu, 10 * cu, 12 * cu, 16 * cu}, 2, 4);
+    if (!rc && maxk > 0)
+        rc = search(&bmf_tuning::smooth_blocks,
+                    {8 * kXcds, cu, 2 * cu, 4 * cu, 8 * cu, 12 * cu, 16 * cu, 32 * cu}, 5, -1);
+    if (rc) return rc;
     // confirmation: the tuned and the starting shapes over the whole frame,
     // alternately (median of 3 * reps runs each); the tuned ones are kept
     // only when they are at least 1 % faster
