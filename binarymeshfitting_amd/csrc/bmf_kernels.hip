@@ -72,8 +72,9 @@ __device__ __forceinline__ int64_t pick(const int64_t (&a)[N], int i) {
 }
 
 // ---- how far k_blocks expands a chunk's noise (see there) ----
-// Largest norm of the noise's Hessian: 48.21 over all positions in a simplex
-// and gradients at its corners, with a margin (tests/test_noise_bounds.py).
+// No Hessian of the noise has a larger norm, at any position and for any
+// gradients: proven by tests/test_noise_bounds_proof.py (the largest that a
+// search finds is 48.21).
 constexpr float kNoiseHess = 50.0f;
 // FP32 error of two noise values and of a gradient over a block, per unit of
 // amplitude: a constant for the kernels' arithmetic (about 76.8 * 4 t^3 g.x
