@@ -25,8 +25,6 @@ namespace {
         if (e_ != hipSuccess) return BMF_EHIP;         \
     } while (0)
 
-int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
-
 bool finite(float v) { return std::isfinite(v); }
 
 template <class T>
@@ -47,14 +45,15 @@ void free_arenas(bmf_ctx* c) {
     c->d_spheres = c->d_boxes = nullptr;
 }
 
-// The whole device pipeline for chunks [0, n) of the uploaded descriptors.
-// With `ev` (BMF_NUM_STAGES + 1 events) the stage boundaries are recorded.
 // Workgroups of the batched row scan: one per chunk up to two per CU; the
 // kernel strides over the batch and skips the chunks that were not sampled,
-// so a large batch with few sampled chunks does not dispatch a workgroup of
-// 1024 threads per chunk.
+// so a large batch with few sampled chunks does not dispatch a workgroup per
+// chunk.
 int scan_blocks(const bmf_ctx* c, int n) { return std::min(n, 2 * c->cu_count); }
 
+// The whole device pipeline for chunks [0, n) of the uploaded descriptors, or
+// for the single descriptor `one`.  With `ev` (BMF_NUM_STAGES + 1 events) the
+// stage boundaries are recorded.
 int enqueue_pipeline(bmf_ctx* c, const Arenas& A, int n, int maxk, int allow_cull, int reset, int sample_blocks,
                      int row_blocks, int scan_blocks, int smooth_blocks, hipEvent_t* ev = nullptr,
                      const bmf_chunk_desc* one = nullptr) {

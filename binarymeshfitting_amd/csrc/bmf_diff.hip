@@ -926,7 +926,7 @@ __global__ void __launch_bounds__(64) k_nn_query(const float* __restrict__ pos, 
             break;
         }
     }
-    // each vertex's lowest (distance, index) over its 8 lanes
+    // each vertex's lowest (distance, index) over its kPart lanes
     auto take = [&](float od, int oi, int os) {
         if (od < bd || (od == bd && oi < bi)) {
             bd = od;

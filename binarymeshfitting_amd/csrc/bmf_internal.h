@@ -223,7 +223,7 @@ hipError_t launch_plan(const Arenas& A, int n, int allow_cull, int reset_bumps, 
                        const bmf_chunk_desc* one = nullptr);
 // adaptive: signs everywhere and densities where the surface reads them (terrain, CSG); 0: every density
 // kind: the sampler the device struct holds for this launch (BMF_SAMPLER_*)
-// slab: the sampler is a 2D noise field (its columns are evaluated once per tile)
+// slab: the sampler is a 2D noise field (its columns are evaluated in a pass of their own)
 hipError_t launch_sample(const Arenas& A, int n, int blocks, int adaptive, int kind, int slab, hipStream_t s);
 // refine: give early-labelled edge endpoints their full density (after an adaptive terrain launch_sample)
 hipError_t launch_count(const Arenas& A, int blocks, int refine, hipStream_t s);

@@ -239,7 +239,7 @@ __device__ __forceinline__ void plan_counters(const Arenas& A, int n, const int6
 // sums over all of them (two descriptors per thread at most, 32-bit wave
 // scans) and writes the records of its own kPlanSlice.  One block that wrote
 // every record took 14 us for 512 descriptors and 33 for 1,536 (a thread's
-// records are 120 bytes apart, written and read again across the scan);
+// records lie side by side, written and read again across the scan);
 // this takes 6.7 and 9.9 (5.4 for one).  A single descriptor may come with the
 // launch (`by_value`), which saves its copy to the arena.
 __global__ void __launch_bounds__(kPlanThreads) k_plan(Arenas A, int n, int allow_cull, int reset_bumps,
@@ -439,7 +439,7 @@ __device__ __forceinline__ void sample_coords(const ChunkGeom& G, uint32_t i, ui
 //
 // A quad of lanes shares a centre, an octave each, so that a wave's chain is
 // one octave long.  Bound by VALU issue: 512 chunks of 64^3 cells, 64 sampled
-// (17.6 M samples, 5 octaves) take 42 us here and 61 in k_terrain; evaluating
+// (17.6 M samples, 5 octaves) take 43 us here and 61 in k_terrain; evaluating
 // every sample's octaves until its sign was certain (1.38 on average) took
 // 202, and 23 instead of 13 for the endpoints that it left.
 // ------------------------------------------------------------------------
@@ -654,9 +654,9 @@ __global__ void __launch_bounds__(kRowThreads) k_blocks(Arenas A, int n) {
 // and their bit in the `exact` bitmap; the others only their label (k_count
 // finishes the densities of those that are endpoints of a sign-changing
 // edge).  Labels and every density that a mesh reads are those of the full
-// evaluation, bit for bit.  Bound by VALU issue (49 of 69 us on the batch
-// above).  kTerrainDirect: short lists lose less to octaves that an early
-// decision would have spared than to the rounds' barriers.
+// evaluation, bit for bit.  Bound by VALU issue (61 us on the batch above).
+// kTerrainDirect: short lists lose less to octaves that an early decision would
+// have spared than to the rounds' barriers.
 // ------------------------------------------------------------------------
 constexpr int kTerrainSamples = kWordWaves * kItemSamples;
 constexpr int kTerrainDirect = 1024;  // open samples up to which all octaves run at once
@@ -829,16 +829,17 @@ __global__ void __launch_bounds__(kRowThreads) k_terrain(Arenas A, int n) {
 }
 
 // ------------------------------------------------------------------------
-// sample: every sampler but the adaptive terrain, one wave per WORDS label
-// words (all of them in a chunk's first item, and so on): no barrier and no
-// LDS but the CSG primitives.  The words per wave balance the chip's last
-// round against the wave's own set-up.  Bound by VALU issue where a sampler is
-// evaluated, by HBM where densities only pass through.
+// sample: the other samplers but CSG (k_csg), one wave per WORDS label words
+// (all of them in a chunk's first item, and so on): no barrier and no LDS.  The
+// words per wave balance the chip's last round against the wave's own set-up.
+// Bound by VALU issue where a sampler is evaluated, by HBM where densities only
+// pass through.
 //   terrain in full  129^3 samples, 5 octaves: 52 us (tiles of 2,048
 //                    samples per workgroup, 1,049 of them: 95)
 //   external         48 chunks of 41^3: 12 us (tiles: 52)
 //   2D noise field   from the columns of k_columns
-//   CSG              with the item's own primitives, see below
+//   implicit shapes  whole passes of one chunk of 16^3 cells 80 us, of 64^3 83,
+//                    64 of 64^3 125 (tiles: 130, 144, 380)
 // ------------------------------------------------------------------------
 constexpr int kSampleImplicit = 0, kSampleTerrain = 1, kSampleField2 = 2, kSampleField3 = 3, kSampleExternal = 4;
 

@@ -185,17 +185,6 @@ __device__ __forceinline__ void block_scan32(const uint32_t (&v)[N], int64_t (&e
     __syncthreads();  // the scratch may be reused
 }
 
-// Chunk j whose half-open range [prefix[j], prefix[j+1]) holds g.
-__device__ __forceinline__ int find_chunk(const int64_t* __restrict__ prefix, int n, int64_t g) {
-    int lo = 0, hi = n;
-    while (hi - lo > 1) {
-        int mid = (lo + hi) >> 1;
-        if (prefix[mid] <= g) lo = mid;
-        else hi = mid;
-    }
-    return lo;
-}
-
 // The largest j in [0, n) with at(j) <= g, for at non-decreasing and
 // at(0) <= g, by one wave: 64 probes a round, two dependent loads up to 4,096
 // entries where a binary search has twelve.

@@ -6,8 +6,8 @@
 //
 // The reference walks the world octree recursively (stitch_cell, the face
 // and edge recursions, stitch_indexes: WorldStitcher.cpp:184-572); here the
-// same dual cells are enumerated point by point, one thread per candidate
-// point, in a fixed order (the chunks of the leaf list in order, the lattice
+// same dual cells are enumerated point by point, the candidate points in a
+// fixed order (the chunks of the leaf list in order, the lattice
 // points of each chunk's closed cube [0, dim]^3 on the cube's boundary in
 // x-major order):
 //   - integer geometry in units of the finest unit node: a node at level l
@@ -19,12 +19,15 @@
 //   - corner c (4*dx + 2*dy + dz) is the unit node of octant c's chunk that
 //     contains the point's octant c, placed where the shell octree places it
 //     (pos + MCD * size/2 + MCD * size/4 + ..., FP32 in that order), valued
-//     by the sampler there (every octave);
+//     by the sampler there;
 //   - marching cubes as stitch_indexes: crossing (v1 - v0) * mu + v0,
 //     mu = (0 - s0) / (s1 - s0), triangles from the tri_table.
-// Three launches: count (triangles per candidate, and per 256-candidate
-// tile), a one-workgroup scan of the tile totals, emit (recomputes the
-// cells of candidates with triangles and writes them at their offsets).
+// Four launches: the world's root and deepest level, count (triangles per
+// candidate, and per 256-candidate tile: a thread per candidate finds its
+// chunks, 8 lanes its corners' signs, of the terrain by no more octaves than
+// they take to be certain), a one-workgroup scan of the tile totals, emit (the
+// cells of the candidates with triangles again, 8 lanes each and every octave,
+// written at their offsets).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
