@@ -427,7 +427,7 @@ struct DmcWave {
 // chunks that smooth, writes its ring.  QEF placement is bound by the
 // normals (a pass over the primitives per edge point): the item's own list
 // keeps the few that can win.  64 chunks of 64^3 cells, 300 primitives,
-// 326,882 vertices: 110 us, with the plane's rows and the chunk's list 169.
+// 326,882 vertices: 106 us, with the plane's rows and the chunk's list 169.
 // ------------------------------------------------------------------------
 __device__ void place_vertex(const Arenas& A, const ChunkMeta& M, const SamplerDev& S, const uint16_t* csg,
                              const float4* s_csg, const uint16_t* ids, int ns, int nb, int x, int y, int z, int p,

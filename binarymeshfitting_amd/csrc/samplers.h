@@ -364,7 +364,7 @@ __device__ __forceinline__ bool cull_csg(const SamplerDev& S, const uint16_t* __
 // Their ids instead, which take a sixteenth of the room: the spheres' from 0
 // on, the boxes' from the next multiple of four.  The primitives themselves are
 // then read by the whole wave at once, through scalar loads.  kCsgIds: 2 KiB per
-// wave, the most that costs neither kernel a workgroup per CU.
+// wave, which costs neither kernel a workgroup per CU.
 constexpr int kCsgIds = 1024;
 __device__ __forceinline__ bool cull_csg_ids(const SamplerDev& S, const uint16_t* __restrict__ list, int ns, int nb,
                                              const float (&lo)[3], const float (&hi)[3], float reach, uint16_t* ids,
